@@ -132,11 +132,35 @@ __device__ __forceinline__ cd csub(cd a, cd b) { return cd{a.x - b.x, a.y - b.y}
 __device__ __forceinline__ cd cconj(cd a) { return cd{a.x, -a.y}; }
 __device__ __forceinline__ cd cscale(cd a, double s) { return cd{a.x * s, a.y * s}; }
 
-// Butterfly reductions over the 64 lanes of a wave (every lane gets the result;
-// the order of the additions is fixed).
+// A double of another lane by data-parallel primitives: quad_perm, row mirrors.
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Halves (ROWS = 32) or odd and even 16-lane rows (16) of a wave added, in every lane
+// as (lower + upper).
+template <int ROWS>
+__device__ __forceinline__ double swap_add(double v) {
+    const unsigned long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    const auto l = ROWS == 32 ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false) : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = ROWS == 32 ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false) : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __longlong_as_double(((unsigned long long)h[0] << 32) | l[0]) + __longlong_as_double(((unsigned long long)h[1] << 32) | l[1]);
+}
+
+// Reductions over the 64 lanes of a wave (every lane gets the result; the order of
+// the additions is fixed).  The sum runs on register moves inside rows of 16 lanes
+// and on row swaps: six rounds of LDS permutes per value cost the observables of a
+// small grid about 2 us.
 __device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v += dpp64<0xB1>(v);   // lanes i, i ^ 1
+    v += dpp64<0x4E>(v);   // i ^ 2
+    v += dpp64<0x141>(v);  // the other four of eight lanes (half-row mirror: each four agree by now)
+    v += dpp64<0x140>(v);  // the other eight of sixteen (row mirror)
+    return swap_add<32>(swap_add<16>(v));
 }
 __device__ __forceinline__ double wave_min(double v) {
     for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
@@ -941,116 +965,6 @@ __global__ __launch_bounds__(64) void k_coul_w_mfma(CoulArgs a, int N1) {
     }
 }
 
-// Observables with the mean field (Observables_MPI.h:286-304, if_resolution.cpp:125-192):
-// eigenvectors of the renormalised H (cyclic Jacobi), its shell gradient and
-// H_ren D^+ for Current2.  One thread per k, nb <= 4.
-template <int NB>
-__global__ __launch_bounds__(256) void k_coul_obs(const double *Hr, const double *Dp, const int *nbr, const double *wb, int n_nbr,
-                                                   int nk, int nkp, int dherm, double *Uexc, double *GE, double *Q, double *Ek) {
-    constexpr int NP = NB * NB;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nk) return;
-    cd A[NB][NB], V[NB][NB];
-#pragma unroll
-    for (int i = 0; i < NB; i++) {
-        A[i][i] = mk(Hr[i * (size_t)nkp + k], 0.0);
-        V[i][i] = mk(1.0, 0.0);
-#pragma unroll
-        for (int j = i + 1; j < NB; j++) {
-            const int p = pair_index(i, j, NB);
-            A[i][j] = mk(Hr[(NB + 2 * p) * (size_t)nkp + k], Hr[(NB + 2 * p + 1) * (size_t)nkp + k]);
-            A[j][i] = cconj(A[i][j]);
-            V[i][j] = V[j][i] = mk(0.0, 0.0);
-        }
-    }
-    for (int sweep = 0; sweep < 20; sweep++) {
-        double off = 0, tot = 0;
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const double v = A[i][j].x * A[i][j].x + A[i][j].y * A[i][j].y;
-                tot += v;
-                if (i != j) off += v;
-            }
-        if (off <= 1e-30 * tot) break;
-#pragma unroll
-        for (int p = 0; p < NB; p++)
-#pragma unroll
-            for (int q = p + 1; q < NB; q++) {
-                const double mag = sqrt(A[p][q].x * A[p][q].x + A[p][q].y * A[p][q].y);
-                if (mag == 0.0) continue;
-                const cd e = mk(A[p][q].x / mag, A[p][q].y / mag);
-                const double th = 0.5 * (A[q][q].x - A[p][p].x) / mag;
-                const double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-                const double cs = 1.0 / sqrt(t * t + 1.0), sn = t * cs;
-#pragma unroll
-                for (int r = 0; r < NB; r++) {
-                    cd x = A[r][p], y = A[r][q];
-                    A[r][p] = csub(cscale(x, cs), cscale(cmul(cconj(e), y), sn));
-                    A[r][q] = cadd(cscale(cmul(e, x), sn), cscale(y, cs));
-                    x = V[r][p]; y = V[r][q];
-                    V[r][p] = csub(cscale(x, cs), cscale(cmul(cconj(e), y), sn));
-                    V[r][q] = cadd(cscale(cmul(e, x), sn), cscale(y, cs));
-                }
-#pragma unroll
-                for (int r = 0; r < NB; r++) {
-                    cd x = A[p][r], y = A[q][r];
-                    A[p][r] = csub(cscale(x, cs), cscale(cmul(e, y), sn));
-                    A[q][r] = cadd(cscale(cmul(cconj(e), x), sn), cscale(y, cs));
-                }
-            }
-    }
-    // ascending eigenvalues; Uexc rows are conj(v_a)
-    int ord[NB];
-#pragma unroll
-    for (int i = 0; i < NB; i++) ord[i] = i;
-    for (int i = 0; i < NB; i++)
-        for (int j = i + 1; j < NB; j++)
-            if (A[ord[j]][ord[j]].x < A[ord[i]][ord[i]].x) { int tt = ord[i]; ord[i] = ord[j]; ord[j] = tt; }
-    double *u = Uexc + (size_t)k * NB * NB * 2;
-    for (int a2 = 0; a2 < NB; a2++) Ek[(size_t)k * NB + a2] = A[ord[a2]][ord[a2]].x;
-    for (int a2 = 0; a2 < NB; a2++)
-        for (int b = 0; b < NB; b++) {
-            const cd v = V[b][ord[a2]];
-            u[(a2 * NB + b) * 2] = v.x;
-            u[(a2 * NB + b) * 2 + 1] = -v.y;
-        }
-    // gradient of the renormalised H on the shell stencil (packed Hermitian)
-    for (int x = 0; x < 3; x++)
-        for (int e = 0; e < NP; e++) {
-            const double h0 = Hr[e * (size_t)nkp + k];
-            double g = 0.0;
-            for (int n = 0; n < n_nbr; n++) g += wb[n * 3 + x] * (Hr[e * (size_t)nkp + nbr[(size_t)n * nkp + k]] - h0);
-            GE[((size_t)k * 3 + x) * NP + e] = g;
-        }
-    // Q_x = H_ren D_x^+ (D symmetric, packed)
-    for (int x = 0; x < 3; x++)
-        for (int i = 0; i < NB; i++)
-            for (int j = 0; j < NB; j++) {
-                cd acc = mk(0, 0);
-                for (int kc = 0; kc < NB; kc++) {
-                    cd h, d;
-                    if (i == kc) h = mk(Hr[i * (size_t)nkp + k], 0.0);
-                    else {
-                        const int p = pair_index(min(i, kc), max(i, kc), NB);
-                        h = mk(Hr[(NB + 2 * p) * (size_t)nkp + k], Hr[(NB + 2 * p + 1) * (size_t)nkp + k]);
-                        if (i > kc) h = cconj(h);
-                    }
-                    if (j == kc) d = mk(Dp[(x * NP + j) * (size_t)nkp + k], 0.0);
-                    else {
-                        const int p = pair_index(min(j, kc), max(j, kc), NB);
-                        d = mk(Dp[(x * NP + NB + 2 * p) * (size_t)nkp + k], Dp[(x * NP + NB + 2 * p + 1) * (size_t)nkp + k]);
-                        if (dherm && j > kc) d = cconj(d);
-                    }
-                    acc = cadd(acc, cmul(h, cconj(d)));
-                }
-                double *q = Q + ((((size_t)k * 3 + x) * NB + i) * NB + j) * 2;
-                q[0] = acc.x;
-                q[1] = acc.y;
-            }
-}
-
 // ================================================================ nb in 5..32: one workgroup per k
 // Threads per k: 32 for nb <= 8 (eight k per workgroup), one wavefront for
 // nb <= 16, four for nb <= 32.  The LDS GEMM of the VALU form (nb <= 8) runs on a
@@ -1775,17 +1689,32 @@ __global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB) void k_sta
 }
 
 // ================================================================ observables
-// Values per partial: pop[nb], j1 re x3, j2 (re,im) x3, tabs (re,im) x3 -> nb + 15,
-// plus min and max of the population diagnostics.
+// Values per partial: pop[nb], J1 re x3, J2 (re,im) x3, TAbs (re,im) x3 -> nb + 15,
+// plus min and max of the population diagnostics.  J2_x = sum_ij P_ij (H D_x^+)_ij
+// is taken as sum_jc conj(D_x,jc) W_jc with W = conj(P) H (P is Hermitian), so the
+// packed operators are read instead of a table of products: 80 nb^2 bytes per k
+// (P, H, U, three components of D and of the gradient of H).
+constexpr int kObsSums = 15;         // J1, J2, TAbs
+constexpr int kObsThreads = 256;
+constexpr int kObsMaxBlocks = 1024;  // wave kernels: a block walks its share of the grid
+
 struct ObsArgs {
-    const double *P;     // state
-    const double *U;     // full complex AoS
-    const double *GE;    // [k][3][NP] packed Hermitian gradient of H (may be null)
-    const double *Q;     // [k][3][nb][nb] complex: H D^+ (Current2)
-    const double *DT;    // [k][3][nch][nb-nch] complex: D on the core<->non-core block
-    double *part;        // [nblocks][nv + 2] (sums with Kahan compensation collapsed)
-    int nk, nb, nch, ncc;
-    size_t sk, se;       // state strides: element e of k at k*sk + e*se
+    const double *P;     // state, packed
+    const double *U;     // full complex AoS (not read with the mean field)
+    const double *GE;    // packed Hermitian gradient of H, components x stride dxs (may be null: J1 = 0)
+    const double *H;     // packed H, or the renormalised H of the mean field
+    const double *D;     // packed dipole, components x stride dxs
+    const int *eidx;     // packed element -> (i, j, comp) (wave layout)
+    double *part;        // [nv + 2][gridDim.x] block partials
+    unsigned *count;     // finished blocks (0 between launches)
+    double *out;         // [nv + 2] results, host memory mapped to the device
+    int nk, nkp, nb, nch, ncc, dherm;
+    size_t dxs;
+    // mean field: stencil of the gradient of the renormalised H; its eigenvalues [nk][nb]
+    const int *nbr;
+    const double *wb;
+    int n_nbr;
+    double *Ek;
 };
 
 struct Kahan {
@@ -1798,183 +1727,510 @@ struct Kahan {
     }
 };
 
-__device__ __forceinline__ cd load_p(const ObsArgs &o, int k, int i, int j) {
-    const int nb = o.nb;
-    if (i == j) return mk(o.P[k * o.sk + i * o.se], 0.0);
-    const int a = min(i, j), b = max(i, j);
-    const int p = pair_index(a, b, nb);
-    cd v = mk(o.P[k * o.sk + (nb + 2 * p) * o.se], o.P[k * o.sk + (nb + 2 * p + 1) * o.se]);
-    return (i < j) ? v : cconj(v);
-}
+// Accesses of the block partials at device scope, one by one: a device-scope fence
+// per block instead writes back and invalidates the XCD's whole L2 each time
+// (8 bands, 200 x 200, 1024 blocks: 203 us with the fence).
+__device__ __forceinline__ void put_agent(double *p, double v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ double get_agent(const double *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// One workgroup of T threads walks its k points and stages each k's full P (from
-// the packed state) and U in its LDS, so the population quadratic form and the
-// current / absorption sums read their matrix operands from LDS.  T = 256 for
-// large band counts: the k's loads and sums are spread over four waves, and the
-// population form of band c over S = T / 32 lanes (terms ii = s, s + S, ...,
-// summed by shuffles), so no lane walks a long chain of dependent loads.
-constexpr int kObsMaxBlocks = 8192;
-
-template <int T>
-__global__ __launch_bounds__(T) void k_observables(ObsArgs o) {
-    extern __shared__ double obs_lds[];
-    constexpr int S = T / 32, NW = T / 64;
-    const int lane = threadIdx.x, wave = lane >> 6;
-    const int nb = o.nb, NP = nb * nb, NN = nb * nb, nch = o.nch;
-    // U rows padded to nb + 1: lanes of consecutive bands start 4 banks apart
-    const int LU = nb + 1;
-    cd *Pl = reinterpret_cast<cd *>(obs_lds), *Ul = Pl + NN;
-    double *red = reinterpret_cast<double *>(Ul + nb * LU);  // [NW][17] cross-wave partials, then [32] populations
-    Kahan pop, j1[3], j2[6], ta[6];
-    double pmin = 1.0, pmax = 0.0;
-    const int pc = lane / S, ps = lane % S;  // band and term slice of the population form
-    for (int k = blockIdx.x; k < o.nk; k += gridDim.x) {
-        __syncthreads();  // the previous k's LDS reads are done
-        for (int t = lane; t < NN; t += T) {
-            Pl[t] = load_p(o, k, t / nb, t % nb);
-            double ur, ui;
-            ld2<false>(o.U, ((size_t)k * NN + t) * 2, ((size_t)k * NN + t) * 2 + 1, true, ur, ui);
-            Ul[(t / nb) * LU + t % nb] = mk(ur, ui);
-        }
-        __syncthreads();
-        // population of band c = Re (conj(U) P_sym U^T)_cc (InitParameters.h:264-335)
-        {
-            double sre = 0.0;
-            if (pc < nb) {
-                const cd *uc = Ul + pc * LU;
-                cd sacc = mk(0.0, 0.0);
-                for (int ii = ps; ii < nb; ii += S) {
-                    cd t = mk(0.0, 0.0);
-#pragma unroll 4
-                    for (int jj = 0; jj < nb; jj++) t = cadd(t, cmul(Pl[ii * nb + jj], uc[jj]));
-                    sacc = cadd(sacc, cmul(cconj(uc[ii]), t));
-                }
-                sre = sacc.x;
-            }
+// The block's sums (every thread's `acc`, the first N of the kObsSums values, the
+// rest being zero; `pmin`, `pmax`; pops[g * stride + band] of
+// the block's ng groups in LDS, written before the call) to its partials, and, in
+// the block that finishes last, the partials to the results: one wave per value,
+// each lane a strided subset with Kahan compensation, the 64 (sum, compensation)
+// pairs combined with error-free two-sums.  The additions run in a fixed order.
+// One launch instead of a reduction kernel and a copy to the host after it: a
+// 70 x 70 grid of 3 bands spent 10 us on the second kernel and 4 us on the copy.
+template <int N>
+__device__ __forceinline__ void obs_finish(const ObsArgs &o, double (&acc)[N], double pmin, double pmax, const double *pops,
+                                           int ng, int stride) {
+    constexpr int NW = kObsThreads / 64;
+    __shared__ double red[NW][kObsSums + 2];
+    __shared__ int last;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nb = o.nb, nv = nb + kObsSums, G = gridDim.x;
 #pragma unroll
-            for (int off = S / 2; off > 0; off >>= 1) sre += __shfl_xor(sre, off, 64);
-            if (pc < nb && ps == 0) {
-                pop.add(sre);
-                const double hv = (pc < o.ncc) ? 1. - sre : sre;
-                pmax = fmax(pmax, fabs(hv));
-                pmin = fmin(pmin, hv);
-            }
-        }
-        // Current1: sum_ij P_ij gradH_ij (real: P and gradH are Hermitian)
-        if (o.GE) {
-            for (int e = lane; e < NP; e += T) {
-                const double pe = o.P[k * o.sk + e * o.se];
-                const double wgt = (e < nb) ? 1.0 : 2.0;   // a pair carries (i,j) and (j,i)
-                // Re(P_ij G_ij): re*re - im*im over the (re, im) doubles of the pair
-                const double sgn = (e >= nb && ((e - nb) & 1)) ? -1.0 : 1.0;
-                for (int x = 0; x < 3; x++) j1[x].add(wgt * sgn * pe * o.GE[((size_t)k * 3 + x) * NP + e]);
-            }
-        }
-        // Current2: sum_ij P_ij (H D^+)_ij
-        for (int t = lane; t < NN; t += T) {
-            const cd pij = Pl[t];
-            for (int x = 0; x < 3; x++) {
-                double qr, qi;
-                ld2<false>(o.Q, (((size_t)k * 3 + x) * NN + t) * 2, (((size_t)k * 3 + x) * NN + t) * 2 + 1, true, qr, qi);
-                cd v = cmul(pij, mk(qr, qi));
-                j2[2 * x].add(v.x);
-                j2[2 * x + 1].add(v.y);
-            }
-        }
-        // Transient absorption: -2 sum_{i<nch<=j} D_ij P_ij (Observables_MPI.h:559-569)
-        const int nblk = nch * (nb - nch);
-        for (int t = lane; t < nblk; t += T) {
-            const int i = t / (nb - nch), j = nch + t % (nb - nch);
-            const cd pij = Pl[i * nb + j];
-            for (int x = 0; x < 3; x++) {
-                const double *d = o.DT + (((size_t)k * 3 + x) * nblk + t) * 2;
-                cd v = cmul(mk(d[0], d[1]), pij);
-                ta[2 * x].add(-2. * v.x);
-                ta[2 * x + 1].add(-2. * v.y);
-            }
-        }
-    }
-    // Lane sums by shuffle, then across the waves in wave order, in a fixed order.
-    __syncthreads();
-    double *pw = red + wave * 17;
-    for (int x = 0; x < 3; x++) {
-        const double v = wave_sum(j1[x].s);
-        if ((lane & 63) == 0) pw[x] = v;
-    }
-    for (int x = 0; x < 6; x++) {
-        const double v = wave_sum(j2[x].s), w = wave_sum(ta[x].s);
-        if ((lane & 63) == 0) { pw[3 + x] = v; pw[9 + x] = w; }
+    for (int x = 0; x < kObsSums; x++) {
+        const double v = x < N ? wave_sum(acc[x < N ? x : 0]) : 0.0;
+        if (lane == 0) red[wave][x] = v;
     }
     const double mn = wave_min(pmin), mx = wave_max(pmax);
-    if ((lane & 63) == 0) { pw[15] = mn; pw[16] = mx; }
-    double *pops = red + NW * 17;
-    if (pc < nb && ps == 0) pops[pc] = pop.s;
-    __syncthreads();
-    const int nv = nb + 15;
-    double *out = o.part + (size_t)blockIdx.x * (nv + 2);
-    if (lane < nb) out[lane] = pops[lane];
-    if (lane < 17) {
-        double v = red[lane];
-        for (int w = 1; w < NW; w++) {
-            const double u = red[w * 17 + lane];
-            v = lane == 15 ? fmin(v, u) : lane == 16 ? fmax(v, u) : v + u;
-        }
-        out[nb + lane] = v;  // nb+0..2 J1, +3..8 J2, +9..14 TAbs, nv and nv+1 min and max
+    if (lane == 0) {
+        red[wave][kObsSums] = mn;
+        red[wave][kObsSums + 1] = mx;
     }
+    __syncthreads();
+    if (t < nb) {
+        double v = 0.0;
+        for (int g = 0; g < ng; g++) v += pops[g * stride + t];
+        put_agent(o.part + (size_t)t * G + blockIdx.x, v);
+    } else if (t >= 64 && t < 64 + kObsSums + 2) {
+        const int x = t - 64;
+        double v = red[0][x];
+        for (int w = 1; w < NW; w++) v = x == kObsSums ? fmin(v, red[w][x]) : x > kObsSums ? fmax(v, red[w][x]) : v + red[w][x];
+        put_agent(o.part + (size_t)(nb + x) * G + blockIdx.x, v);
+    }
+    // the block's partials have reached the device's coherence point (every wave
+    // waits for its own agent-scope stores) before its arrival is counted
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (t == 0) last = atomicAdd(o.count, 1u) == (unsigned)(G - 1);
+    __syncthreads();
+    if (!last) return;
+    for (int c = wave; c < nv + 2; c += NW) {
+        const double *p = o.part + (size_t)c * G;
+        if (c < nv) {
+            Kahan k;
+#pragma unroll 4
+            for (int b = lane; b < G; b += 64) k.add(get_agent(p + b));
+            double s = k.s, lo = -k.c;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                // both lanes of a pair form the same sum: the operands in lane order
+                const double s2 = __shfl_xor(s, off, 64), l2 = __shfl_xor(lo, off, 64);
+                const bool first = (lane & off) == 0;
+                const double a = first ? s : s2, b = first ? s2 : s, sum = a + b, bp = sum - a;
+                lo = (first ? lo : l2) + (first ? l2 : lo) + ((a - (sum - bp)) + (b - bp));
+                s = sum;
+            }
+            if (lane == 0) o.out[c] = s + lo;
+        } else {
+            double v = c == nv ? 1.0 : 0.0;
+            for (int b = lane; b < G; b += 64) v = c == nv ? fmin(v, get_agent(p + b)) : fmax(v, get_agent(p + b));
+            v = c == nv ? wave_min(v) : wave_max(v);
+            if (lane == 0) o.out[c] = v;
+        }
+    }
+    if (t == 0) *o.count = 0;
 }
 
-// Final reduction of the per-block partials: one workgroup per value.  Each
-// thread sums a strided subset with Kahan compensation, and the 256 (sum,
-// compensation) pairs are combined pairwise with an error-free two-sum, so the
-// result keeps the compensated accuracy; the last two values are the
-// population diagnostics' min and max.
-__global__ __launch_bounds__(256) void k_obs_final(const double *part, int nparts, int nv, double *out) {
-    __shared__ double shi[256], slo[256];
-    const int c = blockIdx.x, t = threadIdx.x;
-    const size_t stride = (size_t)nv + 2;
-    if (c < nv) {
-        double s = 0.0, comp = 0.0;
-        for (int b = t; b < nparts; b += 256) {
-            const double yv = part[(size_t)b * stride + c] - comp;
-            const double q = s + yv;
-            comp = (q - s) - yv;
-            s = q;
-        }
-        shi[t] = s;
-        slo[t] = -comp;
-        __syncthreads();
-        for (int h = 128; h > 0; h >>= 1) {
-            if (t < h) {
-                const double a = shi[t], b = shi[t + h];
-                const double sum = a + b, bp = sum - a;
-                const double err = (a - (sum - bp)) + (b - bp);
-                shi[t] = sum;
-                slo[t] = slo[t] + slo[t + h] + err;
+// Eigenvalues (ascending) and eigenvectors (columns of V) of a Hermitian matrix by
+// cyclic Jacobi; every index is a compile-time constant, so A and V stay in
+// registers (a run-time column order put them in scratch memory).
+template <int NB>
+__device__ __forceinline__ void jacobi_small(cd (&A)[NB][NB], cd (&V)[NB][NB], double (&w)[NB]) {
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) V[i][j] = mk(i == j ? 1.0 : 0.0, 0.0);
+    for (int sweep = 0; sweep < 20; sweep++) {
+        double off = 0, tot = 0;
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const double v = A[i][j].x * A[i][j].x + A[i][j].y * A[i][j].y;
+                tot += v;
+                if (i != j) off += v;
             }
-            __syncthreads();
-        }
-        if (t == 0) out[c] = shi[0] + slo[0];
-    } else {
-        const bool mn = c == nv;
-        double v = mn ? 1.0 : 0.0;
-        for (int b = t; b < nparts; b += 256) {
-            const double x = part[(size_t)b * stride + c];
-            v = mn ? fmin(v, x) : fmax(v, x);
-        }
-        shi[t] = v;
-        __syncthreads();
-        for (int h = 128; h > 0; h >>= 1) {
-            if (t < h) shi[t] = mn ? fmin(shi[t], shi[t + h]) : fmax(shi[t], shi[t + h]);
-            __syncthreads();
-        }
-        if (t == 0) out[c] = shi[0];
+        if (off <= 1e-30 * tot) break;
+#pragma unroll
+        for (int p = 0; p < NB; p++)
+#pragma unroll
+            for (int q = p + 1; q < NB; q++) {
+                const double mag = sqrt(A[p][q].x * A[p][q].x + A[p][q].y * A[p][q].y);
+                if (mag == 0.0) continue;
+                const cd e = mk(A[p][q].x / mag, A[p][q].y / mag);
+                const double th = 0.5 * (A[q][q].x - A[p][p].x) / mag;
+                const double t = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
+                const double cs = 1.0 / sqrt(t * t + 1.0), sn = t * cs;
+#pragma unroll
+                for (int r = 0; r < NB; r++) {
+                    cd x = A[r][p], y = A[r][q];
+                    A[r][p] = csub(cscale(x, cs), cscale(cmul(cconj(e), y), sn));
+                    A[r][q] = cadd(cscale(cmul(e, x), sn), cscale(y, cs));
+                    x = V[r][p]; y = V[r][q];
+                    V[r][p] = csub(cscale(x, cs), cscale(cmul(cconj(e), y), sn));
+                    V[r][q] = cadd(cscale(cmul(e, x), sn), cscale(y, cs));
+                }
+#pragma unroll
+                for (int r = 0; r < NB; r++) {
+                    cd x = A[p][r], y = A[q][r];
+                    A[p][r] = csub(cscale(x, cs), cscale(cmul(e, y), sn));
+                    A[q][r] = cadd(cscale(cmul(cconj(e), x), sn), cscale(y, cs));
+                }
+            }
     }
+#pragma unroll
+    for (int i = 0; i < NB; i++) w[i] = A[i][i].x;
+    // exchange sort of (w, column): the same exchanges as sorting an index list
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = i + 1; j < NB; j++) {
+            const bool sw = w[j] < w[i];
+            const double wi = w[i];
+            w[i] = sw ? w[j] : wi;
+            w[j] = sw ? wi : w[j];
+#pragma unroll
+            for (int r = 0; r < NB; r++) {
+                const cd x = V[r][i], y = V[r][j];
+                V[r][i] = mk(sw ? y.x : x.x, sw ? y.y : x.y);
+                V[r][j] = mk(sw ? x.x : y.x, sw ? x.y : y.y);
+            }
+        }
+}
+
+// nb <= 4: a thread per k, all matrices in registers; the SoA tables are read
+// coalesced.  COUL: populations in the eigenbasis of the renormalised H and the
+// currents of that H (Observables_MPI.h:286-304, if_resolution.cpp:125-192), its
+// shell gradient contracted with P neighbour by neighbour; the eigenvalues are
+// kept for edus_renorm_energies.  Bound by the latency of its loads and of the
+// final sums: 60 x 60 k of 3 bands 23 us (two kernels of a wave per k) -> 13;
+// with the mean field, 300 x 300, 345 us (tables written, then read) -> 46.
+template <int NB, bool COUL>
+__global__ __launch_bounds__(kObsThreads) void k_obs_small(ObsArgs o) {
+    constexpr int NP = NB * NB;
+    __shared__ double pops[kObsThreads / 64][NB];
+    const size_t nkp = o.nkp;
+    double pop[NB], acc[kObsSums], pmin = 1.0, pmax = 0.0;
+#pragma unroll
+    for (int c = 0; c < NB; c++) pop[c] = 0.0;
+#pragma unroll
+    for (int x = 0; x < kObsSums; x++) acc[x] = 0.0;
+    const int k = blockIdx.x * kObsThreads + threadIdx.x;
+    if (k < o.nk) {
+        double y[NP], h[NP];
+#pragma unroll
+        for (int e = 0; e < NP; e++) {
+            y[e] = o.P[e * nkp + k];
+            h[e] = o.H[e * nkp + k];
+        }
+        cd U[NB][NB];
+        if constexpr (COUL) {
+            cd A[NB][NB], V[NB][NB];
+            double w[NB];
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                A[i][i] = mk(h[i], 0.0);
+#pragma unroll
+                for (int j = i + 1; j < NB; j++) {
+                    const int p = pair_index(i, j, NB);
+                    A[i][j] = mk(h[NB + 2 * p], h[NB + 2 * p + 1]);
+                    A[j][i] = cconj(A[i][j]);
+                }
+            }
+            jacobi_small<NB>(A, V, w);
+#pragma unroll
+            for (int a = 0; a < NB; a++) {
+                o.Ek[(size_t)k * NB + a] = w[a];
+#pragma unroll
+                for (int b = 0; b < NB; b++) U[a][b] = cconj(V[b][a]);
+            }
+        } else {
+            const double *u = o.U + (size_t)k * NP * 2;
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int b = 0; b < NB; b++) {
+                    double re, im;
+                    ld2<false>(u, (a * NB + b) * 2, (a * NB + b) * 2 + 1, true, re, im);
+                    U[a][b] = mk(re, im);
+                }
+        }
+        cd P[NB][NB], H[NB][NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            P[i][i] = mk(y[i], 0.0);
+            H[i][i] = mk(h[i], 0.0);
+#pragma unroll
+            for (int j = i + 1; j < NB; j++) {
+                const int p = pair_index(i, j, NB);
+                P[i][j] = mk(y[NB + 2 * p], y[NB + 2 * p + 1]);
+                P[j][i] = cconj(P[i][j]);
+                H[i][j] = mk(h[NB + 2 * p], h[NB + 2 * p + 1]);
+                H[j][i] = cconj(H[i][j]);
+            }
+        }
+        // population of band c = Re (conj(U) P U^T)_cc (InitParameters.h:264-335)
+#pragma unroll
+        for (int c = 0; c < NB; c++) {
+            double s = 0.0;
+#pragma unroll
+            for (int i = 0; i < NB; i++) {
+                cd t = mk(0.0, 0.0);
+#pragma unroll
+                for (int j = 0; j < NB; j++) t = cadd(t, cmul(P[i][j], U[c][j]));
+                s += U[c][i].x * t.x + U[c][i].y * t.y;
+            }
+            pop[c] = s;
+            const double hv = (c < o.ncc) ? 1. - s : s;
+            pmax = fmax(pmax, fabs(hv));
+            pmin = fmin(pmin, hv);
+        }
+        // Current1: sum_ij P_ij gradH_ij (real: both Hermitian; a pair counts twice)
+        if (o.GE) {
+            if constexpr (COUL) {
+                double j1[3] = {0.0, 0.0, 0.0};
+                for (int n = 0; n < o.n_nbr; n++) {
+                    const int kn = o.nbr[(size_t)n * nkp + k];
+                    double s = 0.0;
+#pragma unroll
+                    for (int e = 0; e < NP; e++) {
+                        const double f = e < NB ? y[e] : ((e - NB) & 1) ? -2. * y[e] : 2. * y[e];
+                        s += f * (o.H[e * nkp + kn] - h[e]);
+                    }
+#pragma unroll
+                    for (int x = 0; x < 3; x++) j1[x] += o.wb[n * 3 + x] * s;
+                }
+#pragma unroll
+                for (int x = 0; x < 3; x++) acc[x] = j1[x];
+            } else {
+#pragma unroll
+                for (int x = 0; x < 3; x++) {
+                    double s = 0.0;
+#pragma unroll
+                    for (int e = 0; e < NP; e++) {
+                        const double f = e < NB ? y[e] : ((e - NB) & 1) ? -2. * y[e] : 2. * y[e];
+                        s += f * o.GE[x * o.dxs + e * nkp + k];
+                    }
+                    acc[x] = s;
+                }
+            }
+        }
+        // W = conj(P) H; Current2 = sum_jc conj(D_jc) W_jc and the transient
+        // absorption -2 sum_{i<nch<=j} D_ij P_ij (Observables_MPI.h:559-569, 726-775)
+        cd W[NB][NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int c = 0; c < NB; c++) {
+                cd s = mk(0.0, 0.0);
+#pragma unroll
+                for (int i = 0; i < NB; i++) s = cadd(s, cmul(P[i][j], H[i][c]));
+                W[j][c] = s;
+            }
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            const double *d = o.D + x * o.dxs + k;
+            cd s = mk(0.0, 0.0), ta = mk(0.0, 0.0);
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                s = cadd(s, cscale(W[j][j], d[j * nkp]));
+#pragma unroll
+                for (int c = j + 1; c < NB; c++) {
+                    const int p = pair_index(j, c, NB);
+                    const cd v = mk(d[(NB + 2 * p) * nkp], d[(NB + 2 * p + 1) * nkp]);
+                    s = cadd(s, cadd(cmul(cconj(v), W[j][c]), cmul(o.dherm ? v : cconj(v), W[c][j])));
+                    if (j < o.nch && c >= o.nch) ta = cadd(ta, cmul(v, P[j][c]));
+                }
+            }
+            acc[3 + 2 * x] = s.x;
+            acc[4 + 2 * x] = s.y;
+            acc[9 + 2 * x] = -2. * ta.x;
+            acc[10 + 2 * x] = -2. * ta.y;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NB; c++) {
+        const double v = wave_sum(pop[c]);
+        if ((threadIdx.x & 63) == 0) pops[threadIdx.x >> 6][c] = v;
+    }
+    obs_finish(o, acc, pmin, pmax, &pops[0][0], kObsThreads / 64, NB);
+}
+
+// nb 5..32: the stage kernels' thread groups (TPK threads per k), P, U and H of
+// the k in LDS, T = P U^T and W = conj(P) H on the stage kernels' product tiles.
+// All operands of a k are requested together; a lane multiplies its packed
+// elements of D and of the gradient by what it finds in LDS.  Memory-bound at 32
+// bands (80 KB per k): 128 x 128 k take 446 us (2.9 TB/s), where the form that
+// took the population with nb LDS reads per term and read a table of H D^+ took
+// 1168; 16 bands 200 x 200 534 -> 233 us, 8 bands 99 -> 74.  Registers decide how
+// many blocks a CU holds: without TAbs (no core bands) its six compensated sums
+// are compiled out.
+template <int NBT>
+__host__ __device__ constexpr int obs_lds_doubles() {
+    return (kObsThreads / WaveGeom<NBT>::TPK) * (3 * NBT * WaveGeom<NBT>::LD * 2 + NBT) + (NBT == 32 ? 64 : 0);
+}
+
+template <int NBT, bool TA>
+__global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_wave(ObsArgs o) {
+    extern __shared__ double smem_d[];
+    constexpr int TPK = WaveGeom<NBT>::TPK, KPB = kObsThreads / TPK, PER = WaveGeom<NBT>::PER, LD = WaveGeom<NBT>::LD, MAT = NBT * LD;
+    constexpr int RBR = WaveGeom<NBT>::RBR, RBC = WaveGeom<NBT>::RBC;
+    static_assert(PER % 2 == 0, "a thread owns pairs of packed elements");
+    const int grp = threadIdx.x / TPK, lane = threadIdx.x % TPK;
+    const int nb = o.nb, NP = nb * nb, nch = o.nch;
+    cd *A = reinterpret_cast<cd *>(smem_d) + (size_t)grp * 3 * MAT, *B = A + MAT, *C = B + MAT;
+    double *pops = smem_d + (size_t)KPB * 3 * MAT * 2;    // [KPB][NBT], written at the end
+    double *popw = pops + KPB * NBT;                      // NBT = 32: [2][32] per-k halves of the population
+    for (int t = lane; t < 3 * MAT; t += TPK) A[t] = mk(0.0, 0.0);
+    auto elem = [&](int m) { return 2 * (lane + TPK * (m >> 1)) + (m & 1); };
+    int code0[PER];
+#pragma unroll
+    for (int m = 0; m < PER; m++) code0[m] = o.eidx[min(elem(m), NP - 1)];
+    constexpr int NS = TA ? kObsSums : 9;
+    Kahan pop, acc[NS];
+    double pmin = 1.0, pmax = 0.0;
+    auto band = [&](int c, double sre) {
+        pop.add(sre);
+        const double hv = (c < o.ncc) ? 1. - sre : sre;
+        pmax = fmax(pmax, fabs(hv));
+        pmin = fmin(pmin, hv);
+    };
+    for (int k0 = blockIdx.x * KPB; k0 < o.nk; k0 += gridDim.x * KPB) {
+        const bool live = k0 + grp < o.nk;
+        const int k = min(k0 + grp, o.nk - 1);
+        const size_t base = (size_t)k * NP;
+        // the lane's elements, decoded anew for each k: their LDS addresses kept live
+        // over the loop took the registers of a third block per CU
+        int code[PER], eo[PER];
+        bool v2[PER / 2];
+#pragma unroll
+        for (int m = 0; m < PER; m++) {
+            code[m] = code0[m];
+            asm volatile("" : "+v"(code[m]));
+            eo[m] = min(elem(m), NP - 1);
+        }
+#pragma unroll
+        for (int q = 0; q < PER / 2; q++) v2[q] = NP % 2 == 0 && elem(2 * q + 1) < NP;
+        auto row = [&](int m) { return code[m] & 255; };
+        auto col = [&](int m) { return (code[m] >> 8) & 255; };
+        auto imag = [&](int m) { return (code[m] >> 16) != 0; };
+        double y[PER], h[PER], ur[PER], ui[PER], s[NS];
+#pragma unroll
+        for (int q = 0; q < PER / 2; q++) {
+            const int m = 2 * q;
+            const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
+            ld2<false>(o.P, o0, o1, v2[q], y[m], y[m + 1]);
+            ld2<true>(o.H, o0, o1, v2[q], h[m], h[m + 1]);
+        }
+#pragma unroll
+        for (int m = 0; m < PER; m++) {
+            const size_t t = base + min(lane + TPK * m, NP - 1);
+            ld2<true>(o.U, 2 * t, 2 * t + 1, true, ur[m], ui[m]);
+        }
+#pragma unroll
+        for (int x = 0; x < NS; x++) s[x] = 0.0;
+        if (o.GE) {  // J1: sum_ij P_ij gradH_ij (real: both Hermitian; a pair counts twice)
+            const double *ge = o.GE + (size_t)k * 3 * NP;
+            double g[PER][3];
+#pragma unroll
+            for (int q = 0; q < PER / 2; q++)
+#pragma unroll
+                for (int x = 0; x < 3; x++)
+                    ld2<true>(ge + (size_t)x * NP, eo[2 * q], eo[2 * q + 1], v2[q], g[2 * q][x], g[2 * q + 1][x]);
+#pragma unroll
+            for (int m = 0; m < PER; m++) {
+                const double f = elem(m) >= NP ? 0.0 : row(m) == col(m) ? y[m] : imag(m) ? -2. * y[m] : 2. * y[m];
+#pragma unroll
+                for (int x = 0; x < 3; x++) s[x] += f * g[m][x];
+            }
+        }
+        __syncthreads();  // the previous k's LDS reads are done
+#pragma unroll
+        for (int m = 0; m < PER; m++) {
+            const int i = row(m), j = col(m), c = imag(m);
+            double *Ad = reinterpret_cast<double *>(A), *Cd = reinterpret_cast<double *>(C);
+            const int up = 2 * (i * LD + j) + c, lo = 2 * (j * LD + i) + c;
+            Ad[up] = y[m];
+            Cd[up] = h[m];
+            if (i != j) {
+                Ad[lo] = c ? -y[m] : y[m];
+                Cd[lo] = c ? -h[m] : h[m];
+            } else {  // W has replaced P here: the diagonal's imaginary part is zero again
+                Ad[up + 1] = 0.0;
+            }
+            const int t = min(lane + TPK * m, NP - 1);
+            lds_put(B + (t / nb) * LD + t % nb, mk(ur[m], ui[m]));
+        }
+        __syncthreads();
+        // population of band c = Re (conj(U) P U^T)_cc = Re sum_i conj(U_ci) T_ic
+        cd pij[PER];
+        if constexpr (TA) {
+#pragma unroll
+            for (int m = 0; m < PER; m++) pij[m] = lds_get(A + row(m) * LD + col(m));
+        }
+        double d[PER][3];  // in flight during the products
+#pragma unroll
+        for (int q = 0; q < PER / 2; q++)
+#pragma unroll
+            for (int x = 0; x < 3; x++)
+                ld2<true>(o.D + x * o.dxs, base + eo[2 * q], base + eo[2 * q + 1], v2[q], d[2 * q][x], d[2 * q + 1][x]);
+        if constexpr (NBT >= 16) {
+            int r0, c0;
+            mfma_tile<NBT>(lane, r0, c0);
+            v4d cre, cim;
+            gemm_mfma<NBT, 0, 0, double>(A, B, lane, cre, cim);
+            const int cb = c0 + (lane & 15);
+            double ps = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const cd u = lds_get(B + cb * LD + r0 + mfma_row<double>(lane & 63, i));
+                ps += u.x * cre[i] + u.y * cim[i];
+            }
+            ps += __shfl_xor(ps, 16, 64);
+            ps += __shfl_xor(ps, 32, 64);
+            if constexpr (NBT == 32) {
+                if ((lane & 63) < 16) popw[(r0 >> 4) * 32 + cb] = ps;
+            } else if (live && lane < nb) {
+                band(lane, ps);
+            }
+            gemm_mfma<NBT, 1, 1, double>(A, C, lane, cre, cim);  // W = conj(P) H
+            __syncthreads();
+            store_mfma<NBT, double>(A, lane, cre, cim);
+        } else {
+            cd r[RBR][RBC];
+            gemm_lds<NBT, 0, 0>(A, B, lane, r);
+            constexpr int GR = WaveGeom<NBT>::GR, GC = WaveGeom<NBT>::GC;
+            static_assert(RBC == 1, "one column per lane");
+            const int rr = lane / GC, c = lane % GC;
+            double ps = 0.0;
+#pragma unroll
+            for (int i = 0; i < RBR; i++) {
+                const cd u = lds_get(B + c * LD + rr + i * GR);
+                ps += u.x * r[i][0].x + u.y * r[i][0].y;
+            }
+#pragma unroll
+            for (int off = GC; off < TPK; off <<= 1) ps += __shfl_xor(ps, off, 64);
+            if (live && lane < nb) band(lane, ps);
+            gemm_lds<NBT, 1, 1>(A, C, lane, r);
+            __syncthreads();
+            store_block<NBT>(A, lane, r);
+        }
+        __syncthreads();
+        if constexpr (NBT == 32) {
+            if (live && lane < nb) band(lane, popw[lane] + popw[32 + lane]);
+        }
+        // J2: conj(D_jc) W_jc + conj(D_cj) W_cj per element of the upper triangle, the
+        // lower one being D_jc or its conjugate; TAbs
+#pragma unroll
+        for (int m = 0; m < PER; m++) {
+            if (elem(m) >= NP) continue;
+            const int i = row(m), j = col(m);
+            const bool im = imag(m);
+            const cd wu = lds_get(A + i * LD + j), wl = lds_get(A + j * LD + i);
+            cd w;
+            if (i == j) w = wu;
+            else if (!im) w = cadd(wu, wl);
+            else if (o.dherm) w = mk(wu.y - wl.y, wl.x - wu.x);
+            else w = mk(wu.y + wl.y, -(wu.x + wl.x));
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                s[3 + 2 * x] += d[m][x] * w.x;
+                s[4 + 2 * x] += d[m][x] * w.y;
+            }
+            if (TA && i < nch && j >= nch) {
+                const cd p = im ? mk(-pij[m].y, pij[m].x) : pij[m];
+#pragma unroll
+                for (int x = 0; x < 3; x++) {
+                    s[TA ? 9 + 2 * x : 0] += -2. * d[m][x] * p.x;
+                    s[TA ? 10 + 2 * x : 0] += -2. * d[m][x] * p.y;
+                }
+            }
+        }
+        if (live) {
+#pragma unroll
+            for (int x = 0; x < NS; x++) acc[x].add(s[x]);
+        }
+    }
+    if (lane < nb) pops[grp * NBT + lane] = pop.s;
+    double sums[NS];
+#pragma unroll
+    for (int x = 0; x < NS; x++) sums[x] = acc[x].s;
+    obs_finish(o, sums, pmin, pmax, pops, KPB, NBT);
 }
 
 // ================================================================ setup helpers
-// Q_x = H D_x^+ per k (Current2's sum_kc H_ik conj(D_jk), Observables_MPI.h:726-775)
-// from the packed operators: full complex [k][3][nb][nb].  Element e of k sits at
-// k*sk + e*se, component x of D at x*dxs.
 // FP32 copy of an operator table (mixed-precision mode), grid-stride.
 __global__ __launch_bounds__(256) void k_to_float(const double *src, float *dst, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = (float)src[i];
@@ -1999,37 +2255,6 @@ __global__ void k_pack(const double *__restrict__ src, long long n, int nb, int 
         dst[k * sk + e * se] = re;
         dst[k * sk + (e + 1) * se] = im;
     }
-}
-
-// D on the core <-> non-core block (rows i < nch, columns j >= nch) for the
-// transient absorption, [k][3][nch (nb - nch)] complex, from a chunk of the
-// reference [k][nb][nb][3] table.
-__global__ void k_pack_dt(const double *__restrict__ src, int kc, int nb, int nch, double *__restrict__ dst) {
-    const int nblk = nch * (nb - nch);
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)kc * 3 * nblk) return;
-    const int r = (int)(t % (3 * nblk)), x = r / nblk, q = r % nblk, i = q / (nb - nch), j = nch + q % (nb - nch);
-    const size_t k = (size_t)(t / (3 * nblk));
-    const double *d = src + (((k * nb + i) * nb + j) * 3 + x) * 2;
-    dst[2 * t] = d[0];
-    dst[2 * t + 1] = d[1];
-}
-
-__global__ void k_build_q(const double *Hp, const double *Dp, int nk, int nb, size_t sk, size_t se, size_t dxs, int dherm, double *Q) {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (long long)nk * 3 * nb * nb) return;
-    const int j = (int)(id % nb), i = (int)((id / nb) % nb), x = (int)((id / ((long long)nb * nb)) % 3);
-    const long long k = id / (3LL * nb * nb);
-    auto el = [&](const double *base, int a, int b, bool herm) -> cd {
-        if (a == b) return mk(base[k * sk + a * se], 0.0);
-        const int p = pair_index(min(a, b), max(a, b), nb);
-        const cd v = mk(base[k * sk + (nb + 2 * p) * se], base[k * sk + (nb + 2 * p + 1) * se]);
-        return (a < b || !herm) ? v : cconj(v);
-    };
-    cd acc = mk(0.0, 0.0);
-    for (int kc = 0; kc < nb; kc++) acc = cadd(acc, cmul(el(Hp, i, kc, true), cconj(el(Dp + x * dxs, j, kc, dherm != 0))));
-    Q[2 * id] = acc.x;
-    Q[2 * id + 1] = acc.y;
 }
 
 // ================================================================ captured steps
@@ -2072,22 +2297,60 @@ __global__ __launch_bounds__(256) void k_diag_dp(const double *Y, const double *
 // ================================================================ k-resolved snapshots
 // Element (ic, jc) of conj(U) P_sym U^T per k, P_sym from the stored upper
 // triangle, diagonal forced real (get_P_in_dia_vect, InitParameters.h:264-335).
-__global__ void k_eigen_element(const double *Y, const double *U, int nk, int nb, size_t sk, size_t se, int ic, int jc, double *out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nk) return;
+// L lanes per k: each takes every L-th packed element and forms what it and its
+// mirror contribute, conj(U_ic,i) P_ij U_jc,j + conj(U_ic,j) conj(P_ij) U_jc,i; the
+// two rows of U sit in LDS.  L = 1 for the SoA layout (nb <= 4), whose loads are
+// coalesced over k; a thread per k in the k-major layout read 8 nb^2 bytes with a
+// stride of 8 nb^2 (32 bands, 128 x 128: 619 us -> 27, 5.6 TB/s of 150 MB).
+constexpr int kElemThreads = 256;
+
+template <int L>
+__global__ __launch_bounds__(kElemThreads) void k_eigen_element(const double *__restrict__ Y, const double *__restrict__ U,
+                                                                const int *__restrict__ eidx, int nk, int nb, size_t sk, size_t se,
+                                                                int ic, int jc, double *__restrict__ out) {
+    constexpr int KPB = kElemThreads / L;
+    __shared__ cd rows[L > 1 ? KPB : 1][2][L > 1 ? EDUS_MAX_NB + 1 : 1];
+    const int g = threadIdx.x / L, l = threadIdx.x % L, NP = nb * nb;
+    const int kk = blockIdx.x * KPB + g, k = min(kk, nk - 1);
     const double *u = U + (size_t)k * nb * nb * 2;
-    auto pel = [&](int i, int j) -> cd {
-        if (i == j) return mk(Y[k * sk + i * se], 0.0);
-        const int a = min(i, j), b = max(i, j), p = pair_index(a, b, nb);
-        const cd v = mk(Y[k * sk + (nb + 2 * p) * se], Y[k * sk + (nb + 2 * p + 1) * se]);
-        return (i < j) ? v : cconj(v);
-    };
     cd acc = mk(0.0, 0.0);
-    for (int ii = 0; ii < nb; ii++) {
-        cd m = mk(0.0, 0.0);
-        for (int jj = 0; jj < nb; jj++) m = cadd(m, cmul(pel(ii, jj), mk(u[(jc * nb + jj) * 2], u[(jc * nb + jj) * 2 + 1])));
-        acc = cadd(acc, cmul(mk(u[(ic * nb + ii) * 2], -u[(ic * nb + ii) * 2 + 1]), m));
+    if constexpr (L == 1) {
+        auto pel = [&](int i, int j) -> cd {
+            if (i == j) return mk(Y[k * sk + i * se], 0.0);
+            const int a = min(i, j), b = max(i, j), p = pair_index(a, b, nb);
+            const cd v = mk(Y[k * sk + (nb + 2 * p) * se], Y[k * sk + (nb + 2 * p + 1) * se]);
+            return (i < j) ? v : cconj(v);
+        };
+        for (int ii = 0; ii < nb; ii++) {
+            cd m = mk(0.0, 0.0);
+            for (int jj = 0; jj < nb; jj++) m = cadd(m, cmul(pel(ii, jj), mk(u[(jc * nb + jj) * 2], u[(jc * nb + jj) * 2 + 1])));
+            acc = cadd(acc, cmul(mk(u[(ic * nb + ii) * 2], -u[(ic * nb + ii) * 2 + 1]), m));
+        }
+    } else {
+        for (int t = l; t < 2 * nb; t += L) {
+            const int r = t >= nb, i = t - r * nb;
+            const double *q = u + ((size_t)(r ? jc : ic) * nb + i) * 2;
+            rows[g][r][i] = mk(q[0], q[1]);
+        }
+        __syncthreads();
+        const cd *a = rows[g][0], *b = rows[g][1];
+        const double *yk = Y + (size_t)k * NP;
+#pragma unroll 4
+        for (int e = l; e < NP; e += L) {
+            const int code = eidx[e], i = code & 255, j = (code >> 8) & 255;
+            const double v = yk[e];
+            const cd w = cmul(cconj(a[i]), b[j]), x = cmul(cconj(a[j]), b[i]);
+            if (i == j) acc = cadd(acc, cscale(w, v));
+            else if (code >> 16) acc = cadd(acc, mk(v * (x.y - w.y), v * (w.x - x.x)));
+            else acc = cadd(acc, cscale(cadd(w, x), v));
+        }
+#pragma unroll
+        for (int off = L / 2; off > 0; off >>= 1) {
+            acc.x += __shfl_xor(acc.x, off, 64);
+            acc.y += __shfl_xor(acc.y, off, 64);
+        }
     }
+    if (kk >= nk || l != 0) return;
     if (ic == jc) acc.y = 0.0;
     out[2 * (size_t)k] = acc.x;
     out[2 * (size_t)k + 1] = acc.y;
@@ -2551,11 +2814,13 @@ struct edus_ctx {
     std::vector<double> wb;  // [n_nbr][3]
     // device buffers
     double *P0 = nullptr, *ACC = nullptr, *YA = nullptr, *YB = nullptr, *HIST = nullptr;
-    double *H = nullptr, *D = nullptr, *U = nullptr, *T = nullptr, *GE = nullptr, *Q = nullptr, *DT = nullptr;
+    double *H = nullptr, *D = nullptr, *U = nullptr, *T = nullptr, *GE = nullptr;
     int *nbr = nullptr;
     double *tab = nullptr;
     size_t tab_cap = 0;
-    double *part = nullptr, *obs = nullptr;
+    double *part = nullptr;           // observables: block partials, finished-block count, results (host memory)
+    unsigned *obs_count = nullptr;
+    double *obs = nullptr;
     int obs_blocks = 0;
     int cur = 0;          // AB/Taylor: state in P0 (0) or YA (1)
     long long nstep = 0;  // steps done (history ring position)
@@ -2569,7 +2834,7 @@ struct edus_ctx {
     double *cxm = nullptr, *sxm = nullptr, *cyn = nullptr, *syn = nullptr, *cS = nullptr, *cF = nullptr;
     double *cX = nullptr, *cX0 = nullptr, *cA = nullptr, *cB = nullptr, *cC = nullptr, *cD = nullptr, *cvh = nullptr;
     double *cEH = nullptr, *cEH0 = nullptr, *cT = nullptr, *cPW0 = nullptr, *cHr = nullptr, *cscreen = nullptr, *cXw = nullptr;
-    double *cUexc = nullptr, *cGE = nullptr, *cQ = nullptr, *dwb = nullptr, *cEk = nullptr;
+    double *dwb = nullptr, *cEk = nullptr;
     bool cEk_valid = false;
     double *snap = nullptr;  // [nk] complex, k-resolved snapshot element
     // adaptive dt: diagonal before the step, block maxima
@@ -2653,6 +2918,50 @@ void launch_pack(const edus_ctx *c, const double *stage, int kc, int cs, int x, 
     const long long n = (long long)kc * c->nb * c->nb;
     hipLaunchKernelGGL(k_pack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, stage, n, c->nb, cs, x, sk, se, dst);
 }
+
+// Pinned host memory that the observables kernels write their results to: slots of
+// one context each in slabs of 64 (an allocation of its own took each context 1 to
+// 2 ms).  A slab whose slots are all back is freed, except the last one, which
+// stays (32 KB); thread-safe.
+class ResultSlots {
+    static constexpr int kSlot = EDUS_MAX_NB + kObsSums + 17, kSlots = 64;  // doubles per slot (512 bytes)
+    struct Slab {
+        double *base;
+        uint64_t used;
+    };
+    std::mutex mu;
+    std::vector<Slab> slabs;
+
+public:
+    double *take() {
+        std::lock_guard<std::mutex> lock(mu);
+        for (Slab &s : slabs)
+            if (~s.used) {
+                const int i = __builtin_ctzll(~s.used);
+                s.used |= 1ull << i;
+                return s.base + (size_t)i * kSlot;
+            }
+        void *p = nullptr;
+        if (hipHostMalloc(&p, (size_t)kSlots * kSlot * sizeof(double), hipHostMallocPortable) != hipSuccess) return nullptr;
+        slabs.push_back({static_cast<double *>(p), 1});
+        return slabs.back().base;
+    }
+    void give(double *p) {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(mu);
+        for (size_t i = 0; i < slabs.size(); i++) {
+            const ptrdiff_t d = p - slabs[i].base;
+            if (d < 0 || d >= (ptrdiff_t)kSlots * kSlot) continue;
+            slabs[i].used &= ~(1ull << (d / kSlot));
+            if (!slabs[i].used && slabs.size() > 1) {
+                (void)hipHostFree(slabs[i].base);
+                slabs.erase(slabs.begin() + i);
+            }
+            return;
+        }
+    }
+};
+ResultSlots g_results;
 
 struct DeviceFree {
     void operator()(double *p) const { (void)hipFree(p); }
@@ -3033,28 +3342,11 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
         return fail(set_err(EDUS_ERR_HIP, "memset operators"));  // padding columns of the SoA layout
     if ((rc = upload_packed(c, p->H, 1, st, stage_k, [&](int k0, int kc) { launch_pack(c, st, kc, 1, 0, sk, sek, c->H + k0 * sk); })))
         return fail(rc);
-    {
-        // D: three packed components [x][state], and its core <-> non-core block.
-        const int nblk = c->nch * (nb - c->nch);
-        const size_t ndt = (size_t)p->nk * 3 * std::max(nblk, 1) * 2;
-        if ((rc = dalloc(c, &c->DT, ndt))) return fail(rc);
-        if (hipMemsetAsync(c->DT, 0, ndt * sizeof(double), c->stream) != hipSuccess) return fail(set_err(EDUS_ERR_HIP, "memset DT"));
-        rc = upload_packed(c, p->D, 3, st, stage_k, [&](int k0, int kc) {
-            for (int x = 0; x < 3; x++) launch_pack(c, st, kc, 3, x, sk, sek, c->D + x * se + k0 * sk);
-            if (nblk > 0) {
-                const long long n = (long long)kc * 3 * nblk;
-                hipLaunchKernelGGL(k_pack_dt, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, (const double *)st, kc, nb, c->nch,
-                                   c->DT + (size_t)k0 * 3 * nblk * 2);
-            }
-        });
-        if (rc) return fail(rc);
-        // Q_x = H D_x^+ for Current2, built on the device from the packed operators.
-        const size_t nq = (size_t)p->nk * 3 * nb * nb;
-        if ((rc = dalloc(c, &c->Q, nq * 2))) return fail(rc);
-        hipLaunchKernelGGL(k_build_q, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, c->stream, (const double *)c->H,
-                           (const double *)c->D, p->nk, nb, sk, sek, se, c->dherm, c->Q);
-        if (hipGetLastError() != hipSuccess) return fail(set_err(EDUS_ERR_HIP, "k_build_q launch"));
-    }
+    // D: three packed components [x][state]
+    rc = upload_packed(c, p->D, 3, st, stage_k, [&](int k0, int kc) {
+        for (int x = 0; x < 3; x++) launch_pack(c, st, kc, 3, x, sk, sek, c->D + x * se + k0 * sk);
+    });
+    if (rc) return fail(rc);
     {
         const size_t nu = (size_t)p->nk * nb * nb * 2;
         if ((rc = dalloc(c, &c->U, nu)) || (rc = dalloc(c, &c->T, (size_t)nb * nb))) return fail(rc);
@@ -3073,11 +3365,13 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
         if (hipGetLastError() != hipSuccess) return fail(set_err(EDUS_ERR_HIP, "k_to_float launch"));
     }
     if (p->gradH) {
-        // packed Hermitian gradient of H, [k][3][NP] (always k-major)
+        // packed Hermitian gradient of H: like D for the SoA layout, [k][3][NP] k-major
         const size_t np3 = (size_t)3 * c->np;
-        if ((rc = dalloc(c, &c->GE, (size_t)p->nk * np3))) return fail(rc);
+        if ((rc = dalloc(c, &c->GE, c->soa ? 3 * se : (size_t)p->nk * np3))) return fail(rc);
         rc = upload_packed(c, p->gradH, 3, st, stage_k, [&](int k0, int kc) {
-            for (int x = 0; x < 3; x++) launch_pack(c, st, kc, 3, x, np3, 1, c->GE + (size_t)k0 * np3 + (size_t)x * c->np);
+            for (int x = 0; x < 3; x++)
+                if (c->soa) launch_pack(c, st, kc, 3, x, sk, sek, c->GE + x * se + k0 * sk);
+                else launch_pack(c, st, kc, 3, x, np3, 1, c->GE + (size_t)k0 * np3 + (size_t)x * c->np);
         });
         if (rc) return fail(rc);
     }
@@ -3094,8 +3388,16 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
         if (hipMemcpyAsync(c->nbr, nbr.data(), nbr.size() * sizeof(int), hipMemcpyHostToDevice, c->stream) != hipSuccess)
             return fail(set_err(EDUS_ERR_HIP, "upload nbr"));
     }
-    c->obs_blocks = std::max(1, std::min(kObsMaxBlocks, p->nk));
-    if ((rc = dalloc(c, &c->part, (size_t)c->obs_blocks * (nb + 17))) || (rc = dalloc(c, &c->obs, nb + 17))) return fail(rc);
+    {
+        // nb <= 4: a thread per k.  Above, blocks that stay resident (from 9 bands
+        // LDS and registers hold three per CU) walk the grid.
+        const int kpb = c->soa ? kObsThreads : kObsThreads / (nb <= 8 ? WaveGeom<8>::TPK : nb <= 16 ? WaveGeom<16>::TPK : WaveGeom<32>::TPK);
+        const int nblk = (p->nk + kpb - 1) / kpb;
+        c->obs_blocks = c->soa ? nblk : std::min(nb <= 8 ? kObsMaxBlocks : 3 * kObsMaxBlocks / 4, nblk);
+        if ((rc = dalloc(c, &c->part, (size_t)c->obs_blocks * (nb + kObsSums + 2))) || (rc = dalloc(c, &c->obs_count, 1))) return fail(rc);
+        if (!(c->obs = g_results.take())) return fail(set_err(EDUS_ERR_NOMEM, "observables result buffer"));
+        if (hipMemsetAsync(c->obs_count, 0, sizeof(unsigned), c->stream) != hipSuccess) return fail(set_err(EDUS_ERR_HIP, "memset count"));
+    }
     {
         if (c->soa && hipMemsetAsync(c->P0, 0, se * sizeof(double), c->stream) != hipSuccess)
             return fail(set_err(EDUS_ERR_HIP, "memset state"));
@@ -3149,8 +3451,7 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
         if ((rc = dalloc(c, &c->cS, (size_t)2 * c->N1 * c->ncut * c->np)) || (rc = dalloc(c, &c->cF, (size_t)4 * nmm * c->np)) ||
             (rc = dalloc(c, &c->cX, (size_t)4 * nmm * nb2 * 2)) || (rc = dalloc(c, &c->cT, (size_t)2 * c->N2 * c->ncut * c->nu * 2)) ||
             (rc = dalloc(c, &c->cEH, nb)) || (rc = dalloc(c, &c->cPW0, se)) || (rc = dalloc(c, &c->cHr, se)) ||
-            (rc = dalloc(c, &c->cUexc, (size_t)p->nk * nb2 * 2)) || (rc = dalloc(c, &c->cGE, (size_t)p->nk * 3 * c->np)) ||
-            (rc = dalloc(c, &c->cQ, (size_t)p->nk * 3 * nb2 * 2)) || (rc = dalloc(c, &c->cEk, (size_t)p->nk * nb)) ||
+            (rc = dalloc(c, &c->cEk, (size_t)p->nk * nb)) ||
             (rc = dalloc(c, &c->cXw, (size_t)2 * c->nu * c->nkp)))
             return fail(rc);
         if ((rc = up(&c->cX0, std::vector<double>((size_t)4 * nmm * nb2 * 2, 0.0))) || (rc = up(&c->cEH0, std::vector<double>(nb, 0.0))) ||
@@ -3194,6 +3495,7 @@ int edus_destroy(edus_ctx *c) {
     if (c->gtab) (void)hipFree(c->gtab);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->tab) (void)hipFree(c->tab);
+    g_results.give(c->obs);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
@@ -3460,8 +3762,14 @@ int edus_eigen_element(edus_ctx *c, int32_t ic, int32_t jc, double *out) {
     if (!out || ic < 0 || jc < 0 || ic >= c->nb || jc >= c->nb) return set_err(EDUS_ERR_INVALID, "bad snapshot element");
     if (!c->snap && (rc = dalloc(c, &c->snap, (size_t)2 * c->nk))) return rc;
     const size_t sk = c->soa ? 1 : (size_t)c->np, se = c->soa ? (size_t)c->nkp : 1;
-    hipLaunchKernelGGL(k_eigen_element, dim3((c->nk + 255) / 256), dim3(256), 0, c->stream, current_state(c), (const double *)c->U, c->nk,
-                       c->nb, sk, se, ic, jc, c->snap);
+    auto go = [&](auto tag) {
+        constexpr int L = decltype(tag)::value, KPB = kElemThreads / L;
+        hipLaunchKernelGGL(k_eigen_element<L>, dim3((c->nk + KPB - 1) / KPB), dim3(kElemThreads), 0, c->stream, current_state(c),
+                           (const double *)c->U, (const int *)c->eidx, c->nk, c->nb, sk, se, ic, jc, c->snap);
+    };
+    if (c->soa) go(std::integral_constant<int, 1>{});
+    else if (c->nb <= 8) go(std::integral_constant<int, 16>{});
+    else go(std::integral_constant<int, 64>{});
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(out, c->snap, (size_t)2 * c->nk * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -3483,36 +3791,37 @@ int edus_observables(edus_ctx *c, double *pop, double *j1, double *j2, double *t
     int rc = check_ctx(c);
     if (rc) return rc;
     ObsArgs o;
-    o.P = current_state(c); o.U = c->U; o.GE = c->GE; o.Q = c->Q; o.DT = c->DT; o.part = c->part;
-    if (c->coul) {
-        const int blocks = (c->nk + 255) / 256;
+    std::memset(&o, 0, sizeof o);
+    o.P = current_state(c); o.U = c->U; o.GE = c->GE; o.H = c->coul ? c->cHr : c->H; o.D = c->D; o.eidx = c->eidx;
+    o.part = c->part; o.count = c->obs_count; o.out = c->obs;
+    o.nk = c->nk; o.nkp = c->nkp; o.nb = c->nb; o.nch = c->nch; o.ncc = c->ncc; o.dherm = c->dherm; o.dxs = (size_t)state_elems(c);
+    o.nbr = c->nbr; o.wb = c->dwb; o.n_nbr = c->n_nbr; o.Ek = c->cEk;
+    const dim3 grid(c->obs_blocks), block(kObsThreads);
+    auto wave = [&](auto tag) {
+        constexpr int NBT = decltype(tag)::value;
+        const size_t lds = obs_lds_doubles<NBT>() * sizeof(double);
+        if (c->nch > 0) hipLaunchKernelGGL((k_obs_wave<NBT, true>), grid, block, lds, c->stream, o);
+        else hipLaunchKernelGGL((k_obs_wave<NBT, false>), grid, block, lds, c->stream, o);
+    };
+    auto small = [&](auto ctag) {
+        constexpr bool COUL = decltype(ctag)::value;
         switch (c->nb) {
-            case 1: hipLaunchKernelGGL(k_coul_obs<1>, dim3(blocks), dim3(256), 0, c->stream, (const double *)c->cHr, (const double *)c->D, (const int *)c->nbr, (const double *)c->dwb, c->n_nbr, c->nk, c->nkp, c->dherm, c->cUexc, c->cGE, c->cQ, c->cEk); break;
-            case 2: hipLaunchKernelGGL(k_coul_obs<2>, dim3(blocks), dim3(256), 0, c->stream, (const double *)c->cHr, (const double *)c->D, (const int *)c->nbr, (const double *)c->dwb, c->n_nbr, c->nk, c->nkp, c->dherm, c->cUexc, c->cGE, c->cQ, c->cEk); break;
-            case 3: hipLaunchKernelGGL(k_coul_obs<3>, dim3(blocks), dim3(256), 0, c->stream, (const double *)c->cHr, (const double *)c->D, (const int *)c->nbr, (const double *)c->dwb, c->n_nbr, c->nk, c->nkp, c->dherm, c->cUexc, c->cGE, c->cQ, c->cEk); break;
-            default: hipLaunchKernelGGL(k_coul_obs<4>, dim3(blocks), dim3(256), 0, c->stream, (const double *)c->cHr, (const double *)c->D, (const int *)c->nbr, (const double *)c->dwb, c->n_nbr, c->nk, c->nkp, c->dherm, c->cUexc, c->cGE, c->cQ, c->cEk); break;
+            case 1: hipLaunchKernelGGL((k_obs_small<1, COUL>), grid, block, 0, c->stream, o); break;
+            case 2: hipLaunchKernelGGL((k_obs_small<2, COUL>), grid, block, 0, c->stream, o); break;
+            case 3: hipLaunchKernelGGL((k_obs_small<3, COUL>), grid, block, 0, c->stream, o); break;
+            default: hipLaunchKernelGGL((k_obs_small<4, COUL>), grid, block, 0, c->stream, o); break;
         }
-        HIP_TRY(hipGetLastError());
-        c->cEk_valid = true;
-        o.U = c->cUexc;
-        o.Q = c->cQ;
-        if (c->GE) o.GE = c->cGE;
-    }
-    o.nk = c->nk; o.nb = c->nb; o.nch = c->nch; o.ncc = c->ncc;
-    o.sk = c->soa ? 1 : c->np;
-    o.se = c->soa ? c->nkp : 1;
-    const size_t obs_lds = (size_t)c->nb * (2 * c->nb + 1) * sizeof(cd) + (4 * 17 + 32) * sizeof(double);
-    if (c->nb > 8)
-        hipLaunchKernelGGL(k_observables<256>, dim3(c->obs_blocks), dim3(256), obs_lds, c->stream, o);
-    else
-        hipLaunchKernelGGL(k_observables<64>, dim3(c->obs_blocks), dim3(64), obs_lds, c->stream, o);
+    };
+    if (c->coul) small(std::true_type{});
+    else if (c->soa) small(std::false_type{});
+    else if (c->nb <= 8) wave(std::integral_constant<int, 8>{});
+    else if (c->nb <= 16) wave(std::integral_constant<int, 16>{});
+    else wave(std::integral_constant<int, 32>{});
     HIP_TRY(hipGetLastError());
-    const int nv = c->nb + 15;
-    hipLaunchKernelGGL(k_obs_final, dim3(nv + 2), dim3(256), 0, c->stream, (const double *)c->part, c->obs_blocks, nv, c->obs);
-    HIP_TRY(hipGetLastError());
-    std::vector<double> h(nv + 2);
-    HIP_TRY(hipMemcpyAsync(h.data(), c->obs, h.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    c->cEk_valid = c->coul != 0;
     HIP_TRY(hipStreamSynchronize(c->stream));
+    const double *h = c->obs;
+    const int nv = c->nb + kObsSums;
     const int nb = c->nb;
     const double inv = 1. / c->nktot;
     if (pop)
