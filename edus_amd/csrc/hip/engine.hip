@@ -77,19 +77,6 @@ struct ConstArgs {
     int pair, pself, npnew;
     const int *pat;
     double wx2;
-    // Coulomb mean field (small-nb kernel only): the mean-field matrix per k,
-    // peak correction against PW0, renormalised H out.
-    int coul, N2, ncut, nu;
-    double n_cond;
-    const double *cxm, *sxm;   // [ncut][N1] cos/sin(2 pi m k1)
-    const double *Tt;          // [2][ncut][nu][N2] complex
-    const double *Xw;          // [2 nu][nkp] mean-field matrix (upper elements, re/im)
-    const double *PW0;         // packed state at t = 0
-    const double *EH;          // [nb] Hartree shift (minus equilibrium)
-    const double *screen;      // [nb*nb] complex
-    double *Hr;                // packed renormalised H (written)
-    int coul_diag;             // Coulomb_diag_basis: the sums ran on PD, corrections in the eigenbasis
-    const double *PD;          // packed state in the eigenbasis, conj(U) P U^T (diagonal basis)
 };
 
 // Per-launch stage data.  `tab` points at the stage's row of the field table:
@@ -415,105 +402,6 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
             P[j][i] = cconj(P[i][j]);
         }
     }
-    // Renormalised H with the Hartree-Fock mean field (RungeKutta.h:69-138):
-    // X_W[i][j] = -sum_mn (X_mn)_{ji} trig(k), minus Screen_const * (P - P0)_{ji}
-    // when n_cond > 1e-20, real diagonal, plus the Hartree shift.
-    cd Hren[NB][NB];
-    if (c.coul && c.coul_diag) {
-        // Diagonal basis (RungeKutta.h:97-124): X_d from the sums over PD, minus
-        // Screen_const[0][0] (PD - P_Bloch_0) on the diagonal (P_Bloch_0: the
-        // filled bands) and conj(Screen_const[0][1]) PD_ji off it; back to the
-        // orbital basis as U^+ X_d U (InitParameters.h:340-370).
-        cd Xd[NB][NB], U[NB][NB];
-        const double *uk = c.U + (size_t)k * NB * NB * 2;
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = 0; j < NB; j++) {
-                double re, im;
-                ld2<false>(uk, (i * NB + j) * 2, (i * NB + j) * 2 + 1, true, re, im);
-                U[i][j] = mk(re, im);
-            }
-        const cd scr0 = mk(c.screen[0], c.screen[1]), scr1c = mk(c.screen[2], -c.screen[3]);
-        int u = 0;
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = i; j < NB; j++, u++) {
-                cd xk = mk(c.Xw[(size_t)(2 * u) * nkp + k], c.Xw[(size_t)(2 * u + 1) * nkp + k]);
-                if (i == j) {
-                    xk = csub(xk, cscale(scr0, c.PD[i * nkp + k] - (i < c.ncc ? 1.0 : 0.0)));
-                    Xd[i][i] = xk;
-                } else {
-                    const int p = pair_index(i, j, NB);
-                    // PD_ji = conj(PD_ij)
-                    const cd pdji = mk(c.PD[(NB + 2 * p) * nkp + k], -c.PD[(NB + 2 * p + 1) * nkp + k]);
-                    xk = csub(xk, cmul(scr1c, pdji));
-                    Xd[i][j] = xk;
-                    Xd[j][i] = cconj(xk);
-                }
-            }
-        cd T1[NB][NB];
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = 0; j < NB; j++) {
-                cd t = mk(0.0, 0.0);
-#pragma unroll
-                for (int l = 0; l < NB; l++) t = cadd(t, cmul(Xd[i][l], U[l][j]));
-                T1[i][j] = t;
-            }
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = i; j < NB; j++) {
-                cd xw = mk(0.0, 0.0);
-#pragma unroll
-                for (int l = 0; l < NB; l++) xw = cadd(xw, cmul(cconj(U[l][i]), T1[l][j]));
-                cd h;
-                if (i == j) {
-                    h = mk(c.H[i * nkp + k] + xw.x + c.EH[i], 0.0);
-                    c.Hr[i * nkp + k] = h.x;
-                } else {
-                    const int p = pair_index(i, j, NB);
-                    h = mk(c.H[(NB + 2 * p) * nkp + k] + xw.x, c.H[(NB + 2 * p + 1) * nkp + k] + xw.y);
-                    c.Hr[(NB + 2 * p) * nkp + k] = h.x;
-                    c.Hr[(NB + 2 * p + 1) * nkp + k] = h.y;
-                }
-                Hren[i][j] = h;
-            }
-    } else if (c.coul) {
-        int u = 0;
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = i; j < NB; j++, u++) {
-                cd xk = mk(c.Xw[(size_t)(2 * u) * nkp + k], c.Xw[(size_t)(2 * u + 1) * nkp + k]);
-                if (c.n_cond > 1e-20) {
-                    const int idx = (i != j) ? i * NB + j : 0;
-                    cd scr = mk(c.screen[2 * idx], -c.screen[2 * idx + 1]);  // conj(Screen_const)
-                    cd dp;
-                    if (i == j) dp = mk(y[i] - c.PW0[i * nkp + k], 0.0);
-                    else {
-                        const int p = pair_index(i, j, NB);
-                        // (P - P0)_{ji} = conj((P - P0)_{ij})
-                        dp = mk(y[NB + 2 * p] - c.PW0[(NB + 2 * p) * nkp + k], -(y[NB + 2 * p + 1] - c.PW0[(NB + 2 * p + 1) * nkp + k]));
-                    }
-                    xk = csub(xk, cmul(scr, dp));
-                }
-                cd h;
-                if (i == j) {
-                    h = mk(c.H[i * nkp + k] + xk.x + c.EH[i], 0.0);
-                    c.Hr[i * nkp + k] = h.x;
-                } else {
-                    const int p = pair_index(i, j, NB);
-                    h = mk(c.H[(NB + 2 * p) * nkp + k] + xk.x, c.H[(NB + 2 * p + 1) * nkp + k] + xk.y);
-                    c.Hr[(NB + 2 * p) * nkp + k] = h.x;
-                    c.Hr[(NB + 2 * p + 1) * nkp + k] = h.y;
-                }
-                Hren[i][j] = h;
-            }
-    }
     // M = H + E.D with the probe on core<->non-core elements (RungeKutta.h:165-168).
 #pragma unroll
     for (int i = 0; i < NB; i++) {
@@ -534,7 +422,6 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
                     dx[x] = (a.dmask >> x & 1) ? mk(ldnt(c.D + (x * NP + NB + 2 * p) * nkp + k), ldnt(c.D + (x * NP + NB + 2 * p + 1) * nkp + k))
                                                : mk(0.0, 0.0);
             }
-            if (c.coul) h = Hren[i][j];
             cd mij = h, mji = cconj(h);
 #pragma unroll
             for (int x = 0; x < 3; x++) {
@@ -744,7 +631,14 @@ struct CoulArgs {
     double *EH;
     const double *EH0;
     double *Tt;                // [2][ncut][nu][N2] complex
-    double *Xw;                // [2 nu][nkp]: mean-field matrix per k (upper elements, re/im)
+    double *Xw;                // [2 nu][nkp]: mean-field matrix per k (upper elements, re/im; diagonal basis)
+};
+// What the renormalised H takes besides: bare H, U, the equilibrium state, the peak
+// correction and its gate.
+struct CoulHArgs {
+    const double *H, *U, *PW0, *screen;
+    double *Hr;
+    double n_cond;
 };
 
 constexpr int kCoulThreads = 256;
@@ -927,22 +821,57 @@ __global__ void k_coul_s3(CoulArgs a) {
     T[(((size_t)1 * a.ncut + m) * a.nu + u) * a.N2 + i2] = ts;
 }
 
-// Mean-field matrix of every k from the column sums (Coulomb.h:510-541):
-// X_W(i1, i2)_u = -sum_m [cos_m(i1) Tc(m, u, i2) + sin_m(i1) Ts(m, u, i2)], stored
-// SoA as Xw[2u + re/im][k], formed as products on the FP64 matrix cores: for each
-// (u, re/im), Xw(i1, i2) = -sum_kk A[i1][kk] B[kk][i2] with A = [cos_m(i1) |
-// sin_m(i1)] and B = [Tc(m, u, i2) ; Ts(m, u, i2)] (K = 2 Ncut).  Rows are i1,
-// columns c = (2u + re/im) N2 + i2; one wave per 16 x 16 tile, its K loads
-// issued before the products (lane l feeds A[row l%16][kk l/16] and
-// B[kk l/16][col l%16] and ends with C[l/16 + 4 i][l%16]).
-__global__ __launch_bounds__(64) void k_coul_w_mfma(CoulArgs a, int N1) {
+// Renormalised H of every k from the column sums (Coulomb.h:510-541, RungeKutta.h:69-138):
+// X_W(i1, i2)_u = -sum_m [cos_m(i1) Tc(m, u, i2) + sin_m(i1) Ts(m, u, i2)] formed as
+// products on the FP64 matrix cores, A[i1][kk] = [cos_m(i1) | sin_m(i1)] and
+// B[kk][c] = [Tc(m, u, i2) ; Ts(m, u, i2)] (K = 2 Ncut), rows i1, one wave per 16 x
+// 16 tile, its K loads issued before the products (lane l feeds A[row l%16][kk l/16]
+// and B[kk l/16][col l%16] and ends with C[l/16 + 4 i][l%16]).
+// Wannier basis (FULL): columns c = e N2 + i2 over the packed elements e, and the
+// tile's lanes go on to Hr = H + X_W, minus Screen_const * (P - P0)_{ji} when n_cond >
+// 1e-20, real diagonal, plus the Hartree shift: the stage kernel then reads Hr like
+// any H.  (Storing X_W and forming Hr in the stage kernel moved 42 instead of 36
+// doubles per k at 3 bands and cost the stage its registers: 300 x 300 AB4, stage
+// 29.7 + this pass 10.0 us -> 23.4 + 12.3.)
+// Diagonal basis: columns c = (2u + re/im) N2 + i2, stored as Xw[2u + re/im][k].
+template <bool FULL>
+__global__ __launch_bounds__(64) void k_coul_w_mfma(CoulArgs a, CoulHArgs h) {
     typedef double v4 __attribute__((ext_vector_type(4)));
     constexpr int KB = 16;  // K terms loaded per block (2 Ncut <= 64)
-    const int lane = threadIdx.x, r0 = blockIdx.x * 16, c0 = blockIdx.y * 16;
-    const int ncut = a.ncut, K = 2 * ncut, ncol = 2 * a.nu * a.N2;
+    const int lane = threadIdx.x, r0 = blockIdx.x * 16, c0 = blockIdx.y * 16, nb = a.nb;
+    const int ncut = a.ncut, K = 2 * ncut, ncol = (FULL ? a.NP : 2 * a.nu) * a.N2, N1 = a.N1;
     const int ra = r0 + (lane & 15), cb = c0 + (lane & 15), kq = lane >> 4;
     const bool rok = ra < N1, cok = cb < ncol;
-    const int i1 = rok ? ra : 0, uc = cok ? cb / a.N2 : 0, i2 = cok ? cb % a.N2 : 0, u = uc >> 1, ri = uc & 1;
+    const int i1 = rok ? ra : 0, uc = cok ? cb / a.N2 : 0, i2 = cok ? cb % a.N2 : 0;
+    // column -> upper element (bi <= bj) and component
+    int bi = 0, bj = 0, ri = 0, u = 0;
+    if (FULL && uc < nb) {
+        bi = bj = uc;
+    } else {
+        ri = FULL ? (uc - nb) & 1 : uc & 1;
+        int q = FULL ? (uc - nb) >> 1 : uc >> 1;
+        const int d = FULL ? 1 : 0;  // pairs i < j, or i <= j
+        while (q >= nb - bi - d) q -= nb - bi++ - d;
+        bj = bi + d + q;
+    }
+    u = bi * nb - bi * (bi - 1) / 2 + bj - bi;
+    // the tile's own operands are in flight during the products
+    const bool diag = bi == bj, scr = FULL && h.n_cond > 1e-20;
+    double hv[4], pr[4], pi[4];
+    if constexpr (FULL) {
+        const int p = diag ? bi : nb + 2 * pair_index(bi, bj, nb);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const size_t k = (size_t)min(r0 + (lane >> 4) + 4 * i, N1 - 1) * a.N2 + i2;
+            hv[i] = h.H[(size_t)uc * a.nkp + k];
+            pr[i] = pi[i] = 0.0;
+            if (scr) {
+                const size_t o = (size_t)p * a.nkp + k, o1 = diag ? o : o + a.nkp;
+                pr[i] = a.Y[o] - h.PW0[o];
+                pi[i] = diag ? 0.0 : a.Y[o1] - h.PW0[o1];
+            }
+        }
+    }
     v4 acc = {0.0, 0.0, 0.0, 0.0};
     for (int k0 = 0; k0 < K; k0 += KB) {
         double av[KB / 4], bv[KB / 4];
@@ -958,11 +887,91 @@ __global__ __launch_bounds__(64) void k_coul_w_mfma(CoulArgs a, int N1) {
             acc = __builtin_amdgcn_mfma_f64_16x16x4f64((rok && kok) ? av[b] : 0.0, (cok && kok) ? bv[b] : 0.0, acc, 0, 0, 0);
         }
     }
+    if (!cok) return;
+    if constexpr (!FULL) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int r = r0 + (lane >> 4) + 4 * i, c = c0 + (lane & 15);
-        if (r < N1 && c < ncol) a.Xw[(size_t)(c / a.N2) * a.nkp + (size_t)r * a.N2 + c % a.N2] = -acc[i];
+        for (int i = 0; i < 4; i++) {
+            const int r = r0 + (lane >> 4) + 4 * i;
+            if (r < N1) a.Xw[(size_t)uc * a.nkp + (size_t)r * a.N2 + i2] = -acc[i];
+        }
+    } else {
+        const int idx = diag ? 0 : bi * nb + bj;
+        const cd s = mk(h.screen[2 * idx], -h.screen[2 * idx + 1]);  // conj(Screen_const)
+        const double eh = diag ? a.EH[bi] : 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = r0 + (lane >> 4) + 4 * i;
+            if (r >= N1) continue;
+            // (P - P0)_{ji} = conj((P - P0)_{ij})
+            const cd x = cmul(s, mk(pr[i], -pi[i]));
+            h.Hr[(size_t)uc * a.nkp + (size_t)r * a.N2 + i2] = hv[i] + (-acc[i] - (ri ? x.y : x.x)) + eh;
+        }
     }
+}
+
+// Diagonal basis (RungeKutta.h:97-124): X_d from the sums over PD, minus
+// Screen_const[0][0] (PD - P_Bloch_0) on the diagonal (P_Bloch_0: the filled bands)
+// and conj(Screen_const[0][1]) PD_ji off it; back to the orbital basis as U^+ X_d U
+// (InitParameters.h:340-370), real diagonal plus the Hartree shift.  Thread per k.
+template <int NB>
+__global__ __launch_bounds__(256) void k_coul_hdiag(CoulArgs a, CoulHArgs h, int ncc) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= a.nk) return;
+    const size_t nkp = a.nkp;
+    const double *PD = a.Y;
+    cd Xd[NB][NB], U[NB][NB];
+    const double *uk = h.U + (size_t)k * NB * NB * 2;
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            double re, im;
+            ld2<false>(uk, (i * NB + j) * 2, (i * NB + j) * 2 + 1, true, re, im);
+            U[i][j] = mk(re, im);
+        }
+    const cd scr0 = mk(h.screen[0], h.screen[1]), scr1c = mk(h.screen[2], -h.screen[3]);
+    int u = 0;
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = i; j < NB; j++, u++) {
+            cd xk = mk(a.Xw[(size_t)(2 * u) * nkp + k], a.Xw[(size_t)(2 * u + 1) * nkp + k]);
+            if (i == j) {
+                Xd[i][i] = csub(xk, cscale(scr0, PD[i * nkp + k] - (i < ncc ? 1.0 : 0.0)));
+            } else {
+                const int p = pair_index(i, j, NB);
+                // PD_ji = conj(PD_ij)
+                const cd pdji = mk(PD[(NB + 2 * p) * nkp + k], -PD[(NB + 2 * p + 1) * nkp + k]);
+                xk = csub(xk, cmul(scr1c, pdji));
+                Xd[i][j] = xk;
+                Xd[j][i] = cconj(xk);
+            }
+        }
+    cd T1[NB][NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            cd t = mk(0.0, 0.0);
+#pragma unroll
+            for (int l = 0; l < NB; l++) t = cadd(t, cmul(Xd[i][l], U[l][j]));
+            T1[i][j] = t;
+        }
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int j = i; j < NB; j++) {
+            cd xw = mk(0.0, 0.0);
+#pragma unroll
+            for (int l = 0; l < NB; l++) xw = cadd(xw, cmul(cconj(U[l][i]), T1[l][j]));
+            if (i == j) {
+                h.Hr[i * nkp + k] = h.H[i * nkp + k] + xw.x + a.EH[i];
+            } else {
+                const int p = pair_index(i, j, NB);
+                h.Hr[(NB + 2 * p) * nkp + k] = h.H[(NB + 2 * p) * nkp + k] + xw.x;
+                h.Hr[(NB + 2 * p + 1) * nkp + k] = h.H[(NB + 2 * p + 1) * nkp + k] + xw.y;
+            }
+        }
 }
 
 // ================================================================ nb in 5..32: one workgroup per k
@@ -2985,7 +2994,7 @@ CoulArgs coul_args(edus_ctx *c, const double *Y) {
     return a;
 }
 
-// Mean-field coefficients of state Y: reduction, X_mn, column sums (4 launches).
+// Mean-field coefficients of state Y: reduction, X_mn, column sums (3 launches).
 int launch_coulomb(edus_ctx *c, const double *Y) {
     CoulArgs a = coul_args(c, Y);
     const int t3 = c->N2 * c->ncut * c->nu;
@@ -2994,40 +3003,51 @@ int launch_coulomb(edus_ctx *c, const double *Y) {
     hipLaunchKernelGGL(k_coul_s1_mfma, dim3((c->np * c->N1 + 15) / 16, (2 * c->ncut + 15) / 16), dim3(64), 0, c->stream, a);
     hipLaunchKernelGGL(k_coul_s2, dim3(c->ncut * c->ncut), dim3(kCoulThreads), 0, c->stream, a);
     hipLaunchKernelGGL(k_coul_s3, dim3((t3 + 63) / 64), dim3(64), 0, c->stream, a);
-    hipLaunchKernelGGL(k_coul_w_mfma, dim3((c->N1 + 15) / 16, (2 * c->nu * c->N2 + 15) / 16), dim3(64), 0, c->stream, a,
-                       c->N1);
     HIP_TRY(hipGetLastError());
     return 0;
 }
 
-// The mean-field sums of the stage input Y: over Y itself (Wannier basis) or over
-// Y in the eigenbasis (Coulomb_diag_basis, RungeKutta.h:41-55).
-int launch_coulomb_of(edus_ctx *c, const double *Y) {
-    if (!c->coul_diag) return launch_coulomb(c, Y);
-    const dim3 grid((c->nk + 255) / 256), block(256);
-    switch (c->nb) {
-        case 1: hipLaunchKernelGGL(k_coul_pdiag<1>, grid, block, 0, c->stream, Y, (const double *)c->U, c->nk, c->nkp, c->cPD); break;
-        case 2: hipLaunchKernelGGL(k_coul_pdiag<2>, grid, block, 0, c->stream, Y, (const double *)c->U, c->nk, c->nkp, c->cPD); break;
-        case 3: hipLaunchKernelGGL(k_coul_pdiag<3>, grid, block, 0, c->stream, Y, (const double *)c->U, c->nk, c->nkp, c->cPD); break;
-        default: hipLaunchKernelGGL(k_coul_pdiag<4>, grid, block, 0, c->stream, Y, (const double *)c->U, c->nk, c->nkp, c->cPD); break;
+// The renormalised H of the stage input Y into c->cHr: the sums over Y itself
+// (Wannier basis) or over Y in the eigenbasis (Coulomb_diag_basis, RungeKutta.h:41-55).
+int launch_mean_field(edus_ctx *c, const double *Y) {
+    CoulHArgs h;
+    h.H = c->H; h.U = c->U; h.PW0 = c->cPW0; h.screen = c->cscreen; h.Hr = c->cHr; h.n_cond = c->n_cond;
+    const int rt = (c->N1 + 15) / 16;
+    int rc;
+    if (!c->coul_diag) {
+        if ((rc = launch_coulomb(c, Y))) return rc;
+        hipLaunchKernelGGL(k_coul_w_mfma<true>, dim3(rt, (c->np * c->N2 + 15) / 16), dim3(64), 0, c->stream, coul_args(c, Y), h);
+        HIP_TRY(hipGetLastError());
+        return 0;
     }
-    HIP_TRY(hipGetLastError());
-    return launch_coulomb(c, c->cPD);
+    const dim3 grid((c->nk + 255) / 256), block(256);
+    auto go = [&](auto tag) -> int {
+        constexpr int NB = decltype(tag)::value;
+        hipLaunchKernelGGL(k_coul_pdiag<NB>, grid, block, 0, c->stream, Y, (const double *)c->U, c->nk, c->nkp, c->cPD);
+        HIP_TRY(hipGetLastError());
+        if ((rc = launch_coulomb(c, c->cPD))) return rc;
+        const CoulArgs a = coul_args(c, c->cPD);
+        hipLaunchKernelGGL(k_coul_w_mfma<false>, dim3(rt, (2 * c->nu * c->N2 + 15) / 16), dim3(64), 0, c->stream, a, h);
+        hipLaunchKernelGGL(k_coul_hdiag<NB>, grid, block, 0, c->stream, a, h, c->ncc);
+        HIP_TRY(hipGetLastError());
+        return 0;
+    };
+    switch (c->nb) {
+        case 1: return go(std::integral_constant<int, 1>{});
+        case 2: return go(std::integral_constant<int, 2>{});
+        case 3: return go(std::integral_constant<int, 3>{});
+        default: return go(std::integral_constant<int, 4>{});
+    }
 }
 
 ConstArgs const_args(const edus_ctx *c) {
     ConstArgs ca;
     std::memset(&ca, 0, sizeof ca);
-    ca.H = c->H; ca.D = c->D; ca.U = c->U; ca.T = c->T; ca.nbr = c->nbr;
+    ca.H = c->coul ? c->cHr : c->H; ca.D = c->D; ca.U = c->U; ca.T = c->T; ca.nbr = c->nbr;
     ca.Hf = c->Hf; ca.Df = c->Df; ca.Uf = c->Uf; ca.eidx = c->eidx;
     ca.nk = c->nk; ca.nkp = c->nkp; ca.nb = c->nb; ca.nch = c->nch; ca.ncc = c->ncc; ca.n_nbr = c->n_nbr;
     ca.diss = c->diss; ca.dherm = c->dherm; ca.wx2 = c->wx2; ca.sw = c->sw; ca.scol = c->scol;
     ca.pair = c->pair; ca.pself = c->pself; ca.npnew = c->npnew; ca.pat = c->nbr + (size_t)std::max(c->n_nbr, 1) * c->nkp;
-    ca.coul = c->coul; ca.N2 = c->N2; ca.ncut = c->ncut; ca.nu = c->nu; ca.n_cond = c->n_cond;
-    ca.cxm = c->cxm; ca.sxm = c->sxm; ca.Tt = c->cT; ca.PW0 = c->cPW0; ca.EH = c->cEH; ca.screen = c->cscreen; ca.Hr = c->cHr;
-    ca.Xw = c->cXw;
-    ca.coul_diag = c->coul_diag;
-    ca.PD = c->cPD;
     return ca;
 }
 
@@ -3036,7 +3056,7 @@ int launch_stage(edus_ctx *c, StageArgs a) {
     a.dmask = c->dmask;
     const ConstArgs ca = const_args(c);
     if (c->coul) {
-        int rc = launch_coulomb_of(c, a.Y);
+        int rc = launch_mean_field(c, a.Y);
         if (rc) return rc;
     }
     if (c->soa) {
@@ -3452,7 +3472,7 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
             (rc = dalloc(c, &c->cX, (size_t)4 * nmm * nb2 * 2)) || (rc = dalloc(c, &c->cT, (size_t)2 * c->N2 * c->ncut * c->nu * 2)) ||
             (rc = dalloc(c, &c->cEH, nb)) || (rc = dalloc(c, &c->cPW0, se)) || (rc = dalloc(c, &c->cHr, se)) ||
             (rc = dalloc(c, &c->cEk, (size_t)p->nk * nb)) ||
-            (rc = dalloc(c, &c->cXw, (size_t)2 * c->nu * c->nkp)))
+            (q->diag_basis && (rc = dalloc(c, &c->cXw, (size_t)2 * c->nu * c->nkp))))
             return fail(rc);
         if ((rc = up(&c->cX0, std::vector<double>((size_t)4 * nmm * nb2 * 2, 0.0))) || (rc = up(&c->cEH0, std::vector<double>(nb, 0.0))) ||
             (rc = upc(&c->dwb, p->nbr_wb, (size_t)std::max(p->n_nbr, 1) * 3)))
