@@ -104,8 +104,22 @@ struct StageArgs {
 // The field-table row of a stage: `tab`, advanced by the device step counter when
 // the launch belongs to a captured step (its arguments are fixed at capture, the
 // counter moves on between replays).
-__device__ __forceinline__ const double *stage_row(const StageArgs &a) {
-    return a.ctr ? a.tab + (size_t)(*a.ctr) * (size_t)a.ctr_stride : a.tab;
+// Read-only while any launch that reads it runs, so its (uniform) loads are scalar.
+typedef const __attribute__((address_space(4))) double *TabRow;
+__device__ __forceinline__ TabRow stage_row(const StageArgs &a) {
+    return (TabRow)(a.ctr ? a.tab + (size_t)(*a.ctr) * (size_t)a.ctr_stride : a.tab);
+}
+
+// Pointers into device memory.  Those of a batch come from a table in memory, and
+// the compiler would have to access through them with flat instructions, which
+// also count as LDS traffic (8 bands, batch: every stage access).
+template <typename T>
+__device__ __forceinline__ const __attribute__((address_space(1))) T *gm(const T *p) {
+    return (const __attribute__((address_space(1))) T *)p;
+}
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(1))) T *gm(T *p) {
+    return (__attribute__((address_space(1))) T *)p;
 }
 
 // ---------------------------------------------------------------- complex helpers
@@ -200,10 +214,10 @@ __host__ __device__ __forceinline__ int pair_index(int i, int j, int nb) { retur
 // Streaming accesses: operators, accumulators, histories and stage outputs are
 // touched once per launch, so they bypass the caches' normal retention and leave
 // L2 to the stage input, whose 12 stencil neighbours are re-read from it.
-__device__ __forceinline__ double ldnt(const double *p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ float ldnt(const float *p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ void stnt(double *p, double v) { __builtin_nontemporal_store(v, p); }
-__device__ __forceinline__ void stnt(float *p, float v) { __builtin_nontemporal_store(v, p); }
+__device__ __forceinline__ double ldnt(const double *p) { return __builtin_nontemporal_load(gm(p)); }
+__device__ __forceinline__ float ldnt(const float *p) { return __builtin_nontemporal_load(gm(p)); }
+__device__ __forceinline__ void stnt(double *p, double v) { __builtin_nontemporal_store(v, gm(p)); }
+__device__ __forceinline__ void stnt(float *p, float v) { __builtin_nontemporal_store(v, gm(p)); }
 
 // Two adjacent packed elements in one access (16 bytes in FP64, 8 in FP32), when
 // `vec` (the pair lies inside the matrix and the array offset is even); else two
@@ -215,13 +229,13 @@ template <> struct Pair<float> { typedef float V __attribute__((ext_vector_type(
 template <bool NT, typename T>
 __device__ __forceinline__ void ld2(const T *p, size_t o0, size_t o1, bool vec, T &a, T &b) {
     if (vec) {
-        const typename Pair<T>::V *q = reinterpret_cast<const typename Pair<T>::V *>(p + o0);
+        const auto *q = gm(reinterpret_cast<const typename Pair<T>::V *>(p + o0));
         const typename Pair<T>::V v = NT ? __builtin_nontemporal_load(q) : *q;
         a = v.x;
         b = v.y;
     } else {
-        a = NT ? ldnt(p + o0) : p[o0];
-        b = NT ? ldnt(p + o1) : p[o1];
+        a = NT ? ldnt(p + o0) : *gm(p + o0);
+        b = NT ? ldnt(p + o1) : *gm(p + o1);
     }
 }
 template <typename T>
@@ -230,64 +244,19 @@ __device__ __forceinline__ void st2(T *p, size_t o0, size_t o1, bool vec, T a, T
         typename Pair<T>::V v;
         v.x = a;
         v.y = b;
-        __builtin_nontemporal_store(v, reinterpret_cast<typename Pair<T>::V *>(p + o0));
+        __builtin_nontemporal_store(v, gm(reinterpret_cast<typename Pair<T>::V *>(p + o0)));
     } else {
         stnt(p + o0, a);
         stnt(p + o1, b);
     }
 }
 
-// ---------------------------------------------------------------- stage update
-// The elementwise tail shared by all kernels.  `kv` is one packed double of the
-// right-hand side, `y` the same double of the stage input, `o` its offset in the
-// state arrays and `h` the stride between history slots.
-// S: storage type of the Adams-Bashforth / Taylor history (double, or float in
-// the mixed form with FP32 stage storage); the state and its update stay FP64.
-template <int MODE, typename S = double>
-__device__ __forceinline__ void stage_update(const StageArgs &a, size_t o, size_t h, double kv, double y) {
-    S *const hist = reinterpret_cast<S *>(a.HIST);
-    if constexpr (MODE == RK1) {
-        stnt(a.ACC + o, y + kv * a.ca);
-        stnt(a.OUT + o, y + kv * a.cb);
-    } else if constexpr (MODE == RK2 || MODE == RK3) {
-        stnt(a.ACC + o, ldnt(a.ACC + o) + kv * a.ca);
-        stnt(a.OUT + o, ldnt(a.P0 + o) + kv * a.cb);
-    } else if constexpr (MODE == RK4S) {
-        stnt(a.OUT + o, ldnt(a.ACC + o) + kv * a.ca);
-    } else if constexpr (MODE == ABM) {
-        // the order-1 history loads are issued together (unrolled to the largest
-        // order, 5) before the sum, which keeps the order of the coefficients
-        stnt(hist + (size_t)a.slot_out * h + o, (S)kv);
-        double hv[5];
-#pragma unroll
-        for (int s = 1; s < 5; s++) hv[s] = (s < a.order) ? (double)ldnt(hist + (size_t)a.slots[s] * h + o) : 0.0;
-        double delta = a.coef[0] * kv;
-#pragma unroll
-        for (int s = 1; s < 5; s++)
-            if (s < a.order) delta += a.coef[s] * hv[s];
-        stnt(a.OUT + o, y + a.dt * delta);
-    } else if constexpr (MODE == RHSO) {
-        a.OUT[o] = kv;
-    } else {  // TAY
-        stnt(hist + (size_t)a.slot_out * h + o, (S)kv);
-        const int n = a.order - 1;
-        double dp[EDUS_MAX_ORDER];
-#pragma unroll
-        for (int i = 0; i < EDUS_MAX_ORDER - 1; i++) dp[i] = (i < n) ? kv - (double)ldnt(hist + (size_t)a.slots[i + 1] * h + o) : 0.0;
-        double delta = kv * a.dt;
-        for (int i = 1; i <= n; i++) {
-            double al = 0.0;
-            for (int p = 0; p < n; p++) al += a.tinv[(i - 1) * n + p] * dp[p];
-            delta += (a.dtp[i] * al) / (double)(i + 1);
-        }
-        stnt(a.OUT + o, y + delta);
-    }
-}
-
-// stage_update of the Adams-Bashforth mode for two adjacent packed elements
-// (o1 = o0 + 1 when vec): the same operations in the same order, with the
-// history and state accessed as pairs.  (The Taylor mode keeps the single form:
-// its runtime-order loops over two elements' differences cost 60 registers.)
+// ---------------------------------------------------------------- stage update (nb >= 5)
+// The Adams-Bashforth tail for two adjacent packed elements (o1 = o0 + 1 when vec),
+// history and state accessed as pairs; the order-1 history loads are issued
+// together before the sum, which keeps the order of the coefficients.  h: stride
+// between history slots.  S: storage type of the history (double, or float in the
+// mixed form with FP32 stage storage); the state and its update stay FP64.
 template <typename S>
 __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0, size_t o1, bool vec, size_t h, double kv0,
                                                   double kv1, double y0, double y1) {
@@ -318,7 +287,7 @@ __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0,
 
 // The Taylor tail for two adjacent packed elements: the history is read as
 // pairs, then each element's update is formed on its own (one set of
-// differences live at a time), in the operation order of stage_update.
+// differences live at a time).
 template <typename S>
 __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0, size_t o1, bool vec, size_t h, double kv0,
                                                   double kv1, double y0, double y1) {
@@ -353,87 +322,101 @@ __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0,
     st2(a.OUT, o0, o1, vec, out[0], out[1]);
 }
 
-// ================================================================ nb <= 4: thread per k
-// DISS: the context has dephasing terms (c.diss); without them the U sandwich
-// and its registers are compiled out.
-template <int NB, int MODE, bool DISS>
-__device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs &a, const int k) {
-    constexpr int NP = NB * NB;
-    if (k >= c.nk) return;
-    const size_t nkp = c.nkp;
-    const double *tab = stage_row(a);
-    const double Ep[3] = {tab[0], tab[1], tab[2]}, Eq[3] = {tab[3], tab[4], tab[5]};
-    const int nn = c.n_nbr;
-    const bool grad = nn > 0 && tab[6 + nn] != 0.0;
-    // The first stencil indices are requested with the state, so the gather at
-    // the end waits for one round trip, not two.
-    constexpr int kPreNbr = NB <= 3 ? 12 : 0;  // a multiple of the batch size below
-    int kpre[kPreNbr > 0 ? kPreNbr : 1];
-    if (grad) {
-#pragma unroll
-        for (int n = 0; n < kPreNbr; n++) kpre[n] = c.nbr[(size_t)min(n, nn - 1) * nkp + k];
-    }
+// ================================================================ nb <= 4: a lane per k and term
+// The right-hand side of a k is a sum of terms that only meet at the end: the
+// commutator, the dephasing sandwich and the field drift.
+// Each term of 64 k has a wave of its own (threadIdx.y: 0 the commutator, then the
+// dephasing if the context has it, then the drift); the terms meet in LDS, and the
+// waves share out the packed elements of the stage update, whose reads (accumulator,
+// base state, histories) are requested with everything else at the start.
+//
+// What bounds it: on small grids one wave's own instruction stream and the latency
+// of its dependent loads (a wave issues an FP64 instruction every 4 cycles, and 60 x
+// 60 k are 57 waves on 1024 SIMDs), on large ones the loads in flight.  Two or three
+// shorter streams side by side shorten both, and every term's registers leave room
+// for more of them.  RK4 stage, one lane doing all of a k's terms -> this form: 3 bands
+// 60 x 60 with dephasing 8.1 -> 4.8 us, 4 bands 251 x 307 34.2 -> 21.9; AB4 with the
+// mean field 300 x 300 23.4 -> 19.3.  Loads are plain: as non-temporal ones they took
+// the 4-band stage to 27.1 us (states of these grids stay in the Infinity Cache).
+// Six stencil rows in flight per wave instead of three took it to 25.9.
+//
+// DISS: the context has dephasing terms (c.diss).
+template <int NB, bool DISS>
+struct SmallGeom {
+    static constexpr int NP = NB * NB;
+    static constexpr int GW = NB <= 2 ? 1 : 2;       // waves of the drift, a part of the stencil each
+    static constexpr int R = 1 + (DISS ? 1 : 0) + GW;  // waves per 64 k
+    static constexpr int EPR = (NP + R - 1) / R;     // packed elements of the update per wave
+    static constexpr int GB = NB <= 2 ? 6 : 3;       // stencil rows in flight together
+};
+constexpr int kSmallMaxThreads = 512;
+// waves per SIMD that the registers have to allow
+template <int NB, bool DISS>
+constexpr int small_wpe() { return (NB <= 2 ? 5 : NB == 3 ? 4 : 3) - (DISS && NB > 2 ? 1 : 0); }
 
-    double y[NP], pre0[NP], pre1[NP];
-#pragma unroll
-    for (int e = 0; e < NP; e++) y[e] = a.Y[e * nkp + k];
-    // the RK stage tails' reads of the accumulator and the step's base state,
-    // requested with the stage input (up to 3 bands; at 4 the registers they
-    // take cost more occupancy than the early request gains)
-    constexpr bool kPreRK = NB <= 3;
-#pragma unroll
-    for (int e = 0; e < NP; e++) {
-        pre0[e] = pre1[e] = 0.0;
-        if constexpr (kPreRK && (MODE == RK2 || MODE == RK3)) {
-            pre0[e] = ldnt(a.ACC + e * nkp + k);
-            pre1[e] = ldnt(a.P0 + e * nkp + k);
-        } else if constexpr (kPreRK && MODE == RK4S) {
-            pre0[e] = ldnt(a.ACC + e * nkp + k);
-        }
-    }
-    cd P[NB][NB], M[NB][NB];
+// An element row of a SoA array at the lane's byte offset: the row address is
+// uniform, so the load needs no address arithmetic in vector registers.
+__device__ __forceinline__ double ldrow(const double *row, unsigned off) {
+    return *gm(reinterpret_cast<const double *>(reinterpret_cast<const char *>(row) + off));
+}
+__device__ __forceinline__ void strow_nt(double *row, unsigned off, double v) {
+    stnt(reinterpret_cast<double *>(reinterpret_cast<char *>(row) + off), v);
+}
+
+// Neighbour n of the lane's k.
+__device__ __forceinline__ int small_index(const ConstArgs &c, int n, unsigned ko) {
+    return *gm(reinterpret_cast<const int *>(reinterpret_cast<const char *>(c.nbr + (size_t)n * c.nkp) + ko / 2));
+}
+
+// Full P from its packed rows.
+template <int NB>
+__device__ __forceinline__ void small_state(const double *Y, size_t nkp, unsigned ko, cd (&P)[NB][NB]) {
 #pragma unroll
     for (int i = 0; i < NB; i++) {
-        P[i][i] = mk(y[i], 0.0);
+        P[i][i] = mk(ldrow(Y + i * nkp, ko), 0.0);
 #pragma unroll
         for (int j = i + 1; j < NB; j++) {
-            const int p = pair_index(i, j, NB);
-            P[i][j] = mk(y[NB + 2 * p], y[NB + 2 * p + 1]);
+            const int p = NB + 2 * pair_index(i, j, NB);
+            P[i][j] = mk(ldrow(Y + p * nkp, ko), ldrow(Y + (p + 1) * nkp, ko));
             P[j][i] = cconj(P[i][j]);
         }
     }
-    // M = H + E.D with the probe on core<->non-core elements (RungeKutta.h:165-168).
+}
+
+// -i[M, rho] in the transposed storage with M = H + E.D, the probe on core<->non-core
+// elements, and the RWA term (RungeKutta.h:158-212), packed.
+template <int NB>
+__device__ __forceinline__ void small_commutator(const ConstArgs &c, const StageArgs &a, TabRow tab, unsigned ko,
+                                                 double (&pv)[NB * NB]) {
+    constexpr int NP = NB * NB;
+    const size_t nkp = c.nkp;
+    const double Ep[3] = {tab[0], tab[1], tab[2]}, Eq[3] = {tab[3], tab[4], tab[5]};
+    cd P[NB][NB], M[NB][NB];
+    small_state<NB>(a.Y, nkp, ko, P);
 #pragma unroll
-    for (int i = 0; i < NB; i++) {
+    for (int i = 0; i < NB; i++)
 #pragma unroll
         for (int j = i; j < NB; j++) {
-            const bool w = (i >= c.nch && j < c.nch) || (i < c.nch && j >= c.nch);
-            const double E[3] = {w ? Eq[0] : Ep[0], w ? Eq[1] : Ep[1], w ? Eq[2] : Ep[2]};
-            cd h, dx[3];
-            if (i == j) {
-                h = mk(ldnt(c.H + i * nkp + k), 0.0);
-#pragma unroll
-                for (int x = 0; x < 3; x++) dx[x] = (a.dmask >> x & 1) ? mk(ldnt(c.D + (x * NP + i) * nkp + k), 0.0) : mk(0.0, 0.0);
-            } else {
-                const int p = pair_index(i, j, NB);
-                h = mk(ldnt(c.H + (NB + 2 * p) * nkp + k), ldnt(c.H + (NB + 2 * p + 1) * nkp + k));
-#pragma unroll
-                for (int x = 0; x < 3; x++)
-                    dx[x] = (a.dmask >> x & 1) ? mk(ldnt(c.D + (x * NP + NB + 2 * p) * nkp + k), ldnt(c.D + (x * NP + NB + 2 * p + 1) * nkp + k))
-                                               : mk(0.0, 0.0);
-            }
-            cd mij = h, mji = cconj(h);
-#pragma unroll
-            for (int x = 0; x < 3; x++) {
-                mij = cadd(mij, cscale(dx[x], E[x]));
-                mji = cadd(mji, cscale(c.dherm ? cconj(dx[x]) : dx[x], E[x]));
-            }
-            M[i][j] = mij;
-            M[j][i] = mji;
+            const int p = i == j ? i : NB + 2 * pair_index(i, j, NB);
+            M[i][j] = mk(ldrow(c.H + p * nkp, ko), i == j ? 0.0 : ldrow(c.H + (p + 1) * nkp, ko));
+            if (i != j) M[j][i] = cconj(M[i][j]);
         }
-    }
-    // -i[M, rho] in the transposed storage (RungeKutta.h:158-212).
-    double pv[NP];
+#pragma unroll
+    for (int x = 0; x < 3; x++)
+        if (a.dmask >> x & 1) {
+#pragma unroll
+            for (int i = 0; i < NB; i++)
+#pragma unroll
+                for (int j = i; j < NB; j++) {
+                    const bool w = (i >= c.nch && j < c.nch) || (i < c.nch && j >= c.nch);
+                    const double E = w ? Eq[x] : Ep[x];
+                    const int p = i == j ? i : NB + 2 * pair_index(i, j, NB);
+                    const double *row = c.D + (size_t)(x * NP + p) * nkp;
+                    const cd d = mk(ldrow(row, ko), i == j ? 0.0 : ldrow(row + nkp, ko));
+                    M[i][j] = cadd(M[i][j], cscale(d, E));
+                    if (i != j) M[j][i] = cadd(M[j][i], cscale(c.dherm ? cconj(d) : d, E));
+                }
+        }
 #pragma unroll
     for (int i = 0; i < NB; i++) {
         cd beta = mk(0.0, 0.0);
@@ -454,115 +437,226 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
             pv[NB + 2 * p] = v.x;
             pv[NB + 2 * p + 1] = v.y;
         }
-    // Dephasing in the eigenbasis (RungeKutta.h:219-254) as
-    // Pv -= conj(U) (T o (conj(U) P U^T)) conj(U) plus the hole source.
-    if constexpr (DISS) {
-        cd U[NB][NB];
-        const double *u = c.U + (size_t)k * NB * NB * 2;
+}
+
+// Dephasing in the eigenbasis (RungeKutta.h:219-254): the hole source minus
+// conj(U) (T o (conj(U) P U^T)) conj(U), packed.
+template <int NB>
+__device__ __forceinline__ void small_dephasing(const ConstArgs &c, const double *Y, unsigned ko, double (&pv)[NB * NB]) {
+    cd P[NB][NB], U[NB][NB];
+    const double *u = c.U + (size_t)(ko / 8) * NB * NB * 2;
 #pragma unroll
-        for (int i = 0; i < NB; i++)
+    for (int i = 0; i < NB; i++)
 #pragma unroll
-            for (int j = 0; j < NB; j++) {  // one 16-byte load per complex entry (the k's U is 16-byte aligned)
-                double re, im;
-                ld2<true>(u, (i * NB + j) * 2, (i * NB + j) * 2 + 1, true, re, im);
-                U[i][j] = mk(re, im);
-            }
-        cd G[NB][NB];
-#pragma unroll
-        for (int ia = 0; ia < NB; ia++)
-#pragma unroll
-            for (int ib = 0; ib < NB; ib++) {
-                cd g = mk(0.0, 0.0);
-#pragma unroll
-                for (int i = 0; i < NB; i++) {
-                    cd t = mk(0.0, 0.0);
-#pragma unroll
-                    for (int j = 0; j < NB; j++) t = cadd(t, cmul(U[ib][j], P[i][j]));
-                    g = cadd(g, cmul(cconj(U[ia][i]), t));
-                }
-                G[ia][ib] = cscale(g, c.T[ia * NB + ib]);
-            }
-#pragma unroll
-        for (int i = 0; i < NB; i++)
-#pragma unroll
-            for (int j = i; j < NB; j++) {
-                cd w = mk(0.0, 0.0);
-#pragma unroll
-                for (int ia = 0; ia < NB; ia++) {
-                    cd t = mk(0.0, 0.0);
-#pragma unroll
-                    for (int ib = 0; ib < NB; ib++) t = cadd(t, cmul(G[ia][ib], cconj(U[ib][j])));
-                    w = cadd(w, cmul(cconj(U[i][ia]), t));
-                }
-                cd hole = mk(0.0, 0.0);
-#pragma unroll
-                for (int v = 0; v < NB; v++)  // static indices keep U in registers
-                    if (v < c.ncc) hole = cadd(hole, cscale(cmul(cconj(U[v][j]), U[v][i]), c.T[v * NB + v]));
-                if (i == j) {
-                    pv[i] = pv[i] - w.x + hole.x;
-                } else {
-                    const int p = pair_index(i, j, NB);
-                    pv[NB + 2 * p] = pv[NB + 2 * p] - w.x + hole.x;
-                    pv[NB + 2 * p + 1] = pv[NB + 2 * p + 1] - w.y + hole.y;
-                }
-            }
-    }
-    // Field drift E.grad_k rho on the shell stencil (RungeKutta.h:258-276).  The
-    // neighbour indices were requested at the start; the rows come GB neighbours
-    // at a time, all in flight together, and the sum keeps the stencil order.
-    if (grad) {
-        constexpr int GB = NB <= 2 ? 6 : NB == 3 ? 4 : 2;
-        double g[NP];
-#pragma unroll
-        for (int e = 0; e < NP; e++) g[e] = 0.0;
-        auto batch = [&](int n0, const int (&kk)[GB]) {
-            double v[GB][NP];
-#pragma unroll
-            for (int j = 0; j < GB; j++)
-#pragma unroll
-                for (int e = 0; e < NP; e++) v[j][e] = a.Y[e * nkp + kk[j]];
-#pragma unroll
-            for (int j = 0; j < GB; j++)
-                if (n0 + j < nn) {
-                    const double cn = tab[6 + n0 + j];
-#pragma unroll
-                    for (int e = 0; e < NP; e++) g[e] += cn * v[j][e];
-                }
-        };
-#pragma unroll
-        for (int n0 = 0; n0 < kPreNbr; n0 += GB) {
-            if (n0 >= nn) break;
-            int kk[GB];
-#pragma unroll
-            for (int j = 0; j < GB; j++) kk[j] = kpre[n0 + j];
-            batch(n0, kk);
+        for (int j = 0; j < NB; j++) {  // one 16-byte load per complex entry (the k's U is 16-byte aligned)
+            double re, im;
+            ld2<true>(u, (i * NB + j) * 2, (i * NB + j) * 2 + 1, true, re, im);
+            U[i][j] = mk(re, im);
         }
-        for (int n0 = kPreNbr; n0 < nn; n0 += GB) {
-            int kk[GB];
+    small_state<NB>(Y, c.nkp, ko, P);
+    cd G[NB][NB];
 #pragma unroll
-            for (int j = 0; j < GB; j++) kk[j] = c.nbr[(size_t)min(n0 + j, nn - 1) * nkp + k];
-            batch(n0, kk);
+    for (int ib = 0; ib < NB; ib++) {
+        cd t[NB];
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            t[i] = mk(0.0, 0.0);
+#pragma unroll
+            for (int j = 0; j < NB; j++) t[i] = cadd(t[i], cmul(U[ib][j], P[i][j]));
         }
 #pragma unroll
-        for (int e = 0; e < NP; e++) pv[e] += g[e];
+        for (int ia = 0; ia < NB; ia++) {
+            cd g = mk(0.0, 0.0);
+#pragma unroll
+            for (int i = 0; i < NB; i++) g = cadd(g, cmul(cconj(U[ia][i]), t[i]));
+            G[ia][ib] = cscale(g, *gm(c.T + ia * NB + ib));
+        }
     }
 #pragma unroll
-    for (int e = 0; e < NP; e++) {
-        const size_t o = e * nkp + k;
-        if constexpr (kPreRK && (MODE == RK2 || MODE == RK3)) {
-            stnt(a.ACC + o, pre0[e] + pv[e] * a.ca);
-            stnt(a.OUT + o, pre1[e] + pv[e] * a.cb);
-        } else if constexpr (kPreRK && MODE == RK4S) {
-            stnt(a.OUT + o, pre0[e] + pv[e] * a.ca);
-        } else {
-            stage_update<MODE>(a, o, (size_t)NP * nkp, pv[e], y[e]);
+    for (int j = 0; j < NB; j++) {
+        cd t[NB];
+#pragma unroll
+        for (int ia = 0; ia < NB; ia++) {
+            t[ia] = mk(0.0, 0.0);
+#pragma unroll
+            for (int ib = 0; ib < NB; ib++) t[ia] = cadd(t[ia], cmul(G[ia][ib], cconj(U[ib][j])));
+        }
+#pragma unroll
+        for (int i = 0; i <= j; i++) {
+            cd w = mk(0.0, 0.0);
+#pragma unroll
+            for (int ia = 0; ia < NB; ia++) w = cadd(w, cmul(cconj(U[i][ia]), t[ia]));
+            cd hole = mk(0.0, 0.0);
+#pragma unroll
+            for (int v = 0; v < NB; v++)  // static indices keep U in registers
+                if (v < c.ncc) hole = cadd(hole, cscale(cmul(cconj(U[v][j]), U[v][i]), *gm(c.T + v * NB + v)));
+            if (i == j) {
+                pv[i] = hole.x - w.x;
+            } else {
+                const int p = pair_index(i, j, NB);
+                pv[NB + 2 * p] = hole.x - w.x;
+                pv[NB + 2 * p + 1] = hole.y - w.y;
+            }
         }
     }
 }
 
+// Field drift E.grad_k rho on the shell stencil (RungeKutta.h:258-276): the rows of
+// neighbours n0..n1-1, GB at a time, all in flight; the sum keeps the stencil order.
+// The first NPRE indices (`pre`) are requested by the caller.
+template <int NB, int GB, int NPRE>
+__device__ __forceinline__ void small_drift(const ConstArgs &c, const double *Y, TabRow tab, unsigned ko, int n0, int n1,
+                                            const int (&pre)[NPRE], double (&g)[NB * NB]) {
+    constexpr int NP = NB * NB;
+    static_assert(NPRE % GB == 0, "whole batches of requested indices");
+    const size_t nkp = c.nkp;
+    auto batch = [&](int n, const unsigned (&off)[GB]) {
+        double v[GB][NP];
+#pragma unroll
+        for (int j = 0; j < GB; j++)
+#pragma unroll
+            for (int e = 0; e < NP; e++) v[j][e] = ldrow(Y + e * nkp, off[j]);
+#pragma unroll
+        for (int j = 0; j < GB; j++)
+            if (n + j < n1) {
+                const double cn = tab[6 + n + j];
+#pragma unroll
+                for (int e = 0; e < NP; e++) g[e] += cn * v[j][e];
+            }
+    };
+#pragma unroll
+    for (int e = 0; e < NP; e++) g[e] = 0.0;
+#pragma unroll
+    for (int q = 0; q < NPRE; q += GB) {
+        if (n0 + q >= n1) break;
+        unsigned off[GB];
+#pragma unroll
+        for (int j = 0; j < GB; j++) off[j] = 8u * (unsigned)pre[q + j];
+        batch(n0 + q, off);
+    }
+    for (int n = n0 + NPRE; n < n1; n += GB) {
+        unsigned off[GB];
+#pragma unroll
+        for (int j = 0; j < GB; j++) off[j] = 8u * (unsigned)small_index(c, min(n + j, n1 - 1), ko);
+        batch(n, off);
+    }
+}
+
+// What the update of a packed element reads besides the right-hand side.
+template <int MODE>
+struct SmallTail {
+    static constexpr int NH = MODE == ABM ? 4 : MODE == TAY ? EDUS_MAX_ORDER - 1 : 0;
+    double y, p0, p1, h[NH > 0 ? NH : 1];
+};
+
+template <int MODE>
+__device__ __forceinline__ void small_tail_load(const StageArgs &a, size_t row, size_t hstride, unsigned ko, SmallTail<MODE> &t) {
+    t.y = t.p0 = t.p1 = 0.0;
+    if constexpr (MODE == RK1 || MODE == ABM || MODE == TAY) t.y = ldrow(a.Y + row, ko);
+    if constexpr (MODE == RK2 || MODE == RK3 || MODE == RK4S) t.p0 = ldrow(a.ACC + row, ko);
+    if constexpr (MODE == RK2 || MODE == RK3) t.p1 = ldrow(a.P0 + row, ko);
+#pragma unroll
+    for (int s = 0; s < SmallTail<MODE>::NH; s++)
+        t.h[s] = s + 1 < a.order ? ldrow(a.HIST + (size_t)a.slots[s + 1] * hstride + row, ko) : 0.0;
+}
+
+template <int MODE>
+__device__ __forceinline__ void small_tail_store(const StageArgs &a, size_t row, size_t hstride, unsigned ko, double kv, const SmallTail<MODE> &t) {
+    if constexpr (MODE == RK1) {
+        strow_nt(a.ACC + row, ko, t.y + kv * a.ca);
+        strow_nt(a.OUT + row, ko, t.y + kv * a.cb);
+    } else if constexpr (MODE == RK2 || MODE == RK3) {
+        strow_nt(a.ACC + row, ko, t.p0 + kv * a.ca);
+        strow_nt(a.OUT + row, ko, t.p1 + kv * a.cb);
+    } else if constexpr (MODE == RK4S) {
+        strow_nt(a.OUT + row, ko, t.p0 + kv * a.ca);
+    } else if constexpr (MODE == ABM) {
+        strow_nt(a.HIST + (size_t)a.slot_out * hstride + row, ko, kv);
+        double delta = a.coef[0] * kv;
+#pragma unroll
+        for (int s = 1; s < 5; s++)
+            if (s < a.order) delta += a.coef[s] * t.h[s - 1];
+        strow_nt(a.OUT + row, ko, t.y + a.dt * delta);
+    } else if constexpr (MODE == TAY) {
+        strow_nt(a.HIST + (size_t)a.slot_out * hstride + row, ko, kv);
+        const int n = a.order - 1;
+        double dp[EDUS_MAX_ORDER];
+#pragma unroll
+        for (int i = 0; i < EDUS_MAX_ORDER - 1; i++) dp[i] = (i < n) ? kv - t.h[i] : 0.0;
+        double delta = kv * a.dt;
+        for (int i = 1; i <= n; i++) {
+            double al = 0.0;
+#pragma unroll
+            for (int p = 0; p < EDUS_MAX_ORDER - 1; p++)
+                if (p < n) al += a.tinv[(i - 1) * n + p] * dp[p];
+            delta += (a.dtp[i] * al) / (double)(i + 1);
+        }
+        strow_nt(a.OUT + row, ko, t.y + delta);
+    } else {
+        strow_nt(a.OUT + row, ko, kv);
+    }
+}
+
+// kk: the lane's k (past the grid: clamped, nothing stored); lk, tk: its place among
+// the workgroup's tk k; term: threadIdx.y, uniform in a wave; lds: [R][NP][tk].
 template <int NB, int MODE, bool DISS>
-__global__ __launch_bounds__(256) void k_stage_small(ConstArgs c, StageArgs a) {
-    stage_small<NB, MODE, DISS>(c, a, xcd_block() * blockDim.x + threadIdx.x);
+__device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs &a, const int kk, const int lk, const int tk, const int term,
+                                            double *lds) {
+    using G = SmallGeom<NB, DISS>;
+    constexpr int NP = G::NP, R = G::R, EPR = G::EPR;
+    const bool store = kk < c.nk;
+    const unsigned ko = 8u * (unsigned)min(kk, c.nk - 1);
+    const size_t nkp = c.nkp;
+    const TabRow tab = stage_row(a);
+    const int nn = c.n_nbr;
+    SmallTail<MODE> tail[EPR];
+#pragma unroll
+    for (int m = 0; m < EPR; m++)
+        if (term + R * m < NP) small_tail_load<MODE>(a, (size_t)(term + R * m) * nkp, NP * nkp, ko, tail[m]);
+    double pv[NP];
+    if (term == 0) small_commutator<NB>(c, a, tab, ko, pv);
+    else if (DISS && term == 1) small_dephasing<NB>(c, a.Y, ko, pv);
+    else if (nn > 0) {
+        // this wave's part of the stencil; its indices come with the field row, not
+        // after the row has told whether the drift is on
+        constexpr int NPRE = 12 / G::GW;
+        const int q = term - (R - G::GW), n0 = nn * q / G::GW, n1 = nn * (q + 1) / G::GW;
+        int pre[NPRE];
+#pragma unroll
+        for (int n = 0; n < NPRE; n++) pre[n] = small_index(c, min(n0 + n, nn - 1), ko);
+        if (tab[6 + nn] != 0.0) {
+            small_drift<NB, G::GB, NPRE>(c, a.Y, tab, ko, n0, n1, pre, pv);
+        } else {
+#pragma unroll
+            for (int e = 0; e < NP; e++) pv[e] = 0.0;
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < NP; e++) pv[e] = 0.0;
+    }
+#pragma unroll
+    for (int e = 0; e < NP; e++) lds[(term * NP + e) * tk + lk] = pv[e];
+    __syncthreads();
+    if (!store) return;
+#pragma unroll
+    for (int m = 0; m < EPR; m++) {
+        const int e = term + R * m;
+        if (e < NP) {
+            double kv = lds[e * tk + lk], g = lds[((R - G::GW) * NP + e) * tk + lk];
+            if constexpr (DISS) kv += lds[(NP + e) * tk + lk];
+            if constexpr (G::GW == 2) g += lds[((R - 1) * NP + e) * tk + lk];
+            kv += g;
+            small_tail_store<MODE>(a, (size_t)e * nkp, NP * nkp, ko, kv, tail[m]);
+        }
+    }
+}
+
+// blockDim = (k per workgroup, SmallGeom::R)
+template <int NB, int MODE, bool DISS>
+__global__ __launch_bounds__(kSmallMaxThreads, (small_wpe<NB, DISS>())) void k_stage_small(ConstArgs c, StageArgs a) {
+    extern __shared__ double smem_d[];
+    const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    stage_small<NB, MODE, DISS>(c, a, xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
 }
 
 // ================================================================ Coulomb mean field
@@ -1248,7 +1342,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     const R *Hop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.H : (const void *)c.Hf);
     const R *Dop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.D : (const void *)c.Df);
     const R *Uop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.U : (const void *)c.Uf);
-    const double *tab = stage_row(a);
+    const TabRow tab = stage_row(a);
     const R Ep[3] = {(R)tab[0], (R)tab[1], (R)tab[2]}, Eq[3] = {(R)tab[3], (R)tab[4], (R)tab[5]};
     const int nn = c.n_nbr;
     const bool grad = tab[6 + nn] != 0.0;
@@ -1274,7 +1368,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     for (int m = 0; m < PER; m++) {
         const int e = kPairs ? min(2 * (lane + TPK * (m >> 1)) + (m & 1), NP - 1) : min(lane + TPK * m, NP - 1);
         eo[m] = e;
-        const int code = c.eidx[e];
+        const int code = *gm(c.eidx + e);
         ei[m] = code & 255;
         ej[m] = (code >> 8) & 255;
         ec[m] = code >> 16;
@@ -1290,7 +1384,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         constexpr int NV = std::extent<std::remove_reference_t<decltype(v)>>::value;
         size_t kn[NV];
 #pragma unroll
-        for (int j = 0; j < NV; j++) kn[j] = (size_t)c.nbr[(size_t)slot(min(j, cnt - 1)) * c.nkp + kk] * NP;
+        for (int j = 0; j < NV; j++) kn[j] = (size_t)*gm(c.nbr + (size_t)slot(min(j, cnt - 1)) * c.nkp + kk) * NP;
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             if constexpr (kPairs) {
@@ -1366,7 +1460,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
                     for (int m = 0; m < PER; m++) g[m] += cn * v[j][m];
                     if constexpr (ROLE == 1) {
-                        const int pj = c.pat[n0 + j];
+                        const int pj = gm(c.pat)[n0 + j];
                         if (pj >= 0) {
                             const double cb = tab[6 + pj];
 #pragma unroll
@@ -1385,11 +1479,11 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             constexpr int GBN = GB < 5 ? 5 : GB;
             for (int t0 = 0; t0 < c.npnew; t0 += GBN) {
                 double v[GBN][PER];
-                gather(kb, [&](int j) { return c.pat[kMaxNbr + t0 + j]; }, c.npnew - t0, v);
+                gather(kb, [&](int j) { return gm(c.pat)[kMaxNbr + t0 + j]; }, c.npnew - t0, v);
 #pragma unroll
                 for (int j = 0; j < GBN; j++)
                     if (t0 + j < c.npnew) {
-                        const double cb = tab[6 + c.pat[kMaxNbr + t0 + j]];
+                        const double cb = tab[6 + gm(c.pat)[kMaxNbr + t0 + j]];
 #pragma unroll
                         for (int m = 0; m < PER; m++) gb[m] += cb * v[j][m];
                     }
@@ -1502,7 +1596,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             for (int i = 0; i < 4; i++) {
                 int ia, ib;
                 mfma_elem<NBT, R>(lane, i, ia, ib);
-                const R t = (ia < nb && ib < nb) ? (R)c.T[ia * nb + ib] : (R)0;
+                const R t = (ia < nb && ib < nb) ? (R)*gm(c.T + ia * nb + ib) : (R)0;
                 cre[i] *= t;
                 cim[i] *= t;
             }
@@ -1532,7 +1626,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     #pragma unroll
                     for (int j = 0; j < RBC; j++) {
                         const int ia = r0 + i * GR, ib = c0 + j * GC;
-                        const R t = (ia < nb && ib < nb) ? (R)c.T[ia * nb + ib] : (R)0;
+                        const R t = (ia < nb && ib < nb) ? (R)*gm(c.T + ia * nb + ib) : (R)0;
                         acc[i][j] = CT{acc[i][j].x * t, acc[i][j].y * t};
                     }
             }
@@ -1556,7 +1650,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             CT hole = CT{0, 0};
             for (int v = 0; v < c.ncc; v++) {
                 const CT uj = C[v * LD + j], ui = C[v * LD + i];
-                const R tv = (R)c.T[v * nb + v];
+                const R tv = (R)*gm(c.T + v * nb + v);
                 // conj(U[v][j]) U[v][i] T[v][v]
                 hole.x += (uj.x * ui.x + uj.y * ui.y) * tv;
                 hole.y += (uj.x * ui.y - uj.y * ui.x) * tv;
@@ -1570,45 +1664,28 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         }
     }
     if (!store) return;  // after the last barrier (a group past the grid serves no pair)
-    if constexpr (kPairs && MODE != RHSO) {
-        S *const outs = reinterpret_cast<S *>(a.OUT);  // RK stages 1-3 write the next stage input
+    static_assert(kPairs, "a lane owns pairs of packed elements");
+    S *const outs = reinterpret_cast<S *>(a.OUT);  // RK stages 1-3 write the next stage input
 #pragma unroll
-        for (int h = 0; h < PER / 2; h++) {
-            const int m = 2 * h;
-            const double k0 = pv[m] + g[m], k1 = pv[m + 1] + g[m + 1];
-            const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-            const bool v2 = pv2[h];
-            if constexpr (MODE == ABM) {
-                stage_update2_abm<S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
-            } else if constexpr (MODE == TAY) {
-                stage_update2_tay<S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
-            } else if constexpr (MODE == RK1) {
-                st2(a.ACC, o0, o1, v2, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
-                st2(outs, o0, o1, v2, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
-            } else if constexpr (MODE == RK2 || MODE == RK3) {
-                st2(a.ACC, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
-                st2(outs, o0, o1, v2, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
-            } else {
-                st2(a.OUT, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int m = 0; m < PER; m++) {
-        const double kv = pv[m] + g[m];
-        const size_t o = base + eo[m];
-        S *const outs = reinterpret_cast<S *>(a.OUT);  // RK stages 1-3 write the next stage input
-        if constexpr (MODE == RK1) {
-            stnt(a.ACC + o, y[m] + kv * a.ca);
-            stnt(outs + o, (S)(y[m] + kv * a.cb));
+    for (int h = 0; h < PER / 2; h++) {
+        const int m = 2 * h;
+        const double k0 = pv[m] + g[m], k1 = pv[m + 1] + g[m + 1];
+        const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
+        const bool v2 = pv2[h];
+        if constexpr (MODE == ABM) {
+            stage_update2_abm<S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+        } else if constexpr (MODE == TAY) {
+            stage_update2_tay<S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+        } else if constexpr (MODE == RK1) {
+            st2(a.ACC, o0, o1, v2, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
+            st2(outs, o0, o1, v2, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK2 || MODE == RK3) {
-            stnt(a.ACC + o, pre0[m] + kv * a.ca);
-            stnt(outs + o, (S)(pre1[m] + kv * a.cb));
+            st2(a.ACC, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2(outs, o0, o1, v2, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK4S) {
-            stnt(a.OUT + o, pre0[m] + kv * a.ca);
+            st2(a.OUT, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
         } else {
-            stage_update<MODE, S>(a, o, (size_t)c.nk * NP, kv, y[m]);
+            st2(a.OUT, o0, o1, v2, k0, k1);
         }
     }
 }
@@ -1649,9 +1726,8 @@ __global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB) void k_sta
 // table, and every instance's arguments sit in a device array.  The stage body
 // is the single-problem kernel's, so a batched step is bit-identical to
 // stepping each problem on its own.
-// Threads per workgroup of the batched small kernel: an instance of a few
-// thousand k then spreads over more CUs (the k past nk, up to the padded nkp,
-// are computed and never read).
+// k per workgroup of the batched small kernel: an instance of a few thousand k
+// then spreads over more CUs.
 constexpr int kSmallBatchThreads = 64;
 
 struct BatchEntry {
@@ -1663,13 +1739,15 @@ template <int MODE>
 __host__ __device__ constexpr int rk4_stage_of() { return MODE == RK1 ? 0 : MODE == RK2 ? 1 : MODE == RK3 ? 2 : 3; }
 
 template <int NB, int MODE, bool DISS>
-__global__ __launch_bounds__(256) void k_stage_small_batch(const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
+__global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) void k_stage_small_batch(const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
+    extern __shared__ double smem_d[];
+    const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int2 w = blk[xcd_block()];
     const BatchEntry &be = E[w.x];
     StageArgs a = be.a[rk4_stage_of<MODE>()];
     a.tab += tab_step;
     a.dmask = dmask[w.x];
-    stage_small<NB, MODE, DISS>(be.c, a, w.y * blockDim.x + threadIdx.x);
+    stage_small<NB, MODE, DISS>(be.c, a, w.y * kSmallBatchThreads + threadIdx.x, threadIdx.x, kSmallBatchThreads, term, smem_d);
 }
 
 template <int NBT, int MODE, typename R, bool PAIR = false>
@@ -2811,7 +2889,7 @@ struct edus_ctx {
     int nk = 0, nkp = 0, nb = 0, np = 0, nch = 0, ncc = 0, n_nbr = 0, stepper = 0, order = 1, diss = 0, dherm = 0;
     int sw = 0, scol = 0;  // strip order of the wave kernels (strip_k)
     int pair = 0, pself = -1, npnew = 0;  // stencil pairs of the wave kernels (ConstArgs::pair)
-    int tpb = 0;           // threads per workgroup of the nb <= 4 kernel (0: by grid size)
+    int tpb = 0;           // k per workgroup of the nb <= 4 kernel (0: small_group's choice)
     int precision = EDUS_PRECISION_FP64;
     float *Hf = nullptr, *Df = nullptr, *Uf = nullptr;  // FP32 operator copies (mixed precision)
     int *eidx = nullptr;  // packed element -> (i, j, comp) of the wave layout
@@ -3051,6 +3129,9 @@ ConstArgs const_args(const edus_ctx *c) {
     return ca;
 }
 
+// k per workgroup of the nb <= 4 kernel: 64 unless edus_autotune picked another.
+int small_group(const edus_ctx *c) { return c->tpb ? c->tpb : 64; }
+
 template <int MODE>
 int launch_stage(edus_ctx *c, StageArgs a) {
     a.dmask = c->dmask;
@@ -3060,17 +3141,19 @@ int launch_stage(edus_ctx *c, StageArgs a) {
         if (rc) return rc;
     }
     if (c->soa) {
-        // A grid of fewer k than 256 per CU runs 64-thread workgroups, so that
-        // more CUs share it (the k past nk, up to the padded nkp, are computed
-        // and never read).
-        const int tpb = c->tpb ? c->tpb : (c->nk < 256 * 256 ? 64 : 256), blocks = (c->nk + tpb - 1) / tpb;
+        const int tpb = small_group(c), blocks = (c->nk + tpb - 1) / tpb;
         auto go = [&](auto dtag) {
             constexpr bool DISS = decltype(dtag)::value;
+            auto nbgo = [&](auto ntag) {
+                constexpr int NB = decltype(ntag)::value, R = SmallGeom<NB, DISS>::R;
+                hipLaunchKernelGGL((k_stage_small<NB, MODE, DISS>), dim3(blocks), dim3(tpb, R), (size_t)R * NB * NB * tpb * sizeof(double),
+                                   c->stream, ca, a);
+            };
             switch (c->nb) {
-                case 1: hipLaunchKernelGGL((k_stage_small<1, MODE, DISS>), dim3(blocks), dim3(tpb), 0, c->stream, ca, a); break;
-                case 2: hipLaunchKernelGGL((k_stage_small<2, MODE, DISS>), dim3(blocks), dim3(tpb), 0, c->stream, ca, a); break;
-                case 3: hipLaunchKernelGGL((k_stage_small<3, MODE, DISS>), dim3(blocks), dim3(tpb), 0, c->stream, ca, a); break;
-                default: hipLaunchKernelGGL((k_stage_small<4, MODE, DISS>), dim3(blocks), dim3(tpb), 0, c->stream, ca, a); break;
+                case 1: nbgo(std::integral_constant<int, 1>{}); break;
+                case 2: nbgo(std::integral_constant<int, 2>{}); break;
+                case 3: nbgo(std::integral_constant<int, 3>{}); break;
+                default: nbgo(std::integral_constant<int, 4>{}); break;
             }
         };
         if (c->nb < 1 || c->nb > 4) return set_err(EDUS_ERR_UNSUPPORTED, "no small kernel for this band count");
@@ -3923,7 +4006,8 @@ int edus_autotune(edus_ctx *c, const double *field6, uint8_t grad_on, int32_t re
     a.OUT = c->YB;  // scratch between steps: the state is not touched
     std::vector<int> cand;
     if (c->soa) {
-        cand = {64, 128, 256};
+        cand = {64, 128};
+        if (c->nb <= 2 && !c->diss) cand.push_back(256);  // with more terms 128 k fill kSmallMaxThreads
     } else {
         cand.push_back(0);
         if (c->scol > 0)
@@ -3965,7 +4049,7 @@ int edus_launch_schedule(edus_ctx *c, int32_t *out) {
     out[1] = c->sw;
     out[2] = c->pair;
     out[3] = c->pair ? c->npnew : 0;
-    out[4] = c->soa ? (c->tpb ? c->tpb : (c->nk < 256 * 256 ? 64 : 256)) : 0;
+    out[4] = c->soa ? small_group(c) : 0;
     return 0;
 }
 
@@ -4029,11 +4113,16 @@ int batch_launch(edus_batch *b, const edus_batch::Cls &k, size_t tab_step) {
     if (k.soa) {
         auto go = [&](auto dtag) {
             constexpr bool DISS = decltype(dtag)::value;
+            auto nbgo = [&](auto ntag) {
+                constexpr int NB = decltype(ntag)::value, R = SmallGeom<NB, DISS>::R;
+                hipLaunchKernelGGL((k_stage_small_batch<NB, MODE, DISS>), grid, dim3(kSmallBatchThreads, R),
+                                   (size_t)R * NB * NB * kSmallBatchThreads * sizeof(double), b->stream, b->entries, k.blk, b->masks, tab_step);
+            };
             switch (k.nb_small) {
-                case 1: hipLaunchKernelGGL((k_stage_small_batch<1, MODE, DISS>), grid, dim3(kSmallBatchThreads), 0, b->stream, b->entries, k.blk, b->masks, tab_step); break;
-                case 2: hipLaunchKernelGGL((k_stage_small_batch<2, MODE, DISS>), grid, dim3(kSmallBatchThreads), 0, b->stream, b->entries, k.blk, b->masks, tab_step); break;
-                case 3: hipLaunchKernelGGL((k_stage_small_batch<3, MODE, DISS>), grid, dim3(kSmallBatchThreads), 0, b->stream, b->entries, k.blk, b->masks, tab_step); break;
-                default: hipLaunchKernelGGL((k_stage_small_batch<4, MODE, DISS>), grid, dim3(kSmallBatchThreads), 0, b->stream, b->entries, k.blk, b->masks, tab_step); break;
+                case 1: nbgo(std::integral_constant<int, 1>{}); break;
+                case 2: nbgo(std::integral_constant<int, 2>{}); break;
+                case 3: nbgo(std::integral_constant<int, 3>{}); break;
+                default: nbgo(std::integral_constant<int, 4>{}); break;
             }
         };
         if (k.diss) go(std::true_type{});

@@ -215,14 +215,14 @@ int edus_last_step_time(edus_ctx *ctx, double *ms, int32_t *nlaunch);
  * stencil pair of k (2q, 2q + 1: every pair's 12-point stencils overlap alike,
  * as on a uniform grid; the BF16x3 form and the FP32-storage Taylor step at 32
  * bands still run one k per workgroup), the stencil rows the second k of a pair
- * fetches itself, and the threads per workgroup of the thread-per-k kernel.  No
- * reference counterpart (a launch diagnostic). */
+ * fetches itself, and the k per workgroup of the 1..4-band kernel (a thread per k
+ * for each of its terms).  No reference counterpart (a launch diagnostic). */
 int edus_launch_schedule(edus_ctx *ctx, int32_t *out);
 
 /* Picks the stage kernels' launch schedule by measurement on the context's own
  * data and keeps it for every later launch: for 5..32 bands the strip width of
  * the workgroup walk over the grid (0 = k order, or 16..256 columns narrower than
- * a grid row), for 1..4 bands the threads per workgroup (64, 128, 256).  Each
+ * a grid row), for 1..4 bands the k per workgroup (64, 128, 256).  Each
  * candidate runs `reps` right-hand-side launches with the field `field6` (as for
  * edus_rhs) into scratch memory; the state and the step results are unaffected
  * (every candidate forms the same sums for every k).  `chosen` (may be NULL)
