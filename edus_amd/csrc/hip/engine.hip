@@ -213,7 +213,10 @@ __host__ __device__ __forceinline__ int pair_index(int i, int j, int nb) { retur
 
 // Streaming accesses: operators, accumulators, histories and stage outputs are
 // touched once per launch, so they bypass the caches' normal retention and leave
-// L2 to the stage input, whose 12 stencil neighbours are re-read from it.
+// L2 to the stage input, whose 12 stencil neighbours are re-read from it.  From 9
+// bands on (plain ones: 16 bands 200 x 200 117 -> 127 us per stage, 32 bands 128 x
+// 128 214 -> 228); below, a grid's arrays fit in the Infinity Cache, which
+// non-temporal accesses pass by (8 bands 200 x 200, plain: 39.1 -> 35.1 us).
 __device__ __forceinline__ double ldnt(const double *p) { return __builtin_nontemporal_load(gm(p)); }
 __device__ __forceinline__ float ldnt(const float *p) { return __builtin_nontemporal_load(gm(p)); }
 __device__ __forceinline__ void stnt(double *p, double v) { __builtin_nontemporal_store(v, gm(p)); }
@@ -238,16 +241,21 @@ __device__ __forceinline__ void ld2(const T *p, size_t o0, size_t o1, bool vec, 
         b = NT ? ldnt(p + o1) : *gm(p + o1);
     }
 }
-template <typename T>
+template <bool NT, typename T>
 __device__ __forceinline__ void st2(T *p, size_t o0, size_t o1, bool vec, T a, T b) {
     if (vec) {
         typename Pair<T>::V v;
         v.x = a;
         v.y = b;
-        __builtin_nontemporal_store(v, gm(reinterpret_cast<typename Pair<T>::V *>(p + o0)));
-    } else {
+        auto *q = gm(reinterpret_cast<typename Pair<T>::V *>(p + o0));
+        if (NT) __builtin_nontemporal_store(v, q);
+        else *q = v;
+    } else if (NT) {
         stnt(p + o0, a);
         stnt(p + o1, b);
+    } else {
+        *gm(p + o0) = a;
+        *gm(p + o1) = b;
     }
 }
 
@@ -257,12 +265,12 @@ __device__ __forceinline__ void st2(T *p, size_t o0, size_t o1, bool vec, T a, T
 // together before the sum, which keeps the order of the coefficients.  h: stride
 // between history slots.  S: storage type of the history (double, or float in the
 // mixed form with FP32 stage storage); the state and its update stay FP64.
-template <typename S>
+template <bool NT, typename S>
 __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0, size_t o1, bool vec, size_t h, double kv0,
                                                   double kv1, double y0, double y1) {
     S *const hist = reinterpret_cast<S *>(a.HIST);
     const size_t so = (size_t)a.slot_out * h;
-    st2(hist, so + o0, so + o1, vec, (S)kv0, (S)kv1);
+    st2<NT>(hist, so + o0, so + o1, vec, (S)kv0, (S)kv1);
     double h0[5], h1[5];
 #pragma unroll
     for (int s = 1; s < 5; s++) {
@@ -270,7 +278,7 @@ __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0,
         if (s < a.order) {
             const size_t sl = (size_t)a.slots[s] * h;
             S u0, u1;
-            ld2<true>(hist, sl + o0, sl + o1, vec, u0, u1);
+            ld2<NT>(hist, sl + o0, sl + o1, vec, u0, u1);
             h0[s] = (double)u0;
             h1[s] = (double)u1;
         }
@@ -282,18 +290,18 @@ __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0,
             d0 += a.coef[s] * h0[s];
             d1 += a.coef[s] * h1[s];
         }
-    st2(a.OUT, o0, o1, vec, y0 + a.dt * d0, y1 + a.dt * d1);
+    st2<NT>(a.OUT, o0, o1, vec, y0 + a.dt * d0, y1 + a.dt * d1);
 }
 
 // The Taylor tail for two adjacent packed elements: the history is read as
 // pairs, then each element's update is formed on its own (one set of
 // differences live at a time).
-template <typename S>
+template <bool NT, typename S>
 __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0, size_t o1, bool vec, size_t h, double kv0,
                                                   double kv1, double y0, double y1) {
     S *const hist = reinterpret_cast<S *>(a.HIST);
     const size_t so = (size_t)a.slot_out * h;
-    st2(hist, so + o0, so + o1, vec, (S)kv0, (S)kv1);
+    st2<NT>(hist, so + o0, so + o1, vec, (S)kv0, (S)kv1);
     const int n = a.order - 1;
     S u0[EDUS_MAX_ORDER - 1], u1[EDUS_MAX_ORDER - 1];
 #pragma unroll
@@ -301,7 +309,7 @@ __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0,
         u0[i] = u1[i] = (S)0;
         if (i < n) {
             const size_t sl = (size_t)a.slots[i + 1] * h;
-            ld2<true>(hist, sl + o0, sl + o1, vec, u0[i], u1[i]);
+            ld2<NT>(hist, sl + o0, sl + o1, vec, u0[i], u1[i]);
         }
     }
     double out[2];
@@ -319,7 +327,7 @@ __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0,
         }
         out[w] = (w ? y1 : y0) + delta;
     }
-    st2(a.OUT, o0, o1, vec, out[0], out[1]);
+    st2<NT>(a.OUT, o0, o1, vec, out[0], out[1]);
 }
 
 // ================================================================ nb <= 4: a lane per k and term
@@ -1337,6 +1345,8 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     constexpr int TPK = WaveGeom<NBT>::TPK, RBR = WaveGeom<NBT>::RBR, RBC = WaveGeom<NBT>::RBC, PER = WaveGeom<NBT>::PER;
     constexpr int LD = WaveGeom<NBT>::LD, MAT = NBT * LD;
     const int nb = c.nb, NP = nb * nb, nmat = wave_mats(c.diss);
+    // non-temporal streams: see ldnt
+    constexpr bool kNT = NBT >= 16;
     constexpr bool kMfma = NBT >= 16;  // 16x16 matrix-core tiles; NBT = 8 stays on the VALU
     CT *A = reinterpret_cast<CT *>(smem), *B = A + MAT, *C = c.diss ? B + MAT : B;
     const R *Hop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.H : (const void *)c.Hf);
@@ -1411,17 +1421,17 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             ld2<false>(Yin, o0, o1, v2, y0, y1);
             y[m] = (double)y0;
             y[m + 1] = (double)y1;
-            ld2<true>(Hop, o0, o1, v2, hv[m], hv[m + 1]);
+            ld2<kNT>(Hop, o0, o1, v2, hv[m], hv[m + 1]);
 #pragma unroll
             for (int x = 0; x < 3; x++) {
-                if (a.dmask >> x & 1) ld2<true>(Dop + (size_t)x * c.nk * NP, o0, o1, v2, dv[m][x], dv[m + 1][x]);
+                if (a.dmask >> x & 1) ld2<kNT>(Dop + (size_t)x * c.nk * NP, o0, o1, v2, dv[m][x], dv[m + 1][x]);
                 else dv[m][x] = dv[m + 1][x] = (R)0;
             }
             if constexpr ((MODE == RK2 || MODE == RK3) && !kLatePre) {
-                ld2<true>(a.ACC, o0, o1, v2, pre0[m], pre0[m + 1]);
-                ld2<true>(a.P0, o0, o1, v2, pre1[m], pre1[m + 1]);
+                ld2<kNT>(a.ACC, o0, o1, v2, pre0[m], pre0[m + 1]);
+                ld2<kNT>(a.P0, o0, o1, v2, pre1[m], pre1[m + 1]);
             } else if constexpr (MODE == RK4S) {
-                ld2<true>(a.ACC, o0, o1, v2, pre0[m], pre0[m + 1]);
+                ld2<kNT>(a.ACC, o0, o1, v2, pre0[m], pre0[m + 1]);
             }
         }
     } else {
@@ -1558,8 +1568,8 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         for (int h = 0; h < PER / 2; h++) {
             const int m = 2 * h;
             const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-            ld2<true>(a.ACC, o0, o1, pv2[h], pre0[m], pre0[m + 1]);
-            ld2<true>(a.P0, o0, o1, pv2[h], pre1[m], pre1[m + 1]);
+            ld2<kNT>(a.ACC, o0, o1, pv2[h], pre0[m], pre0[m + 1]);
+            ld2<kNT>(a.P0, o0, o1, pv2[h], pre1[m], pre1[m + 1]);
         }
     }
     // pv = -i (X_ij - conj(X_ji)) plus the RWA term on core -> non-core pairs; on
@@ -1673,19 +1683,19 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
         const bool v2 = pv2[h];
         if constexpr (MODE == ABM) {
-            stage_update2_abm<S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+            stage_update2_abm<kNT, S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
         } else if constexpr (MODE == TAY) {
-            stage_update2_tay<S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+            stage_update2_tay<kNT, S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
         } else if constexpr (MODE == RK1) {
-            st2(a.ACC, o0, o1, v2, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
-            st2(outs, o0, o1, v2, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
+            st2<kNT>(a.ACC, o0, o1, v2, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
+            st2<kNT>(outs, o0, o1, v2, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK2 || MODE == RK3) {
-            st2(a.ACC, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
-            st2(outs, o0, o1, v2, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
+            st2<kNT>(a.ACC, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2<kNT>(outs, o0, o1, v2, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK4S) {
-            st2(a.OUT, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2<kNT>(a.OUT, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
         } else {
-            st2(a.OUT, o0, o1, v2, k0, k1);
+            st2<kNT>(a.OUT, o0, o1, v2, k0, k1);
         }
     }
 }
