@@ -2741,152 +2741,281 @@ __global__ void k_wannier_finish(const cd *__restrict__ Out, int kc, int nw, dou
 
 // ================================================================ Coulomb coefficient generator
 // W(q) = sum_G V(|q+G|) e^{i (q+G).(d_i - d_j)} on a grid of q (Create_Wq_with_G_sum,
-// Coulomb.h:87-175), one thread per q point, the G list streamed through LDS in
-// tiles (an all-pairs sum: every q meets every G).  The phase is split as
-// e^{i q.beta} e^{i G.beta} with beta_p = b.(d_i - d_j) per band pair p.
-constexpr int kCgTile = 256;
+// Coulomb.h:87-175): an all-pairs sum, every q meets every G.  The phase is split as
+// e^{i q.beta} e^{i G.beta} with beta_p = b.(d_i - d_j) per band pair p; the q factor
+// leaves the sum.  FP64-bound: per (q, G) the potential and two FMAs per pair.
+//   * q + G in two orthonormal components (the lattice's Cholesky frame), the G part
+//     from the table: two additions.
+//   * V = 2 pi / (eps sqrt(Q2 + qTF2) (sqrt(Q2) r0 + 1)) as one square root and one
+//     reciprocal square root, each a hardware estimate and one third-order step,
+//     instead of two square roots and a division.
+//   * Two q per thread share the reads of the G table (LDS, one address per wave).
+//   * A list of G closed under G -> -G gives W(-q) = conj W(q): the second half of a
+//     symmetric set of q is the first one reversed and conjugated.
+//   * Few q: the G list is split over blockIdx.y and the parts added afterwards.
+// 999^2 q, 2849 G, 3 bands: 12.0 ms -> 1.9 ms.
+constexpr int kCgTile = 128;
 constexpr int kCgMaxPair = 6;  // nb <= 4
+constexpr int kCgQ = 2;        // q per thread
+constexpr int kCgThreads = 256;
 
 struct CGenArgs {
     int npair, n_g, N, mode;    // mode 0: grid q = -0.5 + i h (N per direction); 1: list of (ix, iy) on that grid
-    double h, qtf2, eps, r0, rk;
-    double b1[3], b2[3];
+    int gper;                   // G per blockIdx.y
+    double qtf2, r0;
+    // 2 pi / eps, and q = (qx, qy) -> (l11 qx + l21 qy, l22 qy), as [value, rest]: their
+    // rounding would shift every term alike (1e-15 of the coefficients)
+    double scale[2], l11[2], l21[2], l22[2];
     double beta1[kCgMaxPair], beta2[kCgMaxPair];
-    const double *g;            // [n_g][2] crystal offsets
-    const double *gph;          // [n_g][npair][2] e^{i G.beta_p}
+    const double *g;            // [n_g][2 + 2 npair]: components of G, e^{i G.beta_p}
     const int *qlist;           // mode 1: [nq][2]
 };
 
-__global__ __launch_bounds__(256) void k_cgen_w(CGenArgs a, long long iq0, int nq, double *W) {
-    __shared__ double sg[kCgTile * 2];
-    __shared__ double sph[kCgTile * kCgMaxPair * 2];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = t < nq;
-    int ix = 0, iy = 0;
-    if (valid) {
-        if (a.mode == 0) {
-            const long long iq = iq0 + t;
-            ix = (int)(iq / a.N);
-            iy = (int)(iq % a.N);
-        } else {
-            ix = a.qlist[2 * t];
-            iy = a.qlist[2 * t + 1];
+__device__ __forceinline__ void cgen_q(const CGenArgs &a, long long iq, double &qx, double &qy) {
+    int ix, iy;
+    if (a.mode == 0) {
+        ix = (int)(iq / a.N);
+        iy = (int)(iq % a.N);
+    } else {
+        ix = a.qlist[2 * iq];
+        iy = a.qlist[2 * iq + 1];
+    }
+    // Grid_and_Simpson (integrationWeight.h:5-8): q_i = -0.5 + i / (N - 1), formed so
+    // that q_{N-1-i} = -q_i exactly: with i h the rounding of h shifts all q alike, and
+    // a W taken from the mirrored q would see the shift with the wrong sign (1e-14 of
+    // the q ~ 0 correction)
+    qx = (double)(2 * ix - (a.N - 1)) / (double)(2 * (a.N - 1));
+    qy = (double)(2 * iy - (a.N - 1)) / (double)(2 * (a.N - 1));
+}
+
+// 1 / sqrt(x) for a normal x > 0: the hardware's estimate y, then the series
+// y (1 - e)^(-1/2) = y (1 + e/2 + 3 e^2/8 + ...) with e = 1 - x y^2 (the cubic term
+// changed no digit).
+__device__ __forceinline__ double rsqrt_step(double x, double &m, double &ep) {
+    const double y = __builtin_amdgcn_rsq(x);
+    m = x * y;  // ~ sqrt(x)
+    const double e = __builtin_fma(-m, y, 1.0);
+    ep = e * __builtin_fma(0.375, e, 0.5);
+    return y;
+}
+
+// V(|q + G|) without the scale, Q2 = |q + G|^2 (Coloumb_THh_F, Coulomb.h:60-84).
+template <bool RK>
+__device__ __forceinline__ double cgen_v(double q2, double qtf2, double r0) {
+    double u = q2 + qtf2, m, ep;
+    if constexpr (RK) {
+        rsqrt_step(fmax(q2, 1e-290), m, ep);   // q = 0 and G = 0: sqrt is 0 to within 1e-145
+        const double t = __builtin_fma(__builtin_fma(m, ep, m), r0, 1.0);
+        u = u * t * t;
+    }
+    const double y = rsqrt_step(u, m, ep), v = __builtin_fma(y, ep, y);
+    return u == 0.0 ? __builtin_inf() : v;  // q = 0 without screening
+}
+
+// part[y][t][1 + 2 npair]: sums of q number iq0 + t over the G of blockIdx.y.
+template <int NPAIR, bool RK>
+__global__ __launch_bounds__(kCgThreads) void k_cgen_w(CGenArgs a, long long iq0, int nq, double *part) {
+    constexpr int ROW = 2 + 2 * NPAIR, NW = 1 + 2 * NPAIR;
+    __shared__ double sg[kCgTile * ROW];
+    const int t0 = blockIdx.x * kCgThreads * kCgQ + threadIdx.x;
+    double x[kCgQ], y[kCgQ], w[kCgQ][NW];
+#pragma unroll
+    for (int j = 0; j < kCgQ; j++) {
+        double qx, qy;
+        cgen_q(a, iq0 + min(t0 + j * kCgThreads, nq - 1), qx, qy);
+        x[j] = __builtin_fma(a.l11[0], qx, __builtin_fma(a.l21[0], qy, __builtin_fma(a.l11[1], qx, a.l21[1] * qy)));
+        y[j] = __builtin_fma(a.l22[0], qy, a.l22[1] * qy);
+#pragma unroll
+        for (int c = 0; c < NW; c++) w[j][c] = 0.0;
+    }
+    const int gend = min(a.n_g, (int)(blockIdx.y + 1) * a.gper);
+    for (int g0 = blockIdx.y * a.gper; g0 < gend; g0 += kCgTile) {
+        const int nt = min(kCgTile, gend - g0);
+        __syncthreads();
+        for (int i = threadIdx.x; i < nt * ROW; i += kCgThreads) sg[i] = a.g[(size_t)g0 * ROW + i];
+        __syncthreads();
+#pragma unroll 2
+        for (int j = 0; j < nt; j++) {
+            const double *s = sg + j * ROW;
+#pragma unroll
+            for (int q = 0; q < kCgQ; q++) {
+                const double cx = x[q] + s[0], cy = y[q] + s[1];
+                const double v = cgen_v<RK>(__builtin_fma(cx, cx, cy * cy), a.qtf2, a.r0);
+                w[q][0] += v;
+#pragma unroll
+                for (int p = 0; p < 2 * NPAIR; p++) w[q][1 + p] = __builtin_fma(v, s[2 + p], w[q][1 + p]);
+            }
         }
     }
-    // Grid_and_Simpson (integrationWeight.h:5-8): q_i = -0.5 + i h
-    const double qx = -0.5 + ix * a.h, qy = -0.5 + iy * a.h;
-    double pr[kCgMaxPair], pi[kCgMaxPair], wr[kCgMaxPair], wi[kCgMaxPair];
+#pragma unroll
+    for (int j = 0; j < kCgQ; j++) {
+        const int t = t0 + j * kCgThreads;
+        if (t >= nq) continue;
+        double *o = part + ((size_t)blockIdx.y * nq + t) * NW;
+#pragma unroll
+        for (int c = 0; c < NW; c++) o[c] = w[j][c];
+    }
+}
+
+// W of q number iq0 + t from the ny parts, times e^{i q.beta} and the scale; mirror:
+// its conjugate also goes to the q of the same place from the end of the ntot.
+__global__ __launch_bounds__(256) void k_cgen_finish(CGenArgs a, long long iq0, int nq, int ny, long long ntot, int mirror,
+                                                     const double *part, double *W) {
+    const int t = blockIdx.x * 256 + threadIdx.x, nw = 1 + 2 * a.npair;
+    if (t >= nq) return;
+    double qx, qy;
+    cgen_q(a, iq0 + t, qx, qy);
+    auto sum = [&](int c) {
+        double s = 0.0;
+        for (int b = 0; b < ny; b++) s += part[((size_t)b * nq + t) * nw + c];
+        return __builtin_isinf(s) ? s * a.scale[0] : __builtin_fma(s, a.scale[0], s * a.scale[1]);
+    };
+    double *o = W + (size_t)(iq0 + t) * nw, *m = W + (size_t)(ntot - 1 - iq0 - t) * nw;
+    const bool both = mirror && m != o;
+    o[0] = sum(0);
+    if (both) m[0] = o[0];
     for (int p = 0; p < a.npair; p++) {
         double s, c;
         sincos(qx * a.beta1[p] + qy * a.beta2[p], &s, &c);
-        pr[p] = c;
-        pi[p] = s;
-        wr[p] = wi[p] = 0.0;
-    }
-    double w00 = 0.0;
-    const double twopi = 2 * M_PI;
-    for (int g0 = 0; g0 < a.n_g; g0 += kCgTile) {
-        const int nt = min(kCgTile, a.n_g - g0);
-        __syncthreads();
-        for (int i = threadIdx.x; i < nt * 2; i += blockDim.x) sg[i] = a.g[(size_t)g0 * 2 + i];
-        for (int i = threadIdx.x; i < nt * a.npair * 2; i += blockDim.x) sph[i] = a.gph[(size_t)g0 * a.npair * 2 + i];
-        __syncthreads();
-        for (int j = 0; j < nt; j++) {
-            const double c1 = qx + sg[2 * j], c2 = qy + sg[2 * j + 1];
-            const double x = a.b1[0] * c1 + a.b2[0] * c2, y = a.b1[1] * c1 + a.b2[1] * c2, z = a.b1[2] * c1 + a.b2[2] * c2;
-            const double q2 = x * x + y * y + z * z;
-            // Coloumb_THh_F (Coulomb.h:60-84)
-            const double den = (a.rk != 0.0) ? a.eps * sqrt(q2 + a.qtf2) * (sqrt(q2) * a.r0 + 1.0) : a.eps * sqrt(q2 + a.qtf2);
-            const double V = twopi / den;
-            w00 += V;
-            for (int p = 0; p < a.npair; p++) {
-                const double gr = sph[(j * a.npair + p) * 2], gi = sph[(j * a.npair + p) * 2 + 1];
-                const double er = pr[p] * gr - pi[p] * gi, ei = pr[p] * gi + pi[p] * gr;
-                wr[p] += V * er;
-                wi[p] += V * ei;
-            }
+        const cd w = cmul(mk(c, s), mk(sum(1 + 2 * p), sum(2 + 2 * p)));
+        o[1 + 2 * p] = w.x;
+        o[2 + 2 * p] = w.y;
+        if (both) {
+            m[1 + 2 * p] = w.x;
+            m[2 + 2 * p] = -w.y;
         }
     }
-    if (!valid) return;
-    const int nw = 1 + 2 * a.npair;
-    double *o = W + (size_t)t * nw;
-    o[0] = w00;
-    for (int p = 0; p < a.npair; p++) {
-        o[1 + 2 * p] = wr[p];
-        o[2 + 2 * p] = wi[p];
+}
+
+// T[t][j] = sum_ix wt[ix][t] W[ix][j], j = (iy, c) (first pass of the separable Simpson
+// integral, Fourier_Coulomb.cpp:230-265 with Coulomb.h:182-232): trig_t = cos(2 pi m q),
+// t < ncut, sin(2 pi (t - ncut) q) otherwise, with the weights in wt (rows padded with
+// zeros to ldt, a multiple of 16 TT).  On the FP64 matrix cores: a workgroup owns 16 j
+// and 16 TT trig rows, its four waves every fourth slice of four ix, added in wave
+// order.  W is read once per 16 TT rows instead of once per row.
+constexpr int kCgTT = 3;
+__global__ __launch_bounds__(256) void k_cgen_pass1(const double *__restrict__ W, const double *__restrict__ wt, int N, int ldt, int ntrig,
+                                                    int J, double *__restrict__ T) {
+    typedef double v4 __attribute__((ext_vector_type(4)));
+    __shared__ double red[3][kCgTT][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j0 = blockIdx.x * 16, t0 = blockIdx.y * 16 * kCgTT;
+    const int l = lane & 15, kq = lane >> 4, jc = min(j0 + l, J - 1);
+    v4 acc[kCgTT];
+#pragma unroll
+    for (int u = 0; u < kCgTT; u++) acc[u] = v4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int s = wave * 4; s < N; s += 16) {
+        const int ix = s + kq, ic = min(ix, N - 1);
+        double b = W[(size_t)ic * J + jc], av[kCgTT];
+#pragma unroll
+        for (int u = 0; u < kCgTT; u++) av[u] = wt[(size_t)ic * ldt + t0 + 16 * u + l];
+        if (ix >= N) b = 0.0;
+#pragma unroll
+        for (int u = 0; u < kCgTT; u++) acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(ix < N ? av[u] : 0.0, b, acc[u], 0, 0, 0);
     }
+    if (wave > 0) {
+#pragma unroll
+        for (int u = 0; u < kCgTT; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) red[wave - 1][u][i][lane] = acc[u][i];
+    }
+    __syncthreads();
+    if (wave > 0 || j0 + l >= J) return;
+#pragma unroll
+    for (int u = 0; u < kCgTT; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int t = t0 + 16 * u + kq + 4 * i;
+            if (t < ntrig) T[(size_t)t * J + j0 + l] = ((acc[u][i] + red[0][u][i][lane]) + red[1][u][i][lane]) + red[2][u][i][lane];
+        }
 }
 
-// T[t][iy][c] = sum_ix w[ix] trig_t(ix) W[ix][iy][c], trig_t = cos(2 pi m q), t < ncut,
-// sin(2 pi (t - ncut) q) otherwise (first pass of the separable Simpson integral,
-// Fourier_Coulomb.cpp:230-265 with Coulomb.h:182-232).
-__global__ void k_cgen_pass1(const double *W, const double *wtrig, int N, int ntrig, int nw, double *T) {
-    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (long long)ntrig * nw * N) return;
-    const int iy = (int)(id % N), c = (int)((id / N) % nw), t = (int)(id / ((long long)N * nw));
-    double s = 0.0;
-    for (int ix = 0; ix < N; ix++) s += wtrig[(size_t)t * N + ix] * W[((size_t)ix * N + iy) * nw + c];
-    T[((size_t)t * N + iy) * nw + c] = s;
-}
-
-// S[t1][t2][c] = sum_iy w[iy] trig_t2(iy) T[t1][iy][c].
-__global__ void k_cgen_pass2(const double *T, const double *wtrig, int N, int ntrig, int nw, double *S) {
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= ntrig * ntrig * nw) return;
-    const int c = id % nw, t2 = (id / nw) % ntrig, t1 = id / (nw * ntrig);
-    double s = 0.0;
-    for (int iy = 0; iy < N; iy++) s += wtrig[(size_t)t2 * N + iy] * T[((size_t)t1 * N + iy) * nw + c];
-    S[id] = s;
+// S[t1][t2][c] = sum_iy wtrig[t2][iy] T[t1][iy][c]: a wave per (t1, t2), lanes over iy.
+__global__ __launch_bounds__(256) void k_cgen_pass2(const double *T, const double *wtrig, int N, int ntrig, int nw, double *S) {
+    constexpr int NWMAX = 1 + 2 * kCgMaxPair;
+    const int id = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (id >= ntrig * ntrig) return;
+    const int t1 = id / ntrig, t2 = id % ntrig;
+    double s[NWMAX];
+#pragma unroll
+    for (int c = 0; c < NWMAX; c++) s[c] = 0.0;
+    for (int iy = lane; iy < N; iy += 64) {
+        const double w = wtrig[(size_t)t2 * N + iy];
+        const double *p = T + ((size_t)t1 * N + iy) * nw;
+#pragma unroll
+        for (int c = 0; c < NWMAX; c++)
+            if (c < nw) s[c] += w * p[c];
+    }
+#pragma unroll
+    for (int c = 0; c < NWMAX; c++)
+        if (c < nw) {
+            const double v = wave_sum(s[c]);
+            if (lane == 0) S[(size_t)id * nw + c] = v;
+        }
 }
 
 // Correction around q = 0 (Fourier_Coulomb.cpp:375-456): per listed point,
-// (W0 - Fourier series) * dk2 for the entries ic <= jc, block partial sums.
-__global__ __launch_bounds__(256) void k_cgen_peak(const double *W0, const int *qlist, int np, int nb, int ncut, double h, double dk2,
-                                                   const double *A, const double *B, const double *C, const double *D, double *part) {
-    __shared__ double red[256];
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nb2 = nb * nb, npair = nb * (nb - 1) / 2, nw = 1 + 2 * npair;
-    double qx = 0, qy = 0;
-    if (t < np) {
-        qx = -0.5 + qlist[2 * t] * h;
-        qy = -0.5 + qlist[2 * t + 1] * h;
-    }
-    int p = 0;
-    for (int ic = 0; ic < nb; ic++)
-        for (int jc = ic; jc < nb; jc++) {
-            const int idx = ic * nb + jc;
-            double vr = 0, vi = 0;
-            if (t < np) {
-                // Fourier_series_Coloumb (Coulomb.h:235-267)
-                for (int m = 0; m < ncut; m++) {
-                    double sm, cm;
-                    sincos(2 * M_PI * m * qx, &sm, &cm);
-                    for (int n = 0; n < ncut; n++) {
-                        double sn, cn;
-                        sincos(2 * M_PI * n * qy, &sn, &cn);
-                        const size_t r = ((size_t)(n + ncut * m) * nb2 + idx) * 2;
-                        vr += A[r] * cm * cn + B[r] * cm * sn + C[r] * sm * cn + D[r] * sm * sn;
-                        vi += A[r + 1] * cm * cn + B[r + 1] * cm * sn + C[r + 1] * sm * cn + D[r + 1] * sm * sn;
+// (W0 - Fourier series) * dk2 for the entries ic <= jc, block partial sums.  A thread's
+// cos and sin of 2 pi n qy wait in LDS, NC of them at a time, and all entries are
+// summed in one walk over (m, n) (each entry of each n formed its own before:
+// 1.01 -> 0.43 ms at 9999^2 points of the q grid).
+constexpr int kCgPeakThreads = 128, kCgPeakNC = 16;
+template <int NB>
+__global__ __launch_bounds__(kCgPeakThreads) void k_cgen_peak(const double *W0, const int *qlist, int np, int ncut, int Np, double dk2,
+                                                              const double *A, const double *B, const double *C, const double *D,
+                                                              double *part) {
+    constexpr int NB2 = NB * NB, NE = NB * (NB + 1) / 2, NW = 1 + NB * (NB - 1), NWV = kCgPeakThreads / 64;
+    __shared__ double tc[kCgPeakNC][kCgPeakThreads], ts[kCgPeakNC][kCgPeakThreads];
+    __shared__ double red[NWV][2 * NE];
+    const int th = threadIdx.x, t = blockIdx.x * kCgPeakThreads + th, tt = min(t, np - 1);
+    const double qx = (double)(2 * qlist[2 * tt] - (Np - 1)) / (2 * (Np - 1)), qy = (double)(2 * qlist[2 * tt + 1] - (Np - 1)) / (2 * (Np - 1));
+    double vr[NE], vi[NE];
+#pragma unroll
+    for (int e = 0; e < NE; e++) vr[e] = vi[e] = 0.0;
+    // Fourier_series_Coloumb (Coulomb.h:235-267)
+    for (int n0 = 0; n0 < ncut; n0 += kCgPeakNC) {
+        const int nn = min(kCgPeakNC, ncut - n0);
+        for (int n = 0; n < nn; n++) sincos(2 * M_PI * (n0 + n) * qy, &ts[n][th], &tc[n][th]);
+        for (int m = 0; m < ncut; m++) {
+            double sm, cm;
+            sincos(2 * M_PI * m * qx, &sm, &cm);
+            for (int n = 0; n < nn; n++) {
+                const double cn = tc[n][th], sn = ts[n][th], f0 = cm * cn, f1 = cm * sn, f2 = sm * cn, f3 = sm * sn;
+                const size_t r0 = (size_t)(n0 + n + ncut * m) * NB2 * 2;
+                int e = 0;
+#pragma unroll
+                for (int ic = 0; ic < NB; ic++)
+#pragma unroll
+                    for (int jc = ic; jc < NB; jc++, e++) {
+                        const size_t r = r0 + 2 * (ic * NB + jc);
+                        vr[e] += A[r] * f0 + B[r] * f1 + C[r] * f2 + D[r] * f3;
+                        vi[e] += A[r + 1] * f0 + B[r + 1] * f1 + C[r + 1] * f2 + D[r + 1] * f3;
                     }
-                }
-                const double *w = W0 + (size_t)t * nw;
-                double wr = w[0], wi = 0.0;
-                if (jc != ic) { wr = w[1 + 2 * p]; wi = w[2 + 2 * p]; }
-                vr = (wr - vr) * dk2;
-                vi = (wi - vi) * dk2;
-            }
-            if (jc != ic) p++;
-            for (int comp = 0; comp < 2; comp++) {
-                red[threadIdx.x] = comp ? vi : vr;
-                __syncthreads();
-                for (int s = 128; s > 0; s >>= 1) {
-                    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-                    __syncthreads();
-                }
-                if (threadIdx.x == 0) part[((size_t)blockIdx.x * nb2 + idx) * 2 + comp] = red[0];
-                __syncthreads();
             }
         }
+    }
+    const double *w = W0 + (size_t)tt * NW;
+    int e = 0, p = 0;
+#pragma unroll
+    for (int ic = 0; ic < NB; ic++)
+#pragma unroll
+        for (int jc = ic; jc < NB; jc++, e++) {
+            const double wr = jc == ic ? w[0] : w[1 + 2 * p], wi = jc == ic ? 0.0 : w[2 + 2 * p];
+            if (jc != ic) p++;
+            const double r = wave_sum(t < np ? (wr - vr[e]) * dk2 : 0.0), i = wave_sum(t < np ? (wi - vi[e]) * dk2 : 0.0);
+            if ((th & 63) == 0) {
+                red[th >> 6][2 * e] = r;
+                red[th >> 6][2 * e + 1] = i;
+            }
+        }
+    __syncthreads();
+    if (th < 2 * NE) {
+        double v = 0.0;
+        for (int b = 0; b < NWV; b++) v += red[b][th];
+        int ic = 0, q = th >> 1;
+        while (q >= NB - ic) q -= NB - ic++;
+        part[((size_t)blockIdx.x * NB2 + ic * NB + ic + q) * 2 + (th & 1)] = v;
+    }
 }
 
 }  // namespace
@@ -4444,24 +4573,62 @@ int edus_coulomb_coefficients(const edus_coulomb_gen *g, double *Ao, double *Bo,
             vh[(pjc[p] * nb + pic[p]) * 2] = r;
         }
     }
-    // per-G data: offsets and e^{i G.beta_p}
-    std::vector<double> gd((size_t)g->n_g * 2), gph((size_t)g->n_g * std::max(npair, 1) * 2, 0.0);
+    // The lattice's Cholesky frame: q b1 + q' b2 = (l11 q + l21 q', l22 q') in
+    // orthonormal components of the plane.
+    auto two = [](long double v, double (&o)[2]) {
+        o[0] = (double)v;
+        o[1] = (double)(v - (long double)o[0]);
+    };
+    long double l11, l21, l22;
+    {
+        long double g11 = 0, g12 = 0, g22 = 0, c2 = 0;
+        for (int x = 0; x < 3; x++) {
+            const long double u = g->b1[(x + 1) % 3], v = g->b1[(x + 2) % 3], p = g->b2[(x + 1) % 3], r = g->b2[(x + 2) % 3];
+            g11 += (long double)g->b1[x] * g->b1[x];
+            g12 += (long double)g->b1[x] * g->b2[x];
+            g22 += (long double)g->b2[x] * g->b2[x];
+            c2 += (u * r - v * p) * (u * r - v * p);
+        }
+        l11 = sqrtl(g11);
+        l21 = g11 > 0 ? g12 / l11 : 0.0L;
+        l22 = g11 > 0 ? sqrtl(c2) / l11 : sqrtl(g22);
+    }
+    two(l11, a.l11);
+    two(l21, a.l21);
+    two(l22, a.l22);
+    two((long double)twopi / g->eps_area, a.scale);
+    // per-G data: components and e^{i G.beta_p}
+    const int grow = 2 + 2 * npair;
+    std::vector<double> gd((size_t)g->n_g * grow);
     for (int ig = 0; ig < g->n_g; ig++) {
         const double gx = g->g[2 * ig], gy = g->g[2 * ig + 1];
-        gd[2 * ig] = gx;
-        gd[2 * ig + 1] = gy;
+        double *r = &gd[(size_t)ig * grow];
+        r[0] = (double)(l11 * gx + l21 * gy);
+        r[1] = (double)(l22 * gy);
         for (int p = 0; p < npair; p++) {
             const double ph = gx * a.beta1[p] + gy * a.beta2[p];
-            gph[((size_t)ig * npair + p) * 2] = std::cos(ph);
-            gph[((size_t)ig * npair + p) * 2 + 1] = std::sin(ph);
+            r[2 + 2 * p] = std::cos(ph);
+            r[3 + 2 * p] = std::sin(ph);
         }
+    }
+    // Is the list of G closed under G -> -G (as every shell |G| < R is)?
+    bool gsym;
+    {
+        std::vector<std::pair<int, int>> l(g->n_g), m(g->n_g);
+        for (int ig = 0; ig < g->n_g; ig++) {
+            l[ig] = {g->g[2 * ig], g->g[2 * ig + 1]};
+            m[ig] = {-g->g[2 * ig], -g->g[2 * ig + 1]};
+        }
+        std::sort(l.begin(), l.end());
+        std::sort(m.begin(), m.end());
+        gsym = l == m;
     }
     // Simpson weights and trig tables (integrationWeight.h:5-18)
     auto simpson = [](int n, std::vector<double> &q, std::vector<double> &w) {
         q.resize(n);
         w.resize(n);
-        const double h = 2 * 0.5 / (n - 1), hs = 3 * (n - 1);
-        for (int i = 0; i < n; i++) q[i] = -0.5 + i * h;
+        const double hs = 3 * (n - 1);
+        for (int i = 0; i < n; i++) q[i] = (double)(2 * i - (n - 1)) / (double)(2 * (n - 1));  // as cgen_q
         w[0] = 1 / hs;
         for (int i = 1; i < n; i += 2) w[i] = 4.0 / hs;
         for (int i = 2; i < n; i += 2) w[i] = 2.0 / hs;
@@ -4469,52 +4636,75 @@ int edus_coulomb_coefficients(const edus_coulomb_gen *g, double *Ao, double *Bo,
     };
     std::vector<double> q, w;
     simpson(N, q, w);
-    std::vector<double> wtrig((size_t)ntrig * N);
+    const int ldt = (ntrig + 16 * kCgTT - 1) / (16 * kCgTT) * (16 * kCgTT);
+    std::vector<double> wtrig((size_t)ntrig * N), wt((size_t)N * ldt, 0.0);  // [t][i], and [i][t] padded with zeros
     for (int t = 0; t < ntrig; t++)
         for (int i = 0; i < N; i++) {
             const int m = t < nc ? t : t - nc;
             const double arg = 2 * M_PI * m * q[i];
-            wtrig[(size_t)t * N + i] = w[i] * (t < nc ? std::cos(arg) : std::sin(arg));
+            wt[(size_t)i * ldt + t] = wtrig[(size_t)t * N + i] = w[i] * (t < nc ? std::cos(arg) : std::sin(arg));
         }
     const size_t nq = (size_t)N * N;
-    double *dG = nullptr, *dPh = nullptr, *dW = nullptr, *dTr = nullptr, *dT = nullptr, *dS = nullptr, *dCoef = nullptr, *dW0 = nullptr,
-           *dPart = nullptr;
+    double *dG = nullptr, *dW = nullptr, *dTr = nullptr, *dWt = nullptr, *dT = nullptr, *dS = nullptr, *dCoef = nullptr, *dW0 = nullptr,
+           *dPart = nullptr, *dSum = nullptr;
     int *dQl = nullptr;
     auto cleanup = [&]() {
-        for (void *p : {(void *)dG, (void *)dPh, (void *)dW, (void *)dTr, (void *)dT, (void *)dS, (void *)dCoef, (void *)dW0, (void *)dPart,
-                        (void *)dQl})
+        for (void *p : {(void *)dG, (void *)dW, (void *)dTr, (void *)dWt, (void *)dT, (void *)dS, (void *)dCoef, (void *)dW0, (void *)dPart,
+                        (void *)dSum, (void *)dQl})
             (void)hipFree(p);
     };
     auto fail = [&](int code, const std::string &m) {
         cleanup();
         return set_err(code, m);
     };
-    if (hipMalloc(&dG, gd.size() * 8) != hipSuccess || hipMalloc(&dPh, gph.size() * 8) != hipSuccess ||
-        hipMalloc(&dW, nq * nw * 8) != hipSuccess || hipMalloc(&dTr, wtrig.size() * 8) != hipSuccess ||
+    // A set of n q: chunks of blocks of q, the G list in gs parts when the chunk alone
+    // would leave the chip idle (four waves per SIMD: 1024 blocks).
+    const long long chunk = 1LL << 21;
+    auto blocks_of = [](long long n) { return (int)((n + kCgThreads * kCgQ - 1) / (kCgThreads * kCgQ)); };
+    auto split_of = [&](long long n) { return (int)std::max<long long>(1, std::min<long long>({16, 1024 / blocks_of(n), g->n_g / kCgTile})); };
+    auto sums_of = [&](long long n) { return (size_t)std::min(n, chunk) * split_of(std::min(n, chunk)) * nw * 8; };
+    const long long half = gsym ? (long long)(nq + 1) / 2 : (long long)nq;
+    if (hipMalloc(&dG, gd.size() * 8) != hipSuccess || hipMalloc(&dW, nq * nw * 8) != hipSuccess ||
+        hipMalloc(&dTr, wtrig.size() * 8) != hipSuccess || hipMalloc(&dWt, wt.size() * 8) != hipSuccess ||
         hipMalloc(&dT, (size_t)ntrig * N * nw * 8) != hipSuccess || hipMalloc(&dS, (size_t)ntrig * ntrig * nw * 8) != hipSuccess ||
-        hipMalloc(&dCoef, (size_t)4 * nmm * nb2 * 2 * 8) != hipSuccess)
+        hipMalloc(&dCoef, (size_t)4 * nmm * nb2 * 2 * 8) != hipSuccess || hipMalloc(&dSum, sums_of(half)) != hipSuccess)
         return fail(EDUS_ERR_NOMEM, "coefficient generator buffers");
     if (hipMemcpy(dG, gd.data(), gd.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dPh, gph.data(), gph.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(dWt, wt.data(), wt.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(dTr, wtrig.data(), wtrig.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
         return fail(EDUS_ERR_HIP, "coefficient generator upload");
-    a.npair = npair; a.n_g = g->n_g; a.N = N; a.mode = 0; a.h = 2 * 0.5 / (N - 1);
-    a.qtf2 = g->qtf * g->qtf; a.eps = g->eps_area; a.r0 = g->r0; a.rk = g->rytova_keldysh ? 1.0 : 0.0;
-    for (int x = 0; x < 3; x++) { a.b1[x] = g->b1[x]; a.b2[x] = g->b2[x]; }
-    a.g = dG; a.gph = dPh; a.qlist = nullptr;
+    a.npair = npair; a.n_g = g->n_g; a.N = N; a.mode = 0;
+    a.qtf2 = g->qtf * g->qtf; a.r0 = g->r0;
+    a.g = dG; a.qlist = nullptr;
+    // sums over G of q numbers [q0, q0 + n) and W from them (of a set of ntot; mirror:
+    // its second half comes from the first)
+    auto lattice_sum = [&](CGenArgs c, long long q0, int n, long long ntot, bool mirror, double *W) {
+        const int gs = split_of(n);
+        c.gper = (g->n_g + gs - 1) / gs;
+        const dim3 grid(blocks_of(n), gs), block(kCgThreads);
+        auto go = [&](auto ptag) {
+            constexpr int NPAIR = decltype(ptag)::value;
+            if (g->rytova_keldysh) hipLaunchKernelGGL((k_cgen_w<NPAIR, true>), grid, block, 0, 0, c, q0, n, dSum);
+            else hipLaunchKernelGGL((k_cgen_w<NPAIR, false>), grid, block, 0, 0, c, q0, n, dSum);
+        };
+        if (npair == 0) go(std::integral_constant<int, 0>{});
+        else if (npair == 1) go(std::integral_constant<int, 1>{});
+        else if (npair == 3) go(std::integral_constant<int, 3>{});
+        else go(std::integral_constant<int, 6>{});
+        hipLaunchKernelGGL(k_cgen_finish, dim3((n + 255) / 256), dim3(256), 0, 0, c, q0, n, gs, ntot, mirror ? 1 : 0, (const double *)dSum, W);
+    };
     // W on the Simpson grid, in chunks with a progress line each
-    const long long chunk = 1LL << 21;
-    for (long long q0 = 0; q0 < (long long)nq; q0 += chunk) {
-        const int n = (int)std::min<long long>(chunk, (long long)nq - q0);
-        hipLaunchKernelGGL(k_cgen_w, dim3((n + 255) / 256), dim3(256), 0, 0, a, q0, n, dW + (size_t)q0 * nw);
+    for (long long q0 = 0; q0 < half; q0 += chunk) {
+        const int n = (int)std::min<long long>(chunk, half - q0);
+        lattice_sum(a, q0, n, (long long)nq, gsym, dW);
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) return fail(EDUS_ERR_HIP, "k_cgen_w");
-        if (g->verbose) std::fprintf(stderr, "Coulomb coefficients: %lld / %zu q points\n", q0 + n, nq);
+        if (g->verbose) std::fprintf(stderr, "Coulomb coefficients: %lld / %lld q points\n", q0 + n, half);
     }
     {
-        const long long n1 = (long long)ntrig * nw * N;
-        hipLaunchKernelGGL(k_cgen_pass1, dim3((unsigned)((n1 + 255) / 256)), dim3(256), 0, 0, (const double *)dW, (const double *)dTr, N, ntrig, nw, dT);
-        const int n2 = ntrig * ntrig * nw;
-        hipLaunchKernelGGL(k_cgen_pass2, dim3((n2 + 255) / 256), dim3(256), 0, 0, (const double *)dT, (const double *)dTr, N, ntrig, nw, dS);
+        const int J = N * nw;
+        hipLaunchKernelGGL(k_cgen_pass1, dim3((J + 15) / 16, ldt / (16 * kCgTT)), dim3(256), 0, 0, (const double *)dW, (const double *)dWt, N,
+                           ldt, ntrig, J, dT);
+        hipLaunchKernelGGL(k_cgen_pass2, dim3((ntrig * ntrig + 3) / 4), dim3(256), 0, 0, (const double *)dT, (const double *)dTr, N, ntrig, nw, dS);
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) return fail(EDUS_ERR_HIP, "k_cgen_pass");
     }
     std::vector<double> S((size_t)ntrig * ntrig * nw);
@@ -4545,14 +4735,14 @@ int edus_coulomb_coefficients(const edus_coulomb_gen *g, double *Ao, double *Bo,
         const double lmin = 0.5 * (g11 + g22) - std::sqrt(0.25 * (g11 - g22) * (g11 - g22) + g12 * g12);
         const double rc = (lmin > 0) ? g->q_peak / std::sqrt(lmin) : 1.0;
         const int lo = std::max(0, (int)std::floor((0.5 - rc) / hp) - 2), hi = std::min(Np - 1, (int)std::ceil((0.5 + rc) / hp) + 2);
-        const double qp2 = g->q_peak * g->q_peak;
+        const double qp2 = g->q_peak * g->q_peak, qmin2 = std::pow(10, -17);
         for (int ix = lo; ix <= hi; ix++)
             for (int iy = lo; iy <= hi; iy++) {
                 const double qx = -0.5 + ix * hp, qy = -0.5 + iy * hp;
                 double cart[3];
                 for (int x = 0; x < 3; x++) cart[x] = g->b1[x] * qx + g->b2[x] * qy;
                 const double q2 = cart[0] * cart[0] + cart[1] * cart[1] + cart[2] * cart[2];
-                if (q2 < qp2 && q2 > std::pow(10, -17)) {
+                if (q2 < qp2 && q2 > qmin2) {
                     ql.push_back(ix);
                     ql.push_back(iy);
                 }
@@ -4560,26 +4750,41 @@ int edus_coulomb_coefficients(const edus_coulomb_gen *g, double *Ao, double *Bo,
     }
     const int npk = (int)(ql.size() / 2);
     if (npk > 0) {
-        const int nblk = (npk + 255) / 256;
+        const int nblk = (npk + kCgPeakThreads - 1) / kCgPeakThreads;
         std::vector<double> coef((size_t)4 * nmm * nb2 * 2);
         std::copy(Ao, Ao + (size_t)nmm * nb2 * 2, coef.begin());
         std::copy(Bo, Bo + (size_t)nmm * nb2 * 2, coef.begin() + (size_t)nmm * nb2 * 2);
         std::copy(Co, Co + (size_t)nmm * nb2 * 2, coef.begin() + (size_t)2 * nmm * nb2 * 2);
         std::copy(Do, Do + (size_t)nmm * nb2 * 2, coef.begin() + (size_t)3 * nmm * nb2 * 2);
+        // the list runs through a disc around 0 in grid order: reversed, it is its mirror image
+        bool qsym = gsym;
+        for (int t = 0; t < npk && qsym; t++)
+            qsym = ql[2 * t] + ql[2 * (npk - 1 - t)] == Np - 1 && ql[2 * t + 1] + ql[2 * (npk - 1 - t) + 1] == Np - 1;
+        const long long phalf = qsym ? (npk + 1) / 2 : npk;
+        (void)hipFree(dSum);
+        dSum = nullptr;
         if (hipMalloc(&dQl, ql.size() * sizeof(int)) != hipSuccess || hipMalloc(&dW0, (size_t)npk * nw * 8) != hipSuccess ||
-            hipMalloc(&dPart, (size_t)nblk * nb2 * 2 * 8) != hipSuccess)
+            hipMalloc(&dSum, sums_of(phalf)) != hipSuccess || hipMalloc(&dPart, (size_t)nblk * nb2 * 2 * 8) != hipSuccess)
             return fail(EDUS_ERR_NOMEM, "peak buffers");
         if (hipMemcpy(dQl, ql.data(), ql.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
             hipMemcpy(dCoef, coef.data(), coef.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
             hipMemset(dPart, 0, (size_t)nblk * nb2 * 2 * 8) != hipSuccess)
             return fail(EDUS_ERR_HIP, "peak upload");
         CGenArgs b = a;
-        b.mode = 1; b.N = Np; b.h = hp; b.qtf2 = 0.0; b.qlist = dQl;
-        hipLaunchKernelGGL(k_cgen_w, dim3(nblk), dim3(256), 0, 0, b, 0LL, npk, dW0);
+        b.mode = 1; b.N = Np; b.qtf2 = 0.0; b.qlist = dQl;
+        for (long long q0 = 0; q0 < phalf; q0 += chunk)
+            lattice_sum(b, q0, (int)std::min(chunk, phalf - q0), npk, qsym, dW0);
         const size_t cs = (size_t)nmm * nb2 * 2;
-        hipLaunchKernelGGL(k_cgen_peak, dim3(nblk), dim3(256), 0, 0, (const double *)dW0, (const int *)dQl, npk, nb, nc, hp,
-                           1. / ((double)Np * Np), (const double *)dCoef, (const double *)(dCoef + cs), (const double *)(dCoef + 2 * cs),
-                           (const double *)(dCoef + 3 * cs), dPart);
+        auto peak = [&](auto tag) {
+            constexpr int NB = decltype(tag)::value;
+            hipLaunchKernelGGL(k_cgen_peak<NB>, dim3(nblk), dim3(kCgPeakThreads), 0, 0, (const double *)dW0, (const int *)dQl, npk, nc, Np,
+                               1. / ((double)Np * Np), (const double *)dCoef, (const double *)(dCoef + cs), (const double *)(dCoef + 2 * cs),
+                               (const double *)(dCoef + 3 * cs), dPart);
+        };
+        if (nb == 1) peak(std::integral_constant<int, 1>{});
+        else if (nb == 2) peak(std::integral_constant<int, 2>{});
+        else if (nb == 3) peak(std::integral_constant<int, 3>{});
+        else peak(std::integral_constant<int, 4>{});
         if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) return fail(EDUS_ERR_HIP, "peak kernels");
         std::vector<double> part((size_t)nblk * nb2 * 2);
         if (hipMemcpy(part.data(), dPart, part.size() * 8, hipMemcpyDeviceToHost) != hipSuccess) return fail(EDUS_ERR_HIP, "download peak");
