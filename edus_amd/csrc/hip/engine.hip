@@ -608,14 +608,13 @@ __device__ __forceinline__ void small_tail_store(const StageArgs &a, size_t row,
 // kk: the lane's k (past the grid: clamped, nothing stored); lk, tk: its place among
 // the workgroup's tk k; term: threadIdx.y, uniform in a wave; lds: [R][NP][tk].
 template <int NB, int MODE, bool DISS>
-__device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs &a, const int kk, const int lk, const int tk, const int term,
+__device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs &a, TabRow tab, const int kk, const int lk, const int tk, const int term,
                                             double *lds) {
     using G = SmallGeom<NB, DISS>;
     constexpr int NP = G::NP, R = G::R, EPR = G::EPR;
     const bool store = kk < c.nk;
     const unsigned ko = 8u * (unsigned)min(kk, c.nk - 1);
     const size_t nkp = c.nkp;
-    const TabRow tab = stage_row(a);
     const int nn = c.n_nbr;
     SmallTail<MODE> tail[EPR];
 #pragma unroll
@@ -664,7 +663,7 @@ template <int NB, int MODE, bool DISS>
 __global__ __launch_bounds__(kSmallMaxThreads, (small_wpe<NB, DISS>())) void k_stage_small(ConstArgs c, StageArgs a) {
     extern __shared__ double smem_d[];
     const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    stage_small<NB, MODE, DISS>(c, a, xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
+    stage_small<NB, MODE, DISS>(c, a, stage_row(a), xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
 }
 
 // ================================================================ Coulomb mean field
@@ -1335,7 +1334,7 @@ __host__ __device__ constexpr int wave_lds_doubles(int diss) {
 // histories: double, or float in the mixed form with FP32 stage storage, where
 // the state at t_n (P0), the RK accumulator and every update stay FP64.
 template <int NBT, int MODE, typename R, typename S = double, bool B3 = false, int ROLE = 0>
-__device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &a, const int k, const int kb, const int lane,
+__device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &a, TabRow tab, const int k, const int kb, const int lane,
                                            double *smem, const bool store, double (&gb)[WaveGeom<NBT>::PER]) {
     using CT = typename CplxOf<R>::T;
     // stage input in S for the RK stages 2-4 (they read YA / YB); the FP64 state otherwise
@@ -1352,7 +1351,6 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     const R *Hop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.H : (const void *)c.Hf);
     const R *Dop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.D : (const void *)c.Df);
     const R *Uop = reinterpret_cast<const R *>(sizeof(R) == 8 ? (const void *)c.U : (const void *)c.Uf);
-    const TabRow tab = stage_row(a);
     const R Ep[3] = {(R)tab[0], (R)tab[1], (R)tab[2]}, Eq[3] = {(R)tab[3], (R)tab[4], (R)tab[5]};
     const int nn = c.n_nbr;
     const bool grad = tab[6 + nn] != 0.0;
@@ -1712,20 +1710,20 @@ __global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB) void k_sta
         // xcd_block and strip_k: bijections of the nk / 2 pairs (the pair grid has
         // half as many columns: strips of sw / 2 pairs)
         const int k = 2 * strip_k(xcd_block(), c.nk >> 1, c.sw >> 1, c.scol >> 1);
-        stage_wave<NBT, MODE, R, S, B3, 1>(c, a, k, k + 1, threadIdx.x, smem_d, true, gb);
+        stage_wave<NBT, MODE, R, S, B3, 1>(c, a, stage_row(a), k, k + 1, threadIdx.x, smem_d, true, gb);
         __syncthreads();  // every lane is done with k's matrices
         // the second call forms its lane-derived indices and addresses anew
         // rather than keeping the first call's live across both
         int lane2 = threadIdx.x;
         asm volatile("" : "+v"(lane2));
-        stage_wave<NBT, MODE, R, S, B3, 2>(c, a, k + 1, -1, lane2, smem_d, true, gb);
+        stage_wave<NBT, MODE, R, S, B3, 2>(c, a, stage_row(a), k + 1, -1, lane2, smem_d, true, gb);
     } else if constexpr (WaveGeom<NBT>::KPB == 1) {
         // xcd_block and strip_k: bijections of [0, nk)
-        stage_wave<NBT, MODE, R, S, B3>(c, a, strip_k(xcd_block(), c.nk, c.sw, c.scol), -1, threadIdx.x, smem_d, true, gb);
+        stage_wave<NBT, MODE, R, S, B3>(c, a, stage_row(a), strip_k(xcd_block(), c.nk, c.sw, c.scol), -1, threadIdx.x, smem_d, true, gb);
     } else {
         const int sub = threadIdx.x / TPK;
         const int kk = xcd_block() * WaveGeom<NBT>::KPB + sub;
-        stage_wave<NBT, MODE, R, S, B3>(c, a, strip_k(min(kk, c.nk - 1), c.nk, c.sw, c.scol), -1, threadIdx.x % TPK,
+        stage_wave<NBT, MODE, R, S, B3>(c, a, stage_row(a), strip_k(min(kk, c.nk - 1), c.nk, c.sw, c.scol), -1, threadIdx.x % TPK,
                                  smem_d + sub * wave_lds_doubles<NBT, R>(c.diss), kk < c.nk, gb);
     }
 }
@@ -1757,7 +1755,7 @@ __global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) vo
     StageArgs a = be.a[rk4_stage_of<MODE>()];
     a.tab += tab_step;
     a.dmask = dmask[w.x];
-    stage_small<NB, MODE, DISS>(be.c, a, w.y * kSmallBatchThreads + threadIdx.x, threadIdx.x, kSmallBatchThreads, term, smem_d);
+    stage_small<NB, MODE, DISS>(be.c, a, (TabRow)a.tab, w.y * kSmallBatchThreads + threadIdx.x, threadIdx.x, kSmallBatchThreads, term, smem_d);
 }
 
 template <int NBT, int MODE, typename R, bool PAIR = false>
@@ -1773,14 +1771,14 @@ __global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB) void k_sta
     double gb[WaveGeom<NBT>::PER];
     if constexpr (PAIR) {  // every instance of the class is paired: block w.y serves pair w.y
         static_assert(WaveGeom<NBT>::KPB == 1, "stencil pairs: one k per workgroup");
-        stage_wave<NBT, MODE, R, double, false, 1>(be.c, a, 2 * w.y, 2 * w.y + 1, threadIdx.x, smem_d, true, gb);
+        stage_wave<NBT, MODE, R, double, false, 1>(be.c, a, (TabRow)a.tab, 2 * w.y, 2 * w.y + 1, threadIdx.x, smem_d, true, gb);
         __syncthreads();  // every lane is done with the first k's matrices
-        stage_wave<NBT, MODE, R, double, false, 2>(be.c, a, 2 * w.y + 1, -1, threadIdx.x, smem_d, true, gb);
+        stage_wave<NBT, MODE, R, double, false, 2>(be.c, a, (TabRow)a.tab, 2 * w.y + 1, -1, threadIdx.x, smem_d, true, gb);
     } else if constexpr (WaveGeom<NBT>::KPB == 1) {
-        stage_wave<NBT, MODE, R>(be.c, a, w.y, -1, threadIdx.x, smem_d, true, gb);
+        stage_wave<NBT, MODE, R>(be.c, a, (TabRow)a.tab, w.y, -1, threadIdx.x, smem_d, true, gb);
     } else {
         const int sub = threadIdx.x / TPK, kk = w.y * WaveGeom<NBT>::KPB + sub;
-        stage_wave<NBT, MODE, R>(be.c, a, min(kk, be.c.nk - 1), -1, threadIdx.x % TPK,
+        stage_wave<NBT, MODE, R>(be.c, a, (TabRow)a.tab, min(kk, be.c.nk - 1), -1, threadIdx.x % TPK,
                                  smem_d + sub * wave_lds_doubles<NBT, R>(be.c.diss), kk < be.c.nk, gb);
     }
 }
