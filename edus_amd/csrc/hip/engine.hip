@@ -30,6 +30,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -2452,10 +2453,49 @@ __global__ __launch_bounds__(kElemThreads) void k_eigen_element(const double *__
 }
 
 // ================================================================ Wannier contraction
-// Out[k][m] = sum_R phase(k,R) Val[R][m], Val = [H | r_x | r_y | r_z] per R.
+// Out[k][c] = sum_R phase(k,R) Val[R][c], the columns c being the nw^2 elements of H
+// and the three components of the upper triangle (i <= j, component fastest) of
+// (r + r^T)/2: D = (r + r^T)/2 (Wannier.h:577-578, save_HUD.cpp:187-191) is linear in
+// r(R), so it is taken before the sum, which then has nw^2 + 3 nw (nw+1)/2 columns
+// instead of 4 nw^2, and a product tile goes straight to the caller's layouts.
 // phase(k,R) = prod_l (-1)^{R_l} w_l[(i_l R_l) mod N_l] for N_l > 1 (k_l = -1/2 + i_l/N_l).
-// Tiled complex GEMM: 64 k x 64 m per block, 16x16 threads with 4x4 outputs.
-constexpr int WT = 64, WK = 8;
+__host__ __device__ inline long long wannier_cols(long long nw) { return nw * nw + 3 * (nw * (nw + 1) / 2); }
+
+// Val[r0 + r][.] of n lattice vectors from the caller's H(R) [n][nw][nw] and r(R)
+// [n][nw][nw][3], and (r0 = 0) the column table: element ij = i nw + j of H as (ij, 1 on
+// the diagonal, else 0), pair i <= j of D as (i nw + j, j nw + i).
+__global__ __launch_bounds__(256) void k_wannier_val(const cd *__restrict__ HR, const cd *__restrict__ rR, int r0, int n, int nw, int ncol,
+                                                     cd *__restrict__ Val, int2 *__restrict__ Col) {
+    const int nw2 = nw * nw;
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)n * nw2) return;
+    const int r = (int)(t / nw2), ij = (int)(t % nw2), i = ij / nw, j = ij % nw;
+    cd *v = Val + (size_t)(r0 + r) * ncol;
+    v[ij] = HR[t];
+    const int ji = j * nw + i, c = nw2 + 3 * (i * nw - i * (i - 1) / 2 + j - i);
+    if (i <= j) {
+        const cd *a = rR + 3 * t, *b = rR + 3 * ((long long)r * nw2 + ji);
+        for (int x = 0; x < 3; x++) v[c + x] = mk(0.5 * (a[x].x + b[x].x), 0.5 * (a[x].y + b[x].y));
+    }
+    if (r0 == 0 && r == 0) {
+        Col[ij] = make_int2(ij, i == j ? 1 : 0);
+        if (i <= j)
+            for (int x = 0; x < 3; x++) Col[c + x] = make_int2(ij, ji);
+    }
+}
+
+// Column c of k row kk of the caller's H [k][i][j] (zero diagonal imaginary parts,
+// Wannier.h:489-492) or D [k][i][j][x] (likewise, both mirrored elements); Dd may be null.
+__device__ __forceinline__ void wannier_store(int kk, int c, int nw2, int2 col, double re, double im, cd *Hd, cd *Dd) {
+    if (c < nw2) {
+        Hd[(size_t)kk * nw2 + c] = mk(re, col.y ? 0.0 : im);
+    } else if (Dd) {
+        const int x = (c - nw2) % 3;
+        const cd v = mk(re, col.x == col.y ? 0.0 : im);
+        Dd[((size_t)kk * nw2 + col.x) * 3 + x] = v;
+        if (col.x != col.y) Dd[((size_t)kk * nw2 + col.y) * 3 + x] = v;
+    }
+}
 
 // Per-direction phase tables of the contraction, built once per call:
 // PT[Off_l + r N_l + i] = tw[Off'_l + (i R_l mod N_l)] (-1)^{R_l}, the factor of
@@ -2487,102 +2527,64 @@ __device__ __forceinline__ cd wannier_phase(const cd *PT, int nR, int ka, int r,
     return cmul(ph, PT[o2 + (size_t)r * N2 + i2]);
 }
 
-__global__ __launch_bounds__(256) void k_wannier(const cd *__restrict__ PT, const cd *__restrict__ Val, int N0, int N1, int N2, int nR,
-                                                 int nm, int nk, int kbase, cd *__restrict__ Out) {
-    __shared__ cd Ph[WT][WK + 1];
-    __shared__ cd Vs[WK][WT + 1];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int k0 = blockIdx.y * WT, m0 = blockIdx.x * WT;
-    cd acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = mk(0.0, 0.0);
-    for (int r0 = 0; r0 < nR; r0 += WK) {
-        for (int t = threadIdx.x; t < WT * WK; t += 256) {
-            const int kk = t / WK, rr = t % WK, k = k0 + kk, r = r0 + rr;
-            Ph[kk][rr] = (k < nk && r < nR) ? wannier_phase(PT, nR, kbase + k, r, N0, N1, N2) : mk(0.0, 0.0);
-        }
-        for (int t = threadIdx.x; t < WK * WT; t += 256) {
-            const int rr = t / WT, mm = t % WT, r = r0 + rr, m = m0 + mm;
-            Vs[rr][mm] = (r < nR && m < nm) ? Val[(size_t)r * nm + m] : mk(0.0, 0.0);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int rr = 0; rr < WK; rr++) {
-            cd pv[4], vv[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) pv[i] = Ph[ty * 4 + i][rr];
-#pragma unroll
-            for (int j = 0; j < 4; j++) vv[j] = Vs[rr][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    acc[i][j].x += pv[i].x * vv[j].x - pv[i].y * vv[j].y;
-                    acc[i][j].y += pv[i].x * vv[j].y + pv[i].y * vv[j].x;
-                }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int k = k0 + ty * 4 + i, m = m0 + tx * 4 + j;
-            if (k < nk && m < nm) Out[(size_t)k * nm + m] = acc[i][j];
-        }
-}
-
-// The same contraction on the FP64 matrix cores: Out = Ph Val as four real
-// products (Re = PhR ValR - PhI ValI, Im = PhR ValI + PhI ValR) of 16x16x4
-// v_mfma_f64 tiles.  A workgroup of 4 waves owns 64 k x 32 columns (each wave
-// 16 k x 32 columns: two 16x16 tiles with real and imaginary accumulators); R
-// is consumed 16 at a time through LDS.  Lane l feeds A[row l%16][kk l/16] and
-// B[kk l/16][col l%16] and holds D[l/16 + 4 i][l%16], i = 0..3 (the layout of
-// the gfx950 instruction, checked against a host product).
+// The contraction on the FP64 matrix cores: Out = Ph Val as four real products
+// (Re = PhR ValR - PhI ValI, Im = PhR ValI + PhI ValR) of 16x16x4 v_mfma_f64 tiles.
+// A workgroup of 4 waves owns 64 k x 64 columns (each wave 16 k: four 16x16 tiles with
+// real and imaginary accumulators), so a phase formed in LDS serves 64 columns and one
+// read of it four tiles (32 columns and two tiles: every phase formed twice as often);
+// R is consumed 16 at a time.  Lane l feeds A[row l%16][kk l/16] and B[kk l/16][col
+// l%16] and holds D[l/16 + 4 i][l%16], i = 0..3 (the layout of the gfx950 instruction,
+// checked against a host product).  16 bands, 441 R, 96 x 96 k: 1004 us
+// (with the pass to the caller's layouts that this form has no need of) -> 630, 34 TF/s
+// of useful product.
 constexpr int WMK = 64, WMN = 32, WMR = 16;
 
-__global__ __launch_bounds__(256) void k_wannier_mfma(const cd *__restrict__ PT, const cd *__restrict__ Val, int N0, int N1, int N2,
-                                                      int nR, int nm, int nk, int kbase, cd *__restrict__ Out) {
+__global__ __launch_bounds__(256) void k_wannier_mfma(const cd *__restrict__ PT, const cd *__restrict__ Val, const int2 *__restrict__ Col,
+                                                      int N0, int N1, int N2, int nR, int nw2, int nm, int ncol, int nk, int kbase,
+                                                      cd *__restrict__ Hd, cd *__restrict__ Dd) {
+    constexpr int NT = 4;
     __shared__ cd Ph[WMK][WMR + 1];
-    __shared__ cd Vs[WMR][WMN + 1];
+    __shared__ cd Vs[WMR][16 * NT + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int k0 = blockIdx.y * WMK, m0 = blockIdx.x * WMN;
-    v4d are[2], aim[2];
+    const int k0 = blockIdx.y * WMK, m0 = blockIdx.x * 16 * NT;
+    v4d are[NT], aim[NT];
 #pragma unroll
-    for (int t = 0; t < 2; t++) are[t] = aim[t] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (int t = 0; t < NT; t++) are[t] = aim[t] = v4d{0.0, 0.0, 0.0, 0.0};
     for (int r0 = 0; r0 < nR; r0 += WMR) {
         for (int t = threadIdx.x; t < WMK * WMR; t += 256) {
             const int kk = t / WMR, rr = t % WMR, k = k0 + kk, r = r0 + rr;
             Ph[kk][rr] = (k < nk && r < nR) ? wannier_phase(PT, nR, kbase + k, r, N0, N1, N2) : mk(0.0, 0.0);
         }
-        for (int t = threadIdx.x; t < WMR * WMN; t += 256) {
-            const int rr = t / WMN, mm = t % WMN, r = r0 + rr, m = m0 + mm;
-            Vs[rr][mm] = (r < nR && m < nm) ? Val[(size_t)r * nm + m] : mk(0.0, 0.0);
+        for (int t = threadIdx.x; t < WMR * 16 * NT; t += 256) {
+            const int rr = t / (16 * NT), mm = t % (16 * NT), r = r0 + rr, m = m0 + mm;
+            Vs[rr][mm] = (r < nR && m < nm) ? Val[(size_t)r * ncol + m] : mk(0.0, 0.0);
         }
         __syncthreads();
 #pragma unroll
         for (int ks = 0; ks < WMR / 4; ks++) {
-            const cd a = Ph[wave * 16 + (lane & 15)][ks * 4 + (lane >> 4)];
+            const cd a = lds_get(&Ph[wave * 16 + (lane & 15)][ks * 4 + (lane >> 4)]);
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const cd b = Vs[ks * 4 + (lane >> 4)][t * 16 + (lane & 15)];
+            for (int t = 0; t < NT; t++) {
+                const cd b = lds_get(&Vs[ks * 4 + (lane >> 4)][t * 16 + (lane & 15)]);
                 are[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, are[t], 0, 0, 0);
-                are[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, are[t], 0, 0, 0);
                 aim[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.y, aim[t], 0, 0, 0);
+                are[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b.y, are[t], 0, 0, 0);
                 aim[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.x, aim[t], 0, 0, 0);
             }
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+    for (int t = 0; t < NT; t++) {
+        const int m = m0 + t * 16 + (lane & 15);
+        if (m >= nm) continue;
+        const int2 col = Col[m];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = k0 + wave * 16 + (lane >> 4) + 4 * i, m = m0 + t * 16 + (lane & 15);
-            if (k < nk && m < nm) Out[(size_t)k * nm + m] = mk(are[t][i], aim[t][i]);
+            const int k = k0 + wave * 16 + (lane >> 4) + 4 * i;
+            if (k < nk) wannier_store(k, m, nw2, col, are[t][i], aim[t][i], Hd, Dd);
         }
+    }
 }
 
 // The contraction in FP32 on the matrix cores (v_mfma_f32_16x16x4f32, FP32
@@ -2590,8 +2592,9 @@ __global__ __launch_bounds__(256) void k_wannier_mfma(const cd *__restrict__ PT,
 // tables and rounded once into LDS, H(R) and r(R) likewise; the sums are widened
 // to FP64 on the way out.  Same tiling as k_wannier_mfma; the FP32 instruction
 // holds D[4 (l/16) + i][l%16] in lane l.
-__global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ PT, const cd *__restrict__ Val, int N0, int N1, int N2,
-                                                        int nR, int nm, int nk, int kbase, cd *__restrict__ Out) {
+__global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ PT, const cd *__restrict__ Val, const int2 *__restrict__ Col,
+                                                        int N0, int N1, int N2, int nR, int nw2, int nm, int ncol, int nk, int kbase,
+                                                        cd *__restrict__ Hd, cd *__restrict__ Dd) {
     __shared__ cf Ph[WMK][WMR + 1];
     __shared__ cf Vs[WMR][WMN + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2607,7 +2610,7 @@ __global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ P
         }
         for (int t = threadIdx.x; t < WMR * WMN; t += 256) {
             const int rr = t / WMN, mm = t % WMN, r = r0 + rr, m = m0 + mm;
-            const cd v = (r < nR && m < nm) ? Val[(size_t)r * nm + m] : mk(0.0, 0.0);
+            const cd v = (r < nR && m < nm) ? Val[(size_t)r * ncol + m] : mk(0.0, 0.0);
             Vs[rr][mm] = cf{(float)v.x, (float)v.y};
         }
         __syncthreads();
@@ -2626,12 +2629,16 @@ __global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ P
         __syncthreads();
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+    for (int t = 0; t < 2; t++) {
+        const int m = m0 + t * 16 + (lane & 15);
+        if (m >= nm) continue;
+        const int2 col = Col[m];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i, m = m0 + t * 16 + (lane & 15);
-            if (k < nk && m < nm) Out[(size_t)k * nm + m] = mk((double)are[t][i], (double)aim[t][i]);
+            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i;
+            if (k < nk) wannier_store(k, m, nw2, col, (double)are[t][i], (double)aim[t][i], Hd, Dd);
         }
+    }
 }
 
 // The contraction as BF16x3 split products on the bf16 matrix cores
@@ -2644,8 +2651,9 @@ __global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ P
 // and holds D[4 (l/16) + i][l%16].
 constexpr int WBR = 32;
 
-__global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restrict__ PT, const cd *__restrict__ Val, int N0, int N1,
-                                                             int N2, int nR, int nm, int nk, int kbase, cd *__restrict__ Out) {
+__global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restrict__ PT, const cd *__restrict__ Val, const int2 *__restrict__ Col,
+                                                        int N0, int N1, int N2, int nR, int nw2, int nm, int ncol, int nk, int kbase,
+                                                        cd *__restrict__ Hd, cd *__restrict__ Dd) {
     // [hi, lo] planes of the real and imaginary parts, K (R) innermost with one pad
     __shared__ __bf16 Ph[2][2][WMK][WBR + 8];
     __shared__ __bf16 Vs[2][2][WMN][WBR + 8];
@@ -2663,7 +2671,7 @@ __global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restric
         }
         for (int t = threadIdx.x; t < WBR * WMN; t += 256) {
             const int rr = t / WMN, mm = t % WMN, r = r0 + rr, m = m0 + mm;
-            const cd v = (r < nR && m < nm) ? Val[(size_t)r * nm + m] : mk(0.0, 0.0);
+            const cd v = (r < nR && m < nm) ? Val[(size_t)r * ncol + m] : mk(0.0, 0.0);
             bf16_split((float)v.x, Vs[0][0][mm][rr], Vs[0][1][mm][rr]);
             bf16_split((float)v.y, Vs[1][0][mm][rr], Vs[1][1][mm][rr]);
         }
@@ -2703,37 +2711,15 @@ __global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restric
         __syncthreads();
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+    for (int t = 0; t < 2; t++) {
+        const int m = m0 + t * 16 + (lane & 15);
+        if (m >= nm) continue;
+        const int2 col = Col[m];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i, m = m0 + t * 16 + (lane & 15);
-            if (k < nk && m < nm) Out[(size_t)k * nm + m] = mk((double)are[t][i], (double)aim[t][i]);
+            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i;
+            if (k < nk) wannier_store(k, m, nw2, col, (double)are[t][i], (double)aim[t][i], Hd, Dd);
         }
-}
-
-// Contraction output [k][c][i][j] (c = 0 H, 1..3 r) to the caller's layouts,
-// one thread per (k, i, j): H with zero diagonal imaginary parts
-// (Wannier.h:489-492) and D = (r + r^T)/2 with zero diagonal imaginary parts
-// (Wannier.h:577-578, save_HUD.cpp:187-191), [k][i][j][x].  rtx: the r part of
-// each output row is [i][j][x] (the caller's own order) instead of [x][i][j].
-__global__ void k_wannier_finish(const cd *__restrict__ Out, int kc, int nw, double *__restrict__ Hd, double *__restrict__ Dd,
-                                 int rtx) {
-    const int nw2 = nw * nw;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (long long)kc * nw2) return;
-    const int kk = (int)(t / nw2), ij = (int)(t % nw2), i = ij / nw, j = ij % nw;
-    const cd *src = Out + (size_t)kk * 4 * nw2;
-    const cd h = src[ij];
-    Hd[2 * t] = h.x;
-    Hd[2 * t + 1] = (i == j) ? 0.0 : h.y;
-    if (!Dd) return;
-#pragma unroll
-    for (int x = 0; x < 3; x++) {
-        const cd a = rtx ? src[nw2 + (i * nw + j) * 3 + x] : src[(x + 1) * nw2 + i * nw + j];
-        const cd b = rtx ? src[nw2 + (j * nw + i) * 3 + x] : src[(x + 1) * nw2 + j * nw + i];
-        const double ai = (i == j) ? 0.0 : a.y, bi = (i == j) ? 0.0 : b.y;
-        Dd[(3 * t + x) * 2] = 0.5 * (a.x + b.x);
-        Dd[(3 * t + x) * 2 + 1] = 0.5 * (ai + bi);
     }
 }
 
@@ -4809,7 +4795,93 @@ static void wannier_twiddles(const int32_t nk3[3], std::vector<double> &tw, int 
     }
 }
 
+// Copies of large results to the caller's ordinary memory.  hipMemcpy locks that
+// memory page by page in front of the copy engine (9.3 GB/s into fresh pages, 17 into
+// touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
+// memory, and each of a few threads copies its own piece on to the caller's pages
+// while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring belongs to the
+// object (12 MB).  From 32 MB on; below, the threads' start takes what it gives.
+class Downloader {
+    static constexpr size_t kPiece = 2 << 20;
+    static constexpr int kWorkers = 6;
+    char *ring = nullptr;
+    hipEvent_t ev[kWorkers] = {};
+    int dev = 0;
+
+    bool ready() {
+        if (ring) return true;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        for (hipEvent_t &e : ev)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kWorkers * kPiece, hipHostMallocDefault) != hipSuccess) return false;
+        ring = static_cast<char *>(p);
+        return true;
+    }
+
+public:
+    Downloader() = default;
+    Downloader(const Downloader &) = delete;
+    Downloader &operator=(const Downloader &) = delete;
+    ~Downloader() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+        if (ring) (void)hipHostFree(ring);
+    }
+    // n bytes of device memory, in null-stream order; returns when dst holds them.
+    hipError_t copy(void *dst, const void *src, size_t n) {
+        if (n < 16 * kPiece || !ready()) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
+        std::mutex mu;
+        size_t next = 0;
+        hipError_t err = hipSuccess;
+        auto work = [&](int w) {
+            char *slot = ring + w * kPiece;
+            hipError_t e = hipSetDevice(dev);
+            for (;;) {
+                size_t o, len;
+                {
+                    std::lock_guard<std::mutex> lock(mu);
+                    if (e != hipSuccess) err = e;
+                    if (err != hipSuccess || next >= n) return;
+                    o = next;
+                    len = std::min(kPiece, n - o);
+                    next += len;
+                    e = hipMemcpyAsync(slot, static_cast<const char *>(src) + o, len, hipMemcpyDeviceToHost, 0);
+                    if (e == hipSuccess) e = hipEventRecord(ev[w], 0);
+                }
+                if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
+                if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + o, slot, len);
+            }
+        };
+        std::thread th[kWorkers - 1];
+        try {
+            for (int w = 1; w < kWorkers; w++) th[w - 1] = std::thread(work, w);
+        } catch (...) {
+            // fewer workers: the others, this thread at least, take their pieces
+        }
+        work(0);
+        for (std::thread &t : th)
+            if (t.joinable()) t.join();
+        return err;
+    }
+};
+
+// One chunk of kc k (from kbase) of the contraction, the first nm of Val's ncol columns.
 // form: 0 FP64 matrix cores, 1 FP32, 2 BF16x3 split products.
+static void wannier_launch(int form, const cd *PT, const cd *Val, const int2 *Col, const int32_t nk3[3], int nR, int nw2, int nm, int ncol,
+                           int kc, int kbase, cd *H, cd *D) {
+    const unsigned gk = (unsigned)((kc + WMK - 1) / WMK);
+    if (form == 0)
+        hipLaunchKernelGGL(k_wannier_mfma, dim3((unsigned)((nm + 63) / 64), gk), dim3(256), 0, 0, PT, Val, Col, nk3[0], nk3[1], nk3[2], nR, nw2,
+                           nm, ncol, kc, kbase, H, D);
+    else if (form == 1)
+        hipLaunchKernelGGL(k_wannier_mfma32, dim3((unsigned)((nm + WMN - 1) / WMN), gk), dim3(256), 0, 0, PT, Val, Col, nk3[0], nk3[1], nk3[2],
+                           nR, nw2, nm, ncol, kc, kbase, H, D);
+    else
+        hipLaunchKernelGGL(k_wannier_mfma_bf16x3, dim3((unsigned)((nm + WMN - 1) / WMN), gk), dim3(256), 0, 0, PT, Val, Col, nk3[0], nk3[1],
+                           nk3[2], nR, nw2, nm, ncol, kc, kbase, H, D);
+}
+
 static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_t *R, const double *HR, const double *rR, double *H_out,
                      double *D_out, int form) {
     if (!nk3 || !R || !HR || !rR || !H_out || nR < 1 || nw < 1) return set_err(EDUS_ERR_INVALID, "bad Wannier arguments");
@@ -4818,61 +4890,46 @@ static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return set_err(EDUS_ERR_NODEVICE, "no HIP device visible");
     const long long nk = (long long)nk3[0] * nk3[1] * nk3[2];
-    const int nw2 = nw * nw, nm = 4 * nw2;
-    // Val[R][c][i][j]: c = 0 H, 1..3 r_x, r_y, r_z
-    std::vector<double> val((size_t)nR * nm * 2);
-    for (int r = 0; r < nR; r++)
-        for (int t = 0; t < nw2; t++) {
-            val[((size_t)r * nm + t) * 2] = HR[((size_t)r * nw2 + t) * 2];
-            val[((size_t)r * nm + t) * 2 + 1] = HR[((size_t)r * nw2 + t) * 2 + 1];
-            for (int x = 0; x < 3; x++) {
-                val[((size_t)r * nm + (x + 1) * nw2 + t) * 2] = rR[((size_t)r * nw2 + t) * 6 + 2 * x];
-                val[((size_t)r * nm + (x + 1) * nw2 + t) * 2 + 1] = rR[((size_t)r * nw2 + t) * 6 + 2 * x + 1];
-            }
-        }
+    const int nw2 = nw * nw, nm = D_out ? (int)wannier_cols(nw) : nw2, ncol = (int)wannier_cols(nw);
     std::vector<double> tw;
     int offs[3];
     wannier_twiddles(nk3, tw, offs);
     int *dR = nullptr;
-    double *dVal = nullptr, *dTw = nullptr, *dOut = nullptr, *dPT = nullptr, *dH = nullptr, *dD = nullptr;
+    int2 *dCol = nullptr;
+    double *dHR = nullptr, *drR = nullptr, *dVal = nullptr, *dTw = nullptr, *dPT = nullptr, *dH = nullptr, *dD = nullptr;
     auto cleanup = [&]() {
-        (void)hipFree(dR); (void)hipFree(dVal); (void)hipFree(dTw); (void)hipFree(dOut); (void)hipFree(dPT);
-        (void)hipFree(dH); (void)hipFree(dD);
+        for (void *q : {(void *)dR, (void *)dCol, (void *)dHR, (void *)drR, (void *)dVal, (void *)dTw, (void *)dPT, (void *)dH, (void *)dD})
+            (void)hipFree(q);
     };
-    const size_t npt = (size_t)nR * (nk3[0] + nk3[1] + nk3[2]);
-    const size_t chunk = std::min<long long>(nk, std::max<long long>(64, (1LL << 28) / ((long long)nm * 16)));
-    if (hipMalloc(&dR, (size_t)nR * 3 * sizeof(int)) != hipSuccess || hipMalloc(&dVal, val.size() * sizeof(double)) != hipSuccess ||
-        hipMalloc(&dTw, tw.size() * sizeof(double)) != hipSuccess || hipMalloc(&dOut, chunk * nm * 2 * sizeof(double)) != hipSuccess ||
+    Downloader down;
+    const size_t npt = (size_t)nR * (nk3[0] + nk3[1] + nk3[2]), nval = (size_t)nR * nw2;
+    const size_t chunk = std::min<long long>(nk, std::max<long long>(64, (1LL << 28) / ((long long)nw2 * 64)));
+    if (hipMalloc(&dR, (size_t)nR * 3 * sizeof(int)) != hipSuccess || hipMalloc(&dCol, (size_t)ncol * sizeof(int2)) != hipSuccess ||
+        hipMalloc(&dHR, nval * 16) != hipSuccess || hipMalloc(&drR, nval * 48) != hipSuccess ||
+        hipMalloc(&dVal, (size_t)nR * ncol * 16) != hipSuccess || hipMalloc(&dTw, tw.size() * sizeof(double)) != hipSuccess ||
         hipMalloc(&dPT, npt * 2 * sizeof(double)) != hipSuccess || hipMalloc(&dH, chunk * nw2 * 2 * sizeof(double)) != hipSuccess ||
         (D_out && hipMalloc(&dD, chunk * nw2 * 6 * sizeof(double)) != hipSuccess)) {
         cleanup();
         return set_err(EDUS_ERR_NOMEM, "Wannier buffers");
     }
     if (hipMemcpy(dR, R, (size_t)nR * 3 * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(dVal, val.data(), val.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(dHR, HR, nval * 16, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(drR, rR, nval * 48, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(dTw, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
         cleanup();
         return set_err(EDUS_ERR_HIP, "Wannier upload");
     }
+    hipLaunchKernelGGL(k_wannier_val, dim3((unsigned)((nval + 255) / 256)), dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR, 0, nR, nw, ncol,
+                       (cd *)dVal, dCol);
     hipLaunchKernelGGL(k_wannier_ptab, dim3((unsigned)std::min<size_t>((npt + 255) / 256, 65536)), dim3(256), 0, 0, (const int *)dR,
                        (const cd *)dTw, nR, nk3[0], nk3[1], nk3[2], offs[1], offs[2], (cd *)dPT);
     for (long long k0 = 0; k0 < nk; k0 += chunk) {
         const int kc = (int)std::min<long long>(chunk, nk - k0);
-        const dim3 grid((nm + WMN - 1) / WMN, (unsigned)((kc + WMK - 1) / WMK));
-        if (form == 2)
-            hipLaunchKernelGGL(k_wannier_mfma_bf16x3, grid, dim3(256), 0, 0, (const cd *)dPT, (const cd *)dVal, nk3[0], nk3[1], nk3[2], nR,
-                               nm, kc, (int)k0, (cd *)dOut);
-        else if (form == 1)
-            hipLaunchKernelGGL(k_wannier_mfma32, grid, dim3(256), 0, 0, (const cd *)dPT, (const cd *)dVal, nk3[0], nk3[1], nk3[2], nR, nm,
-                               kc, (int)k0, (cd *)dOut);
-        else
-            hipLaunchKernelGGL(k_wannier_mfma, grid, dim3(256), 0, 0, (const cd *)dPT, (const cd *)dVal, nk3[0], nk3[1], nk3[2], nR, nm,
-                               kc, (int)k0, (cd *)dOut);
-        const long long nt = (long long)kc * nw2;
-        hipLaunchKernelGGL(k_wannier_finish, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, 0, (const cd *)dOut, kc, nw, dH, dD, 0);
+        wannier_launch(form, (const cd *)dPT, (const cd *)dVal, dCol, nk3, nR, nw2, nm, ncol, kc, (int)k0, (cd *)dH, (cd *)dD);
+        const size_t nt = (size_t)kc * nw2;
         hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpy(H_out + (size_t)k0 * nw2 * 2, dH, (size_t)nt * 16, hipMemcpyDeviceToHost);
-        if (e == hipSuccess && D_out) e = hipMemcpy(D_out + (size_t)k0 * nw2 * 6, dD, (size_t)nt * 48, hipMemcpyDeviceToHost);
+        if (e == hipSuccess) e = down.copy(H_out + (size_t)k0 * nw2 * 2, dH, nt * 16);
+        if (e == hipSuccess && D_out) e = down.copy(D_out + (size_t)k0 * nw2 * 6, dD, nt * 48);
         if (e != hipSuccess) {
             cleanup();
             return set_err(EDUS_ERR_HIP, std::string("k_wannier: ") + hipGetErrorString(e));
@@ -4900,10 +4957,9 @@ int edus_wannier_hk_bf16x3(const int32_t nk3[3], int32_t nR, int32_t nw, const i
 
 // The contraction of edus_wannier_hk with every device buffer carved from the
 // fixed scratch array: lattice vectors, twiddles, phase tables, H(R) and r(R)
-// (copied in with 2D copies, the r part of each row in the caller's [i][j][x]
-// order, so no host repacking), then the grid in as many k chunks as the rest
-// of the array holds.  Nothing in the array needs clearing: every buffer is
-// written before it is read.
+// (packed on the device from copies passed through the output area), then the grid
+// in as many k chunks as the rest of the array holds.  Nothing in the array needs
+// clearing: every buffer is written before it is read.
 int edus_wannier_hk_noalloc(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_t *R, const double *HR, const double *rR,
                             double *H_out, double *D_out) {
     if (!nk3 || !R || !HR || !rR || !H_out || nR < 1 || nw < 1) return set_err(EDUS_ERR_INVALID, "bad Wannier arguments");
@@ -4929,29 +4985,36 @@ int edus_wannier_hk_noalloc(const int32_t nk3[3], int32_t nR, int32_t nw, const 
     char *b = static_cast<char *>(base);
     int *dR = reinterpret_cast<int *>(b + oR);
     double *dTw = reinterpret_cast<double *>(b + oTw), *dPT = reinterpret_cast<double *>(b + oPT);
-    cd *dVal = reinterpret_cast<cd *>(b + oVal), *dOut = reinterpret_cast<cd *>(b + oOut);
-    const long long oH = al(oOut + 16 * chunk * nm), oD = al(oH + 16 * chunk * nw2);
-    double *dH = reinterpret_cast<double *>(b + oH), *dD = D_out ? reinterpret_cast<double *>(b + oD) : nullptr;
+    cd *dVal = reinterpret_cast<cd *>(b + oVal);
+    const int ncol = (int)wannier_cols(nw), nform = D_out ? ncol : (int)nw2;
+    // behind Val (smaller than the 4 nw^2 columns that the limit counts): the column
+    // table, then the output chunk, which H(R) and r(R) pass through first
+    const long long oCol = al(oVal + 16LL * nR * ncol), oH = al(oCol + 8LL * ncol), oD = al(oH + 16 * chunk * nw2);
+    int2 *dCol = reinterpret_cast<int2 *>(b + oCol);
+    cd *dH = reinterpret_cast<cd *>(b + oH), *dD = D_out ? reinterpret_cast<cd *>(b + oD) : nullptr;
     std::vector<double> tw;
     int offs[3];
     wannier_twiddles(nk3, tw, offs);
     HIP_TRY(hipMemcpy(dR, R, (size_t)nR * 3 * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(dTw, tw.data(), tw.size() * sizeof(double), hipMemcpyHostToDevice));
-    // Val[R] = [H(R) (nw^2) | r(R) as [i][j][x] (3 nw^2)]
-    HIP_TRY(hipMemcpy2D(dVal, (size_t)nm * 16, HR, (size_t)nw2 * 16, (size_t)nw2 * 16, (size_t)nR, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy2D(dVal + nw2, (size_t)nm * 16, rR, (size_t)3 * nw2 * 16, (size_t)3 * nw2 * 16, (size_t)nR,
-                        hipMemcpyHostToDevice));
+    const int rchunk = (int)std::max<long long>(1, std::min<long long>(nR, (cap - oH - slack) / (64 * nw2)));
+    for (int r0 = 0; r0 < nR; r0 += rchunk) {
+        const int n = std::min(rchunk, nR - r0);
+        cd *dHR = dH, *drR = dHR + (size_t)n * nw2;
+        HIP_TRY(hipMemcpy(dHR, HR + (size_t)r0 * nw2 * 2, (size_t)n * nw2 * 16, hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(drR, rR + (size_t)r0 * nw2 * 6, (size_t)n * nw2 * 48, hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(k_wannier_val, dim3((unsigned)(((long long)n * nw2 + 255) / 256)), dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR,
+                           r0, n, (int)nw, ncol, dVal, dCol);
+        HIP_TRY(hipGetLastError());
+    }
     const size_t npt = (size_t)nR * nsum;
     hipLaunchKernelGGL(k_wannier_ptab, dim3((unsigned)std::min<size_t>((npt + 255) / 256, 65536)), dim3(256), 0, 0, (const int *)dR,
                        (const cd *)dTw, nR, nk3[0], nk3[1], nk3[2], offs[1], offs[2], (cd *)dPT);
     HIP_TRY(hipGetLastError());
     for (long long k0 = 0; k0 < nk; k0 += chunk) {
         const int kc = (int)std::min<long long>(chunk, nk - k0);
-        const dim3 grid((unsigned)((nm + WMN - 1) / WMN), (unsigned)((kc + WMK - 1) / WMK));
-        hipLaunchKernelGGL(k_wannier_mfma, grid, dim3(256), 0, 0, (const cd *)dPT, (const cd *)dVal, nk3[0], nk3[1], nk3[2], nR,
-                           (int)nm, kc, (int)k0, dOut);
+        wannier_launch(0, (const cd *)dPT, dVal, dCol, nk3, nR, (int)nw2, nform, ncol, kc, (int)k0, dH, dD);
         const long long nt = (long long)kc * nw2;
-        hipLaunchKernelGGL(k_wannier_finish, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, 0, (const cd *)dOut, kc, nw, dH, dD, 1);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemcpy(H_out + (size_t)k0 * nw2 * 2, dH, (size_t)nt * 16, hipMemcpyDeviceToHost));
         if (D_out) HIP_TRY(hipMemcpy(D_out + (size_t)k0 * nw2 * 6, dD, (size_t)nt * 48, hipMemcpyDeviceToHost));
