@@ -68,6 +68,7 @@ struct ConstArgs {
     const int *nbr;      // [n_nbr][nkp]
     const int *eidx;     // packed element e -> i | j << 8 | comp << 16 (wave layout)
     int nk, nkp, nb, nch, ncc, n_nbr, diss, dherm;  // dherm: D_ji = conj(D_ij) (else D_ji = D_ij)
+    int hole;            // some filled band has T_vv != 0 (else the hole source is an exact zero and is not formed)
     int sw, scol;        // wave kernels: strip width and row length of the workgroup order (sw = 0: k order)
     // Wave kernels of one k per workgroup: pair = 1 when every pair of k (2q, 2q+1)
     // has the same stencil overlap (a uniform grid of even length along the
@@ -498,7 +499,7 @@ __device__ __forceinline__ void small_dephasing(const ConstArgs &c, const double
             cd hole = mk(0.0, 0.0);
 #pragma unroll
             for (int v = 0; v < NB; v++)  // static indices keep U in registers
-                if (v < c.ncc) hole = cadd(hole, cscale(cmul(cconj(U[v][j]), U[v][i]), *gm(c.T + v * NB + v)));
+                if (c.hole && v < c.ncc) hole = cadd(hole, cscale(cmul(cconj(U[v][j]), U[v][i]), *gm(c.T + v * NB + v)));
             if (i == j) {
                 pv[i] = hole.x - w.x;
             } else {
@@ -749,50 +750,58 @@ constexpr int kCoulThreads = 256;
 // cores (a thread per output with a sequential sum took 28 us at 300 x 300,
 // bound by the address throughput of its uncoalesced loads): rows r = e N1 + i1
 // (the state row Y[e][i1 N2 + i2], contiguous in i2), columns c = q ncut + n
-// (q = 0: cos, 1: sin), K = N2.  One wave per 16 x 16 tile walks K four at a
-// time with v_mfma_f64_16x16x4f64 (lane l feeds A[row l%16][k l/16] and
+// (q = 0: cos, 1: sin), K = N2.  One workgroup per 16 x 16 tile; its four waves take
+// a quarter of K each and are added in wave order.  A wave walks its quarter four k at
+// a time with v_mfma_f64_16x16x4f64 (lane l feeds A[row l%16][k l/16] and
 // B[k l/16][col l%16] and ends with C[l/16 + 4 i][l%16]); out-of-range rows,
-// columns and k are fed zeros.
-__global__ __launch_bounds__(64) void k_coul_s1_mfma(CoulArgs a) {
+// columns and k are fed zeros.  The pass waits for its loads: one wave per tile with 16
+// of them in flight took 13.8 us at 300 x 300, this form 11.1.
+__global__ __launch_bounds__(256) void k_coul_s1_mfma(CoulArgs a) {
     typedef double v4 __attribute__((ext_vector_type(4)));
-    const int lane = threadIdx.x, r0 = blockIdx.x * 16, c0 = blockIdx.y * 16;
+    constexpr int KB = 12;  // k slices of four whose loads are in flight together
+    __shared__ double red[3][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r0 = blockIdx.x * 16, c0 = blockIdx.y * 16;
     const int nrow = a.NP * a.N1, ncol = 2 * a.ncut;
     const int ra = r0 + (lane & 15), cb = c0 + (lane & 15), kq = lane >> 4;
     const bool rok = ra < nrow, cok = cb < ncol;
     const double *yrow = a.Y + (rok ? (size_t)(ra / a.N1) * a.nkp + (size_t)(ra % a.N1) * a.N2 : 0);
     const int q = cok ? cb / a.ncut : 0, n = cok ? cb % a.ncut : 0;
     const double *trig = (q ? a.syn : a.cyn) + (size_t)n * a.N2;
+    const int per = ((a.N2 + 15) / 16) * 4, kbeg = wave * per, kend = min(a.N2, kbeg + per);
     v4 acc = {0.0, 0.0, 0.0, 0.0};
-    // K in blocks of 32: the block's 16 loads (at a clamped k, always in
-    // bounds) are all issued before its 8 products; values past the edges are
-    // zeroed after loading.
-    for (int k0 = 0; k0 < a.N2; k0 += 32) {
-        double yv[8], tv[8];
+    for (int k0 = kbeg; k0 < kend; k0 += 4 * KB) {
+        double yv[KB], tv[KB];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < KB; u++) {
             const int kc = min(k0 + 4 * u + kq, a.N2 - 1);
             yv[u] = yrow[kc];
             tv[u] = trig[kc];
         }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const bool kok = k0 + 4 * u + kq < a.N2;
+        for (int u = 0; u < KB; u++) {
+            const bool kok = k0 + 4 * u + kq < kend;
             acc = __builtin_amdgcn_mfma_f64_16x16x4f64((rok && kok) ? yv[u] : 0.0, (cok && kok) ? tv[u] : 0.0, acc, 0, 0, 0);
         }
     }
+    if (wave > 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[wave - 1][i][lane] = acc[i];
+    }
+    __syncthreads();
+    if (wave > 0) return;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int r = r0 + (lane >> 4) + 4 * i, c = c0 + (lane & 15);
         if (r < nrow && c < ncol) {
             const int e = r / a.N1, i1 = r % a.N1, qq = c / a.ncut, nn = c % a.ncut;
-            a.S[(((size_t)qq * a.N1 + i1) * a.ncut + nn) * a.NP + e] = acc[i];
+            a.S[(((size_t)qq * a.N1 + i1) * a.ncut + nn) * a.NP + e] = ((acc[i] + red[0][i][lane]) + red[1][i][lane]) + red[2][i][lane];
         }
     }
 }
 
 // F_xy[mm][e] = w (1 + corr_mn) sum_i1 x_m(i1) S_y[i1][n][e]: one workgroup per
 // mm; thread t takes element e = t % NP and every (256/NP)-th term of the sum,
-// and the parts are added in a fixed order per element.  The same workgroup then
+// and the parts are added in a fixed tree per element (10.0 -> 8.6 us at 300 x 300).  The same workgroup then
 // forms X_mn from its F (coul_x_elem) and, for mm = 0, the Hartree shift: X_mn
 // needs no other mode's F, so no launch of its own.
 constexpr int kCoulMaxNP = 16;  // the mean field runs at nb <= 4
@@ -806,6 +815,7 @@ __global__ __launch_bounds__(kCoulThreads) void k_coul_s2(CoulArgs a) {
     const int NP = a.NP, nparts = kCoulThreads / NP, e = t % NP, part = t / NP;
     double cc = 0, cs = 0, sc = 0, ss = 0;
     if (part < nparts) {
+#pragma unroll 4
         for (int i1 = part; i1 < a.N1; i1 += nparts) {
             const double xc = a.cxm[m * a.N1 + i1], xs = a.sxm[m * a.N1 + i1];
             const double yc = a.S[(((size_t)0 * a.N1 + i1) * a.ncut + n) * NP + e];
@@ -820,16 +830,24 @@ __global__ __launch_bounds__(kCoulThreads) void k_coul_s2(CoulArgs a) {
     red[1][t] = cs;
     red[2][t] = sc;
     red[3][t] = ss;
+    // the parts in a fixed tree (one after the other they took half of the pass)
+    int h = 1;
+    while (h < nparts) h *= 2;
+    for (h /= 2; h > 0; h /= 2) {
+        __syncthreads();
+        if (part < h && part + h < nparts) {
+#pragma unroll
+            for (int qd = 0; qd < 4; qd++) red[qd][t] += red[qd][t + h * NP];
+        }
+    }
     __syncthreads();
-    if (t < NP) {
+    if (t < 4 * NP) {
         const double corr = -4 * M_PI * M_PI * (m * m + n * n) / ((double)a.nk * 27);
         const double f = a.w * (1. + corr);
-        for (int qd = 0; qd < 4; qd++) {
-            double v = 0.0;
-            for (int q = 0; q < nparts; q++) v += red[qd][q * NP + t];
-            a.F[((size_t)qd * nmm + mm) * NP + t] = v * f;
-            Fs[qd][t] = v * f;
-        }
+        const int qd = t / NP, el = t % NP;
+        const double v = red[qd][el] * f;
+        a.F[((size_t)qd * nmm + mm) * NP + el] = v;
+        Fs[qd][el] = v;
     }
     __syncthreads();
     if (mm == 0 && t < a.nb) {  // Hartree shift from mode 0 (Coulomb.h:385-410)
@@ -885,7 +903,7 @@ __device__ __forceinline__ void coul_x_elem(const CoulArgs &a, const double (*Fs
 
 // Column sums of the reconstruction for upper element u = (i <= j), which reads
 // (X_mn)_{ji} because the reference stores X_{jc,ic} (Coulomb.h:537).
-__global__ void k_coul_s3(CoulArgs a) {
+__global__ __launch_bounds__(64) void k_coul_s3(CoulArgs a) {
     const int nb = a.nb, nmm = a.ncut * a.ncut, nb2 = nb * nb;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.N2 * a.ncut * a.nu) return;
@@ -897,13 +915,14 @@ __global__ void k_coul_s3(CoulArgs a) {
     }
     const cd *X = reinterpret_cast<const cd *>(a.X);
     cd tc = mk(0, 0), ts = mk(0, 0);
-    // n in blocks of 4: the block's loads (at a clamped n) are issued together,
+    constexpr int NBLK = 10;  // of 4: 6.6 us at 300 x 300, of 10 5.7
+    // n in blocks of NBLK: the block's loads (at a clamped n) are issued together,
     // the sums keep the order of n.
-    for (int n0 = 0; n0 < a.ncut; n0 += 4) {
-        cd xv[4][4];
-        double ycv[4], ysv[4];
+    for (int n0 = 0; n0 < a.ncut; n0 += NBLK) {
+        cd xv[NBLK][4];
+        double ycv[NBLK], ysv[NBLK];
 #pragma unroll
-        for (int b = 0; b < 4; b++) {
+        for (int b = 0; b < NBLK; b++) {
             const int n = min(n0 + b, a.ncut - 1);
             const size_t d = (size_t)(m * a.ncut + n) * nb2 + j * nb + i;
 #pragma unroll
@@ -912,7 +931,7 @@ __global__ void k_coul_s3(CoulArgs a) {
             ysv[b] = a.syn[n * a.N2 + i2];
         }
 #pragma unroll
-        for (int b = 0; b < 4; b++)
+        for (int b = 0; b < NBLK; b++)
             if (n0 + b < a.ncut) {
                 tc = cadd(tc, cadd(cscale(xv[b][0], ycv[b]), cscale(xv[b][1], ysv[b])));
                 ts = cadd(ts, cadd(cscale(xv[b][2], ycv[b]), cscale(xv[b][3], ysv[b])));
@@ -939,7 +958,7 @@ __global__ void k_coul_s3(CoulArgs a) {
 template <bool FULL>
 __global__ __launch_bounds__(64) void k_coul_w_mfma(CoulArgs a, CoulHArgs h) {
     typedef double v4 __attribute__((ext_vector_type(4)));
-    constexpr int KB = 16;  // K terms loaded per block (2 Ncut <= 64)
+    constexpr int KB = 40;  // K terms loaded per block (2 Ncut <= 64)
     const int lane = threadIdx.x, r0 = blockIdx.x * 16, c0 = blockIdx.y * 16, nb = a.nb;
     const int ncut = a.ncut, K = 2 * ncut, ncol = (FULL ? a.NP : 2 * a.nu) * a.N2, N1 = a.N1;
     const int ra = r0 + (lane & 15), cb = c0 + (lane & 15), kq = lane >> 4;
@@ -1455,6 +1474,29 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     // (ROLE 1): every neighbour of k that is also one of kb's adds to kb's sum gb
     // as well, and kb's remaining neighbours are fetched after k's.  Second of a
     // pair (ROLE 2): the sum is gb.
+    // The dephasing's U and rates, requested before the drift and the products that
+    // come first (loaded where they are used, each k waited for them: AB4 step of 13
+    // bands on 61 x 85 k 50.4 us -> 41.9).
+    constexpr bool kPreDiss = NBT == 16 && ROLE == 0;  // elsewhere the registers are taken
+    R ur[kPreDiss ? PER : 1], ui[kPreDiss ? PER : 1], tr[4];
+    if constexpr (kPreDiss) {
+        if (c.diss) {
+            const R *u = Uop + (size_t)k * nb * nb * 2;
+#pragma unroll
+            for (int m = 0; m < PER; m++) {
+                const int t = min(lane + TPK * m, nb * nb - 1);
+                ld2<true>(u, 2 * t, 2 * t + 1, true, ur[m], ui[m]);
+            }
+            if constexpr (kMfma) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    int ia, ib;
+                    mfma_elem<NBT, R>(lane, i, ia, ib);
+                    tr[i] = (ia < nb && ib < nb) ? (R)*gm(c.T + ia * nb + ib) : (R)0;
+                }
+            }
+        }
+    }
     if constexpr (ROLE == 2) {
 #pragma unroll
         for (int m = 0; m < PER; m++) g[m] = gb[m];
@@ -1591,8 +1633,20 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     if (c.diss) {
         __syncthreads();
         // C <- U
-        const R *u = Uop + (size_t)k * nb * nb * 2;
-        for (int t = lane; t < nb * nb; t += TPK) C[(t / nb) * LD + (t % nb)] = CT{ldnt(u + 2 * t), ldnt(u + 2 * t + 1)};
+        if constexpr (kPreDiss) {
+#pragma unroll
+            for (int m = 0; m < PER; m++) {
+                const int t = min(lane + TPK * m, nb * nb - 1);
+                lds_put(C + (t / nb) * LD + (t % nb), CT{ur[m], ui[m]});
+            }
+        } else {
+            const R *u = Uop + (size_t)k * nb * nb * 2;
+            for (int t = lane; t < nb * nb; t += TPK) {
+                R re, im;
+                ld2<true>(u, 2 * t, 2 * t + 1, true, re, im);
+                lds_put(C + (t / nb) * LD + (t % nb), CT{re, im});
+            }
+        }
         __syncthreads();
         if constexpr (kMfma) {
             typename MfmaAcc<R>::T cre, cim;
@@ -1605,7 +1659,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             for (int i = 0; i < 4; i++) {
                 int ia, ib;
                 mfma_elem<NBT, R>(lane, i, ia, ib);
-                const R t = (ia < nb && ib < nb) ? (R)*gm(c.T + ia * nb + ib) : (R)0;
+                const R t = kPreDiss ? tr[i] : (ia < nb && ib < nb) ? (R)*gm(c.T + ia * nb + ib) : (R)0;
                 cre[i] *= t;
                 cim[i] *= t;
             }
@@ -1657,7 +1711,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             const int i = ei[m], j = ej[m];
             const CT w = A[i * LD + j];
             CT hole = CT{0, 0};
-            for (int v = 0; v < c.ncc; v++) {
+            for (int v = 0; v < (c.hole ? c.ncc : 0); v++) {
                 const CT uj = C[v * LD + j], ui = C[v * LD + i];
                 const R tv = (R)*gm(c.T + v * nb + v);
                 // conj(U[v][j]) U[v][i] T[v][v]
@@ -1702,7 +1756,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 // One k per workgroup, or with PAIR (ConstArgs::pair, one k per workgroup only)
 // the stencil pair (2q, 2q + 1).
 template <int NBT, int MODE, typename R, typename S = double, bool B3 = false, bool PAIR = false>
-__global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB) void k_stage_wave(ConstArgs c, StageArgs a) {
+__global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB, (NBT == 16 && !PAIR ? 3 : 1)) void k_stage_wave(ConstArgs c, StageArgs a) {
     extern __shared__ double smem_d[];
     constexpr int TPK = WaveGeom<NBT>::TPK;
     double gb[WaveGeom<NBT>::PER];
@@ -3009,7 +3063,7 @@ struct edus_ctx {
     int dev = 0;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    int nk = 0, nkp = 0, nb = 0, np = 0, nch = 0, ncc = 0, n_nbr = 0, stepper = 0, order = 1, diss = 0, dherm = 0;
+    int nk = 0, nkp = 0, nb = 0, np = 0, nch = 0, ncc = 0, n_nbr = 0, stepper = 0, order = 1, diss = 0, dherm = 0, hole = 0;
     int sw = 0, scol = 0;  // strip order of the wave kernels (strip_k)
     int pair = 0, pself = -1, npnew = 0;  // stencil pairs of the wave kernels (ConstArgs::pair)
     int tpb = 0;           // k per workgroup of the nb <= 4 kernel (0: small_group's choice)
@@ -3201,7 +3255,7 @@ int launch_coulomb(edus_ctx *c, const double *Y) {
     const int t3 = c->N2 * c->ncut * c->nu;
     // 64-thread workgroups: the passes have a few 10^4 outputs each, and small
     // workgroups spread them over all CUs.  Pass 1 runs a wave per 16 x 16 tile.
-    hipLaunchKernelGGL(k_coul_s1_mfma, dim3((c->np * c->N1 + 15) / 16, (2 * c->ncut + 15) / 16), dim3(64), 0, c->stream, a);
+    hipLaunchKernelGGL(k_coul_s1_mfma, dim3((c->np * c->N1 + 15) / 16, (2 * c->ncut + 15) / 16), dim3(256), 0, c->stream, a);
     hipLaunchKernelGGL(k_coul_s2, dim3(c->ncut * c->ncut), dim3(kCoulThreads), 0, c->stream, a);
     hipLaunchKernelGGL(k_coul_s3, dim3((t3 + 63) / 64), dim3(64), 0, c->stream, a);
     HIP_TRY(hipGetLastError());
@@ -3247,9 +3301,18 @@ ConstArgs const_args(const edus_ctx *c) {
     ca.H = c->coul ? c->cHr : c->H; ca.D = c->D; ca.U = c->U; ca.T = c->T; ca.nbr = c->nbr;
     ca.Hf = c->Hf; ca.Df = c->Df; ca.Uf = c->Uf; ca.eidx = c->eidx;
     ca.nk = c->nk; ca.nkp = c->nkp; ca.nb = c->nb; ca.nch = c->nch; ca.ncc = c->ncc; ca.n_nbr = c->n_nbr;
-    ca.diss = c->diss; ca.dherm = c->dherm; ca.wx2 = c->wx2; ca.sw = c->sw; ca.scol = c->scol;
+    ca.diss = c->diss; ca.hole = c->hole; ca.dherm = c->dherm; ca.wx2 = c->wx2; ca.sw = c->sw; ca.scol = c->scol;
     ca.pair = c->pair; ca.pself = c->pself; ca.npnew = c->npnew; ca.pat = c->nbr + (size_t)std::max(c->n_nbr, 1) * c->nkp;
     return ca;
+}
+
+// Whether the stage kernels of a context serve stencil pairs (nb > 8; see
+// stencil_pairs): not in the BF16x3 form, whose split products leave no registers for
+// the second k's stencil sum, and not at 9..16 bands with dephasing, where the
+// dephasing's own operands are worth them more (AB4 step of 16 bands, 100 x 100 k: 81
+// us paired, 66 with one k per workgroup; RK4 stages of 60 x 60 k even).
+bool runs_paired(const edus_ctx *c) {
+    return c->pair && c->precision != EDUS_PRECISION_BF16X3 && !(c->diss && c->nb <= 16);
 }
 
 // k per workgroup of the nb <= 4 kernel: 64 unless edus_autotune picked another.
@@ -3302,13 +3365,11 @@ int launch_stage(edus_ctx *c, StageArgs a) {
             else
                 hipLaunchKernelGGL((k_stage_wave<NBT, MODE, double, double, false, PAIR>), grid, block, lds_d, c->stream, ca, a);
         };
-        // stencil pairs only where a workgroup serves one k (nb > 8; see
-        // stencil_pairs), and where they measured faster: not in the BF16x3 form,
-        // whose split products leave no registers for the second k's stencil
-        // sum, nor in the 32-band Taylor step with FP32 storage (3.73 ms paired,
-        // 3.53 one k per workgroup; its RK4 stages gain: 2.21 against 2.26 ms)
-        const bool pair = c->pair && c->precision != EDUS_PRECISION_BF16X3 &&
-                          !(MODE == TAY && c->nb > 16 && c->precision == EDUS_PRECISION_MIXED32);
+        // stencil pairs where a workgroup serves one k and where they measured
+        // faster (runs_paired), and not in the 32-band Taylor step with FP32 storage
+        // (3.73 ms paired, 3.53 one k per workgroup; its RK4 stages gain: 2.21
+        // against 2.26 ms)
+        const bool pair = runs_paired(c) && !(MODE == TAY && c->nb > 16 && c->precision == EDUS_PRECISION_MIXED32);
         if (c->nb <= 8) go(std::integral_constant<int, 8>{}, std::false_type{});
         else if (c->nb <= 16 && pair) go(std::integral_constant<int, 16>{}, std::true_type{});
         else if (c->nb <= 16) go(std::integral_constant<int, 16>{}, std::false_type{});
@@ -3515,6 +3576,8 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
     c->wb.assign(p->nbr_wb, p->nbr_wb + (size_t)p->n_nbr * 3);
     for (int i = 0; i < nb * nb; i++)
         if (std::fabs(p->T[i]) > 1e-24) c->diss = 1;
+    for (int v = 0; v < c->ncc; v++)
+        if (p->T[v * nb + v] != 0.0) c->hole = 1;
     if (p->stepper == EDUS_STEPPER_TAYLOR) c->tinv.assign(p->taylor_tau_inv, p->taylor_tau_inv + (size_t)(p->order - 1) * (p->order - 1));
     // Adams-Bashforth coefficients (ODE_solver.h:152-179).
     if (p->stepper == EDUS_STEPPER_AB) {
@@ -4327,13 +4390,13 @@ int edus_batch_create(const edus_problem *const *problems, int32_t n, edus_batch
         edus_batch::Cls *hit = nullptr;
         for (auto &k : b->cls)
             if (k.soa == c->soa && k.nb_small == (c->soa ? c->nb : 0) && k.nbt == nbt && k.precision == c->precision &&
-                k.diss == c->diss && k.pair == c->pair)
+                k.diss == c->diss && k.pair == (int)runs_paired(c))
                 hit = &k;
         if (!hit) {
             b->cls.emplace_back();
             hit = &b->cls.back();
             hit->soa = c->soa; hit->nb_small = c->soa ? c->nb : 0; hit->nbt = nbt; hit->precision = c->precision;
-            hit->diss = c->diss; hit->pair = c->pair;
+            hit->diss = c->diss; hit->pair = runs_paired(c);
         }
         hit->members.push_back(i);
     }
@@ -4343,7 +4406,7 @@ int edus_batch_create(const edus_problem *const *problems, int32_t n, edus_batch
             const edus_ctx *c = b->inst[i];
             const int kpb = c->nb <= 8 ? WaveGeom<8>::KPB : c->nb <= 16 ? WaveGeom<16>::KPB : WaveGeom<32>::KPB;
             const int nblk = c->soa    ? (c->nk + kSmallBatchThreads - 1) / kSmallBatchThreads
-                             : c->pair ? c->nk / 2
+                             : runs_paired(c) ? c->nk / 2
                                        : (c->nk + kpb - 1) / kpb;
             for (int q = 0; q < nblk; q++) map.push_back(make_int2(i, q));
         }
