@@ -2518,6 +2518,8 @@ __host__ __device__ inline long long wannier_cols(long long nw) { return nw * nw
 // Val[r0 + r][.] of n lattice vectors from the caller's H(R) [n][nw][nw] and r(R)
 // [n][nw][nw][3], and (r0 = 0) the column table: element ij = i nw + j of H as (ij, 1 on
 // the diagonal, else 0), pair i <= j of D as (i nw + j, j nw + i).
+// PLAIN: Val[r] = [H | r_x | r_y | r_z] as the FP32 and BF16x3 forms take it (no Col).
+template <bool PLAIN>
 __global__ __launch_bounds__(256) void k_wannier_val(const cd *__restrict__ HR, const cd *__restrict__ rR, int r0, int n, int nw, int ncol,
                                                      cd *__restrict__ Val, int2 *__restrict__ Col) {
     const int nw2 = nw * nw;
@@ -2526,6 +2528,10 @@ __global__ __launch_bounds__(256) void k_wannier_val(const cd *__restrict__ HR, 
     const int r = (int)(t / nw2), ij = (int)(t % nw2), i = ij / nw, j = ij % nw;
     cd *v = Val + (size_t)(r0 + r) * ncol;
     v[ij] = HR[t];
+    if constexpr (PLAIN) {
+        for (int x = 0; x < 3; x++) v[(x + 1) * nw2 + ij] = rR[3 * t + x];
+        return;
+    }
     const int ji = j * nw + i, c = nw2 + 3 * (i * nw - i * (i - 1) / 2 + j - i);
     if (i <= j) {
         const cd *a = rR + 3 * t, *b = rR + 3 * ((long long)r * nw2 + ji);
@@ -2644,11 +2650,11 @@ __global__ __launch_bounds__(256) void k_wannier_mfma(const cd *__restrict__ PT,
 // The contraction in FP32 on the matrix cores (v_mfma_f32_16x16x4f32, FP32
 // accumulation): the phases are formed in FP64 from the exact per-direction
 // tables and rounded once into LDS, H(R) and r(R) likewise; the sums are widened
-// to FP64 on the way out.  Same tiling as k_wannier_mfma; the FP32 instruction
-// holds D[4 (l/16) + i][l%16] in lane l.
-__global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ PT, const cd *__restrict__ Val, const int2 *__restrict__ Col,
-                                                        int N0, int N1, int N2, int nR, int nw2, int nm, int ncol, int nk, int kbase,
-                                                        cd *__restrict__ Hd, cd *__restrict__ Dd) {
+// to FP64 on the way out.  A workgroup owns 64 k x 32 columns of
+// Val = [H | r_x | r_y | r_z]; each sum is rounded to FP32 before D = (r + r^T)/2 is
+// taken from it.  The FP32 instruction holds D[4 (l/16) + i][l%16] in lane l.
+__global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ PT, const cd *__restrict__ Val, int N0, int N1, int N2,
+                                                        int nR, int nm, int nk, int kbase, cd *__restrict__ Out) {
     __shared__ cf Ph[WMK][WMR + 1];
     __shared__ cf Vs[WMR][WMN + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -2664,7 +2670,7 @@ __global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ P
         }
         for (int t = threadIdx.x; t < WMR * WMN; t += 256) {
             const int rr = t / WMN, mm = t % WMN, r = r0 + rr, m = m0 + mm;
-            const cd v = (r < nR && m < nm) ? Val[(size_t)r * ncol + m] : mk(0.0, 0.0);
+            const cd v = (r < nR && m < nm) ? Val[(size_t)r * nm + m] : mk(0.0, 0.0);
             Vs[rr][mm] = cf{(float)v.x, (float)v.y};
         }
         __syncthreads();
@@ -2683,16 +2689,12 @@ __global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ P
         __syncthreads();
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int m = m0 + t * 16 + (lane & 15);
-        if (m >= nm) continue;
-        const int2 col = Col[m];
+    for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i;
-            if (k < nk) wannier_store(k, m, nw2, col, (double)are[t][i], (double)aim[t][i], Hd, Dd);
+            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i, m = m0 + t * 16 + (lane & 15);
+            if (k < nk && m < nm) Out[(size_t)k * nm + m] = mk((double)are[t][i], (double)aim[t][i]);
         }
-    }
 }
 
 // The contraction as BF16x3 split products on the bf16 matrix cores
@@ -2705,9 +2707,8 @@ __global__ __launch_bounds__(256) void k_wannier_mfma32(const cd *__restrict__ P
 // and holds D[4 (l/16) + i][l%16].
 constexpr int WBR = 32;
 
-__global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restrict__ PT, const cd *__restrict__ Val, const int2 *__restrict__ Col,
-                                                        int N0, int N1, int N2, int nR, int nw2, int nm, int ncol, int nk, int kbase,
-                                                        cd *__restrict__ Hd, cd *__restrict__ Dd) {
+__global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restrict__ PT, const cd *__restrict__ Val, int N0, int N1,
+                                                             int N2, int nR, int nm, int nk, int kbase, cd *__restrict__ Out) {
     // [hi, lo] planes of the real and imaginary parts, K (R) innermost with one pad
     __shared__ __bf16 Ph[2][2][WMK][WBR + 8];
     __shared__ __bf16 Vs[2][2][WMN][WBR + 8];
@@ -2725,7 +2726,7 @@ __global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restric
         }
         for (int t = threadIdx.x; t < WBR * WMN; t += 256) {
             const int rr = t / WMN, mm = t % WMN, r = r0 + rr, m = m0 + mm;
-            const cd v = (r < nR && m < nm) ? Val[(size_t)r * ncol + m] : mk(0.0, 0.0);
+            const cd v = (r < nR && m < nm) ? Val[(size_t)r * nm + m] : mk(0.0, 0.0);
             bf16_split((float)v.x, Vs[0][0][mm][rr], Vs[0][1][mm][rr]);
             bf16_split((float)v.y, Vs[1][0][mm][rr], Vs[1][1][mm][rr]);
         }
@@ -2765,15 +2766,35 @@ __global__ __launch_bounds__(256) void k_wannier_mfma_bf16x3(const cd *__restric
         __syncthreads();
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int m = m0 + t * 16 + (lane & 15);
-        if (m >= nm) continue;
-        const int2 col = Col[m];
+    for (int t = 0; t < 2; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i;
-            if (k < nk) wannier_store(k, m, nw2, col, (double)are[t][i], (double)aim[t][i], Hd, Dd);
+            const int k = k0 + wave * 16 + 4 * (lane >> 4) + i, m = m0 + t * 16 + (lane & 15);
+            if (k < nk && m < nm) Out[(size_t)k * nm + m] = mk((double)are[t][i], (double)aim[t][i]);
         }
+}
+
+// Output [k][c][i][j] (c = 0 H, 1..3 r) of the FP32 and BF16x3 forms to the caller's layouts,
+// one thread per (k, i, j): H with zero diagonal imaginary parts
+// (Wannier.h:489-492) and D = (r + r^T)/2 with zero diagonal imaginary parts
+// (Wannier.h:577-578, save_HUD.cpp:187-191), [k][i][j][x].
+__global__ void k_wannier_finish(const cd *__restrict__ Out, int kc, int nw, double *__restrict__ Hd, double *__restrict__ Dd) {
+    const int nw2 = nw * nw;
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long long)kc * nw2) return;
+    const int kk = (int)(t / nw2), ij = (int)(t % nw2), i = ij / nw, j = ij % nw;
+    const cd *src = Out + (size_t)kk * 4 * nw2;
+    const cd h = src[ij];
+    Hd[2 * t] = h.x;
+    Hd[2 * t + 1] = (i == j) ? 0.0 : h.y;
+    if (!Dd) return;
+#pragma unroll
+    for (int x = 0; x < 3; x++) {
+        const cd a = src[(x + 1) * nw2 + i * nw + j];
+        const cd b = src[(x + 1) * nw2 + j * nw + i];
+        const double ai = (i == j) ? 0.0 : a.y, bi = (i == j) ? 0.0 : b.y;
+        Dd[(3 * t + x) * 2] = 0.5 * (a.x + b.x);
+        Dd[(3 * t + x) * 2 + 1] = 0.5 * (ai + bi);
     }
 }
 
@@ -4929,22 +4950,14 @@ public:
     }
 };
 
-// One chunk of kc k (from kbase) of the contraction, the first nm of Val's ncol columns.
-// form: 0 FP64 matrix cores, 1 FP32, 2 BF16x3 split products.
-static void wannier_launch(int form, const cd *PT, const cd *Val, const int2 *Col, const int32_t nk3[3], int nR, int nw2, int nm, int ncol,
-                           int kc, int kbase, cd *H, cd *D) {
-    const unsigned gk = (unsigned)((kc + WMK - 1) / WMK);
-    if (form == 0)
-        hipLaunchKernelGGL(k_wannier_mfma, dim3((unsigned)((nm + 63) / 64), gk), dim3(256), 0, 0, PT, Val, Col, nk3[0], nk3[1], nk3[2], nR, nw2,
-                           nm, ncol, kc, kbase, H, D);
-    else if (form == 1)
-        hipLaunchKernelGGL(k_wannier_mfma32, dim3((unsigned)((nm + WMN - 1) / WMN), gk), dim3(256), 0, 0, PT, Val, Col, nk3[0], nk3[1], nk3[2],
-                           nR, nw2, nm, ncol, kc, kbase, H, D);
-    else
-        hipLaunchKernelGGL(k_wannier_mfma_bf16x3, dim3((unsigned)((nm + WMN - 1) / WMN), gk), dim3(256), 0, 0, PT, Val, Col, nk3[0], nk3[1],
-                           nk3[2], nR, nw2, nm, ncol, kc, kbase, H, D);
+// One chunk of kc k (from kbase) of the FP64 contraction, the first nm of Val's ncol columns.
+static void wannier_launch(const cd *PT, const cd *Val, const int2 *Col, const int32_t nk3[3], int nR, int nw2, int nm, int ncol, int kc,
+                           int kbase, cd *H, cd *D) {
+    hipLaunchKernelGGL(k_wannier_mfma, dim3((unsigned)((nm + 63) / 64), (unsigned)((kc + WMK - 1) / WMK)), dim3(256), 0, 0, PT, Val, Col,
+                       nk3[0], nk3[1], nk3[2], nR, nw2, nm, ncol, kc, kbase, H, D);
 }
 
+// form: 0 FP64 matrix cores, 1 FP32, 2 BF16x3 split products.
 static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_t *R, const double *HR, const double *rR, double *H_out,
                      double *D_out, int form) {
     if (!nk3 || !R || !HR || !rR || !H_out || nR < 1 || nw < 1) return set_err(EDUS_ERR_INVALID, "bad Wannier arguments");
@@ -4953,15 +4966,15 @@ static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return set_err(EDUS_ERR_NODEVICE, "no HIP device visible");
     const long long nk = (long long)nk3[0] * nk3[1] * nk3[2];
-    const int nw2 = nw * nw, nm = D_out ? (int)wannier_cols(nw) : nw2, ncol = (int)wannier_cols(nw);
+    const int nw2 = nw * nw, nm = D_out ? (int)wannier_cols(nw) : nw2, ncol = form ? 4 * nw2 : (int)wannier_cols(nw);
     std::vector<double> tw;
     int offs[3];
     wannier_twiddles(nk3, tw, offs);
     int *dR = nullptr;
     int2 *dCol = nullptr;
-    double *dHR = nullptr, *drR = nullptr, *dVal = nullptr, *dTw = nullptr, *dPT = nullptr, *dH = nullptr, *dD = nullptr;
+    double *dHR = nullptr, *drR = nullptr, *dVal = nullptr, *dTw = nullptr, *dPT = nullptr, *dH = nullptr, *dD = nullptr, *dOut = nullptr;
     auto cleanup = [&]() {
-        for (void *q : {(void *)dR, (void *)dCol, (void *)dHR, (void *)drR, (void *)dVal, (void *)dTw, (void *)dPT, (void *)dH, (void *)dD})
+        for (void *q : {(void *)dOut, (void *)dR, (void *)dCol, (void *)dHR, (void *)drR, (void *)dVal, (void *)dTw, (void *)dPT, (void *)dH, (void *)dD})
             (void)hipFree(q);
     };
     Downloader down;
@@ -4971,6 +4984,7 @@ static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_
         hipMalloc(&dHR, nval * 16) != hipSuccess || hipMalloc(&drR, nval * 48) != hipSuccess ||
         hipMalloc(&dVal, (size_t)nR * ncol * 16) != hipSuccess || hipMalloc(&dTw, tw.size() * sizeof(double)) != hipSuccess ||
         hipMalloc(&dPT, npt * 2 * sizeof(double)) != hipSuccess || hipMalloc(&dH, chunk * nw2 * 2 * sizeof(double)) != hipSuccess ||
+        (form && hipMalloc(&dOut, chunk * ncol * 16) != hipSuccess) ||
         (D_out && hipMalloc(&dD, chunk * nw2 * 6 * sizeof(double)) != hipSuccess)) {
         cleanup();
         return set_err(EDUS_ERR_NOMEM, "Wannier buffers");
@@ -4982,14 +4996,22 @@ static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_
         cleanup();
         return set_err(EDUS_ERR_HIP, "Wannier upload");
     }
-    hipLaunchKernelGGL(k_wannier_val, dim3((unsigned)((nval + 255) / 256)), dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR, 0, nR, nw, ncol,
-                       (cd *)dVal, dCol);
+    const dim3 gval((unsigned)((nval + 255) / 256));
+    if (form) hipLaunchKernelGGL(k_wannier_val<true>, gval, dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR, 0, nR, nw, ncol, (cd *)dVal, dCol);
+    else hipLaunchKernelGGL(k_wannier_val<false>, gval, dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR, 0, nR, nw, ncol, (cd *)dVal, dCol);
     hipLaunchKernelGGL(k_wannier_ptab, dim3((unsigned)std::min<size_t>((npt + 255) / 256, 65536)), dim3(256), 0, 0, (const int *)dR,
                        (const cd *)dTw, nR, nk3[0], nk3[1], nk3[2], offs[1], offs[2], (cd *)dPT);
     for (long long k0 = 0; k0 < nk; k0 += chunk) {
         const int kc = (int)std::min<long long>(chunk, nk - k0);
-        wannier_launch(form, (const cd *)dPT, (const cd *)dVal, dCol, nk3, nR, nw2, nm, ncol, kc, (int)k0, (cd *)dH, (cd *)dD);
         const size_t nt = (size_t)kc * nw2;
+        if (form == 0) {
+            wannier_launch((const cd *)dPT, (const cd *)dVal, dCol, nk3, nR, nw2, nm, ncol, kc, (int)k0, (cd *)dH, (cd *)dD);
+        } else {
+            const dim3 grid((ncol + WMN - 1) / WMN, (unsigned)((kc + WMK - 1) / WMK));
+            hipLaunchKernelGGL(form == 1 ? k_wannier_mfma32 : k_wannier_mfma_bf16x3, grid, dim3(256), 0, 0, (const cd *)dPT, (const cd *)dVal,
+                               nk3[0], nk3[1], nk3[2], nR, ncol, kc, (int)k0, (cd *)dOut);
+            hipLaunchKernelGGL(k_wannier_finish, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, 0, (const cd *)dOut, kc, nw, dH, dD);
+        }
         hipError_t e = hipGetLastError();
         if (e == hipSuccess) e = down.copy(H_out + (size_t)k0 * nw2 * 2, dH, nt * 16);
         if (e == hipSuccess && D_out) e = down.copy(D_out + (size_t)k0 * nw2 * 6, dD, nt * 48);
@@ -5066,7 +5088,7 @@ int edus_wannier_hk_noalloc(const int32_t nk3[3], int32_t nR, int32_t nw, const 
         cd *dHR = dH, *drR = dHR + (size_t)n * nw2;
         HIP_TRY(hipMemcpy(dHR, HR + (size_t)r0 * nw2 * 2, (size_t)n * nw2 * 16, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(drR, rR + (size_t)r0 * nw2 * 6, (size_t)n * nw2 * 48, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(k_wannier_val, dim3((unsigned)(((long long)n * nw2 + 255) / 256)), dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR,
+        hipLaunchKernelGGL(k_wannier_val<false>, dim3((unsigned)(((long long)n * nw2 + 255) / 256)), dim3(256), 0, 0, (const cd *)dHR, (const cd *)drR,
                            r0, n, (int)nw, ncol, dVal, dCol);
         HIP_TRY(hipGetLastError());
     }
@@ -5076,7 +5098,7 @@ int edus_wannier_hk_noalloc(const int32_t nk3[3], int32_t nR, int32_t nw, const 
     HIP_TRY(hipGetLastError());
     for (long long k0 = 0; k0 < nk; k0 += chunk) {
         const int kc = (int)std::min<long long>(chunk, nk - k0);
-        wannier_launch(0, (const cd *)dPT, dVal, dCol, nk3, nR, (int)nw2, nform, ncol, kc, (int)k0, dH, dD);
+        wannier_launch((const cd *)dPT, dVal, dCol, nk3, nR, (int)nw2, nform, ncol, kc, (int)k0, dH, dD);
         const long long nt = (long long)kc * nw2;
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipMemcpy(H_out + (size_t)k0 * nw2 * 2, dH, (size_t)nt * 16, hipMemcpyDeviceToHost));
