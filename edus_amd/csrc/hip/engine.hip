@@ -2417,6 +2417,23 @@ __global__ void k_counter_step(int *ctr) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *ctr += 1;
 }
 
+// Packed matrices of k0 .. k0 + n/nb^2 - 1 to the full reference layout [k][i][j], one
+// thread per element (k at k sk + e se in the packed array).
+__global__ __launch_bounds__(256) void k_unpack(const double *__restrict__ Y, long long n, int nb, size_t sk, size_t se, int k0,
+                                                cd *__restrict__ out) {
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (t >= n) return;
+    const int nb2 = nb * nb, ij = (int)(t % nb2), i = ij / nb, j = ij % nb;
+    const double *y = Y + (size_t)(k0 + t / nb2) * sk;
+    if (i == j) {
+        out[t] = mk(y[i * se], 0.0);
+    } else {
+        const size_t e = nb + 2 * (size_t)pair_index(min(i, j), max(i, j), nb);
+        const double re = y[e * se], im = y[(e + 1) * se];
+        out[t] = mk(re, i < j ? im : -im);
+    }
+}
+
 // ================================================================ adaptive dt
 // Diagonal of the state before a step (P_W_prev, RungeKutta.cpp:1-9,139-147 and
 // Taylor_DE_solver_deriv_Polynom.cpp:75-84).  Element e of k sits at k*sk + e*se.
@@ -3122,6 +3139,7 @@ struct edus_ctx {
     double *dwb = nullptr, *cEk = nullptr;
     bool cEk_valid = false;
     double *snap = nullptr;  // [nk] complex, k-resolved snapshot element
+    double *full = nullptr;  // full matrices of a small grid (download_full)
     // adaptive dt: diagonal before the step, block maxima
     double *DG = nullptr, *dpart = nullptr;
     // device-resident field table of a run and the captured RK4 step reading it
@@ -3159,26 +3177,6 @@ void pack_state(const edus_ctx *c, const double *full, std::vector<double> &out)
                 const size_t er = nb + 2 * p;
                 out[c->soa ? er * c->nkp + k : (size_t)k * np + er] = m[(i * nb + j) * 2];
                 out[c->soa ? (er + 1) * c->nkp + k : (size_t)k * np + er + 1] = m[(i * nb + j) * 2 + 1];
-            }
-        }
-    }
-}
-
-void unpack_state(const edus_ctx *c, const std::vector<double> &in, double *full) {
-    const int nb = c->nb, np = c->np;
-    for (int k = 0; k < c->nk; k++) {
-        double *m = full + (size_t)k * nb * nb * 2;
-        auto at = [&](size_t e) { return in[c->soa ? e * c->nkp + k : (size_t)k * np + e]; };
-        for (int i = 0; i < nb; i++) {
-            m[(i * nb + i) * 2] = at(i);
-            m[(i * nb + i) * 2 + 1] = 0.0;
-            for (int j = i + 1; j < nb; j++) {
-                const int p = pair_index(i, j, nb);
-                const double re = at(nb + 2 * p), im = at(nb + 2 * p + 1);
-                m[(i * nb + j) * 2] = re;
-                m[(i * nb + j) * 2 + 1] = im;
-                m[(j * nb + i) * 2] = re;
-                m[(j * nb + i) * 2 + 1] = -im;
             }
         }
     }
@@ -4017,6 +4015,113 @@ int edus_step_taylor(edus_ctx *c, int32_t nsteps, const double *fields, const ui
     return step_multistep(c, nsteps, fields, grad_on, true);
 }
 
+// Copies of large results to the caller's ordinary memory.  hipMemcpy locks that
+// memory page by page in front of the copy engine (9.3 GB/s into fresh pages, 17 into
+// touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
+// memory, and each of a few threads copies its own piece on to the caller's pages
+// while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring belongs to the
+// object (12 MB).  From 32 MB on; below, the threads' start takes what it gives.
+namespace {
+class Downloader {
+    static constexpr size_t kPiece = 2 << 20;
+    static constexpr int kWorkers = 6;
+    char *ring = nullptr;
+    hipEvent_t ev[kWorkers] = {};
+    int dev = 0;
+
+    bool ready() {
+        if (ring) return true;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        for (hipEvent_t &e : ev)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kWorkers * kPiece, hipHostMallocDefault) != hipSuccess) return false;
+        ring = static_cast<char *>(p);
+        return true;
+    }
+
+public:
+    Downloader() = default;
+    Downloader(const Downloader &) = delete;
+    Downloader &operator=(const Downloader &) = delete;
+    ~Downloader() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+        if (ring) (void)hipHostFree(ring);
+    }
+    // n bytes of device memory, in the stream's order; returns when dst holds them.
+    hipError_t copy(void *dst, const void *src, size_t n, hipStream_t st) {
+        if (n < 16 * kPiece || !ready()) {
+            const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
+            return e == hipSuccess ? hipStreamSynchronize(st) : e;
+        }
+        std::mutex mu;
+        size_t next = 0;
+        hipError_t err = hipSuccess;
+        auto work = [&](int w) {
+            char *slot = ring + w * kPiece;
+            hipError_t e = hipSetDevice(dev);
+            for (;;) {
+                size_t o, len;
+                {
+                    std::lock_guard<std::mutex> lock(mu);
+                    if (e != hipSuccess) err = e;
+                    if (err != hipSuccess || next >= n) return;
+                    o = next;
+                    len = std::min(kPiece, n - o);
+                    next += len;
+                    e = hipMemcpyAsync(slot, static_cast<const char *>(src) + o, len, hipMemcpyDeviceToHost, st);
+                    if (e == hipSuccess) e = hipEventRecord(ev[w], st);
+                }
+                if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
+                if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + o, slot, len);
+            }
+        };
+        std::thread th[kWorkers - 1];
+        try {
+            for (int w = 1; w < kWorkers; w++) th[w - 1] = std::thread(work, w);
+        } catch (...) {
+            // fewer workers: the others, this thread at least, take their pieces
+        }
+        work(0);
+        for (std::thread &t : th)
+            if (t.joinable()) t.join();
+        return err;
+    }
+};
+
+// Packed array Y of the context (complete in stream order) to the caller's full
+// matrices: unpacked on the device, 64 MB at a time (unpacking 3600 k of 3 bands on the
+// host took 60 us, 40000 of 16 bands 110 ms).
+int download_full(edus_ctx *c, const double *Y, double *out) {
+    const size_t per = (size_t)c->np * 16;
+    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(c->nk, ((size_t)64 << 20) / per));
+    double *buf = c->full;  // kept by the context up to 4 MB
+    std::unique_ptr<double, DeviceFree> hold;
+    if (!buf) {
+        int rc;
+        if (chunk * per <= ((size_t)4 << 20)) {
+            if ((rc = dalloc(c, &c->full, chunk * per / 8))) return rc;
+            buf = c->full;
+        } else {
+            void *q = nullptr;
+            HIP_TRY(hipMalloc(&q, chunk * per));
+            hold.reset(buf = static_cast<double *>(q));
+        }
+    }
+    Downloader down;
+    const size_t sk = c->soa ? 1 : (size_t)c->np, se = c->soa ? (size_t)c->nkp : 1;
+    for (int k0 = 0; k0 < c->nk; k0 += chunk) {
+        const int kc = std::min(chunk, c->nk - k0);
+        const long long n = (long long)kc * c->np;
+        hipLaunchKernelGGL(k_unpack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, Y, n, c->nb, sk, se, k0, reinterpret_cast<cd *>(buf));
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(down.copy(out + (size_t)k0 * c->np * 2, buf, kc * per, c->stream));
+    }
+    return 0;
+}
+}  // namespace
+
 static const double *current_state(const edus_ctx *c) {
     if (c->stepper == EDUS_STEPPER_RK4) return c->P0;
     return c->cur ? c->YA : c->P0;
@@ -4167,22 +4272,14 @@ int edus_rhs(edus_ctx *c, const double *field6, uint8_t grad_on, double *pv) {
     a.Y = current_state(c);
     a.OUT = c->YB;
     if ((rc = launch_stage<RHSO>(c, a))) return rc;
-    std::vector<double> st(state_elems(c));
-    HIP_TRY(hipMemcpyAsync(st.data(), c->YB, st.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    unpack_state(c, st, pv);
-    return 0;
+    return download_full(c, c->YB, pv);
 }
 
 int edus_get_state(edus_ctx *c, double *rho) {
     int rc = check_ctx(c);
     if (rc) return rc;
     if (!rho) return set_err(EDUS_ERR_INVALID, "null output");
-    std::vector<double> st(state_elems(c));
-    HIP_TRY(hipMemcpyAsync(st.data(), current_state(c), st.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    unpack_state(c, st, rho);
-    return 0;
+    return download_full(c, current_state(c), rho);
 }
 
 int edus_set_state(edus_ctx *c, const double *rho) {
@@ -4879,77 +4976,6 @@ static void wannier_twiddles(const int32_t nk3[3], std::vector<double> &tw, int 
     }
 }
 
-// Copies of large results to the caller's ordinary memory.  hipMemcpy locks that
-// memory page by page in front of the copy engine (9.3 GB/s into fresh pages, 17 into
-// touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
-// memory, and each of a few threads copies its own piece on to the caller's pages
-// while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring belongs to the
-// object (12 MB).  From 32 MB on; below, the threads' start takes what it gives.
-class Downloader {
-    static constexpr size_t kPiece = 2 << 20;
-    static constexpr int kWorkers = 6;
-    char *ring = nullptr;
-    hipEvent_t ev[kWorkers] = {};
-    int dev = 0;
-
-    bool ready() {
-        if (ring) return true;
-        if (hipGetDevice(&dev) != hipSuccess) return false;
-        for (hipEvent_t &e : ev)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-        void *p = nullptr;
-        if (hipHostMalloc(&p, kWorkers * kPiece, hipHostMallocDefault) != hipSuccess) return false;
-        ring = static_cast<char *>(p);
-        return true;
-    }
-
-public:
-    Downloader() = default;
-    Downloader(const Downloader &) = delete;
-    Downloader &operator=(const Downloader &) = delete;
-    ~Downloader() {
-        for (hipEvent_t e : ev)
-            if (e) (void)hipEventDestroy(e);
-        if (ring) (void)hipHostFree(ring);
-    }
-    // n bytes of device memory, in null-stream order; returns when dst holds them.
-    hipError_t copy(void *dst, const void *src, size_t n) {
-        if (n < 16 * kPiece || !ready()) return hipMemcpy(dst, src, n, hipMemcpyDeviceToHost);
-        std::mutex mu;
-        size_t next = 0;
-        hipError_t err = hipSuccess;
-        auto work = [&](int w) {
-            char *slot = ring + w * kPiece;
-            hipError_t e = hipSetDevice(dev);
-            for (;;) {
-                size_t o, len;
-                {
-                    std::lock_guard<std::mutex> lock(mu);
-                    if (e != hipSuccess) err = e;
-                    if (err != hipSuccess || next >= n) return;
-                    o = next;
-                    len = std::min(kPiece, n - o);
-                    next += len;
-                    e = hipMemcpyAsync(slot, static_cast<const char *>(src) + o, len, hipMemcpyDeviceToHost, 0);
-                    if (e == hipSuccess) e = hipEventRecord(ev[w], 0);
-                }
-                if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
-                if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + o, slot, len);
-            }
-        };
-        std::thread th[kWorkers - 1];
-        try {
-            for (int w = 1; w < kWorkers; w++) th[w - 1] = std::thread(work, w);
-        } catch (...) {
-            // fewer workers: the others, this thread at least, take their pieces
-        }
-        work(0);
-        for (std::thread &t : th)
-            if (t.joinable()) t.join();
-        return err;
-    }
-};
-
 // One chunk of kc k (from kbase) of the FP64 contraction, the first nm of Val's ncol columns.
 static void wannier_launch(const cd *PT, const cd *Val, const int2 *Col, const int32_t nk3[3], int nR, int nw2, int nm, int ncol, int kc,
                            int kbase, cd *H, cd *D) {
@@ -5013,8 +5039,8 @@ static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_
             hipLaunchKernelGGL(k_wannier_finish, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, 0, (const cd *)dOut, kc, nw, dH, dD);
         }
         hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = down.copy(H_out + (size_t)k0 * nw2 * 2, dH, nt * 16);
-        if (e == hipSuccess && D_out) e = down.copy(D_out + (size_t)k0 * nw2 * 6, dD, nt * 48);
+        if (e == hipSuccess) e = down.copy(H_out + (size_t)k0 * nw2 * 2, dH, nt * 16, 0);
+        if (e == hipSuccess && D_out) e = down.copy(D_out + (size_t)k0 * nw2 * 6, dD, nt * 48, 0);
         if (e != hipSuccess) {
             cleanup();
             return set_err(EDUS_ERR_HIP, std::string("k_wannier: ") + hipGetErrorString(e));
