@@ -3139,7 +3139,6 @@ struct edus_ctx {
     double *dwb = nullptr, *cEk = nullptr;
     bool cEk_valid = false;
     double *snap = nullptr;  // [nk] complex, k-resolved snapshot element
-    double *full = nullptr;  // full matrices of a small grid (download_full)
     // adaptive dt: diagonal before the step, block maxima
     double *DG = nullptr, *dpart = nullptr;
     // device-resident field table of a run and the captured RK4 step reading it
@@ -3177,6 +3176,26 @@ void pack_state(const edus_ctx *c, const double *full, std::vector<double> &out)
                 const size_t er = nb + 2 * p;
                 out[c->soa ? er * c->nkp + k : (size_t)k * np + er] = m[(i * nb + j) * 2];
                 out[c->soa ? (er + 1) * c->nkp + k : (size_t)k * np + er + 1] = m[(i * nb + j) * 2 + 1];
+            }
+        }
+    }
+}
+
+void unpack_state(const edus_ctx *c, const std::vector<double> &in, double *full) {
+    const int nb = c->nb, np = c->np;
+    for (int k = 0; k < c->nk; k++) {
+        double *m = full + (size_t)k * nb * nb * 2;
+        auto at = [&](size_t e) { return in[c->soa ? e * c->nkp + k : (size_t)k * np + e]; };
+        for (int i = 0; i < nb; i++) {
+            m[(i * nb + i) * 2] = at(i);
+            m[(i * nb + i) * 2 + 1] = 0.0;
+            for (int j = i + 1; j < nb; j++) {
+                const int p = pair_index(i, j, nb);
+                const double re = at(nb + 2 * p), im = at(nb + 2 * p + 1);
+                m[(i * nb + j) * 2] = re;
+                m[(i * nb + j) * 2 + 1] = im;
+                m[(j * nb + i) * 2] = re;
+                m[(j * nb + i) * 2 + 1] = -im;
             }
         }
     }
@@ -4020,7 +4039,7 @@ int edus_step_taylor(edus_ctx *c, int32_t nsteps, const double *fields, const ui
 // touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
 // memory, and each of a few threads copies its own piece on to the caller's pages
 // while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring belongs to the
-// object (12 MB).  From 32 MB on; below, the threads' start takes what it gives.
+// object (12 MB).  From 16 MB on (16.8 MB: 1.24 -> 1.07 ms, 33 MB 2.5 -> 1.6; 8 MB even).
 namespace {
 class Downloader {
     static constexpr size_t kPiece = 2 << 20;
@@ -4051,7 +4070,7 @@ public:
     }
     // n bytes of device memory, in the stream's order; returns when dst holds them.
     hipError_t copy(void *dst, const void *src, size_t n, hipStream_t st) {
-        if (n < 16 * kPiece || !ready()) {
+        if (n < 8 * kPiece || !ready()) {
             const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
             return e == hipSuccess ? hipStreamSynchronize(st) : e;
         }
@@ -4091,30 +4110,32 @@ public:
 };
 
 // Packed array Y of the context (complete in stream order) to the caller's full
-// matrices: unpacked on the device, 64 MB at a time (unpacking 3600 k of 3 bands on the
-// host took 60 us, 40000 of 16 bands 110 ms).
+// matrices.  From 16 MB of them on they are unpacked on the device, up to 64 MB at a
+// time (16.8 MB: 2.0 ms with the host's loop, 1.1 so; 67 MB 14.2, 2.5; 268 MB 49, 8.3).
+// Below, and where the device has no room for the piece, the host unpacks: the piece's
+// allocation and first use take what the kernel gives (0.5 MB: 0.048 and 0.055 ms, 8.2 MB
+// 0.61 and 0.64, the first call 0.79 and 1.05).
 int download_full(edus_ctx *c, const double *Y, double *out) {
     const size_t per = (size_t)c->np * 16;
     const int chunk = (int)std::max<size_t>(1, std::min<size_t>(c->nk, ((size_t)64 << 20) / per));
-    double *buf = c->full;  // kept by the context up to 4 MB
-    std::unique_ptr<double, DeviceFree> hold;
-    if (!buf) {
-        int rc;
-        if (chunk * per <= ((size_t)4 << 20)) {
-            if ((rc = dalloc(c, &c->full, chunk * per / 8))) return rc;
-            buf = c->full;
-        } else {
-            void *q = nullptr;
-            HIP_TRY(hipMalloc(&q, chunk * per));
-            hold.reset(buf = static_cast<double *>(q));
-        }
+    void *q = nullptr;
+    if (c->nk * per < ((size_t)16 << 20) || hipMalloc(&q, chunk * per) != hipSuccess) {
+        if (c->nk * per >= ((size_t)16 << 20)) (void)hipGetLastError();
+        std::vector<double> st(state_elems(c));
+        HIP_TRY(hipMemcpyAsync(st.data(), Y, st.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        unpack_state(c, st, out);
+        return 0;
     }
+    const std::unique_ptr<double, DeviceFree> hold(static_cast<double *>(q));
+    double *buf = hold.get();
     Downloader down;
     const size_t sk = c->soa ? 1 : (size_t)c->np, se = c->soa ? (size_t)c->nkp : 1;
     for (int k0 = 0; k0 < c->nk; k0 += chunk) {
         const int kc = std::min(chunk, c->nk - k0);
         const long long n = (long long)kc * c->np;
-        hipLaunchKernelGGL(k_unpack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, Y, n, c->nb, sk, se, k0, reinterpret_cast<cd *>(buf));
+        hipLaunchKernelGGL(k_unpack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, Y, n, c->nb, sk, se, k0,
+                           reinterpret_cast<cd *>(buf));
         HIP_TRY(hipGetLastError());
         HIP_TRY(down.copy(out + (size_t)k0 * c->np * 2, buf, kc * per, c->stream));
     }

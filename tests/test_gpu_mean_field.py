@@ -1,6 +1,7 @@
 """Right-hand side with the mean field for random tables against the oracle, where
 the passes' tiles end: every band count they take, grids that are and are not
-multiples of 16, both bases, the screening gate off and on."""
+multiples of 16 or longer than one batch of the first pass, both bases, the screening
+gate off and on."""
 import ctypes as C
 
 import numpy as np
@@ -16,7 +17,8 @@ class _Coulomb(C.Structure):
 
 
 @pytest.mark.parametrize("nb,n1,n2,ncut,diag", [(1, 5, 7, 3, False), (2, 16, 16, 8, False), (3, 17, 33, 5, False), (4, 9, 40, 11, False),
-                                                (2, 7, 5, 4, True), (3, 20, 17, 6, True), (4, 16, 18, 3, True)])
+                                                (2, 7, 5, 4, True), (3, 20, 17, 6, True), (4, 16, 18, 3, True), (2, 3, 200, 12, False),
+                                                (1, 2, 385, 4, False)])
 def test_rhs_with_mean_field_matches_oracle(nb, n1, n2, ncut, diag):
     rng = np.random.default_rng(10 * nb + n1)
     nk, ncc, dp, ip = n1 * n2, max(1, nb // 2), C.POINTER(C.c_double), C.POINTER(C.c_int32)
