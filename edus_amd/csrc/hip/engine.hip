@@ -1375,14 +1375,19 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     const int nn = c.n_nbr;
     const bool grad = tab[6 + nn] != 0.0;
 
-    // Lanes past the last packed element (nb < NBT) repeat element NP-1: every
-    // load stays in bounds without a branch, and their LDS and global stores
-    // write the same value to the same address as the lane that owns it.
+    // Lanes past the last packed element (nb < NBT) repeat it: every load stays in
+    // bounds without a branch, and their LDS and global stores write the same value
+    // to the same address as the lane that owns it.
     // With an even number of doubles per thread, a lane owns adjacent pairs of
     // elements (2q, 2q+1), q = lane + TPK m', read and written 16 bytes at a time
     // when nb is even (NP even keeps every pair inside one k and aligned); the
     // pair is a real diagonal pair or the (re, im) of one upper element.
     constexpr bool kPairs = PER % 2 == 0;
+    // With kLast a lane past the end repeats the last pair, so that the choice of
+    // access is the same on every lane (Taylor step of 24 bands on 96 x 100 k with
+    // FP32 operators 149 us -> 131); at 9..16 bands it gained nothing (16 bands RK4
+    // 119.3 us -> 121.1 a stage, 13 bands AB4 42.1 -> 45.8).
+    constexpr bool kLast = NBT != 16;
     // A stencil pair's calls load the RK2/RK3 accumulator and state at t_n after
     // the products, not with the other inputs: the registers then hold kb's
     // stencil sum instead through the gather and the products.
@@ -1394,7 +1399,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     const size_t base = (size_t)k * NP;
 #pragma unroll
     for (int m = 0; m < PER; m++) {
-        const int e = kPairs ? min(2 * (lane + TPK * (m >> 1)) + (m & 1), NP - 1) : min(lane + TPK * m, NP - 1);
+        const int e = kPairs ? min(min(2 * (lane + TPK * (m >> 1)), kLast ? NP - 2 + (NP & 1) : NP - 1) + (m & 1), NP - 1) : min(lane + TPK * m, NP - 1);
         eo[m] = e;
         const int code = *gm(c.eidx + e);
         ei[m] = code & 255;
@@ -1404,15 +1409,15 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         if constexpr (ROLE == 1) gb[m] = 0.0;
     }
 #pragma unroll
-    for (int h = 0; h < (PER > 1 ? PER / 2 : 1); h++) pv2[h] = kPairs && (NP % 2 == 0) && 2 * (lane + TPK * h) + 1 < NP;
+    for (int h = 0; h < (PER > 1 ? PER / 2 : 1); h++) pv2[h] = kPairs && NP % 2 == 0 && (kLast || 2 * (lane + TPK * h) + 1 < NP);
     // Neighbour data of the stage input, GB neighbours per call, their loads all
     // issued before any is used (k's or kb's stencil slots, by `slot`).
     constexpr int GB = WaveGeom<NBT>::GATHER;
-    auto gather = [&](const int kk, auto slot, const int cnt, auto &v) {
+    auto fetch = [&](const auto &row, auto &v) {
         constexpr int NV = std::extent<std::remove_reference_t<decltype(v)>>::value;
         size_t kn[NV];
 #pragma unroll
-        for (int j = 0; j < NV; j++) kn[j] = (size_t)*gm(c.nbr + (size_t)slot(min(j, cnt - 1)) * c.nkp + kk) * NP;
+        for (int j = 0; j < NV; j++) kn[j] = (size_t)row[j] * NP;
 #pragma unroll
         for (int j = 0; j < NV; j++) {
             if constexpr (kPairs) {
@@ -1429,6 +1434,23 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             }
         }
     };
+    auto gather = [&](const int kk, auto slot, const int cnt, auto &v) {
+        constexpr int NV = std::extent<std::remove_reference_t<decltype(v)>>::value;
+        int row[NV];
+#pragma unroll
+        for (int j = 0; j < NV; j++) row[j] = *gm(c.nbr + (size_t)slot(min(j, cnt - 1)) * c.nkp + kk);
+        fetch(row, v);
+    };
+    // Up to 8 bands a wave serves two k and its stencil rows are vector loads, which
+    // return in the order of their requests: the first batch's are requested in front
+    // of the stage's operands, not behind them (8 bands, 200 x 200 k, RK4 stage 36 us
+    // -> 33.7).
+    constexpr bool kRowsFirst = WaveGeom<NBT>::KPB > 1;
+    int row0[kRowsFirst ? GB : 1];
+    if constexpr (kRowsFirst) {
+#pragma unroll
+        for (int j = 0; j < GB; j++) row0[j] = *gm(c.nbr + (size_t)max(min(j, nn - 1), 0) * c.nkp + k);
+    }
     if constexpr (kPairs) {
 #pragma unroll
         for (int h = 0; h < PER / 2; h++) {
@@ -1503,7 +1525,15 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     } else if (grad) {
         for (int n0 = 0; n0 < nn; n0 += GB) {
             double v[GB][PER];
-            gather(k, [&](int j) { return n0 + j; }, nn - n0, v);
+            if constexpr (kRowsFirst) {
+                fetch(row0, v);
+                if (n0 + GB < nn) {
+#pragma unroll
+                    for (int j = 0; j < GB; j++) row0[j] = *gm(c.nbr + (size_t)min(n0 + GB + j, nn - 1) * c.nkp + k);
+                }
+            } else {
+                gather(k, [&](int j) { return n0 + j; }, nn - n0, v);
+            }
 #pragma unroll
             for (int j = 0; j < GB; j++)
                 if (n0 + j < nn) {
@@ -1732,6 +1762,9 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
     for (int h = 0; h < PER / 2; h++) {
         const int m = 2 * h;
+        // A lane that repeats an element of another wave leaves its result to that
+        // one: with kLatePre it may have read the accumulator after the update.
+        if (TPK > 64 && 2 * (lane + TPK * h) >= NP) break;
         const double k0 = pv[m] + g[m], k1 = pv[m + 1] + g[m + 1];
         const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
         const bool v2 = pv2[h];
@@ -1753,10 +1786,14 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     }
 }
 
+// Waves per SIMD that the registers are to allow: some modes otherwise end a few
+// registers above the limit.
+constexpr int wave_occupancy(int nbt, bool pair) { return nbt == 8 ? 4 : nbt == 16 && !pair ? 3 : 1; }
+
 // One k per workgroup, or with PAIR (ConstArgs::pair, one k per workgroup only)
 // the stencil pair (2q, 2q + 1).
 template <int NBT, int MODE, typename R, typename S = double, bool B3 = false, bool PAIR = false>
-__global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB, (NBT == 16 && !PAIR ? 3 : 1)) void k_stage_wave(ConstArgs c, StageArgs a) {
+__global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB, wave_occupancy(NBT, PAIR)) void k_stage_wave(ConstArgs c, StageArgs a) {
     extern __shared__ double smem_d[];
     constexpr int TPK = WaveGeom<NBT>::TPK;
     double gb[WaveGeom<NBT>::PER];
@@ -1814,8 +1851,8 @@ __global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) vo
 }
 
 template <int NBT, int MODE, typename R, bool PAIR = false>
-__global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB) void k_stage_wave_batch(const BatchEntry *E, const int2 *blk,
-                                                                                         const int *dmask, size_t tab_step) {
+__global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB, wave_occupancy(NBT, PAIR)) void k_stage_wave_batch(
+    const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
     extern __shared__ double smem_d[];
     constexpr int TPK = WaveGeom<NBT>::TPK;
     const int2 w = blk[xcd_block()];
