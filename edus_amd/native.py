@@ -413,7 +413,7 @@ class Engine:
 
     def autotune(self, field6, grad_on=True, reps=5):
         """Launch schedule picked by timing (edus_autotune); returns the kept strip
-        width (5..32 bands) or workgroup size (1..4 bands)."""
+        width (5..32 bands) or k per workgroup (1..4 bands)."""
         f = np.ascontiguousarray(field6, dtype=np.float64)
         ch = C.c_int32()
         _check_hip(hip.edus_autotune(self._h, _dptr(f), 1 if grad_on else 0, reps, C.byref(ch)), "edus_autotune")
