@@ -224,13 +224,13 @@ __device__ __forceinline__ float ldnt(const float *p) { return __builtin_nontemp
 __device__ __forceinline__ void stnt(double *p, double v) { __builtin_nontemporal_store(v, gm(p)); }
 __device__ __forceinline__ void stnt(float *p, float v) { __builtin_nontemporal_store(v, gm(p)); }
 
-// Two adjacent packed elements in one access (16 bytes in FP64, 8 in FP32), when
-// `vec` (the pair lies inside the matrix and the array offset is even); else two
-// single accesses at o0 and o1.  Halves the vector memory instructions of the
+// Two adjacent packed elements in one access (16 bytes in FP64, 8 in FP32, at any
+// element's alignment), when `vec` (they are neighbours); else two single accesses
+// at o0 and o1.  Halves the vector memory instructions of the
 // wave kernels, whose address unit is their busiest memory stage.
 template <typename T> struct Pair;
-template <> struct Pair<double> { typedef double V __attribute__((ext_vector_type(2))); };
-template <> struct Pair<float> { typedef float V __attribute__((ext_vector_type(2))); };
+template <> struct Pair<double> { typedef double V __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct Pair<float> { typedef float V __attribute__((ext_vector_type(2), aligned(4))); };
 template <bool NT, typename T>
 __device__ __forceinline__ void ld2(const T *p, size_t o0, size_t o1, bool vec, T &a, T &b) {
     if (vec) {
@@ -1375,31 +1375,31 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     const int nn = c.n_nbr;
     const bool grad = tab[6 + nn] != 0.0;
 
-    // Lanes past the last packed element (nb < NBT) repeat it: every load stays in
-    // bounds without a branch, and their LDS and global stores write the same value
-    // to the same address as the lane that owns it.
     // With an even number of doubles per thread, a lane owns adjacent pairs of
-    // elements (2q, 2q+1), q = lane + TPK m', read and written 16 bytes at a time
-    // when nb is even (NP even keeps every pair inside one k and aligned); the
-    // pair is a real diagonal pair or the (re, im) of one upper element.
+    // elements (2q, 2q+1), q = lane + TPK m', always read and written 16 bytes at a
+    // time (8 in FP32): the memory unit takes any element's alignment, so odd band
+    // counts, whose k start at odd offsets, need no second form.  Lanes past the last
+    // pair repeat it, and the last lane of an odd count takes (NP-2, NP-1): every
+    // load stays in bounds without a branch, and repeated LDS and global stores write
+    // the same value to the same address.  A choice between one wide and two single
+    // accesses in front of each load and store took registers and instructions even
+    // where it always fell the same way: RK4 stage of 8 bands, 200 x 200 k, 33.7 us
+    // -> 29.2, of 16 119 -> 112, of 32 bands, 128 x 128, 216 -> 203; AB4 step of 13
+    // bands with dephasing, 61 x 85, 42.1 -> 38.7; Taylor step of 24 bands, 96 x 100,
+    // FP32 operators 131 -> 110.
     constexpr bool kPairs = PER % 2 == 0;
-    // With kLast a lane past the end repeats the last pair, so that the choice of
-    // access is the same on every lane (Taylor step of 24 bands on 96 x 100 k with
-    // FP32 operators 149 us -> 131); at 9..16 bands it gained nothing (16 bands RK4
-    // 119.3 us -> 121.1 a stage, 13 bands AB4 42.1 -> 45.8).
-    constexpr bool kLast = NBT != 16;
     // A stencil pair's calls load the RK2/RK3 accumulator and state at t_n after
     // the products, not with the other inputs: the registers then hold kb's
     // stencil sum instead through the gather and the products.
     constexpr bool kLatePre = ROLE != 0 && kPairs;
-    bool pv2[PER > 1 ? PER / 2 : 1];
+    const bool cp = kPairs && NP % 2 == 0;  // each pair is (re, im) of one upper element or two diagonal ones
     int eo[PER], ei[PER], ej[PER], ec[PER];
     double y[PER], pv[PER], g[PER], pre0[PER], pre1[PER];
     R hv[PER], dv[PER][3];
     const size_t base = (size_t)k * NP;
 #pragma unroll
     for (int m = 0; m < PER; m++) {
-        const int e = kPairs ? min(min(2 * (lane + TPK * (m >> 1)), kLast ? NP - 2 + (NP & 1) : NP - 1) + (m & 1), NP - 1) : min(lane + TPK * m, NP - 1);
+        const int e = kPairs ? min(2 * (lane + TPK * (m >> 1)), NP - 2) + (m & 1) : min(lane + TPK * m, NP - 1);
         eo[m] = e;
         const int code = *gm(c.eidx + e);
         ei[m] = code & 255;
@@ -1408,8 +1408,6 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         g[m] = pre0[m] = pre1[m] = 0.0;
         if constexpr (ROLE == 1) gb[m] = 0.0;
     }
-#pragma unroll
-    for (int h = 0; h < (PER > 1 ? PER / 2 : 1); h++) pv2[h] = kPairs && NP % 2 == 0 && (kLast || 2 * (lane + TPK * h) + 1 < NP);
     // Neighbour data of the stage input, GB neighbours per call, their loads all
     // issued before any is used (k's or kb's stencil slots, by `slot`).
     constexpr int GB = WaveGeom<NBT>::GATHER;
@@ -1424,7 +1422,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
                 for (int h = 0; h < PER / 2; h++) {
                     YT v0, v1;
-                    ld2<false>(Yin, kn[j] + eo[2 * h], kn[j] + eo[2 * h + 1], pv2[h], v0, v1);
+                    ld2<false>(Yin, kn[j] + eo[2 * h], kn[j] + eo[2 * h + 1], true, v0, v1);
                     v[j][2 * h] = (double)v0;
                     v[j][2 * h + 1] = (double)v1;
                 }
@@ -1444,7 +1442,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     // Up to 8 bands a wave serves two k and its stencil rows are vector loads, which
     // return in the order of their requests: the first batch's are requested in front
     // of the stage's operands, not behind them (8 bands, 200 x 200 k, RK4 stage 36 us
-    // -> 33.7).
+    // -> 33.7; 29.2 with the accesses above).
     constexpr bool kRowsFirst = WaveGeom<NBT>::KPB > 1;
     int row0[kRowsFirst ? GB : 1];
     if constexpr (kRowsFirst) {
@@ -1455,23 +1453,22 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
         for (int h = 0; h < PER / 2; h++) {
             const int m = 2 * h;
-            const bool v2 = pv2[h];
             const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
             YT y0, y1;
-            ld2<false>(Yin, o0, o1, v2, y0, y1);
+            ld2<false>(Yin, o0, o1, true, y0, y1);
             y[m] = (double)y0;
             y[m + 1] = (double)y1;
-            ld2<kNT>(Hop, o0, o1, v2, hv[m], hv[m + 1]);
+            ld2<kNT>(Hop, o0, o1, true, hv[m], hv[m + 1]);
 #pragma unroll
             for (int x = 0; x < 3; x++) {
-                if (a.dmask >> x & 1) ld2<kNT>(Dop + (size_t)x * c.nk * NP, o0, o1, v2, dv[m][x], dv[m + 1][x]);
+                if (a.dmask >> x & 1) ld2<kNT>(Dop + (size_t)x * c.nk * NP, o0, o1, true, dv[m][x], dv[m + 1][x]);
                 else dv[m][x] = dv[m + 1][x] = (R)0;
             }
             if constexpr ((MODE == RK2 || MODE == RK3) && !kLatePre) {
-                ld2<kNT>(a.ACC, o0, o1, v2, pre0[m], pre0[m + 1]);
-                ld2<kNT>(a.P0, o0, o1, v2, pre1[m], pre1[m + 1]);
+                ld2<kNT>(a.ACC, o0, o1, true, pre0[m], pre0[m + 1]);
+                ld2<kNT>(a.P0, o0, o1, true, pre1[m], pre1[m + 1]);
             } else if constexpr (MODE == RK4S) {
-                ld2<kNT>(a.ACC, o0, o1, v2, pre0[m], pre0[m + 1]);
+                ld2<kNT>(a.ACC, o0, o1, true, pre0[m], pre0[m + 1]);
             }
         }
     } else {
@@ -1581,7 +1578,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         R *Ad = reinterpret_cast<R *>(A), *Bd = reinterpret_cast<R *>(B);
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            if (kPairs && (m & 1) == 0 && pv2[m >> 1] && eo[m] >= nb) {
+            if (kPairs && (m & 1) == 0 && cp && eo[m] >= nb) {
                 const int i = ei[m], j = ej[m];
                 const bool w = (i >= c.nch && j < c.nch) || (i < c.nch && j >= c.nch);
                 const R E[3] = {w ? Eq[0] : Ep[0], w ? Eq[1] : Ep[1], w ? Eq[2] : Ep[2]};
@@ -1599,7 +1596,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
                 lds_put(B + j * LD + i, CT{dr, c.dherm ? -di : -hv[m + 1] + ddi});
                 continue;
             }
-            if (kPairs && (m & 1) == 1 && pv2[m >> 1] && eo[m - 1] >= nb) continue;  // written with m - 1
+            if (kPairs && (m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // written with m - 1
             const int i = ei[m], j = ej[m], comp = ec[m];
             const bool w = (i >= c.nch && j < c.nch) || (i < c.nch && j >= c.nch);
             const R E[3] = {w ? Eq[0] : Ep[0], w ? Eq[1] : Ep[1], w ? Eq[2] : Ep[2]};  // selects, no pointer
@@ -1639,21 +1636,21 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         for (int h = 0; h < PER / 2; h++) {
             const int m = 2 * h;
             const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-            ld2<kNT>(a.ACC, o0, o1, pv2[h], pre0[m], pre0[m + 1]);
-            ld2<kNT>(a.P0, o0, o1, pv2[h], pre1[m], pre1[m + 1]);
+            ld2<kNT>(a.ACC, o0, o1, true, pre0[m], pre0[m + 1]);
+            ld2<kNT>(a.P0, o0, o1, true, pre1[m], pre1[m + 1]);
         }
     }
     // pv = -i (X_ij - conj(X_ji)) plus the RWA term on core -> non-core pairs; on
     // the diagonal this is 2 Im X_ii.
 #pragma unroll
     for (int m = 0; m < PER; m++) {
-        if (kPairs && (m & 1) == 1 && pv2[m >> 1] && eo[m - 1] >= nb) continue;  // formed with m - 1
+        if (kPairs && (m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // formed with m - 1
         const int i = ei[m], j = ej[m];
         const CT xij = lds_get(C + i * LD + j), xji = lds_get(C + j * LD + i), pij = lds_get(A + i * LD + j);
         const double bre = (double)xij.x - (double)xji.x, bim = (double)xij.y + (double)xji.y;
         const double wr = (i < c.nch && j >= c.nch) ? c.wx2 : 0.0;
         const double vr = bim + -wr * (double)pij.y, vi = -bre + wr * (double)pij.x;
-        if (kPairs && (m & 1) == 0 && pv2[m >> 1] && eo[m] >= nb) {
+        if (kPairs && (m & 1) == 0 && cp && eo[m] >= nb) {
             pv[m] = vr;
             pv[m + 1] = vi;
         } else {
@@ -1737,7 +1734,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         }
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            if (kPairs && (m & 1) == 1 && pv2[m >> 1] && eo[m - 1] >= nb) continue;  // formed with m - 1
+            if (kPairs && (m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // formed with m - 1
             const int i = ei[m], j = ej[m];
             const CT w = A[i * LD + j];
             CT hole = CT{0, 0};
@@ -1748,7 +1745,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
                 hole.x += (uj.x * ui.x + uj.y * ui.y) * tv;
                 hole.y += (uj.x * ui.y - uj.y * ui.x) * tv;
             }
-            if (kPairs && (m & 1) == 0 && pv2[m >> 1] && eo[m] >= nb) {
+            if (kPairs && (m & 1) == 0 && cp && eo[m] >= nb) {
                 pv[m] = pv[m] - (double)w.x + (double)hole.x;
                 pv[m + 1] = pv[m + 1] - (double)w.y + (double)hole.y;
             } else {
@@ -1767,21 +1764,20 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         if (TPK > 64 && 2 * (lane + TPK * h) >= NP) break;
         const double k0 = pv[m] + g[m], k1 = pv[m + 1] + g[m + 1];
         const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-        const bool v2 = pv2[h];
         if constexpr (MODE == ABM) {
-            stage_update2_abm<kNT, S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+            stage_update2_abm<kNT, S>(a, o0, o1, true, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
         } else if constexpr (MODE == TAY) {
-            stage_update2_tay<kNT, S>(a, o0, o1, v2, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+            stage_update2_tay<kNT, S>(a, o0, o1, true, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
         } else if constexpr (MODE == RK1) {
-            st2<kNT>(a.ACC, o0, o1, v2, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
-            st2<kNT>(outs, o0, o1, v2, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
+            st2<kNT>(a.ACC, o0, o1, true, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
+            st2<kNT>(outs, o0, o1, true, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK2 || MODE == RK3) {
-            st2<kNT>(a.ACC, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
-            st2<kNT>(outs, o0, o1, v2, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
+            st2<kNT>(a.ACC, o0, o1, true, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2<kNT>(outs, o0, o1, true, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK4S) {
-            st2<kNT>(a.OUT, o0, o1, v2, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2<kNT>(a.OUT, o0, o1, true, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
         } else {
-            st2<kNT>(a.OUT, o0, o1, v2, k0, k1);
+            st2<kNT>(a.OUT, o0, o1, true, k0, k1);
         }
     }
 }
