@@ -62,7 +62,7 @@ def build_engine():
     os.makedirs(LIB, exist_ok=True)
     out = os.path.join(LIB, "libedus_hip.so")
     srcs = [os.path.join(CSRC, "hip", f) for f in ("engine.hip", "stream.hip")]
-    headers = [os.path.join(ROOT, "include", "edus.h")]
+    headers = [os.path.join(ROOT, "include", "edus.h"), os.path.join(CSRC, "hip", "offsets.hpp")]
     _run_stable([HIPCC, *HIP_FLAGS, *srcs, "-o", out, "-lrocsolver", "-lrocblas"], srcs + headers)
     return out
 

@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "../../../include/edus.h"
+#include "offsets.hpp"
 
 namespace {
 
@@ -364,23 +365,26 @@ constexpr int kSmallMaxThreads = 512;
 template <int NB, bool DISS>
 constexpr int small_wpe() { return (NB <= 2 ? 5 : NB == 3 ? 4 : 3) - (DISS && NB > 2 ? 1 : 0); }
 
-// An element row of a SoA array at the lane's byte offset: the row address is
-// uniform, so the load needs no address arithmetic in vector registers.
-__device__ __forceinline__ double ldrow(const double *row, unsigned off) {
+// An element row of a SoA array at the lane's byte offset (SmallOff): the row address
+// is uniform, so a 32-bit offset needs no address arithmetic in vector registers.
+template <typename O>
+__device__ __forceinline__ double ldrow(const double *row, O off) {
     return *gm(reinterpret_cast<const double *>(reinterpret_cast<const char *>(row) + off));
 }
-__device__ __forceinline__ void strow_nt(double *row, unsigned off, double v) {
+template <typename O>
+__device__ __forceinline__ void strow_nt(double *row, O off, double v) {
     stnt(reinterpret_cast<double *>(reinterpret_cast<char *>(row) + off), v);
 }
 
 // Neighbour n of the lane's k.
-__device__ __forceinline__ int small_index(const ConstArgs &c, int n, unsigned ko) {
+template <typename O>
+__device__ __forceinline__ int small_index(const ConstArgs &c, int n, O ko) {
     return *gm(reinterpret_cast<const int *>(reinterpret_cast<const char *>(c.nbr + (size_t)n * c.nkp) + ko / 2));
 }
 
 // Full P from its packed rows.
 template <int NB>
-__device__ __forceinline__ void small_state(const double *Y, size_t nkp, unsigned ko, cd (&P)[NB][NB]) {
+__device__ __forceinline__ void small_state(const double *Y, size_t nkp, SmallOff<NB> ko, cd (&P)[NB][NB]) {
 #pragma unroll
     for (int i = 0; i < NB; i++) {
         P[i][i] = mk(ldrow(Y + i * nkp, ko), 0.0);
@@ -396,7 +400,7 @@ __device__ __forceinline__ void small_state(const double *Y, size_t nkp, unsigne
 // -i[M, rho] in the transposed storage with M = H + E.D, the probe on core<->non-core
 // elements, and the RWA term (RungeKutta.h:158-212), packed.
 template <int NB>
-__device__ __forceinline__ void small_commutator(const ConstArgs &c, const StageArgs &a, TabRow tab, unsigned ko,
+__device__ __forceinline__ void small_commutator(const ConstArgs &c, const StageArgs &a, TabRow tab, SmallOff<NB> ko,
                                                  double (&pv)[NB * NB]) {
     constexpr int NP = NB * NB;
     const size_t nkp = c.nkp;
@@ -452,7 +456,7 @@ __device__ __forceinline__ void small_commutator(const ConstArgs &c, const Stage
 // Dephasing in the eigenbasis (RungeKutta.h:219-254): the hole source minus
 // conj(U) (T o (conj(U) P U^T)) conj(U), packed.
 template <int NB>
-__device__ __forceinline__ void small_dephasing(const ConstArgs &c, const double *Y, unsigned ko, double (&pv)[NB * NB]) {
+__device__ __forceinline__ void small_dephasing(const ConstArgs &c, const double *Y, SmallOff<NB> ko, double (&pv)[NB * NB]) {
     cd P[NB][NB], U[NB][NB];
     const double *u = c.U + (size_t)(ko / 8) * NB * NB * 2;
 #pragma unroll
@@ -515,12 +519,12 @@ __device__ __forceinline__ void small_dephasing(const ConstArgs &c, const double
 // neighbours n0..n1-1, GB at a time, all in flight; the sum keeps the stencil order.
 // The first NPRE indices (`pre`) are requested by the caller.
 template <int NB, int GB, int NPRE>
-__device__ __forceinline__ void small_drift(const ConstArgs &c, const double *Y, TabRow tab, unsigned ko, int n0, int n1,
+__device__ __forceinline__ void small_drift(const ConstArgs &c, const double *Y, TabRow tab, SmallOff<NB> ko, int n0, int n1,
                                             const int (&pre)[NPRE], double (&g)[NB * NB]) {
     constexpr int NP = NB * NB;
     static_assert(NPRE % GB == 0, "whole batches of requested indices");
     const size_t nkp = c.nkp;
-    auto batch = [&](int n, const unsigned (&off)[GB]) {
+    auto batch = [&](int n, const SmallOff<NB> (&off)[GB]) {
         double v[GB][NP];
 #pragma unroll
         for (int j = 0; j < GB; j++)
@@ -539,15 +543,15 @@ __device__ __forceinline__ void small_drift(const ConstArgs &c, const double *Y,
 #pragma unroll
     for (int q = 0; q < NPRE; q += GB) {
         if (n0 + q >= n1) break;
-        unsigned off[GB];
+        SmallOff<NB> off[GB];
 #pragma unroll
-        for (int j = 0; j < GB; j++) off[j] = 8u * (unsigned)pre[q + j];
+        for (int j = 0; j < GB; j++) off[j] = small_offset<NB>(pre[q + j]);
         batch(n0 + q, off);
     }
     for (int n = n0 + NPRE; n < n1; n += GB) {
-        unsigned off[GB];
+        SmallOff<NB> off[GB];
 #pragma unroll
-        for (int j = 0; j < GB; j++) off[j] = 8u * (unsigned)small_index(c, min(n + j, n1 - 1), ko);
+        for (int j = 0; j < GB; j++) off[j] = small_offset<NB>(small_index(c, min(n + j, n1 - 1), ko));
         batch(n, off);
     }
 }
@@ -559,8 +563,8 @@ struct SmallTail {
     double y, p0, p1, h[NH > 0 ? NH : 1];
 };
 
-template <int MODE>
-__device__ __forceinline__ void small_tail_load(const StageArgs &a, size_t row, size_t hstride, unsigned ko, SmallTail<MODE> &t) {
+template <int MODE, typename O>
+__device__ __forceinline__ void small_tail_load(const StageArgs &a, size_t row, size_t hstride, O ko, SmallTail<MODE> &t) {
     t.y = t.p0 = t.p1 = 0.0;
     if constexpr (MODE == RK1 || MODE == ABM || MODE == TAY) t.y = ldrow(a.Y + row, ko);
     if constexpr (MODE == RK2 || MODE == RK3 || MODE == RK4S) t.p0 = ldrow(a.ACC + row, ko);
@@ -570,8 +574,8 @@ __device__ __forceinline__ void small_tail_load(const StageArgs &a, size_t row, 
         t.h[s] = s + 1 < a.order ? ldrow(a.HIST + (size_t)a.slots[s + 1] * hstride + row, ko) : 0.0;
 }
 
-template <int MODE>
-__device__ __forceinline__ void small_tail_store(const StageArgs &a, size_t row, size_t hstride, unsigned ko, double kv, const SmallTail<MODE> &t) {
+template <int MODE, typename O>
+__device__ __forceinline__ void small_tail_store(const StageArgs &a, size_t row, size_t hstride, O ko, double kv, const SmallTail<MODE> &t) {
     if constexpr (MODE == RK1) {
         strow_nt(a.ACC + row, ko, t.y + kv * a.ca);
         strow_nt(a.OUT + row, ko, t.y + kv * a.cb);
@@ -615,7 +619,7 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
     using G = SmallGeom<NB, DISS>;
     constexpr int NP = G::NP, R = G::R, EPR = G::EPR;
     const bool store = kk < c.nk;
-    const unsigned ko = 8u * (unsigned)min(kk, c.nk - 1);
+    const SmallOff<NB> ko = small_offset<NB>(min(kk, c.nk - 1));
     const size_t nkp = c.nkp;
     const int nn = c.n_nbr;
     SmallTail<MODE> tail[EPR];
@@ -3579,6 +3583,8 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
     *out = nullptr;
     const int nb = p->nb;
     if (p->nk < 1 || nb < 1 || nb > EDUS_MAX_NB) return set_err(EDUS_ERR_INVALID, "nk/nb out of range");
+    const long long padded = nb <= 4 ? ((long long)p->nk + 255) / 256 * 256 : (long long)p->nk;
+    if (padded * nb * nb > kMaxStateElems) return set_err(EDUS_ERR_UNSUPPORTED, "grid too large: nk nb^2 must stay below 2^31");
     if (p->nch < 0 || p->nch > nb || p->ncc < p->nch || p->ncc > nb) return set_err(EDUS_ERR_INVALID, "core/filled band counts out of range");
     if (p->n_nbr < 0 || p->n_nbr > kMaxNbr) return set_err(EDUS_ERR_INVALID, "neighbour count out of range (0..64)");
     if (!p->H || !p->D || !p->U || !p->T || !p->rho0 || (p->n_nbr > 0 && (!p->nbr || !p->nbr_wb)))
@@ -3627,7 +3633,7 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
         return fail(set_err(EDUS_ERR_UNSUPPORTED, "mixed precision is implemented for nb >= 5"));
     if (c->precision == EDUS_PRECISION_BF16X3 && nb <= 8)
         return fail(set_err(EDUS_ERR_UNSUPPORTED, "EDUS_PRECISION_BF16X3 runs on the matrix-core tiles of nb >= 9"));
-    c->nkp = c->soa ? ((p->nk + 255) / 256) * 256 : p->nk;
+    c->nkp = (int)padded;
     // Wave kernels: walk the grid in strips (strip_k) when a strip's two previous
     // rows of packed state, the stencil's reach, fit in kStripL2Bytes while whole
     // rows would not (512 x 512 k at 32 bands: 64-column strips).
