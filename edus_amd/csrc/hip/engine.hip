@@ -740,6 +740,8 @@ struct CoulArgs {
     double *Tt;                // [2][ncut][nu][N2] complex
     double *Xw;                // [2 nu][nkp]: mean-field matrix per k (upper elements, re/im; diagonal basis)
 };
+// The peak correction is on once a band holds carriers (RungeKutta.h:69-138).
+__host__ __device__ __forceinline__ bool mean_field_gate(double n_cond) { return n_cond > 1e-20; }
 // What the renormalised H takes besides: bare H, U, the equilibrium state, the peak
 // correction and its gate.
 struct CoulHArgs {
@@ -981,7 +983,7 @@ __global__ __launch_bounds__(64) void k_coul_w_mfma(CoulArgs a, CoulHArgs h) {
     }
     u = bi * nb - bi * (bi - 1) / 2 + bj - bi;
     // the tile's own operands are in flight during the products
-    const bool diag = bi == bj, scr = FULL && h.n_cond > 1e-20;
+    const bool diag = bi == bj, scr = FULL && mean_field_gate(h.n_cond);
     double hv[4], pr[4], pi[4];
     if constexpr (FULL) {
         const int p = diag ? bi : nb + 2 * pair_index(bi, bj, nb);
@@ -4314,6 +4316,7 @@ int edus_observables(edus_ctx *c, double *pop, double *j1, double *j2, double *t
             const double v = (i < c->ncc) ? 1.0 - h[i] * inv : h[i] * inv;
             if (v > nc) nc = v;
         }
+        if (mean_field_gate(nc) != mean_field_gate(c->n_cond)) drop_graph(c);  // a captured step holds the gate
         c->n_cond = nc;
     }
     return 0;

@@ -50,6 +50,31 @@ def test_graph_steps_with_mean_field(tmp_path):
     _compare(s, 40, [10, 30])
 
 
+def test_graph_steps_follow_the_mean_field_gate(tmp_path):
+    """The peak correction starts with the observables that find carriers, between two
+    chunks of the same table: the captured step has to change with it."""
+    s = N.Setup(Hh.coulomb_input(str(tmp_path), nk=24, dt=0.1, nsteps=200, pump_int=5e13))
+    P0 = s.array("rho0", True).reshape(-1, 3, 3)
+    Uc = s.array("U", True).reshape(-1, 3, 3)[:, 2, :]
+    P = P0 + 0.02 * np.einsum("k,ki,kj->kij", np.cos(np.arange(len(P0))) ** 2, Uc, np.conj(Uc))
+    a, b = N.Engine(s.problem()), N.Engine(s.problem())
+    f, g = s.fields(0, 24)
+    b.set_field_table(f, g)
+    shut = N.Engine(s.problem())  # no observables: its gate stays shut
+    for e in (a, b, shut):
+        e.set_state(P)
+    for lo, hi in ((0, 8), (8, 16), (16, 24)):
+        a.step(f[lo:hi], g[lo:hi])
+        shut.step(f[lo:hi], g[lo:hi])
+        b.step_graph(hi - lo)
+        np.testing.assert_array_equal(b.get_state(), a.get_state())
+        assert np.array_equal(a.get_state(), shut.get_state()) == (lo == 0)  # the gate opened and matters
+        oa, ob = a.observables(), b.observables()
+        assert oa["pop"][2] > 1e-3
+        for key in oa:
+            np.testing.assert_array_equal(ob[key], oa[key])
+
+
 def test_graph_path_rejects_other_steppers(tmp_path):
     s = N.Setup(tb_input(str(tmp_path), nk=8, stepper="Adams_Bashforth 4\n"))
     e = N.Engine(s.problem())
