@@ -2914,11 +2914,16 @@ __device__ __forceinline__ double rsqrt_step(double x, double &m, double &ep) {
     return y;
 }
 
-// V(|q + G|) without the scale, Q2 = |q + G|^2 (Coloumb_THh_F, Coulomb.h:60-84).
-template <bool RK>
+// V(|q + G|) without the scale, Q2 = |q + G|^2 (Coloumb_THh_F, Coulomb.h:60-84).  The
+// fast forms take (q^2 + qTF^2) (|q| r0 + 1)^2 as a whole, which has to be a normal
+// number with |q| r0 + 1 > 0 (edus_coulomb_coefficients looks the parameters over); the
+// general one is the formula as it stands.
+enum CgForm { CG_PLAIN, CG_RYTOVA, CG_GENERAL };
+template <int FORM>
 __device__ __forceinline__ double cgen_v(double q2, double qtf2, double r0) {
     double u = q2 + qtf2, m, ep;
-    if constexpr (RK) {
+    if constexpr (FORM == CG_GENERAL) return 1.0 / (sqrt(u) * (r0 != 0.0 ? sqrt(q2) * r0 + 1.0 : 1.0));
+    if constexpr (FORM == CG_RYTOVA) {
         rsqrt_step(fmax(q2, 1e-290), m, ep);   // q = 0 and G = 0: sqrt is 0 to within 1e-145
         const double t = __builtin_fma(__builtin_fma(m, ep, m), r0, 1.0);
         u = u * t * t;
@@ -2928,7 +2933,7 @@ __device__ __forceinline__ double cgen_v(double q2, double qtf2, double r0) {
 }
 
 // part[y][t][1 + 2 npair]: sums of q number iq0 + t over the G of blockIdx.y.
-template <int NPAIR, bool RK>
+template <int NPAIR, int FORM>
 __global__ __launch_bounds__(kCgThreads) void k_cgen_w(CGenArgs a, long long iq0, int nq, double *part) {
     constexpr int ROW = 2 + 2 * NPAIR, NW = 1 + 2 * NPAIR;
     __shared__ double sg[kCgTile * ROW];
@@ -2955,7 +2960,7 @@ __global__ __launch_bounds__(kCgThreads) void k_cgen_w(CGenArgs a, long long iq0
 #pragma unroll
             for (int q = 0; q < kCgQ; q++) {
                 const double cx = x[q] + s[0], cy = y[q] + s[1];
-                const double v = cgen_v<RK>(__builtin_fma(cx, cx, cy * cy), a.qtf2, a.r0);
+                const double v = cgen_v<FORM>(__builtin_fma(cx, cx, cy * cy), a.qtf2, a.r0);
                 w[q][0] += v;
 #pragma unroll
                 for (int p = 0; p < 2 * NPAIR; p++) w[q][1 + p] = __builtin_fma(v, s[2 + p], w[q][1 + p]);
@@ -4902,7 +4907,21 @@ int edus_coulomb_coefficients(const edus_coulomb_gen *g, double *Ao, double *Bo,
         hipMemcpy(dTr, wtrig.data(), wtrig.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
         return fail(EDUS_ERR_HIP, "coefficient generator upload");
     a.npair = npair; a.n_g = g->n_g; a.N = N; a.mode = 0;
-    a.qtf2 = g->qtf * g->qtf; a.r0 = g->r0;
+    a.qtf2 = g->qtf * g->qtf; a.r0 = g->rytova_keldysh ? g->r0 : 0.0;
+    int form = CG_GENERAL;
+    {
+        // the largest (q^2 + qTF^2) (|q| r0 + 1)^2 of the sums, and no lattice or screening
+        // so small that its square is not a normal number
+        double gx = 0, gy = 0;
+        for (int ig = 0; ig < g->n_g; ig++) {
+            gx = std::max(gx, std::fabs((double)g->g[2 * ig]));
+            gy = std::max(gy, std::fabs((double)g->g[2 * ig + 1]));
+        }
+        const double b1 = (double)l11, b2 = std::hypot((double)l21, (double)l22), qm = (gx + 0.5) * b1 + (gy + 0.5) * b2, t = qm * a.r0 + 1.0;
+        if (a.r0 >= 0.0 && (qm * qm + a.qtf2) * t * t < 1e300 && a.r0 < 1e100 && b1 > 1e-100 && l22 > 1e-100 &&
+            (a.qtf2 == 0.0 || a.qtf2 > 1e-290))
+            form = g->rytova_keldysh ? CG_RYTOVA : CG_PLAIN;
+    }
     a.g = dG; a.qlist = nullptr;
     // sums over G of q numbers [q0, q0 + n) and W from them (of a set of ntot; mirror:
     // its second half comes from the first)
@@ -4912,8 +4931,9 @@ int edus_coulomb_coefficients(const edus_coulomb_gen *g, double *Ao, double *Bo,
         const dim3 grid(blocks_of(n), gs), block(kCgThreads);
         auto go = [&](auto ptag) {
             constexpr int NPAIR = decltype(ptag)::value;
-            if (g->rytova_keldysh) hipLaunchKernelGGL((k_cgen_w<NPAIR, true>), grid, block, 0, 0, c, q0, n, dSum);
-            else hipLaunchKernelGGL((k_cgen_w<NPAIR, false>), grid, block, 0, 0, c, q0, n, dSum);
+            if (form == CG_RYTOVA) hipLaunchKernelGGL((k_cgen_w<NPAIR, CG_RYTOVA>), grid, block, 0, 0, c, q0, n, dSum);
+            else if (form == CG_PLAIN) hipLaunchKernelGGL((k_cgen_w<NPAIR, CG_PLAIN>), grid, block, 0, 0, c, q0, n, dSum);
+            else hipLaunchKernelGGL((k_cgen_w<NPAIR, CG_GENERAL>), grid, block, 0, 0, c, q0, n, dSum);
         };
         if (npair == 0) go(std::integral_constant<int, 0>{});
         else if (npair == 1) go(std::integral_constant<int, 1>{});
