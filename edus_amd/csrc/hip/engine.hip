@@ -16,7 +16,7 @@
 // Kernels: fused RHS + stage update per RK4 stage / Adams-Bashforth step /
 // Taylor step (RungeKutta.h:7-355, RungeKutta.cpp, Linear_Multistep_ODE_solvers.cpp,
 // Taylor_DE_solver_deriv_Polynom.cpp), wave-per-k observable reductions with
-// Kahan-compensated partials (Observables_MPI.h:217-775) and the Wannier phase
+// error-compensated sums over the grid (Observables_MPI.h:217-775) and the Wannier phase
 // contraction (Wannier.h:278-471).
 #include <hip/hip_runtime.h>
 #include <rocblas/rocblas.h>
@@ -1894,7 +1894,7 @@ struct ObsArgs {
     const double *H;     // packed H, or the renormalised H of the mean field
     const double *D;     // packed dipole, components x stride dxs
     const int *eidx;     // packed element -> (i, j, comp) (wave layout)
-    double *part;        // [nv + 2][gridDim.x] block partials
+    double *part;        // [2 nv + 2][gridDim.x] block partials (obs_put)
     unsigned *count;     // finished blocks (0 between launches)
     double *out;         // [nv + 2] results, host memory mapped to the device
     int nk, nkp, nb, nch, ncc, dherm;
@@ -1906,15 +1906,37 @@ struct ObsArgs {
     double *Ek;
 };
 
-struct Kahan {
-    double s = 0.0, c = 0.0;
+// A running sum and the rounding errors of its additions (error-free two-sum): s + e is
+// the sum as if formed in twice the precision and rounded at the end.
+struct Sum2 {
+    double s = 0.0, e = 0.0;
     __device__ __forceinline__ void add(double v) {
-        double yv = v - c;
-        double t = s + yv;
-        c = (t - s) - yv;
+        const double t = s + v, b = t - s;
+        e += (s - (t - b)) + (v - b);
         s = t;
     }
 };
+// The sums of lane groups OFF apart, in all their lanes (operands in lane order, so that
+// all form the same sum); the groups of OFF lanes hold one sum each.
+template <int OFF>
+__device__ __forceinline__ double lane_xor(double v) {
+    if constexpr (OFF == 1) return dpp64<0xB1>(v);
+    else if constexpr (OFF == 2) return dpp64<0x4E>(v);
+    else if constexpr (OFF == 4) return dpp64<0x141>(v);  // half-row mirror
+    else if constexpr (OFF == 8) return dpp64<0x140>(v);  // row mirror
+    else return __shfl_xor(v, OFF, 64);
+}
+template <int OFF>
+__device__ __forceinline__ void sum2_xor(Sum2 &a) {
+    const double s2 = lane_xor<OFF>(a.s), e2 = lane_xor<OFF>(a.e);
+    const bool first = (threadIdx.x & OFF) == 0;
+    Sum2 r;
+    r.s = first ? a.s : s2;
+    r.e = first ? a.e : e2;
+    r.add(first ? s2 : a.s);
+    r.e += first ? e2 : a.e;
+    a = r;
+}
 
 // Accesses of the block partials at device scope, one by one: a device-scope fence
 // per block instead writes back and invalidates the XCD's whole L2 each time
@@ -1922,41 +1944,73 @@ struct Kahan {
 __device__ __forceinline__ void put_agent(double *p, double v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ double get_agent(const double *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// The block's sums (every thread's `acc`, the first N of the kObsSums values, the
-// rest being zero; `pmin`, `pmax`; pops[g * stride + band] of
-// the block's ng groups in LDS, written before the call) to its partials, and, in
-// the block that finishes last, the partials to the results: one wave per value,
-// each lane a strided subset with Kahan compensation, the 64 (sum, compensation)
-// pairs combined with error-free two-sums.  The additions run in a fixed order.
-// One launch instead of a reduction kernel and a copy to the host after it: a
-// 70 x 70 grid of 3 bands spent 10 us on the second kernel and 4 us on the copy.
-template <int N>
-__device__ __forceinline__ void obs_finish(const ObsArgs &o, double (&acc)[N], double pmin, double pmax, const double *pops,
-                                           int ng, int stride) {
-    constexpr int NW = kObsThreads / 64;
-    __shared__ double red[NW][kObsSums + 2];
-    __shared__ int last;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nb = o.nb, nv = nb + kObsSums, G = gridDim.x;
+// Partials of a block: value c < nb + kObsSums as (sum, error) at rows 2c and 2c + 1 of
+// `part`, then min and max, a column per block.
+__device__ __forceinline__ void obs_put(const ObsArgs &o, int c, const Sum2 &v) {
+    double *p = o.part + (size_t)(2 * c) * gridDim.x + blockIdx.x;
+    put_agent(p, v.s);
+    put_agent(p + gridDim.x, v.e);
+}
+
+// Sums of N values over the block's threads (thread t: s[x] + e[x]; HAS_E = false: e is
+// zero) as the partials c0, c0 + 1, ..., V of them at a time through `buf` in LDS
+// (obs_buf doubles): eight lanes per value take 32 threads' terms each.  Every addition
+// keeps its error: J1, J2 and TAbs cancel over the grid.  Six rounds of lane exchanges
+// per value instead, with the errors, are 3.5 times the instructions.
+constexpr int kObsRow = kObsThreads + 8;  // eight values' rows start in different LDS banks
+template <int V, bool HAS_E>
+constexpr int obs_buf() { return V * (HAS_E ? 2 : 1) * kObsRow; }
+
+template <int V, bool HAS_E, int N>
+__device__ __forceinline__ void obs_block_sums(const ObsArgs &o, int c0, const double (&s)[N], const double (&e)[N], double *buf) {
+    const int t = threadIdx.x, x = t >> 3;
+    static_assert(V * 8 <= kObsThreads, "eight lanes per value");
 #pragma unroll
-    for (int x = 0; x < kObsSums; x++) {
-        const double v = x < N ? wave_sum(acc[x < N ? x : 0]) : 0.0;
-        if (lane == 0) red[wave][x] = v;
+    for (int r = 0; r < N; r += V) {
+        __syncthreads();  // the buffer's last use is over
+#pragma unroll
+        for (int v = 0; v < V; v++)
+            if (r + v < N) {
+                buf[v * kObsRow + t] = s[r + v < N ? r + v : 0];
+                if (HAS_E) buf[(V + v) * kObsRow + t] = e[r + v < N ? r + v : 0];
+            }
+        __syncthreads();
+        Sum2 a;
+        const bool mine = x < V && r + x < N;
+        if (mine) {
+#pragma unroll 8
+            for (int i = t & 7; i < kObsThreads; i += 8) {
+                a.add(buf[x * kObsRow + i]);
+                if (HAS_E) a.e += buf[(V + x) * kObsRow + i];
+            }
+        }
+        sum2_xor<1>(a);
+        sum2_xor<2>(a);
+        sum2_xor<4>(a);
+        if (mine && (t & 7) == 0) obs_put(o, c0 + r + x, a);
     }
+}
+
+// After the block's sums: `pmin`, `pmax` to its partials, and, in the block that
+// finishes last, the partials of the first nsum values to the results (the rest are
+// zero): one wave per value, each lane a strided subset, errors kept, the additions in a
+// fixed order.  One launch instead of a reduction kernel and a copy to the host after
+// it: a 70 x 70 grid of 3 bands spent 10 us on the second kernel and 4 us on the copy.
+__device__ __forceinline__ void obs_finish(const ObsArgs &o, int nsum, double pmin, double pmax) {
+    constexpr int NW = kObsThreads / 64;
+    __shared__ double red[NW][2];
+    __shared__ int last;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nv = o.nb + kObsSums, G = gridDim.x;
     const double mn = wave_min(pmin), mx = wave_max(pmax);
     if (lane == 0) {
-        red[wave][kObsSums] = mn;
-        red[wave][kObsSums + 1] = mx;
+        red[wave][0] = mn;
+        red[wave][1] = mx;
     }
     __syncthreads();
-    if (t < nb) {
-        double v = 0.0;
-        for (int g = 0; g < ng; g++) v += pops[g * stride + t];
-        put_agent(o.part + (size_t)t * G + blockIdx.x, v);
-    } else if (t >= 64 && t < 64 + kObsSums + 2) {
-        const int x = t - 64;
-        double v = red[0][x];
-        for (int w = 1; w < NW; w++) v = x == kObsSums ? fmin(v, red[w][x]) : x > kObsSums ? fmax(v, red[w][x]) : v + red[w][x];
-        put_agent(o.part + (size_t)(nb + x) * G + blockIdx.x, v);
+    if (t < 2) {
+        double v = red[0][t];
+        for (int w = 1; w < NW; w++) v = t == 0 ? fmin(v, red[w][0]) : fmax(v, red[w][1]);
+        put_agent(o.part + (size_t)(2 * nv + t) * G + blockIdx.x, v);
     }
     // the block's partials have reached the device's coherence point (every wave
     // waits for its own agent-scope stores) before its arrival is counted
@@ -1966,23 +2020,25 @@ __device__ __forceinline__ void obs_finish(const ObsArgs &o, double (&acc)[N], d
     __syncthreads();
     if (!last) return;
     for (int c = wave; c < nv + 2; c += NW) {
-        const double *p = o.part + (size_t)c * G;
         if (c < nv) {
-            Kahan k;
+            const double *p = o.part + (size_t)(2 * c) * G;
+            Sum2 a;
+            if (c < nsum) {
 #pragma unroll 4
-            for (int b = lane; b < G; b += 64) k.add(get_agent(p + b));
-            double s = k.s, lo = -k.c;
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                // both lanes of a pair form the same sum: the operands in lane order
-                const double s2 = __shfl_xor(s, off, 64), l2 = __shfl_xor(lo, off, 64);
-                const bool first = (lane & off) == 0;
-                const double a = first ? s : s2, b = first ? s2 : s, sum = a + b, bp = sum - a;
-                lo = (first ? lo : l2) + (first ? l2 : lo) + ((a - (sum - bp)) + (b - bp));
-                s = sum;
+                for (int b = lane; b < G; b += 64) {
+                    a.add(get_agent(p + b));
+                    a.e += get_agent(p + G + b);
+                }
+                sum2_xor<1>(a);
+                sum2_xor<2>(a);
+                sum2_xor<4>(a);
+                sum2_xor<8>(a);
+                sum2_xor<16>(a);
+                sum2_xor<32>(a);
             }
-            if (lane == 0) o.out[c] = s + lo;
+            if (lane == 0) o.out[c] = a.s + a.e;
         } else {
+            const double *p = o.part + (size_t)(nv + c) * G;
             double v = c == nv ? 1.0 : 0.0;
             for (int b = lane; b < G; b += 64) v = c == nv ? fmin(v, get_agent(p + b)) : fmax(v, get_agent(p + b));
             v = c == nv ? wave_min(v) : wave_max(v);
@@ -2066,16 +2122,20 @@ __device__ __forceinline__ void jacobi_small(cd (&A)[NB][NB], cd (&V)[NB][NB], d
 // kept for edus_renorm_energies.  Bound by the latency of its loads and of the
 // final sums: 60 x 60 k of 3 bands 23 us (two kernels of a wave per k) -> 13;
 // with the mean field, 300 x 300, 345 us (tables written, then read) -> 46.
+// Waves per SIMD: at 3 and 4 bands the compiler would give up loads in flight for one
+// more (4 bands 1000 x 1000 k, whole call: 373 us, 318 with two; 3 bands 300 x 300 44.8,
+// 42.5 with three).
+constexpr int obs_wpe(int nb, int other) { return nb == 4 ? 2 : nb == 3 ? 3 : other; }
 template <int NB, bool COUL>
-__global__ __launch_bounds__(kObsThreads) void k_obs_small(ObsArgs o) {
+__global__ __launch_bounds__(kObsThreads) __attribute__((amdgpu_waves_per_eu(obs_wpe(NB, 1), obs_wpe(NB, 8)))) void k_obs_small(ObsArgs o) {
     constexpr int NP = NB * NB;
-    __shared__ double pops[kObsThreads / 64][NB];
+    constexpr int V = NB + kObsSums;  // up to 40 KB of LDS, and four blocks per CU
+    __shared__ double buf[obs_buf<V, false>()];
     const size_t nkp = o.nkp;
-    double pop[NB], acc[kObsSums], pmin = 1.0, pmax = 0.0;
+    double val[NB + kObsSums], pmin = 1.0, pmax = 0.0;  // populations, J1, J2, TAbs
+    double *const acc = val + NB;
 #pragma unroll
-    for (int c = 0; c < NB; c++) pop[c] = 0.0;
-#pragma unroll
-    for (int x = 0; x < kObsSums; x++) acc[x] = 0.0;
+    for (int x = 0; x < NB + kObsSums; x++) val[x] = 0.0;
     const int k = blockIdx.x * kObsThreads + threadIdx.x;
     if (k < o.nk) {
         double y[NP], h[NP];
@@ -2141,7 +2201,7 @@ __global__ __launch_bounds__(kObsThreads) void k_obs_small(ObsArgs o) {
                 for (int j = 0; j < NB; j++) t = cadd(t, cmul(P[i][j], U[c][j]));
                 s += U[c][i].x * t.x + U[c][i].y * t.y;
             }
-            pop[c] = s;
+            val[c] = s;
             const double hv = (c < o.ncc) ? 1. - s : s;
             pmax = fmax(pmax, fabs(hv));
             pmin = fmin(pmin, hv);
@@ -2209,12 +2269,8 @@ __global__ __launch_bounds__(kObsThreads) void k_obs_small(ObsArgs o) {
             acc[10 + 2 * x] = -2. * ta.y;
         }
     }
-#pragma unroll
-    for (int c = 0; c < NB; c++) {
-        const double v = wave_sum(pop[c]);
-        if ((threadIdx.x & 63) == 0) pops[threadIdx.x >> 6][c] = v;
-    }
-    obs_finish(o, acc, pmin, pmax, &pops[0][0], kObsThreads / 64, NB);
+    obs_block_sums<V, false>(o, 0, val, val, buf);
+    obs_finish(o, NB + kObsSums, pmin, pmax);
 }
 
 // nb 5..32: the stage kernels' thread groups (TPK threads per k), P, U and H of
@@ -2226,9 +2282,15 @@ __global__ __launch_bounds__(kObsThreads) void k_obs_small(ObsArgs o) {
 // 1168; 16 bands 200 x 200 534 -> 233 us, 8 bands 99 -> 74.  Registers decide how
 // many blocks a CU holds: without TAbs (no core bands) its six compensated sums
 // are compiled out.
+constexpr int kObsWaveV = 9;  // sums per round of obs_block_sums, in the matrices' LDS
+template <int NBT>
+__host__ __device__ constexpr int obs_mat_doubles() {
+    constexpr int mats = (kObsThreads / WaveGeom<NBT>::TPK) * 3 * NBT * WaveGeom<NBT>::LD * 2, sums = obs_buf<kObsWaveV, true>();
+    return mats > sums ? mats : sums;
+}
 template <int NBT>
 __host__ __device__ constexpr int obs_lds_doubles() {
-    return (kObsThreads / WaveGeom<NBT>::TPK) * (3 * NBT * WaveGeom<NBT>::LD * 2 + NBT) + (NBT == 32 ? 64 : 0);
+    return obs_mat_doubles<NBT>() + (kObsThreads / WaveGeom<NBT>::TPK) * 2 * NBT + (NBT == 32 ? 64 : 0);
 }
 
 template <int NBT, bool TA>
@@ -2240,15 +2302,15 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
     const int grp = threadIdx.x / TPK, lane = threadIdx.x % TPK;
     const int nb = o.nb, NP = nb * nb, nch = o.nch;
     cd *A = reinterpret_cast<cd *>(smem_d) + (size_t)grp * 3 * MAT, *B = A + MAT, *C = B + MAT;
-    double *pops = smem_d + (size_t)KPB * 3 * MAT * 2;    // [KPB][NBT], written at the end
-    double *popw = pops + KPB * NBT;                      // NBT = 32: [2][32] per-k halves of the population
+    Sum2 *pops = reinterpret_cast<Sum2 *>(smem_d + obs_mat_doubles<NBT>());  // [KPB][NBT], written at the end
+    double *popw = reinterpret_cast<double *>(pops + KPB * NBT);                // NBT = 32: [2][32] per-k halves of the population
     for (int t = lane; t < 3 * MAT; t += TPK) A[t] = mk(0.0, 0.0);
     auto elem = [&](int m) { return 2 * (lane + TPK * (m >> 1)) + (m & 1); };
     int code0[PER];
 #pragma unroll
     for (int m = 0; m < PER; m++) code0[m] = o.eidx[min(elem(m), NP - 1)];
     constexpr int NS = TA ? kObsSums : 9;
-    Kahan pop, acc[NS];
+    Sum2 pop, acc[NS];
     double pmin = 1.0, pmax = 0.0;
     auto band = [&](int c, double sre) {
         pop.add(sre);
@@ -2275,7 +2337,7 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
         auto row = [&](int m) { return code[m] & 255; };
         auto col = [&](int m) { return (code[m] >> 8) & 255; };
         auto imag = [&](int m) { return (code[m] >> 16) != 0; };
-        double y[PER], h[PER], ur[PER], ui[PER], s[NS];
+        double y[PER], h[PER], ur[PER], ui[PER];
 #pragma unroll
         for (int q = 0; q < PER / 2; q++) {
             const int m = 2 * q;
@@ -2288,8 +2350,6 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
             const size_t t = base + min(lane + TPK * m, NP - 1);
             ld2<true>(o.U, 2 * t, 2 * t + 1, true, ur[m], ui[m]);
         }
-#pragma unroll
-        for (int x = 0; x < NS; x++) s[x] = 0.0;
         if (o.GE) {  // J1: sum_ij P_ij gradH_ij (real: both Hermitian; a pair counts twice)
             const double *ge = o.GE + (size_t)k * 3 * NP;
             double g[PER][3];
@@ -2300,9 +2360,10 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
                     ld2<true>(ge + (size_t)x * NP, eo[2 * q], eo[2 * q + 1], v2[q], g[2 * q][x], g[2 * q + 1][x]);
 #pragma unroll
             for (int m = 0; m < PER; m++) {
-                const double f = elem(m) >= NP ? 0.0 : row(m) == col(m) ? y[m] : imag(m) ? -2. * y[m] : 2. * y[m];
+                if (!live || elem(m) >= NP) continue;
+                const double f = row(m) == col(m) ? y[m] : imag(m) ? -2. * y[m] : 2. * y[m];
 #pragma unroll
-                for (int x = 0; x < 3; x++) s[x] += f * g[m][x];
+                for (int x = 0; x < 3; x++) acc[x].add(f * g[m][x]);
             }
         }
         __syncthreads();  // the previous k's LDS reads are done
@@ -2384,7 +2445,7 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
         // lower one being D_jc or its conjugate; TAbs
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            if (elem(m) >= NP) continue;
+            if (!live || elem(m) >= NP) continue;
             const int i = row(m), j = col(m);
             const bool im = imag(m);
             const cd wu = lds_get(A + i * LD + j), wl = lds_get(A + j * LD + i);
@@ -2395,28 +2456,37 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
             else w = mk(wu.y + wl.y, -(wu.x + wl.x));
 #pragma unroll
             for (int x = 0; x < 3; x++) {
-                s[3 + 2 * x] += d[m][x] * w.x;
-                s[4 + 2 * x] += d[m][x] * w.y;
+                acc[3 + 2 * x].add(d[m][x] * w.x);
+                acc[4 + 2 * x].add(d[m][x] * w.y);
             }
             if (TA && i < nch && j >= nch) {
                 const cd p = im ? mk(-pij[m].y, pij[m].x) : pij[m];
 #pragma unroll
                 for (int x = 0; x < 3; x++) {
-                    s[TA ? 9 + 2 * x : 0] += -2. * d[m][x] * p.x;
-                    s[TA ? 10 + 2 * x : 0] += -2. * d[m][x] * p.y;
+                    acc[TA ? 9 + 2 * x : 0].add(-2. * d[m][x] * p.x);
+                    acc[TA ? 10 + 2 * x : 0].add(-2. * d[m][x] * p.y);
                 }
             }
         }
-        if (live) {
-#pragma unroll
-            for (int x = 0; x < NS; x++) acc[x].add(s[x]);
-        }
     }
-    if (lane < nb) pops[grp * NBT + lane] = pop.s;
-    double sums[NS];
+    if (lane < nb) pops[grp * NBT + lane] = pop;
+    double s[NS], e[NS];
 #pragma unroll
-    for (int x = 0; x < NS; x++) sums[x] = acc[x].s;
-    obs_finish(o, sums, pmin, pmax, pops, KPB, NBT);
+    for (int x = 0; x < NS; x++) {
+        s[x] = acc[x].s;
+        e[x] = acc[x].e;
+    }
+    obs_block_sums<kObsWaveV, true>(o, nb, s, e, smem_d);
+    if (threadIdx.x < nb) {
+        Sum2 a;
+        for (int g = 0; g < KPB; g++) {
+            const Sum2 v = pops[g * NBT + threadIdx.x];
+            a.add(v.s);
+            a.e += v.e;
+        }
+        obs_put(o, threadIdx.x, a);
+    }
+    obs_finish(o, nb + NS, pmin, pmax);
 }
 
 // ================================================================ setup helpers
@@ -3767,7 +3837,7 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
         const int kpb = c->soa ? kObsThreads : kObsThreads / (nb <= 8 ? WaveGeom<8>::TPK : nb <= 16 ? WaveGeom<16>::TPK : WaveGeom<32>::TPK);
         const int nblk = (p->nk + kpb - 1) / kpb;
         c->obs_blocks = c->soa ? nblk : std::min(nb <= 8 ? kObsMaxBlocks : 3 * kObsMaxBlocks / 4, nblk);
-        if ((rc = dalloc(c, &c->part, (size_t)c->obs_blocks * (nb + kObsSums + 2))) || (rc = dalloc(c, &c->obs_count, 1))) return fail(rc);
+        if ((rc = dalloc(c, &c->part, (size_t)c->obs_blocks * 2 * (nb + kObsSums + 1))) || (rc = dalloc(c, &c->obs_count, 1))) return fail(rc);
         if (!(c->obs = g_results.take())) return fail(set_err(EDUS_ERR_NOMEM, "observables result buffer"));
         if (hipMemsetAsync(c->obs_count, 0, sizeof(unsigned), c->stream) != hipSuccess) return fail(set_err(EDUS_ERR_HIP, "memset count"));
     }
