@@ -26,6 +26,8 @@ HIP_FLAGS = [
     # MFMA accumulators in ordinary VGPRs: the stage kernels then need no AGPRs
     # on top of their VGPRs and keep 4 waves per SIMD (8-17 % faster at 32 bands)
     "-mllvm", "-amdgpu-mfma-vgpr-form",
+    # accesses through a type whose alignment the address does not have
+    "-Werror=align-mismatch",
     "-Wno-unused-result",
 ]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off", "-Wall", "-Wno-unused-variable"]

@@ -229,13 +229,15 @@ __device__ __forceinline__ void stnt(float *p, float v) { __builtin_nontemporal_
 // element's alignment), when `vec` (they are neighbours); else two single accesses
 // at o0 and o1.  Halves the vector memory instructions of the
 // wave kernels, whose address unit is their busiest memory stage.
+// The pointers are cast to the pair type in one go: a template that deduces it (gm)
+// would drop its alignment and promise 16 bytes.
 template <typename T> struct Pair;
 template <> struct Pair<double> { typedef double V __attribute__((ext_vector_type(2), aligned(8))); };
 template <> struct Pair<float> { typedef float V __attribute__((ext_vector_type(2), aligned(4))); };
 template <bool NT, typename T>
 __device__ __forceinline__ void ld2(const T *p, size_t o0, size_t o1, bool vec, T &a, T &b) {
     if (vec) {
-        const auto *q = gm(reinterpret_cast<const typename Pair<T>::V *>(p + o0));
+        const auto *q = (const __attribute__((address_space(1))) typename Pair<T>::V *)(p + o0);
         const typename Pair<T>::V v = NT ? __builtin_nontemporal_load(q) : *q;
         a = v.x;
         b = v.y;
@@ -250,7 +252,7 @@ __device__ __forceinline__ void st2(T *p, size_t o0, size_t o1, bool vec, T a, T
         typename Pair<T>::V v;
         v.x = a;
         v.y = b;
-        auto *q = gm(reinterpret_cast<typename Pair<T>::V *>(p + o0));
+        auto *q = (__attribute__((address_space(1))) typename Pair<T>::V *)(p + o0);
         if (NT) __builtin_nontemporal_store(v, q);
         else *q = v;
     } else if (NT) {
