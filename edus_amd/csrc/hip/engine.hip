@@ -669,7 +669,7 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
 // blockDim = (k per workgroup, SmallGeom::R)
 template <int NB, int MODE, bool DISS>
 __global__ __launch_bounds__(kSmallMaxThreads, (small_wpe<NB, DISS>())) void k_stage_small(ConstArgs c, StageArgs a) {
-    extern __shared__ double smem_d[];
+    extern __shared__ __align__(16) double smem_d[];
     const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
     stage_small<NB, MODE, DISS>(c, a, stage_row(a), xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
 }
@@ -1206,7 +1206,7 @@ __device__ __forceinline__ void mfma_tile(int t, int &r0, int &c0) {
 }
 
 // LDS complex element access: an FP64 complex moves as one 16-byte access
-// (ds_read_b128 / ds_write_b128; the matrices start 16-byte aligned and every
+// (ds_read_b128 / ds_write_b128; the LDS arrays are declared 16-byte aligned and every
 // element is 16 bytes) rather than two 8-byte halves, whose 32-lane passes put
 // rows r and r + 1 of neighbouring K slices on one bank.
 template <typename T>
@@ -1798,7 +1798,7 @@ constexpr int wave_occupancy(int nbt, bool pair) { return nbt == 8 ? 4 : nbt == 
 // the stencil pair (2q, 2q + 1).
 template <int NBT, int MODE, typename R, typename S = double, bool B3 = false, bool PAIR = false>
 __global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB, wave_occupancy(NBT, PAIR)) void k_stage_wave(ConstArgs c, StageArgs a) {
-    extern __shared__ double smem_d[];
+    extern __shared__ __align__(16) double smem_d[];
     constexpr int TPK = WaveGeom<NBT>::TPK;
     double gb[WaveGeom<NBT>::PER];
     if constexpr (PAIR) {
@@ -1844,7 +1844,7 @@ __host__ __device__ constexpr int rk4_stage_of() { return MODE == RK1 ? 0 : MODE
 
 template <int NB, int MODE, bool DISS>
 __global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) void k_stage_small_batch(const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
-    extern __shared__ double smem_d[];
+    extern __shared__ __align__(16) double smem_d[];
     const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int2 w = blk[xcd_block()];
     const BatchEntry &be = E[w.x];
@@ -1857,7 +1857,7 @@ __global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) vo
 template <int NBT, int MODE, typename R, bool PAIR = false>
 __global__ __launch_bounds__(WaveGeom<NBT>::TPK * WaveGeom<NBT>::KPB, wave_occupancy(NBT, PAIR)) void k_stage_wave_batch(
     const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
-    extern __shared__ double smem_d[];
+    extern __shared__ __align__(16) double smem_d[];
     constexpr int TPK = WaveGeom<NBT>::TPK;
     const int2 w = blk[xcd_block()];
     const BatchEntry &be = E[w.x];
@@ -2297,7 +2297,7 @@ __host__ __device__ constexpr int obs_lds_doubles() {
 
 template <int NBT, bool TA>
 __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_wave(ObsArgs o) {
-    extern __shared__ double smem_d[];
+    extern __shared__ __align__(16) double smem_d[];
     constexpr int TPK = WaveGeom<NBT>::TPK, KPB = kObsThreads / TPK, PER = WaveGeom<NBT>::PER, LD = WaveGeom<NBT>::LD, MAT = NBT * LD;
     constexpr int RBR = WaveGeom<NBT>::RBR, RBC = WaveGeom<NBT>::RBC;
     static_assert(PER % 2 == 0, "a thread owns pairs of packed elements");
@@ -2731,8 +2731,8 @@ __global__ __launch_bounds__(256) void k_wannier_mfma(const cd *__restrict__ PT,
                                                       int N0, int N1, int N2, int nR, int nw2, int nm, int ncol, int nk, int kbase,
                                                       cd *__restrict__ Hd, cd *__restrict__ Dd) {
     constexpr int NT = 4;
-    __shared__ cd Ph[WMK][WMR + 1];
-    __shared__ cd Vs[WMR][16 * NT + 1];
+    __shared__ __align__(16) cd Ph[WMK][WMR + 1];
+    __shared__ __align__(16) cd Vs[WMR][16 * NT + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int k0 = blockIdx.y * WMK, m0 = blockIdx.x * 16 * NT;
     v4d are[NT], aim[NT];
