@@ -3210,6 +3210,81 @@ __global__ __launch_bounds__(kCgPeakThreads) void k_cgen_peak(const double *W0, 
     }
 }
 
+// Copies of large results to the caller's ordinary memory.  hipMemcpy locks that
+// memory page by page in front of the copy engine (9.3 GB/s into fresh pages, 17 into
+// touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
+// memory, and each of a few threads copies its own piece on to the caller's pages
+// while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring (12 MB) belongs
+// to the object, made by its first large copy.  From 16 MB on (16.8 MB: 1.24 -> 1.07 ms,
+// 33 MB 2.5 -> 1.6; 8 MB even).
+class Downloader {
+    static constexpr size_t kPiece = 2 << 20;
+    static constexpr int kWorkers = 6;
+    char *ring = nullptr;
+    hipEvent_t ev[kWorkers] = {};
+    int dev = 0;
+
+    bool ready() {
+        if (ring) return true;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        for (hipEvent_t &e : ev)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, kWorkers * kPiece, hipHostMallocDefault) != hipSuccess) return false;
+        ring = static_cast<char *>(p);
+        return true;
+    }
+
+public:
+    Downloader() = default;
+    Downloader(const Downloader &) = delete;
+    Downloader &operator=(const Downloader &) = delete;
+    ~Downloader() {
+        for (hipEvent_t e : ev)
+            if (e) (void)hipEventDestroy(e);
+        if (ring) (void)hipHostFree(ring);
+    }
+    // n bytes of device memory, in the stream's order; returns when dst holds them.
+    hipError_t copy(void *dst, const void *src, size_t n, hipStream_t st) {
+        if (n < 8 * kPiece || !ready()) {
+            const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
+            return e == hipSuccess ? hipStreamSynchronize(st) : e;
+        }
+        std::mutex mu;
+        size_t next = 0;
+        hipError_t err = hipSuccess;
+        auto work = [&](int w) {
+            char *slot = ring + w * kPiece;
+            hipError_t e = hipSetDevice(dev);
+            for (;;) {
+                size_t o, len;
+                {
+                    std::lock_guard<std::mutex> lock(mu);
+                    if (e != hipSuccess) err = e;
+                    if (err != hipSuccess || next >= n) return;
+                    o = next;
+                    len = std::min(kPiece, n - o);
+                    next += len;
+                    e = hipMemcpyAsync(slot, static_cast<const char *>(src) + o, len, hipMemcpyDeviceToHost, st);
+                    if (e == hipSuccess) e = hipEventRecord(ev[w], st);
+                }
+                if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
+                if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + o, slot, len);
+            }
+        };
+        std::thread th[kWorkers - 1];
+        try {
+            for (int w = 1; w < kWorkers; w++) th[w - 1] = std::thread(work, w);
+        } catch (...) {
+            // fewer workers: the others, this thread at least, take their pieces
+        }
+        work(0);
+        for (std::thread &t : th)
+            if (t.joinable()) t.join();
+        return err;
+    }
+};
+
 }  // namespace
 
 // ==================================================================== context
@@ -3236,6 +3311,7 @@ struct edus_ctx {
     int *nbr = nullptr;
     double *tab = nullptr;
     size_t tab_cap = 0;
+    Downloader down;                  // large results to the host
     double *part = nullptr;           // observables: block partials, finished-block count, results (host memory)
     unsigned *obs_count = nullptr;
     double *obs = nullptr;
@@ -4152,102 +4228,24 @@ int edus_step_taylor(edus_ctx *c, int32_t nsteps, const double *fields, const ui
     return step_multistep(c, nsteps, fields, grad_on, true);
 }
 
-// Copies of large results to the caller's ordinary memory.  hipMemcpy locks that
-// memory page by page in front of the copy engine (9.3 GB/s into fresh pages, 17 into
-// touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
-// memory, and each of a few threads copies its own piece on to the caller's pages
-// while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring belongs to the
-// object (12 MB).  From 16 MB on (16.8 MB: 1.24 -> 1.07 ms, 33 MB 2.5 -> 1.6; 8 MB even).
 namespace {
-class Downloader {
-    static constexpr size_t kPiece = 2 << 20;
-    static constexpr int kWorkers = 6;
-    char *ring = nullptr;
-    hipEvent_t ev[kWorkers] = {};
-    int dev = 0;
-
-    bool ready() {
-        if (ring) return true;
-        if (hipGetDevice(&dev) != hipSuccess) return false;
-        for (hipEvent_t &e : ev)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-        void *p = nullptr;
-        if (hipHostMalloc(&p, kWorkers * kPiece, hipHostMallocDefault) != hipSuccess) return false;
-        ring = static_cast<char *>(p);
-        return true;
-    }
-
-public:
-    Downloader() = default;
-    Downloader(const Downloader &) = delete;
-    Downloader &operator=(const Downloader &) = delete;
-    ~Downloader() {
-        for (hipEvent_t e : ev)
-            if (e) (void)hipEventDestroy(e);
-        if (ring) (void)hipHostFree(ring);
-    }
-    // n bytes of device memory, in the stream's order; returns when dst holds them.
-    hipError_t copy(void *dst, const void *src, size_t n, hipStream_t st) {
-        if (n < 8 * kPiece || !ready()) {
-            const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
-            return e == hipSuccess ? hipStreamSynchronize(st) : e;
-        }
-        std::mutex mu;
-        size_t next = 0;
-        hipError_t err = hipSuccess;
-        auto work = [&](int w) {
-            char *slot = ring + w * kPiece;
-            hipError_t e = hipSetDevice(dev);
-            for (;;) {
-                size_t o, len;
-                {
-                    std::lock_guard<std::mutex> lock(mu);
-                    if (e != hipSuccess) err = e;
-                    if (err != hipSuccess || next >= n) return;
-                    o = next;
-                    len = std::min(kPiece, n - o);
-                    next += len;
-                    e = hipMemcpyAsync(slot, static_cast<const char *>(src) + o, len, hipMemcpyDeviceToHost, st);
-                    if (e == hipSuccess) e = hipEventRecord(ev[w], st);
-                }
-                if (e == hipSuccess) e = hipEventSynchronize(ev[w]);
-                if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + o, slot, len);
-            }
-        };
-        std::thread th[kWorkers - 1];
-        try {
-            for (int w = 1; w < kWorkers; w++) th[w - 1] = std::thread(work, w);
-        } catch (...) {
-            // fewer workers: the others, this thread at least, take their pieces
-        }
-        work(0);
-        for (std::thread &t : th)
-            if (t.joinable()) t.join();
-        return err;
-    }
-};
-
 // Packed array Y of the context (complete in stream order) to the caller's full
 // matrices.  From 16 MB of them on they are unpacked on the device, up to 64 MB at a
-// time (16.8 MB: 2.0 ms with the host's loop, 1.1 so; 67 MB 14.2, 2.5; 268 MB 49, 8.3).
-// Below, and where the device has no room for the piece, the host unpacks: the piece's
-// allocation and first use take what the kernel gives (0.5 MB: 0.048 and 0.055 ms, 8.2 MB
-// 0.61 and 0.64, the first call 0.79 and 1.05).
+// time, into the accumulator (scratch between steps for every stepper).  Nothing is
+// allocated or freed on the device: that waits for every stream of it (an 82 MB state
+// beside another context's steps: 259 ms with a buffer of the call's own, 4 as now).
+// Below, the host unpacks.
 int download_full(edus_ctx *c, const double *Y, double *out) {
     const size_t per = (size_t)c->np * 16;
-    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(c->nk, ((size_t)64 << 20) / per));
-    void *q = nullptr;
-    if (c->nk * per < ((size_t)16 << 20) || hipMalloc(&q, chunk * per) != hipSuccess) {
-        if (c->nk * per >= ((size_t)16 << 20)) (void)hipGetLastError();
+    if (c->nk * per < ((size_t)16 << 20)) {
         std::vector<double> st(state_elems(c));
         HIP_TRY(hipMemcpyAsync(st.data(), Y, st.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         unpack_state(c, st, out);
         return 0;
     }
-    const std::unique_ptr<double, DeviceFree> hold(static_cast<double *>(q));
-    double *buf = hold.get();
-    Downloader down;
+    const int chunk = (int)std::min<size_t>(state_elems(c) / (2 * (size_t)c->np), ((size_t)64 << 20) / per);
+    double *buf = c->ACC;
     const size_t sk = c->soa ? 1 : (size_t)c->np, se = c->soa ? (size_t)c->nkp : 1;
     for (int k0 = 0; k0 < c->nk; k0 += chunk) {
         const int kc = std::min(chunk, c->nk - k0);
@@ -4255,7 +4253,7 @@ int download_full(edus_ctx *c, const double *Y, double *out) {
         hipLaunchKernelGGL(k_unpack, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, Y, n, c->nb, sk, se, k0,
                            reinterpret_cast<cd *>(buf));
         HIP_TRY(hipGetLastError());
-        HIP_TRY(down.copy(out + (size_t)k0 * c->np * 2, buf, kc * per, c->stream));
+        HIP_TRY(c->down.copy(out + (size_t)k0 * c->np * 2, buf, kc * per, c->stream));
     }
     return 0;
 }
