@@ -3246,7 +3246,9 @@ public:
     }
     // n bytes of device memory, in the stream's order; returns when dst holds them.
     hipError_t copy(void *dst, const void *src, size_t n, hipStream_t st) {
-        if (n < 8 * kPiece || !ready()) {
+        const bool ring_used = n >= 8 * kPiece && ready();
+        if (!ring_used) {
+            if (n >= 8 * kPiece) (void)hipGetLastError();  // the ring's: this copy does without it
             const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
             return e == hipSuccess ? hipStreamSynchronize(st) : e;
         }

@@ -13,6 +13,27 @@ from helpers import N
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("nb,nk", [(1, 7), (3, 1001), (4, 65535), (4, 65536), (3, 466033 + 5), (5, 50001), (16, 4097), (17, 14513), (32, 1024),
+                                   (32, 4099)])
+def test_state_round_trip(nb, nk):
+    rng = np.random.default_rng(nb)
+    P = rng.normal(size=(nk, nb, nb)) + 1j * rng.normal(size=(nk, nb, nb))
+    P += P.swapaxes(1, 2).conj()
+    dp = C.POINTER(C.c_double)
+    unit, zero = np.broadcast_to(np.eye(nb) + 0j, (nk, nb, nb)).copy(), np.zeros((nk, nb, nb, 3), complex)
+    T, w = np.zeros((nb, nb)), np.zeros((1, 3))
+    p = N.Problem()
+    p.nk, p.nb, p.nch, p.ncc, p.n_nbr, p.stepper, p.order = nk, nb, 0, 1, 0, N.STEPPER_RK4, 4
+    nbr = np.zeros((nk, 1), np.int32)
+    p.nbr, p.nbr_wb = nbr.ctypes.data_as(C.POINTER(C.c_int32)), w.ctypes.data_as(dp)
+    p.H, p.D, p.U, p.T, p.rho0 = (a.ctypes.data_as(dp) for a in (unit, zero, unit, T, P))
+    p.dt, p.j_norm, p.tabs_norm, p.nktot = 0.01, 1.0, 1.0, float(nk)
+    eng = N.Engine(p)
+    assert np.array_equal(eng.get_state(), P)
+    eng.set_state(P[::-1])
+    assert np.array_equal(eng.get_state(), P[::-1])
+
+
 def _engine(P):
     nk, nb = P.shape[:2]
     dp = C.POINTER(C.c_double)
@@ -25,18 +46,6 @@ def _engine(P):
     p.H, p.D, p.U, p.T, p.rho0 = (a.ctypes.data_as(dp) for a in (unit, zero, unit, T, P))
     p.dt, p.j_norm, p.tabs_norm, p.nktot = 0.01, 1.0, 1.0, float(nk)
     return N.Engine(p)
-
-
-@pytest.mark.parametrize("nb,nk", [(1, 7), (3, 1001), (4, 65535), (4, 65536), (3, 466033 + 5), (5, 50001), (16, 4097), (17, 14513), (32, 1024),
-                                   (32, 4099)])
-def test_state_round_trip(nb, nk):
-    rng = np.random.default_rng(nb)
-    P = rng.normal(size=(nk, nb, nb)) + 1j * rng.normal(size=(nk, nb, nb))
-    P += P.swapaxes(1, 2).conj()
-    eng = _engine(P)
-    assert np.array_equal(eng.get_state(), P)
-    eng.set_state(P[::-1])
-    assert np.array_equal(eng.get_state(), P[::-1])
 
 
 def test_transfer_does_not_wait_for_another_context():
