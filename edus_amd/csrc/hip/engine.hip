@@ -1768,7 +1768,9 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     for (int h = 0; h < PER / 2; h++) {
         const int m = 2 * h;
         // A lane that repeats an element of another wave leaves its result to that
-        // one: with kLatePre it may have read the accumulator after the update.
+        // one: with kLatePre it may have read the accumulator after the update.  The
+        // two lanes that share element NP-2 of an odd count are of one wave
+        // (odd_tail_in_one_wave), whose reads all precede its stores.
         if (TPK > 64 && 2 * (lane + TPK * h) >= NP) break;
         const double k0 = pv[m] + g[m], k1 = pv[m + 1] + g[m + 1];
         const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
@@ -1793,6 +1795,15 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 // Waves per SIMD that the registers are to allow: some modes otherwise end a few
 // registers above the limit.
 constexpr int wave_occupancy(int nbt, bool pair) { return nbt == 8 ? 4 : nbt == 16 && !pair ? 3 : 1; }
+
+// Odd band counts of a tile whose k spans several waves: the last lane, (NP - 1) / 2 in
+// the order of pairs, takes elements (NP-2, NP-1), and the lane before it owns NP-2.
+constexpr bool odd_tail_in_one_wave(int lo, int hi) {
+    for (int nb = lo | 1; nb <= hi; nb += 2)
+        if ((nb * nb - 1) / 2 % 64 == 0) return false;
+    return true;
+}
+static_assert(WaveGeom<16>::TPK == 64 && odd_tail_in_one_wave(17, 32), "element NP-2 needs one owner");
 
 // One k per workgroup, or with PAIR (ConstArgs::pair, one k per workgroup only)
 // the stencil pair (2q, 2q + 1).
