@@ -200,6 +200,16 @@ __device__ __forceinline__ int xcd_block() {
 // large matrices would not fit.  A bijection of [0, nk); sw = 0 keeps k = L.
 constexpr long long kStripL2Bytes = 1 << 20;
 
+// 1..4 bands: above so many bytes of a stage (its neighbour table and kStageArrays states'
+// worth of state, accumulator, base state, output, H and one component of D) the Infinity
+// Cache (256 MB) no longer keeps them from one stage to the next, and the operators,
+// accumulator and histories are read as non-temporal streams.
+// RK4 step, plain and so: 4 bands 600 x 600 k (294 MB) 303 and 345 us, 3 bands 800 x 800
+// (307 MB) 293 and 324, 1 band 2000 x 2000 (384 MB) 329 and 289, 3 bands 1000 x 1000 (480
+// MB) 513 and 489.
+constexpr int kStageArrays = 6;
+constexpr double kStageCacheBytes = 340e6;
+
 __device__ __forceinline__ int strip_k(int L, int nk, int sw, int scol) {
     if (sw == 0) return L;
     const int nrow = nk / scol, nfull = scol / sw, per = nrow * sw, s = L / per;
@@ -349,11 +359,12 @@ __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0,
 // shorter streams side by side shorten both, and every term's registers leave room
 // for more of them.  RK4 stage, one lane doing all of a k's terms -> this form: 3 bands
 // 60 x 60 with dephasing 8.1 -> 4.8 us, 4 bands 251 x 307 34.2 -> 21.9; AB4 with the
-// mean field 300 x 300 23.4 -> 19.3.  Loads are plain: as non-temporal ones they took
-// the 4-band stage to 27.1 us (states of these grids stay in the Infinity Cache).
+// mean field 300 x 300 23.4 -> 19.3.  Loads are plain, but for U, while a stage's arrays
+// stay in the Infinity Cache: as non-temporal ones they took the 4-band stage to 27.1 us.
 // Six stencil rows in flight per wave instead of three took it to 25.9.
 //
-// DISS: the context has dephasing terms (c.diss).
+// DISS: the context has dephasing terms (c.diss).  NT: the arrays of a stage exceed the
+// caches (kStageCacheBytes).
 template <int NB, bool DISS>
 struct SmallGeom {
     static constexpr int NP = NB * NB;
@@ -369,9 +380,10 @@ constexpr int small_wpe() { return (NB <= 2 ? 5 : NB == 3 ? 4 : 3) - (DISS && NB
 
 // An element row of a SoA array at the lane's byte offset (SmallOff): the row address
 // is uniform, so a 32-bit offset needs no address arithmetic in vector registers.
-template <typename O>
+template <bool NT = false, typename O>
 __device__ __forceinline__ double ldrow(const double *row, O off) {
-    return *gm(reinterpret_cast<const double *>(reinterpret_cast<const char *>(row) + off));
+    const double *p = reinterpret_cast<const double *>(reinterpret_cast<const char *>(row) + off);
+    return NT ? ldnt(p) : *gm(p);
 }
 template <typename O>
 __device__ __forceinline__ void strow_nt(double *row, O off, double v) {
@@ -401,7 +413,7 @@ __device__ __forceinline__ void small_state(const double *Y, size_t nkp, SmallOf
 
 // -i[M, rho] in the transposed storage with M = H + E.D, the probe on core<->non-core
 // elements, and the RWA term (RungeKutta.h:158-212), packed.
-template <int NB>
+template <int NB, bool NT>
 __device__ __forceinline__ void small_commutator(const ConstArgs &c, const StageArgs &a, TabRow tab, SmallOff<NB> ko,
                                                  double (&pv)[NB * NB]) {
     constexpr int NP = NB * NB;
@@ -414,7 +426,7 @@ __device__ __forceinline__ void small_commutator(const ConstArgs &c, const Stage
 #pragma unroll
         for (int j = i; j < NB; j++) {
             const int p = i == j ? i : NB + 2 * pair_index(i, j, NB);
-            M[i][j] = mk(ldrow(c.H + p * nkp, ko), i == j ? 0.0 : ldrow(c.H + (p + 1) * nkp, ko));
+            M[i][j] = mk(ldrow<NT>(c.H + p * nkp, ko), i == j ? 0.0 : ldrow<NT>(c.H + (p + 1) * nkp, ko));
             if (i != j) M[j][i] = cconj(M[i][j]);
         }
 #pragma unroll
@@ -428,7 +440,7 @@ __device__ __forceinline__ void small_commutator(const ConstArgs &c, const Stage
                     const double E = w ? Eq[x] : Ep[x];
                     const int p = i == j ? i : NB + 2 * pair_index(i, j, NB);
                     const double *row = c.D + (size_t)(x * NP + p) * nkp;
-                    const cd d = mk(ldrow(row, ko), i == j ? 0.0 : ldrow(row + nkp, ko));
+                    const cd d = mk(ldrow<NT>(row, ko), i == j ? 0.0 : ldrow<NT>(row + nkp, ko));
                     M[i][j] = cadd(M[i][j], cscale(d, E));
                     if (i != j) M[j][i] = cadd(M[j][i], cscale(c.dherm ? cconj(d) : d, E));
                 }
@@ -565,15 +577,15 @@ struct SmallTail {
     double y, p0, p1, h[NH > 0 ? NH : 1];
 };
 
-template <int MODE, typename O>
+template <int MODE, bool NT, typename O>
 __device__ __forceinline__ void small_tail_load(const StageArgs &a, size_t row, size_t hstride, O ko, SmallTail<MODE> &t) {
     t.y = t.p0 = t.p1 = 0.0;
     if constexpr (MODE == RK1 || MODE == ABM || MODE == TAY) t.y = ldrow(a.Y + row, ko);
-    if constexpr (MODE == RK2 || MODE == RK3 || MODE == RK4S) t.p0 = ldrow(a.ACC + row, ko);
-    if constexpr (MODE == RK2 || MODE == RK3) t.p1 = ldrow(a.P0 + row, ko);
+    if constexpr (MODE == RK2 || MODE == RK3 || MODE == RK4S) t.p0 = ldrow<NT>(a.ACC + row, ko);
+    if constexpr (MODE == RK2 || MODE == RK3) t.p1 = ldrow<NT>(a.P0 + row, ko);
 #pragma unroll
     for (int s = 0; s < SmallTail<MODE>::NH; s++)
-        t.h[s] = s + 1 < a.order ? ldrow(a.HIST + (size_t)a.slots[s + 1] * hstride + row, ko) : 0.0;
+        t.h[s] = s + 1 < a.order ? ldrow<NT>(a.HIST + (size_t)a.slots[s + 1] * hstride + row, ko) : 0.0;
 }
 
 template <int MODE, typename O>
@@ -615,7 +627,7 @@ __device__ __forceinline__ void small_tail_store(const StageArgs &a, size_t row,
 
 // kk: the lane's k (past the grid: clamped, nothing stored); lk, tk: its place among
 // the workgroup's tk k; term: threadIdx.y, uniform in a wave; lds: [R][NP][tk].
-template <int NB, int MODE, bool DISS>
+template <int NB, int MODE, bool DISS, bool NT>
 __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs &a, TabRow tab, const int kk, const int lk, const int tk, const int term,
                                             double *lds) {
     using G = SmallGeom<NB, DISS>;
@@ -627,9 +639,9 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
     SmallTail<MODE> tail[EPR];
 #pragma unroll
     for (int m = 0; m < EPR; m++)
-        if (term + R * m < NP) small_tail_load<MODE>(a, (size_t)(term + R * m) * nkp, NP * nkp, ko, tail[m]);
+        if (term + R * m < NP) small_tail_load<MODE, NT>(a, (size_t)(term + R * m) * nkp, NP * nkp, ko, tail[m]);
     double pv[NP];
-    if (term == 0) small_commutator<NB>(c, a, tab, ko, pv);
+    if (term == 0) small_commutator<NB, NT>(c, a, tab, ko, pv);
     else if (DISS && term == 1) small_dephasing<NB>(c, a.Y, ko, pv);
     else if (nn > 0) {
         // this wave's part of the stencil; its indices come with the field row, not
@@ -667,11 +679,11 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
 }
 
 // blockDim = (k per workgroup, SmallGeom::R)
-template <int NB, int MODE, bool DISS>
+template <int NB, int MODE, bool DISS, bool NT>
 __global__ __launch_bounds__(kSmallMaxThreads, (small_wpe<NB, DISS>())) void k_stage_small(ConstArgs c, StageArgs a) {
     extern __shared__ __align__(16) double smem_d[];
     const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    stage_small<NB, MODE, DISS>(c, a, stage_row(a), xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
+    stage_small<NB, MODE, DISS, NT>(c, a, stage_row(a), xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
 }
 
 // ================================================================ Coulomb mean field
@@ -1862,7 +1874,7 @@ __global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) vo
     StageArgs a = be.a[rk4_stage_of<MODE>()];
     a.tab += tab_step;
     a.dmask = dmask[w.x];
-    stage_small<NB, MODE, DISS>(be.c, a, (TabRow)a.tab, w.y * kSmallBatchThreads + threadIdx.x, threadIdx.x, kSmallBatchThreads, term, smem_d);
+    stage_small<NB, MODE, DISS, false>(be.c, a, (TabRow)a.tab, w.y * kSmallBatchThreads + threadIdx.x, threadIdx.x, kSmallBatchThreads, term, smem_d);
 }
 
 template <int NBT, int MODE, typename R, bool PAIR = false>
@@ -3308,6 +3320,7 @@ struct edus_ctx {
     int nk = 0, nkp = 0, nb = 0, np = 0, nch = 0, ncc = 0, n_nbr = 0, stepper = 0, order = 1, diss = 0, dherm = 0, hole = 0;
     int sw = 0, scol = 0;  // strip order of the wave kernels (strip_k)
     int pair = 0, pself = -1, npnew = 0;  // stencil pairs of the wave kernels (ConstArgs::pair)
+    bool streamed = false; // nb <= 4: a stage's arrays exceed the caches (kStageCacheBytes)
     int tpb = 0;           // k per workgroup of the nb <= 4 kernel (0: small_group's choice)
     int precision = EDUS_PRECISION_FP64;
     float *Hf = nullptr, *Df = nullptr, *Uf = nullptr;  // FP32 operator copies (mixed precision)
@@ -3575,8 +3588,9 @@ int launch_stage(edus_ctx *c, StageArgs a) {
             constexpr bool DISS = decltype(dtag)::value;
             auto nbgo = [&](auto ntag) {
                 constexpr int NB = decltype(ntag)::value, R = SmallGeom<NB, DISS>::R;
-                hipLaunchKernelGGL((k_stage_small<NB, MODE, DISS>), dim3(blocks), dim3(tpb, R), (size_t)R * NB * NB * tpb * sizeof(double),
-                                   c->stream, ca, a);
+                const size_t lds = (size_t)R * NB * NB * tpb * sizeof(double);
+                if (c->streamed) hipLaunchKernelGGL((k_stage_small<NB, MODE, DISS, true>), dim3(blocks), dim3(tpb, R), lds, c->stream, ca, a);
+                else hipLaunchKernelGGL((k_stage_small<NB, MODE, DISS, false>), dim3(blocks), dim3(tpb, R), lds, c->stream, ca, a);
             };
             switch (c->nb) {
                 case 1: nbgo(std::integral_constant<int, 1>{}); break;
@@ -3802,6 +3816,7 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
     if (c->precision == EDUS_PRECISION_BF16X3 && nb <= 8)
         return fail(set_err(EDUS_ERR_UNSUPPORTED, "EDUS_PRECISION_BF16X3 runs on the matrix-core tiles of nb >= 9"));
     c->nkp = (int)padded;
+    c->streamed = c->soa && (double)c->nkp * (4. * p->n_nbr + 8. * c->np * kStageArrays) > kStageCacheBytes;
     // Wave kernels: walk the grid in strips (strip_k) when a strip's two previous
     // rows of packed state, the stencil's reach, fit in kStripL2Bytes while whole
     // rows would not (512 x 512 k at 32 bands: 64-column strips).
