@@ -375,8 +375,11 @@ struct SmallGeom {
 };
 constexpr int kSmallMaxThreads = 512;
 // waves per SIMD that the registers have to allow
-template <int NB, bool DISS>
-constexpr int small_wpe() { return (NB <= 2 ? 5 : NB == 3 ? 4 : 3) - (DISS && NB > 2 ? 1 : 0); }
+template <int NB, int MODE, bool DISS>
+constexpr int small_wpe() {
+    if (MODE == TAY && NB == 2) return 4;  // up to seven histories per element
+    return (NB <= 2 ? 5 : NB == 3 ? 4 : 3) - (DISS && NB > 2 ? 1 : 0);
+}
 
 // An element row of a SoA array at the lane's byte offset (SmallOff): the row address
 // is uniform, so a 32-bit offset needs no address arithmetic in vector registers.
@@ -637,9 +640,16 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
     const size_t nkp = c.nkp;
     const int nn = c.n_nbr;
     SmallTail<MODE> tail[EPR];
+    auto load_tail = [&] {
 #pragma unroll
-    for (int m = 0; m < EPR; m++)
-        if (term + R * m < NP) small_tail_load<MODE, NT>(a, (size_t)(term + R * m) * nkp, NP * nkp, ko, tail[m]);
+        for (int m = 0; m < EPR; m++)
+            if (term + R * m < NP) small_tail_load<MODE, NT>(a, (size_t)(term + R * m) * nkp, NP * nkp, ko, tail[m]);
+    };
+    // At 4 bands the Taylor step's histories do not fit beside the terms' registers:
+    // they are requested behind them (600 x 600 k, without dephasing: 187 us spilling,
+    // 110 so, 169 with one lane doing all of a k's terms).
+    constexpr bool kLateTail = MODE == TAY && NB == 4;
+    if constexpr (!kLateTail) load_tail();
     double pv[NP];
     if (term == 0) small_commutator<NB, NT>(c, a, tab, ko, pv);
     else if (DISS && term == 1) small_dephasing<NB>(c, a.Y, ko, pv);
@@ -663,6 +673,7 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
     }
 #pragma unroll
     for (int e = 0; e < NP; e++) lds[(term * NP + e) * tk + lk] = pv[e];
+    if constexpr (kLateTail) load_tail();
     __syncthreads();
     if (!store) return;
 #pragma unroll
@@ -680,7 +691,7 @@ __device__ __forceinline__ void stage_small(const ConstArgs &c, const StageArgs 
 
 // blockDim = (k per workgroup, SmallGeom::R)
 template <int NB, int MODE, bool DISS, bool NT>
-__global__ __launch_bounds__(kSmallMaxThreads, (small_wpe<NB, DISS>())) void k_stage_small(ConstArgs c, StageArgs a) {
+__global__ __launch_bounds__(kSmallMaxThreads, (small_wpe<NB, MODE, DISS>())) void k_stage_small(ConstArgs c, StageArgs a) {
     extern __shared__ __align__(16) double smem_d[];
     const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
     stage_small<NB, MODE, DISS, NT>(c, a, stage_row(a), xcd_block() * blockDim.x + threadIdx.x, threadIdx.x, blockDim.x, term, smem_d);
@@ -1866,7 +1877,7 @@ template <int MODE>
 __host__ __device__ constexpr int rk4_stage_of() { return MODE == RK1 ? 0 : MODE == RK2 ? 1 : MODE == RK3 ? 2 : 3; }
 
 template <int NB, int MODE, bool DISS>
-__global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, DISS>())) void k_stage_small_batch(const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
+__global__ __launch_bounds__(kSmallBatchThreads * 4, (small_wpe<NB, MODE, DISS>())) void k_stage_small_batch(const BatchEntry *E, const int2 *blk, const int *dmask, size_t tab_step) {
     extern __shared__ __align__(16) double smem_d[];
     const int term = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int2 w = blk[xcd_block()];
