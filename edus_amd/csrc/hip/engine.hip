@@ -4495,6 +4495,11 @@ int edus_autotune(edus_ctx *c, const double *field6, uint8_t grad_on, int32_t re
             for (int w : {16, 32, 64, 128, 256})
                 if (w < c->scol) cand.push_back(w);
     }
+    // 1..4 bands: the right-hand sides of 64 and 128 k per workgroup are even, and a
+    // choice by their noise can cost the step, whose kernel holds more (4 bands 1000 x
+    // 1000, AB4 step 290 and 372 us; 3 bands, Taylor 159 and 180): a larger one has to
+    // gain 3 %.
+    const float gain = c->soa ? 0.97f : 1.f;
     int &knob = c->soa ? c->tpb : c->sw;
     const int before = knob;
     int best = cand[0];
@@ -4509,7 +4514,7 @@ int edus_autotune(edus_ctx *c, const double *field6, uint8_t grad_on, int32_t re
         HIP_TRY(hipEventSynchronize(c->ev1));
         float ms = 0.f;
         HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-        if (i == 0 || ms < best_ms) { best_ms = ms; best = cand[i]; }
+        if (i == 0 || ms < gain * best_ms) { best_ms = ms; best = cand[i]; }
     }
     knob = best;
     if (best != before) drop_graph(c);  // a captured step holds the old launch shape

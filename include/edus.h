@@ -223,8 +223,9 @@ int edus_launch_schedule(edus_ctx *ctx, int32_t *out);
 /* Picks the stage kernels' launch schedule by measurement on the context's own
  * data and keeps it for every later launch: for 5..32 bands the strip width of
  * the workgroup walk over the grid (0 = k order, or 16..256 columns narrower than
- * a grid row), for 1..4 bands the k per workgroup (64, 128, 256).  Each
- * candidate runs `reps` right-hand-side launches with the field `field6` (as for
+ * a grid row), for 1..4 bands the k per workgroup (64 or 128, and 256 up to 2
+ * bands without dephasing; more than 64 where that gains 3 %).  Each candidate
+ * runs `reps` right-hand-side launches with the field `field6` (as for
  * edus_rhs) into scratch memory; the state and the step results are unaffected
  * (every candidate forms the same sums for every k).  `chosen` (may be NULL)
  * receives the strip width or the workgroup size kept.  No reference
