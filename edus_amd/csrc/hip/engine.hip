@@ -3249,11 +3249,14 @@ __global__ __launch_bounds__(kCgPeakThreads) void k_cgen_peak(const double *W0, 
 // touched ones, where pinned memory takes 56); here pieces go through a ring of pinned
 // memory, and each of a few threads copies its own piece on to the caller's pages
 // while the next pieces are under way (151 MB: 15 -> 4.5 ms).  The ring (12 MB) belongs
-// to the object, made by its first large copy.  From 16 MB on (16.8 MB: 1.24 -> 1.07 ms,
-// 33 MB 2.5 -> 1.6; 8 MB even).
+// to the object, made by its first copy of kRingFrom bytes (16.8 MB: 1.24 -> 1.07 ms, 33
+// MB 2.5 -> 1.6; 8 MB even).  An object of one call frees it again, which takes 1 to 2 ms
+// with the call's other buffers: for_call (a Wannier call with 28 MB of results 2.4 ms
+// without, 3.4 with; 44 MB even; 56 MB 6.3 and 3.2).
 class Downloader {
     static constexpr size_t kPiece = 2 << 20;
     static constexpr int kWorkers = 6;
+    const size_t from;
     char *ring = nullptr;
     hipEvent_t ev[kWorkers] = {};
     int dev = 0;
@@ -3270,7 +3273,10 @@ class Downloader {
     }
 
 public:
-    Downloader() = default;
+    static constexpr size_t kRingFrom = 16 << 20;
+    explicit Downloader(size_t ring_from = kRingFrom) : from(ring_from) {}
+    // the least copy that takes the ring, in a call with so many bytes of results
+    static size_t for_call(size_t total) { return total >= (48u << 20) ? kRingFrom : (size_t)-1; }
     Downloader(const Downloader &) = delete;
     Downloader &operator=(const Downloader &) = delete;
     ~Downloader() {
@@ -3280,9 +3286,9 @@ public:
     }
     // n bytes of device memory, in the stream's order; returns when dst holds them.
     hipError_t copy(void *dst, const void *src, size_t n, hipStream_t st) {
-        const bool ring_used = n >= 8 * kPiece && ready();
-        if (!ring_used) {
-            if (n >= 8 * kPiece) (void)hipGetLastError();  // the ring's: this copy does without it
+        const bool large = n >= from;
+        if (!large || !ready()) {
+            if (large) (void)hipGetLastError();  // the ring's: this copy does without it
             const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
             return e == hipSuccess ? hipStreamSynchronize(st) : e;
         }
@@ -5200,7 +5206,7 @@ static int wannier_hk(const int32_t nk3[3], int32_t nR, int32_t nw, const int32_
         for (void *q : {(void *)dOut, (void *)dR, (void *)dCol, (void *)dHR, (void *)drR, (void *)dVal, (void *)dTw, (void *)dPT, (void *)dH, (void *)dD})
             (void)hipFree(q);
     };
-    Downloader down;
+    Downloader down(Downloader::for_call((size_t)nk * nw2 * (D_out ? 64 : 16)));
     const size_t npt = (size_t)nR * (nk3[0] + nk3[1] + nk3[2]), nval = (size_t)nR * nw2;
     const size_t chunk = std::min<long long>(nk, std::max<long long>(64, (1LL << 28) / ((long long)nw2 * 64)));
     if (hipMalloc(&dR, (size_t)nR * 3 * sizeof(int)) != hipSuccess || hipMalloc(&dCol, (size_t)ncol * sizeof(int2)) != hipSuccess ||
