@@ -7,15 +7,15 @@
 //     k point is stored packed: nb real diagonal entries, then (re, im) of the
 //     strict upper triangle in row-major pair order -> nb*nb doubles.  This is
 //     lossless and halves the HBM traffic of the reference's full complex arrays.
-//   * nb <= 4: "SoA" -- element e of k at e*nkp + k (one thread per k, coalesced).
-//     nb >= 5: "AoS" -- k-major, nb*nb contiguous doubles (one wavefront per k).
+//   * nb <= 4: "SoA" -- element e of k at e*nkp + k (a lane per k and term, coalesced).
+//     nb >= 5: "AoS" -- k-major, nb*nb contiguous doubles (32, 64 or 256 threads per k).
 //   * H is packed like the state (upper triangle, as the RHS reads it);
 //     D components are packed by their upper triangle, the lower one being D_ij
 //     (symmetric tables) or conj(D_ij) (Hermitian tables); U is full complex.
 //
 // Kernels: fused RHS + stage update per RK4 stage / Adams-Bashforth step /
 // Taylor step (RungeKutta.h:7-355, RungeKutta.cpp, Linear_Multistep_ODE_solvers.cpp,
-// Taylor_DE_solver_deriv_Polynom.cpp), wave-per-k observable reductions with
+// Taylor_DE_solver_deriv_Polynom.cpp), observables in one launch with
 // error-compensated sums over the grid (Observables_MPI.h:217-775) and the Wannier phase
 // contraction (Wannier.h:278-471).
 #include <hip/hip_runtime.h>
@@ -236,56 +236,52 @@ __device__ __forceinline__ void stnt(double *p, double v) { __builtin_nontempora
 __device__ __forceinline__ void stnt(float *p, float v) { __builtin_nontemporal_store(v, gm(p)); }
 
 // Two adjacent packed elements in one access (16 bytes in FP64, 8 in FP32, at any
-// element's alignment), when `vec` (they are neighbours); else two single accesses
-// at o0 and o1.  Halves the vector memory instructions of the
-// wave kernels, whose address unit is their busiest memory stage.
+// element's alignment).  Halves the vector memory instructions of the wave kernels,
+// whose address unit is their busiest memory stage.
 // The pointers are cast to the pair type in one go: a template that deduces it (gm)
 // would drop its alignment and promise 16 bytes.
 template <typename T> struct Pair;
 template <> struct Pair<double> { typedef double V __attribute__((ext_vector_type(2), aligned(8))); };
 template <> struct Pair<float> { typedef float V __attribute__((ext_vector_type(2), aligned(4))); };
 template <bool NT, typename T>
-__device__ __forceinline__ void ld2(const T *p, size_t o0, size_t o1, bool vec, T &a, T &b) {
+__device__ __forceinline__ void ld2(const T *p, size_t o, T &a, T &b) {
+    const auto *q = (const __attribute__((address_space(1))) typename Pair<T>::V *)(p + o);
+    const typename Pair<T>::V v = NT ? __builtin_nontemporal_load(q) : *q;
+    a = v.x;
+    b = v.y;
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void st2(T *p, size_t o, T a, T b) {
+    typename Pair<T>::V v;
+    v.x = a;
+    v.y = b;
+    auto *q = (__attribute__((address_space(1))) typename Pair<T>::V *)(p + o);
+    if (NT) __builtin_nontemporal_store(v, q);
+    else *q = v;
+}
+// The elements at o0 and o1, in one access where they are neighbours (`vec`).
+template <bool NT, typename T>
+__device__ __forceinline__ void ld2_or_two(const T *p, size_t o0, size_t o1, bool vec, T &a, T &b) {
     if (vec) {
-        const auto *q = (const __attribute__((address_space(1))) typename Pair<T>::V *)(p + o0);
-        const typename Pair<T>::V v = NT ? __builtin_nontemporal_load(q) : *q;
-        a = v.x;
-        b = v.y;
+        ld2<NT>(p, o0, a, b);
     } else {
         a = NT ? ldnt(p + o0) : *gm(p + o0);
         b = NT ? ldnt(p + o1) : *gm(p + o1);
     }
 }
-template <bool NT, typename T>
-__device__ __forceinline__ void st2(T *p, size_t o0, size_t o1, bool vec, T a, T b) {
-    if (vec) {
-        typename Pair<T>::V v;
-        v.x = a;
-        v.y = b;
-        auto *q = (__attribute__((address_space(1))) typename Pair<T>::V *)(p + o0);
-        if (NT) __builtin_nontemporal_store(v, q);
-        else *q = v;
-    } else if (NT) {
-        stnt(p + o0, a);
-        stnt(p + o1, b);
-    } else {
-        *gm(p + o0) = a;
-        *gm(p + o1) = b;
-    }
-}
 
 // ---------------------------------------------------------------- stage update (nb >= 5)
-// The Adams-Bashforth tail for two adjacent packed elements (o1 = o0 + 1 when vec),
+// The Adams-Bashforth tail for the packed elements o0 and o0 + 1,
 // history and state accessed as pairs; the order-1 history loads are issued
 // together before the sum, which keeps the order of the coefficients.  h: stride
 // between history slots.  S: storage type of the history (double, or float in the
 // mixed form with FP32 stage storage); the state and its update stay FP64.
 template <bool NT, typename S>
-__device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0, size_t o1, bool vec, size_t h, double kv0,
+__device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0, size_t h, double kv0,
                                                   double kv1, double y0, double y1) {
     S *const hist = reinterpret_cast<S *>(a.HIST);
     const size_t so = (size_t)a.slot_out * h;
-    st2<NT>(hist, so + o0, so + o1, vec, (S)kv0, (S)kv1);
+    st2<NT>(hist, so + o0, (S)kv0, (S)kv1);
     double h0[5], h1[5];
 #pragma unroll
     for (int s = 1; s < 5; s++) {
@@ -293,7 +289,7 @@ __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0,
         if (s < a.order) {
             const size_t sl = (size_t)a.slots[s] * h;
             S u0, u1;
-            ld2<NT>(hist, sl + o0, sl + o1, vec, u0, u1);
+            ld2<NT>(hist, sl + o0, u0, u1);
             h0[s] = (double)u0;
             h1[s] = (double)u1;
         }
@@ -305,18 +301,18 @@ __device__ __forceinline__ void stage_update2_abm(const StageArgs &a, size_t o0,
             d0 += a.coef[s] * h0[s];
             d1 += a.coef[s] * h1[s];
         }
-    st2<NT>(a.OUT, o0, o1, vec, y0 + a.dt * d0, y1 + a.dt * d1);
+    st2<NT>(a.OUT, o0, y0 + a.dt * d0, y1 + a.dt * d1);
 }
 
 // The Taylor tail for two adjacent packed elements: the history is read as
 // pairs, then each element's update is formed on its own (one set of
 // differences live at a time).
 template <bool NT, typename S>
-__device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0, size_t o1, bool vec, size_t h, double kv0,
+__device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0, size_t h, double kv0,
                                                   double kv1, double y0, double y1) {
     S *const hist = reinterpret_cast<S *>(a.HIST);
     const size_t so = (size_t)a.slot_out * h;
-    st2<NT>(hist, so + o0, so + o1, vec, (S)kv0, (S)kv1);
+    st2<NT>(hist, so + o0, (S)kv0, (S)kv1);
     const int n = a.order - 1;
     S u0[EDUS_MAX_ORDER - 1], u1[EDUS_MAX_ORDER - 1];
 #pragma unroll
@@ -324,7 +320,7 @@ __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0,
         u0[i] = u1[i] = (S)0;
         if (i < n) {
             const size_t sl = (size_t)a.slots[i + 1] * h;
-            ld2<NT>(hist, sl + o0, sl + o1, vec, u0[i], u1[i]);
+            ld2<NT>(hist, sl + o0, u0[i], u1[i]);
         }
     }
     double out[2];
@@ -342,7 +338,7 @@ __device__ __forceinline__ void stage_update2_tay(const StageArgs &a, size_t o0,
         }
         out[w] = (w ? y1 : y0) + delta;
     }
-    st2<NT>(a.OUT, o0, o1, vec, out[0], out[1]);
+    st2<NT>(a.OUT, o0, out[0], out[1]);
 }
 
 // ================================================================ nb <= 4: a lane per k and term
@@ -481,7 +477,7 @@ __device__ __forceinline__ void small_dephasing(const ConstArgs &c, const double
 #pragma unroll
         for (int j = 0; j < NB; j++) {  // one 16-byte load per complex entry (the k's U is 16-byte aligned)
             double re, im;
-            ld2<true>(u, (i * NB + j) * 2, (i * NB + j) * 2 + 1, true, re, im);
+            ld2<true>(u, (i * NB + j) * 2, re, im);
             U[i][j] = mk(re, im);
         }
     small_state<NB>(Y, c.nkp, ko, P);
@@ -748,15 +744,14 @@ __global__ __launch_bounds__(256) void k_coul_pdiag(const double *__restrict__ Y
 // k = (i1, i2) (Coulomb.h:273-350):
 //   S_y[i1][n][e] = sum_i2 y_n(i2) P_e(i1, i2)                     (y = cos, sin)
 //   F_xy[mm][e]   = w (1 + corr_mn) sum_i1 x_m(i1) S_y[i1][n][e]    (4 combinations)
-// then X_mn from A..D minus the equilibrium (Coulomb.h:413-470) and the column
-// sums of the reconstruction (Coulomb.h:510-541), the row sum being done per k
-// inside the RHS kernel.
+// then X_mn from A..D minus the equilibrium (Coulomb.h:413-470), the column sums of
+// the reconstruction and its row sum with the renormalised H (Coulomb.h:510-541).
 struct CoulArgs {
     const double *Y;
     int nk, nkp, nb, NP, N1, N2, ncut, nu;
     double w;
     const double *cxm, *sxm, *cyn, *syn;
-    double *S, *F;
+    double *S;
     double *X;                 // [4][ncut^2][nb][nb] complex
     const double *X0;
     const double *A, *B, *C, *D, *vh;  // complex
@@ -832,8 +827,8 @@ __global__ __launch_bounds__(256) void k_coul_s1_mfma(CoulArgs a) {
 
 // F_xy[mm][e] = w (1 + corr_mn) sum_i1 x_m(i1) S_y[i1][n][e]: one workgroup per
 // mm; thread t takes element e = t % NP and every (256/NP)-th term of the sum,
-// and the parts are added in a fixed tree per element (10.0 -> 8.6 us at 300 x 300).  The same workgroup then
-// forms X_mn from its F (coul_x_elem) and, for mm = 0, the Hartree shift: X_mn
+// and the parts are added in a fixed tree per element (10.0 -> 8.6 us at 300 x 300).
+// The same workgroup then forms X_mn from its F (coul_x_elem) and, for mm = 0, the Hartree shift: X_mn
 // needs no other mode's F, so no launch of its own.
 constexpr int kCoulMaxNP = 16;  // the mean field runs at nb <= 4
 
@@ -842,7 +837,7 @@ __device__ __forceinline__ void coul_x_elem(const CoulArgs &a, const double (*Fs
 __global__ __launch_bounds__(kCoulThreads) void k_coul_s2(CoulArgs a) {
     __shared__ double red[4][kCoulThreads];
     __shared__ double Fs[4][kCoulMaxNP];
-    const int nmm = a.ncut * a.ncut, mm = blockIdx.x, m = mm / a.ncut, n = mm % a.ncut, t = threadIdx.x;
+    const int mm = blockIdx.x, m = mm / a.ncut, n = mm % a.ncut, t = threadIdx.x;
     const int NP = a.NP, nparts = kCoulThreads / NP, e = t % NP, part = t / NP;
     double cc = 0, cs = 0, sc = 0, ss = 0;
     if (part < nparts) {
@@ -876,9 +871,7 @@ __global__ __launch_bounds__(kCoulThreads) void k_coul_s2(CoulArgs a) {
         const double corr = -4 * M_PI * M_PI * (m * m + n * n) / ((double)a.nk * 27);
         const double f = a.w * (1. + corr);
         const int qd = t / NP, el = t % NP;
-        const double v = red[qd][el] * f;
-        a.F[((size_t)qd * nmm + mm) * NP + el] = v;
-        Fs[qd][el] = v;
+        Fs[qd][el] = red[qd][el] * f;
     }
     __syncthreads();
     if (mm == 0 && t < a.nb) {  // Hartree shift from mode 0 (Coulomb.h:385-410)
@@ -1078,7 +1071,7 @@ __global__ __launch_bounds__(256) void k_coul_hdiag(CoulArgs a, CoulHArgs h, int
 #pragma unroll
         for (int j = 0; j < NB; j++) {
             double re, im;
-            ld2<false>(uk, (i * NB + j) * 2, (i * NB + j) * 2 + 1, true, re, im);
+            ld2<false>(uk, (i * NB + j) * 2, re, im);
             U[i][j] = mk(re, im);
         }
     const cd scr0 = mk(h.screen[0], h.screen[1]), scr1c = mk(h.screen[2], -h.screen[3]);
@@ -1418,19 +1411,19 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
     // -> 29.2, of 16 119 -> 112, of 32 bands, 128 x 128, 216 -> 203; AB4 step of 13
     // bands with dephasing, 61 x 85, 42.1 -> 38.7; Taylor step of 24 bands, 96 x 100,
     // FP32 operators 131 -> 110.
-    constexpr bool kPairs = PER % 2 == 0;
+    static_assert(PER % 2 == 0, "a lane owns pairs of packed elements");
     // A stencil pair's calls load the RK2/RK3 accumulator and state at t_n after
     // the products, not with the other inputs: the registers then hold kb's
     // stencil sum instead through the gather and the products.
-    constexpr bool kLatePre = ROLE != 0 && kPairs;
-    const bool cp = kPairs && NP % 2 == 0;  // each pair is (re, im) of one upper element or two diagonal ones
+    constexpr bool kLatePre = ROLE != 0;
+    const bool cp = NP % 2 == 0;  // each pair is (re, im) of one upper element or two diagonal ones
     int eo[PER], ei[PER], ej[PER], ec[PER];
     double y[PER], pv[PER], g[PER], pre0[PER], pre1[PER];
     R hv[PER], dv[PER][3];
     const size_t base = (size_t)k * NP;
 #pragma unroll
     for (int m = 0; m < PER; m++) {
-        const int e = kPairs ? min(2 * (lane + TPK * (m >> 1)), NP - 2) + (m & 1) : min(lane + TPK * m, NP - 1);
+        const int e = min(2 * (lane + TPK * (m >> 1)), NP - 2) + (m & 1);
         eo[m] = e;
         const int code = *gm(c.eidx + e);
         ei[m] = code & 255;
@@ -1449,17 +1442,12 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         for (int j = 0; j < NV; j++) kn[j] = (size_t)row[j] * NP;
 #pragma unroll
         for (int j = 0; j < NV; j++) {
-            if constexpr (kPairs) {
 #pragma unroll
-                for (int h = 0; h < PER / 2; h++) {
-                    YT v0, v1;
-                    ld2<false>(Yin, kn[j] + eo[2 * h], kn[j] + eo[2 * h + 1], true, v0, v1);
-                    v[j][2 * h] = (double)v0;
-                    v[j][2 * h + 1] = (double)v1;
-                }
-            } else {
-#pragma unroll
-                for (int m = 0; m < PER; m++) v[j][m] = (double)Yin[kn[j] + eo[m]];
+            for (int h = 0; h < PER / 2; h++) {
+                YT v0, v1;
+                ld2<false>(Yin, kn[j] + eo[2 * h], v0, v1);
+                v[j][2 * h] = (double)v0;
+                v[j][2 * h + 1] = (double)v1;
             }
         }
     };
@@ -1480,50 +1468,27 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
         for (int j = 0; j < GB; j++) row0[j] = *gm(c.nbr + (size_t)max(min(j, nn - 1), 0) * c.nkp + k);
     }
-    if constexpr (kPairs) {
 #pragma unroll
-        for (int h = 0; h < PER / 2; h++) {
-            const int m = 2 * h;
-            const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-            YT y0, y1;
-            ld2<false>(Yin, o0, o1, true, y0, y1);
-            y[m] = (double)y0;
-            y[m + 1] = (double)y1;
-            ld2<kNT>(Hop, o0, o1, true, hv[m], hv[m + 1]);
+    for (int h = 0; h < PER / 2; h++) {
+        const int m = 2 * h;
+        const size_t o0 = base + eo[m];
+        YT y0, y1;
+        ld2<false>(Yin, o0, y0, y1);
+        y[m] = (double)y0;
+        y[m + 1] = (double)y1;
+        ld2<kNT>(Hop, o0, hv[m], hv[m + 1]);
 #pragma unroll
-            for (int x = 0; x < 3; x++) {
-                if (a.dmask >> x & 1) ld2<kNT>(Dop + (size_t)x * c.nk * NP, o0, o1, true, dv[m][x], dv[m + 1][x]);
-                else dv[m][x] = dv[m + 1][x] = (R)0;
-            }
-            if constexpr ((MODE == RK2 || MODE == RK3) && !kLatePre) {
-                ld2<kNT>(a.ACC, o0, o1, true, pre0[m], pre0[m + 1]);
-                ld2<kNT>(a.P0, o0, o1, true, pre1[m], pre1[m + 1]);
-            } else if constexpr (MODE == RK4S) {
-                ld2<kNT>(a.ACC, o0, o1, true, pre0[m], pre0[m + 1]);
-            }
+        for (int x = 0; x < 3; x++) {
+            if (a.dmask >> x & 1) ld2<kNT>(Dop + (size_t)x * c.nk * NP, o0, dv[m][x], dv[m + 1][x]);
+            else dv[m][x] = dv[m + 1][x] = (R)0;
         }
-    } else {
-#pragma unroll
-        for (int m = 0; m < PER; m++) {
-            const int e = eo[m];
-            y[m] = (double)Yin[base + e];
-            hv[m] = ldnt(Hop + base + e);
-#pragma unroll
-            for (int x = 0; x < 3; x++) dv[m][x] = (a.dmask >> x & 1) ? ldnt(Dop + (size_t)x * c.nk * NP + base + e) : (R)0;
-            if constexpr (MODE == RK2 || MODE == RK3) {
-                pre0[m] = ldnt(a.ACC + base + e);
-                pre1[m] = ldnt(a.P0 + base + e);
-            } else if constexpr (MODE == RK4S) {
-                pre0[m] = ldnt(a.ACC + base + e);
-            }
+        if constexpr ((MODE == RK2 || MODE == RK3) && !kLatePre) {
+            ld2<kNT>(a.ACC, o0, pre0[m], pre0[m + 1]);
+            ld2<kNT>(a.P0, o0, pre1[m], pre1[m + 1]);
+        } else if constexpr (MODE == RK4S) {
+            ld2<kNT>(a.ACC, o0, pre0[m], pre0[m + 1]);
         }
     }
-    // Field drift E.grad_k rho on the shell stencil (RungeKutta.h:258-276).  The
-    // neighbours are fetched GB at a time: their index and data loads are all in
-    // flight together, and the sum keeps the stencil order.  First of a pair
-    // (ROLE 1): every neighbour of k that is also one of kb's adds to kb's sum gb
-    // as well, and kb's remaining neighbours are fetched after k's.  Second of a
-    // pair (ROLE 2): the sum is gb.
     // The dephasing's U and rates, requested before the drift and the products that
     // come first (loaded where they are used, each k waited for them: AB4 step of 13
     // bands on 61 x 85 k 50.4 us -> 41.9).
@@ -1535,7 +1500,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
             for (int m = 0; m < PER; m++) {
                 const int t = min(lane + TPK * m, nb * nb - 1);
-                ld2<true>(u, 2 * t, 2 * t + 1, true, ur[m], ui[m]);
+                ld2<true>(u, 2 * t, ur[m], ui[m]);
             }
             if constexpr (kMfma) {
 #pragma unroll
@@ -1547,6 +1512,12 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             }
         }
     }
+    // Field drift E.grad_k rho on the shell stencil (RungeKutta.h:258-276).  The
+    // neighbours are fetched GB at a time: their index and data loads are all in
+    // flight together, and the sum keeps the stencil order.  First of a pair
+    // (ROLE 1): every neighbour of k that is also one of kb's adds to kb's sum gb
+    // as well, and kb's remaining neighbours are fetched after k's.  Second of a
+    // pair (ROLE 2): the sum is gb.
     if constexpr (ROLE == 2) {
 #pragma unroll
         for (int m = 0; m < PER; m++) g[m] = gb[m];
@@ -1609,7 +1580,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         R *Ad = reinterpret_cast<R *>(A), *Bd = reinterpret_cast<R *>(B);
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            if (kPairs && (m & 1) == 0 && cp && eo[m] >= nb) {
+            if ((m & 1) == 0 && cp && eo[m] >= nb) {
                 const int i = ei[m], j = ej[m];
                 const bool w = (i >= c.nch && j < c.nch) || (i < c.nch && j >= c.nch);
                 const R E[3] = {w ? Eq[0] : Ep[0], w ? Eq[1] : Ep[1], w ? Eq[2] : Ep[2]};
@@ -1627,7 +1598,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
                 lds_put(B + j * LD + i, CT{dr, c.dherm ? -di : -hv[m + 1] + ddi});
                 continue;
             }
-            if (kPairs && (m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // written with m - 1
+            if ((m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // written with m - 1
             const int i = ei[m], j = ej[m], comp = ec[m];
             const bool w = (i >= c.nch && j < c.nch) || (i < c.nch && j >= c.nch);
             const R E[3] = {w ? Eq[0] : Ep[0], w ? Eq[1] : Ep[1], w ? Eq[2] : Ep[2]};  // selects, no pointer
@@ -1666,22 +1637,22 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
 #pragma unroll
         for (int h = 0; h < PER / 2; h++) {
             const int m = 2 * h;
-            const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-            ld2<kNT>(a.ACC, o0, o1, true, pre0[m], pre0[m + 1]);
-            ld2<kNT>(a.P0, o0, o1, true, pre1[m], pre1[m + 1]);
+            const size_t o0 = base + eo[m];
+            ld2<kNT>(a.ACC, o0, pre0[m], pre0[m + 1]);
+            ld2<kNT>(a.P0, o0, pre1[m], pre1[m + 1]);
         }
     }
     // pv = -i (X_ij - conj(X_ji)) plus the RWA term on core -> non-core pairs; on
     // the diagonal this is 2 Im X_ii.
 #pragma unroll
     for (int m = 0; m < PER; m++) {
-        if (kPairs && (m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // formed with m - 1
+        if ((m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // formed with m - 1
         const int i = ei[m], j = ej[m];
         const CT xij = lds_get(C + i * LD + j), xji = lds_get(C + j * LD + i), pij = lds_get(A + i * LD + j);
         const double bre = (double)xij.x - (double)xji.x, bim = (double)xij.y + (double)xji.y;
         const double wr = (i < c.nch && j >= c.nch) ? c.wx2 : 0.0;
         const double vr = bim + -wr * (double)pij.y, vi = -bre + wr * (double)pij.x;
-        if (kPairs && (m & 1) == 0 && cp && eo[m] >= nb) {
+        if ((m & 1) == 0 && cp && eo[m] >= nb) {
             pv[m] = vr;
             pv[m + 1] = vi;
         } else {
@@ -1701,7 +1672,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
             const R *u = Uop + (size_t)k * nb * nb * 2;
             for (int t = lane; t < nb * nb; t += TPK) {
                 R re, im;
-                ld2<true>(u, 2 * t, 2 * t + 1, true, re, im);
+                ld2<true>(u, 2 * t, re, im);
                 lds_put(C + (t / nb) * LD + (t % nb), CT{re, im});
             }
         }
@@ -1765,7 +1736,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         }
 #pragma unroll
         for (int m = 0; m < PER; m++) {
-            if (kPairs && (m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // formed with m - 1
+            if ((m & 1) == 1 && cp && eo[m - 1] >= nb) continue;  // formed with m - 1
             const int i = ei[m], j = ej[m];
             const CT w = A[i * LD + j];
             CT hole = CT{0, 0};
@@ -1776,7 +1747,7 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
                 hole.x += (uj.x * ui.x + uj.y * ui.y) * tv;
                 hole.y += (uj.x * ui.y - uj.y * ui.x) * tv;
             }
-            if (kPairs && (m & 1) == 0 && cp && eo[m] >= nb) {
+            if ((m & 1) == 0 && cp && eo[m] >= nb) {
                 pv[m] = pv[m] - (double)w.x + (double)hole.x;
                 pv[m + 1] = pv[m + 1] - (double)w.y + (double)hole.y;
             } else {
@@ -1785,7 +1756,6 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         }
     }
     if (!store) return;  // after the last barrier (a group past the grid serves no pair)
-    static_assert(kPairs, "a lane owns pairs of packed elements");
     S *const outs = reinterpret_cast<S *>(a.OUT);  // RK stages 1-3 write the next stage input
 #pragma unroll
     for (int h = 0; h < PER / 2; h++) {
@@ -1796,21 +1766,21 @@ __device__ __forceinline__ void stage_wave(const ConstArgs &c, const StageArgs &
         // (odd_tail_in_one_wave), whose reads all precede its stores.
         if (TPK > 64 && 2 * (lane + TPK * h) >= NP) break;
         const double k0 = pv[m] + g[m], k1 = pv[m + 1] + g[m + 1];
-        const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
+        const size_t o0 = base + eo[m];
         if constexpr (MODE == ABM) {
-            stage_update2_abm<kNT, S>(a, o0, o1, true, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+            stage_update2_abm<kNT, S>(a, o0, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
         } else if constexpr (MODE == TAY) {
-            stage_update2_tay<kNT, S>(a, o0, o1, true, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
+            stage_update2_tay<kNT, S>(a, o0, (size_t)c.nk * NP, k0, k1, y[m], y[m + 1]);
         } else if constexpr (MODE == RK1) {
-            st2<kNT>(a.ACC, o0, o1, true, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
-            st2<kNT>(outs, o0, o1, true, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
+            st2<kNT>(a.ACC, o0, y[m] + k0 * a.ca, y[m + 1] + k1 * a.ca);
+            st2<kNT>(outs, o0, (S)(y[m] + k0 * a.cb), (S)(y[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK2 || MODE == RK3) {
-            st2<kNT>(a.ACC, o0, o1, true, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
-            st2<kNT>(outs, o0, o1, true, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
+            st2<kNT>(a.ACC, o0, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2<kNT>(outs, o0, (S)(pre1[m] + k0 * a.cb), (S)(pre1[m + 1] + k1 * a.cb));
         } else if constexpr (MODE == RK4S) {
-            st2<kNT>(a.OUT, o0, o1, true, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
+            st2<kNT>(a.OUT, o0, pre0[m] + k0 * a.ca, pre0[m + 1] + k1 * a.ca);
         } else {
-            st2<kNT>(a.OUT, o0, o1, true, k0, k1);
+            st2<kNT>(a.OUT, o0, k0, k1);
         }
     }
 }
@@ -2208,7 +2178,7 @@ __global__ __launch_bounds__(kObsThreads) __attribute__((amdgpu_waves_per_eu(obs
 #pragma unroll
                 for (int b = 0; b < NB; b++) {
                     double re, im;
-                    ld2<false>(u, (a * NB + b) * 2, (a * NB + b) * 2 + 1, true, re, im);
+                    ld2<false>(u, (a * NB + b) * 2, re, im);
                     U[a][b] = mk(re, im);
                 }
         }
@@ -2378,13 +2348,13 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
         for (int q = 0; q < PER / 2; q++) {
             const int m = 2 * q;
             const size_t o0 = base + eo[m], o1 = base + eo[m + 1];
-            ld2<false>(o.P, o0, o1, v2[q], y[m], y[m + 1]);
-            ld2<true>(o.H, o0, o1, v2[q], h[m], h[m + 1]);
+            ld2_or_two<false>(o.P, o0, o1, v2[q], y[m], y[m + 1]);
+            ld2_or_two<true>(o.H, o0, o1, v2[q], h[m], h[m + 1]);
         }
 #pragma unroll
         for (int m = 0; m < PER; m++) {
             const size_t t = base + min(lane + TPK * m, NP - 1);
-            ld2<true>(o.U, 2 * t, 2 * t + 1, true, ur[m], ui[m]);
+            ld2<true>(o.U, 2 * t, ur[m], ui[m]);
         }
         if (o.GE) {  // J1: sum_ij P_ij gradH_ij (real: both Hermitian; a pair counts twice)
             const double *ge = o.GE + (size_t)k * 3 * NP;
@@ -2393,7 +2363,7 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
             for (int q = 0; q < PER / 2; q++)
 #pragma unroll
                 for (int x = 0; x < 3; x++)
-                    ld2<true>(ge + (size_t)x * NP, eo[2 * q], eo[2 * q + 1], v2[q], g[2 * q][x], g[2 * q + 1][x]);
+                    ld2_or_two<true>(ge + (size_t)x * NP, eo[2 * q], eo[2 * q + 1], v2[q], g[2 * q][x], g[2 * q + 1][x]);
 #pragma unroll
             for (int m = 0; m < PER; m++) {
                 if (!live || elem(m) >= NP) continue;
@@ -2431,7 +2401,7 @@ __global__ __launch_bounds__(kObsThreads, TA ? 2 : NBT == 8 ? 4 : 3) void k_obs_
         for (int q = 0; q < PER / 2; q++)
 #pragma unroll
             for (int x = 0; x < 3; x++)
-                ld2<true>(o.D + x * o.dxs, base + eo[2 * q], base + eo[2 * q + 1], v2[q], d[2 * q][x], d[2 * q + 1][x]);
+                ld2_or_two<true>(o.D + x * o.dxs, base + eo[2 * q], base + eo[2 * q + 1], v2[q], d[2 * q][x], d[2 * q + 1][x]);
         if constexpr (NBT >= 16) {
             int r0, c0;
             mfma_tile<NBT>(lane, r0, c0);
@@ -3368,7 +3338,7 @@ struct edus_ctx {
     int coul = 0, coul_diag = 0, N1 = 0, N2 = 0, ncut = 0, nu = 0;
     double *cPD = nullptr;  // diagonal basis: packed state in the eigenbasis
     double n_cond = 0.0;
-    double *cxm = nullptr, *sxm = nullptr, *cyn = nullptr, *syn = nullptr, *cS = nullptr, *cF = nullptr;
+    double *cxm = nullptr, *sxm = nullptr, *cyn = nullptr, *syn = nullptr, *cS = nullptr;
     double *cX = nullptr, *cX0 = nullptr, *cA = nullptr, *cB = nullptr, *cC = nullptr, *cD = nullptr, *cvh = nullptr;
     double *cEH = nullptr, *cEH0 = nullptr, *cT = nullptr, *cPW0 = nullptr, *cHr = nullptr, *cscreen = nullptr, *cXw = nullptr;
     double *dwb = nullptr, *cEk = nullptr;
@@ -3516,7 +3486,7 @@ CoulArgs coul_args(edus_ctx *c, const double *Y) {
     CoulArgs a;
     a.Y = Y; a.nk = c->nk; a.nkp = c->nkp; a.nb = c->nb; a.NP = c->np; a.N1 = c->N1; a.N2 = c->N2; a.ncut = c->ncut; a.nu = c->nu;
     a.w = 1.0 / (double)c->nk;
-    a.cxm = c->cxm; a.sxm = c->sxm; a.cyn = c->cyn; a.syn = c->syn; a.S = c->cS; a.F = c->cF; a.X = c->cX; a.X0 = c->cX0;
+    a.cxm = c->cxm; a.sxm = c->sxm; a.cyn = c->cyn; a.syn = c->syn; a.S = c->cS; a.X = c->cX; a.X0 = c->cX0;
     a.A = c->cA; a.B = c->cB; a.C = c->cC; a.D = c->cD; a.vh = c->cvh; a.EH = c->cEH; a.EH0 = c->cEH0; a.Tt = c->cT;
     a.Xw = c->cXw;
     return a;
@@ -3526,8 +3496,8 @@ CoulArgs coul_args(edus_ctx *c, const double *Y) {
 int launch_coulomb(edus_ctx *c, const double *Y) {
     CoulArgs a = coul_args(c, Y);
     const int t3 = c->N2 * c->ncut * c->nu;
-    // 64-thread workgroups: the passes have a few 10^4 outputs each, and small
-    // workgroups spread them over all CUs.  Pass 1 runs a wave per 16 x 16 tile.
+    // Pass 1: a workgroup of four waves per 16 x 16 tile; pass 3: 64-thread workgroups,
+    // which spread its few 10^4 outputs over all CUs.
     hipLaunchKernelGGL(k_coul_s1_mfma, dim3((c->np * c->N1 + 15) / 16, (2 * c->ncut + 15) / 16), dim3(256), 0, c->stream, a);
     hipLaunchKernelGGL(k_coul_s2, dim3(c->ncut * c->ncut), dim3(kCoulThreads), 0, c->stream, a);
     hipLaunchKernelGGL(k_coul_s3, dim3((t3 + 63) / 64), dim3(64), 0, c->stream, a);
@@ -3582,8 +3552,10 @@ ConstArgs const_args(const edus_ctx *c) {
 // Whether the stage kernels of a context serve stencil pairs (nb > 8; see
 // stencil_pairs): not in the BF16x3 form, whose split products leave no registers for
 // the second k's stencil sum, and not at 9..16 bands with dephasing, where the
-// dephasing's own operands are worth them more (AB4 step of 16 bands, 100 x 100 k: 81
-// us paired, 66 with one k per workgroup; RK4 stages of 60 x 60 k even).
+// dephasing's own operands are worth them more.  16 bands, paired and one k per
+// workgroup, per step: RK4 60 x 60 k 104 and 107 us, 200 x 200 844 and 743, 320 x 320
+// 2077 and 1894 (MIXED 586 and 556 at 200 x 200, MIXED32 542 and 510), AB4 238 and 221
+// at 200 x 200; 12 bands 802 and 739 (RK4), MIXED and MIXED32 even.
 bool runs_paired(const edus_ctx *c) {
     return c->pair && c->precision != EDUS_PRECISION_BF16X3 && !(c->diss && c->nb <= 16);
 }
@@ -4014,7 +3986,7 @@ int edus_create(const edus_problem *p, edus_ctx **out) {
             (rc = upc(&c->cC, q->C, (size_t)nmm * nb2 * 2)) || (rc = upc(&c->cD, q->D, (size_t)nmm * nb2 * 2)) ||
             (rc = upc(&c->cscreen, q->screen, (size_t)nb2 * 2)) || (rc = upc(&c->cvh, q->v_hartree, (size_t)nb2 * 2)))
             return fail(rc);
-        if ((rc = dalloc(c, &c->cS, (size_t)2 * c->N1 * c->ncut * c->np)) || (rc = dalloc(c, &c->cF, (size_t)4 * nmm * c->np)) ||
+        if ((rc = dalloc(c, &c->cS, (size_t)2 * c->N1 * c->ncut * c->np)) ||
             (rc = dalloc(c, &c->cX, (size_t)4 * nmm * nb2 * 2)) || (rc = dalloc(c, &c->cT, (size_t)2 * c->N2 * c->ncut * c->nu * 2)) ||
             (rc = dalloc(c, &c->cEH, nb)) || (rc = dalloc(c, &c->cPW0, se)) || (rc = dalloc(c, &c->cHr, se)) ||
             (rc = dalloc(c, &c->cEk, (size_t)p->nk * nb)) ||
