@@ -2127,7 +2127,7 @@ __device__ __forceinline__ void jacobi_small(cd (&A)[NB][NB], cd (&V)[NB][NB], d
 // shell gradient contracted with P neighbour by neighbour; the eigenvalues are
 // kept for edus_renorm_energies.  Bound by the latency of its loads and of the
 // final sums: 60 x 60 k of 3 bands 23 us (two kernels of a wave per k) -> 13;
-// with the mean field, 300 x 300, 345 us (tables written, then read) -> 46.
+// with the mean field, 300 x 300, 345 us (tables written, then read) -> 43.
 // Waves per SIMD: at 3 and 4 bands the compiler would give up loads in flight for one
 // more (4 bands 1000 x 1000 k, whole call: 373 us, 318 with two; 3 bands 300 x 300 44.8,
 // 42.5 with three).
@@ -2283,11 +2283,12 @@ __global__ __launch_bounds__(kObsThreads) __attribute__((amdgpu_waves_per_eu(obs
 // the k in LDS, T = P U^T and W = conj(P) H on the stage kernels' product tiles.
 // All operands of a k are requested together; a lane multiplies its packed
 // elements of D and of the gradient by what it finds in LDS.  Memory-bound at 32
-// bands (80 KB per k): 128 x 128 k take 446 us (2.9 TB/s), where the form that
-// took the population with nb LDS reads per term and read a table of H D^+ took
-// 1168; 16 bands 200 x 200 534 -> 233 us, 8 bands 99 -> 74.  Registers decide how
-// many blocks a CU holds: without TAbs (no core bands) its six compensated sums
-// are compiled out.
+// bands (80 KB per k): 128 x 128 k take 297 us (4.5 TB/s), where the form that took
+// the population with nb LDS reads per term and read a table of H D^+ took 1168; 16
+// bands 200 x 200 534 -> 167 us, 8 bands 99 -> 60.  With the matrices 8 bytes off the
+// boundary of their 16-byte LDS accesses a whole call takes 461 us at 32 bands, not 313,
+// and 212 at 16, not 178.  Registers decide how many
+// blocks a CU holds: without TAbs (no core bands) its six sums are compiled out.
 constexpr int kObsWaveV = 9;  // sums per round of obs_block_sums, in the matrices' LDS
 template <int NBT>
 __host__ __device__ constexpr int obs_mat_doubles() {
@@ -2944,7 +2945,7 @@ __global__ void k_wannier_finish(const cd *__restrict__ Out, int kc, int nw, dou
 //   * A list of G closed under G -> -G gives W(-q) = conj W(q): the second half of a
 //     symmetric set of q is the first one reversed and conjugated.
 //   * Few q: the G list is split over blockIdx.y and the parts added afterwards.
-// 999^2 q, 2849 G, 3 bands: 12.0 ms -> 1.9 ms.
+// 999^2 q, 2849 G, 3 bands, with the correction around q = 0: 13.2 ms -> 2.0 ms.
 constexpr int kCgTile = 128;
 constexpr int kCgMaxPair = 6;  // nb <= 4
 constexpr int kCgQ = 2;        // q per thread

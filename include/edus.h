@@ -121,7 +121,9 @@ typedef struct edus_problem {
 
 /* Creates a context on the current HIP device and uploads the problem.
  * Replaces: allocate_arr.cpp, the per-thread copies main_MPI.cpp:143-227,
- * CalculateIndicesMPI/Organize_kspace (one device holds the whole grid). */
+ * CalculateIndicesMPI/Organize_kspace (one device holds the whole grid).
+ * nk nb^2 (nk rounded up to 256 at 1..4 bands) has to stay below 2^31:
+ * EDUS_ERR_UNSUPPORTED otherwise. */
 int edus_create(const edus_problem *p, edus_ctx **out);
 
 /* Frees every device buffer of the context. */
